@@ -1,0 +1,21 @@
+// FPUOp and TropicalFPUOp: which kernel runs a launch, and the instances of the max-plus product.
+//
+// Floating-point FPUOp runs on the FP32 / FP64 matrix instructions (fpu_mfma.hpp: the same bits at two to six times the
+// speed); the vector-ALU kernel (fpu_gemm.hpp) keeps what has no matrix instruction -- the max-plus product, the
+// integers -- and the lane grids other than 8 x 8, which are a way of dealing outputs out to lanes of the vector ALUs.
+#include "fpu_instances.inc"
+
+int family_fpu(const InstanceKey& key, const GemmArgs& args, dim3 grid, hipStream_t stream, int mode, InstanceInfo* info,
+               hipError_t* err) {
+  if ((key.variant >> 4) != 0) return family_fpu_lanes(key, args, grid, stream, mode, info, err);
+  if ((key.variant & 1) == 0) {
+    for (FamilyFn fn : {family_fpu_mfma_f32_large, family_fpu_mfma_f32_small, family_fpu_mfma_f64, family_fpu_mfma_mixed, family_fpu_integers})
+      if (fn(key, args, grid, stream, mode, info, err)) return 1;
+    return 0;
+  }
+  GK_FPU_T(64, 64, 32, 2, 2, float, 0, 1, "64x64x32_w2x2_f32_tropical")
+  GK_FPU_T(64, 64, 32, 2, 2, float, 1, 1, "64x64x32_w2x2_f32_tropical_checked")
+  return 0;
+}
+
+}  // namespace gk

@@ -2,6 +2,9 @@
 // reference (src/operator.jl:35-153) together with the kernels that drive them
 // (src/kernel.jl:10-129, 147-350).
 //
+// Runs the max-plus product, the integers and the lane grids other than 8 x 8; floating-point FPUOp on the square grid
+// runs on the matrix instructions (fpu_mfma.hpp), which give the same bits.
+//
 // Every output element is one accumulator updated by a scalar fused multiply-add per k, in
 // ascending k, exactly like FPUOp.mma (src/operator.jl:139-153), so results are bit-identical to
 // a sequential fma loop on the host.  The accumulator type TACC is the element type of C and D and
@@ -108,13 +111,11 @@ __device__ __forceinline__ TACC fpu_fma(TACC a, TACC b, TACC c) {
 }
 
 template <int BM_, int BN_, int BK_, int WAVES_M_, int WAVES_N_, typename TIN_, bool A_KMAJOR_, bool B_KMAJOR_, bool CHECKED_,
-          bool TROPICAL_, typename TACC_ = float, bool FUSED_ = true, int LANES_M_ = 8>
+          bool TROPICAL_, typename TACC_ = float, int LANES_M_ = 8>
 struct FpuGemmConfig {
   // the lane grid of a wave: lane l stands at row l % LANES_M, column l / LANES_M of it (reference src/operator.jl:61)
   static constexpr int LANES_M = LANES_M_, LANES_N = kWaveSize / LANES_M_;
   static_assert(LANES_M_ > 0 && kWaveSize % LANES_M_ == 0, "the lane grid is LANES_M x (64 / LANES_M)");
-  // FUSED: the kernel carries the eight transform hooks and the bias; without, none of that code exists
-  static constexpr bool FUSED = FUSED_;
   static constexpr int BM = BM_, BN = BN_, BK = BK_, WAVES_M = WAVES_M_, WAVES_N = WAVES_N_;
   static constexpr bool A_KMAJOR = A_KMAJOR_, B_KMAJOR = B_KMAJOR_, CHECKED = CHECKED_, TROPICAL = TROPICAL_;
   typedef TIN_ TIN;
@@ -130,12 +131,10 @@ struct FpuGemmConfig {
   static constexpr int LDS_BYTES = (BK * LDA_S + BK * LDB_S) * (int)sizeof(TACC);
   static constexpr int A_CHUNKS = BM * BK / 4, B_CHUNKS = BN * BK / 4;
   static constexpr int A_PER_THREAD = A_CHUNKS / THREADS, B_PER_THREAD = B_CHUNKS / THREADS;
-  // K tiles whose global loads are in flight (in registers) while the current one is multiplied: the fma chain
-  // of a tile is shorter than the memory latency, so one tile ahead left every tile waiting for its loads
-  // (256^3 on 16 workgroups: 19.4 us with one tile in flight)
-  // -- four tiles without hooks, two with; the bounds-checked and the 64-bit kernels stay with one (their
-  // per-element loads and wide registers make deeper buffers expensive to compile and to hold)
-  static constexpr int DEPTH = (CHECKED_ || sizeof(TIN_) > 4) ? 1 : (FUSED_ ? 2 : 4);
+  // K tiles whose global loads are in flight (in registers) while the current one is multiplied: the fma chain of a tile
+  // is shorter than the memory latency.  The bounds-checked and the 64-bit kernels stay with one (their per-element
+  // loads and wide registers make deeper buffers expensive to compile and to hold)
+  static constexpr int DEPTH = (CHECKED_ || sizeof(TIN_) > 4) ? 1 : 2;
   static_assert(WTM % LANES_M == 0 && WTN % LANES_N == 0 && TM >= 1 && TN >= 1 && TM % CWM == 0 && TN % CWN == 0,
                 "the lane grid divides the wave tile and a lane owns whole chunks");
   static_assert(LANES_M_ != 8 || (TM >= 2 && TN >= 2), "8 x 8 lanes: a lane owns whole chunks of 2 or 4 outputs");
@@ -214,8 +213,8 @@ __global__ void __launch_bounds__(Cfg::THREADS) fpu_gemm_kernel(const GemmArgs a
   const TIN* B = (const TIN*)args.b;
   const TACC* C = (const TACC*)args.c;
   const bool zero_ab = (args.a_kind == 0 /* Layout.Zero */);
-  const bool xf_a = Cfg::FUSED && (args.t[H_GL2SH_A].n > 0 || args.t[H_SH2RF_A].n > 0);
-  const bool xf_b = Cfg::FUSED && (args.t[H_GL2SH_B].n > 0 || args.t[H_SH2RF_B].n > 0);
+  const bool xf_a = (args.t[H_GL2SH_A].n > 0 || args.t[H_SH2RF_A].n > 0);
+  const bool xf_b = (args.t[H_GL2SH_B].n > 0 || args.t[H_SH2RF_B].n > 0);
 
   // accumulators: acc[i][j] is row wm*WTM + (i/CW)*LANES_M*CW + CW*ly + i%CW (CW = 4, or fewer), columns likewise with lx
   constexpr int CWM = Cfg::CWM, CWN = Cfg::CWN;
@@ -244,11 +243,9 @@ __global__ void __launch_bounds__(Cfg::THREADS) fpu_gemm_kernel(const GemmArgs a
 #pragma unroll
     for (int q = 0; q < TM * TN; ++q) acc[q % TM][q / TM] = flat[q];
   };
-  if constexpr (Cfg::FUSED) {
-    if (args.c_mode != 0) {
-      hook_acc(args.t[H_GL2SH_C]);
-      hook_acc(args.t[H_SH2RF_C]);
-    }
+  if (args.c_mode != 0) {
+    hook_acc(args.t[H_GL2SH_C]);
+    hook_acc(args.t[H_SH2RF_C]);
   }
 
   constexpr int DEPTH = Cfg::DEPTH;
@@ -273,20 +270,18 @@ __global__ void __launch_bounds__(Cfg::THREADS) fpu_gemm_kernel(const GemmArgs a
     TIN x[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) x[e] = v[e];
-    if constexpr (Cfg::FUSED) {
-      if (xf) {
-        TAR y[4];
+    if (xf) {
+      TAR y[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) y[e] = (TAR)x[e];
-        if (t0.n > 0) {
-          apply_list_regs_t<TAR, 4>(t0, y);
+      for (int e = 0; e < 4; ++e) y[e] = (TAR)x[e];
+      if (t0.n > 0) {
+        apply_list_regs_t<TAR, 4>(t0, y);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) y[e] = (TAR)(TIN)y[e];       // rounded to the operand's type between the hooks
-        }
-        if (t1.n > 0) apply_list_regs_t<TAR, 4>(t1, y);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) x[e] = (TIN)y[e];
+        for (int e = 0; e < 4; ++e) y[e] = (TAR)(TIN)y[e];       // rounded to the operand's type between the hooks
       }
+      if (t1.n > 0) apply_list_regs_t<TAR, 4>(t1, y);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = (TIN)y[e];
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -372,29 +367,27 @@ __global__ void __launch_bounds__(Cfg::THREADS) fpu_gemm_kernel(const GemmArgs a
   // epilogue: transform, bias, transform, store (a chunk of consecutive rows per vector store); the bias of
   // Epilogue.Bias is fp32 (reference src/epilogue.jl:44-52) and only offered with fp32 accumulators
   TACC* D = (TACC*)args.d;
-  if constexpr (Cfg::FUSED) {
-    hook_acc(args.t[H_RF2SH_D]);
-    if constexpr (std::is_same<TACC, float>::value) {
-      if (args.epi_kind == 1) {
+  hook_acc(args.t[H_RF2SH_D]);
+  if constexpr (std::is_same<TACC, float>::value) {
+    if (args.epi_kind == 1) {
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const int cc = col_of(j);
-          const float bv = args.bias[Cfg::CHECKED ? (cc < args.N ? cc : 0) : cc];
+      for (int j = 0; j < TN; ++j) {
+        const int cc = col_of(j);
+        const float bv = args.bias[Cfg::CHECKED ? (cc < args.N ? cc : 0) : cc];
 #pragma unroll
-          for (int i = 0; i < TM; ++i) acc[i][j] = acc[i][j] + bv;
-        }
-      } else if (args.epi_kind == 2) {
+        for (int i = 0; i < TM; ++i) acc[i][j] = acc[i][j] + bv;
+      }
+    } else if (args.epi_kind == 2) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          const int r = row_of(i);
-          const float bv = args.bias[Cfg::CHECKED ? (r < args.M ? r : 0) : r];
+      for (int i = 0; i < TM; ++i) {
+        const int r = row_of(i);
+        const float bv = args.bias[Cfg::CHECKED ? (r < args.M ? r : 0) : r];
 #pragma unroll
-          for (int j = 0; j < TN; ++j) acc[i][j] = acc[i][j] + bv;
-        }
+        for (int j = 0; j < TN; ++j) acc[i][j] = acc[i][j] + bv;
       }
     }
-    hook_acc(args.t[H_SH2GL_D]);
   }
+  hook_acc(args.t[H_SH2GL_D]);
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
     const int cc = col_of(j);

@@ -1,12 +1,11 @@
-// Instances of the vector-ALU GEMM for the element types of FPUOp beyond fp32 accumulation
-// (reference configs/configs.jl:489-497): Float32 -> Float64, Float64, Int16, Int32, Int64.
+// Instances of the vector-ALU GEMM for the integer types of FPUOp (reference configs/configs.jl:489-497).
 #include "fpu_gemm.hpp"
 #include "registry.hpp"
 
 namespace gk {
 
-int family_fpu_types(const InstanceKey& key, const GemmArgs& args, dim3 grid, hipStream_t stream, int mode, InstanceInfo* info,
-                     hipError_t* err) {
+int family_fpu_integers(const InstanceKey& key, const GemmArgs& args, dim3 grid, hipStream_t stream, int mode, InstanceInfo* info,
+                        hipError_t* err) {
   // key.variant: bit 0 tropical (fp32 only, not here), bit 1 bounds-checked
 #define GK_FPU(TIN, TACC, akm_, bkm_, chk_, NAME)                                                                          \
   if (key.BM == 64 && key.BN == 64 && key.BK == 32 && key.waves_m == 2 && key.waves_n == 2 &&                             \
@@ -24,8 +23,6 @@ int family_fpu_types(const InstanceKey& key, const GemmArgs& args, dim3 grid, hi
   GK_FPU(TIN, TACC, 0, 0, 1, "fpu_gemm_nt_64x64x32_w2x2_" TAG "_checked")    \
   GK_FPU(TIN, TACC, 1, 1, 1, "fpu_gemm_tn_64x64x32_w2x2_" TAG "_checked")    \
   GK_FPU(TIN, TACC, 1, 0, 1, "fpu_gemm_tt_64x64x32_w2x2_" TAG "_checked")
-  GK_FPU_T(float, double, "f32_f64")
-  GK_FPU_T(double, double, "f64")
   GK_FPU_T(short, short, "i16")
   GK_FPU_T(int, int, "i32")
   GK_FPU_T(long long, long long, "i64")

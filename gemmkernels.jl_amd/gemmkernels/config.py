@@ -174,13 +174,16 @@ def default_block_shape(operator, gemm_shape, tile_sized: bool = True, gett: boo
     ``b_kmajor``: B is stored K x N ('N'); they admit the tiles with a side of 192."""
     M, N, K = gemm_shape["M"], gemm_shape["N"], gemm_shape["K"]
     if operator.kind in (Operator.FPU, Operator.FPU_TROPICAL):
-        # a small Float32 product in whole 32 x 32 x 32 tiles: four times the workgroups of the 64 x 64 tile
-        # (256^3: 64 workgroups instead of 16) with 2 x 2 outputs per lane on four waves, so that a lane works
-        # through 4 fma chains instead of 16 (every output is still one fma chain in k: the same bits)
-        if (operator.kind == Operator.FPU and operator.CT.name == "Float32" and operator.AT.name == "Float32" and tile_sized
-                and M % 32 == 0 and N % 32 == 0 and K % 32 == 0 and -(-M // 64) * -(-N // 64) < NUM_CUS // 2):
-            return NT(M=32, N=32, K=32)
-        return NT(M=64, N=64, K=32)
+        costs = _FPU_TILE_COST.get((operator.CT.name, operator.AT.name), {}) if operator.kind == Operator.FPU else {}
+        fitting = [t for t in costs if not tile_sized or (M % t[0] == 0 and N % t[1] == 0 and K % t[2] == 0)]
+        if not fitting:
+            return NT(M=64, N=64, K=32)
+
+        def fpu_cost(t):
+            rounds = -(-(-(-M // t[0]) * -(-N // t[1])) // NUM_CUS)
+            return costs[t][0] if rounds == 1 else costs[t][1] * rounds
+        best = min(fitting, key=fpu_cost)
+        return NT(M=best[0], N=best[1], K=best[2])
     if operator.kind in (Operator.MFMA_COMPLEX, Operator.MFMA_DUAL):
         # complex tiles, in complex elements
         table = _complex_tiles(operator, planar, a_kmajor, b_kmajor)
@@ -243,6 +246,14 @@ def _rounds(t, tiles):
     return 1.0 + 0.36 * (per_cu - 1.0)
 
 
+# FPUOp on the FP32 / FP64 matrix instructions: time of a tile per 1000 k, in microseconds, when every CU has one tile at most
+# and per tile when a CU has several (they are bound by the matrix cores, so the tiles of a CU add up, and a launch
+# takes as long as the CU with the most).  Measured, e.g. Float32: 2048^3 134 us on 128 x 128 (256 tiles), 142 on 64 x 64 (1024);
+# 2560^3 324 against 302 (400 and 1600 tiles: 2 and 7 rounds); 1024^3 68, 24.5 and 26 us on 128 x 128, 64 x 64 (256 tiles) and
+# 32 x 32 (1024); 768^3 53, 19 and 17 (576 tiles of 32 x 32).  Float64: 1000^3 41.3 us on 64 x 64, 41.1 on 32 x 32; 2048^3 270, 305.
+_FPU_TILE_COST = {("Float32", "Float32"): {(128, 128, 32): (65.0, 63.0), (64, 64, 32): (21.0, 17.8), (32, 32, 32): (9.0, 6.1)},
+                  ("Float64", "Float64"): {(64, 64, 32): (38.0, 33.0), (32, 32, 32): (14.0, 9.8)}}
+
 # complex / dual tiles (complex elements) -> waves: one real product of the real views of A and B, whose real tile
 # has twice the rows and columns; the same table for every transpose
 _COMPLEX_PAIR_TILES = [((128, 128, 64), (2, 4)), ((64, 64, 64), (2, 2)), ((64, 64, 32), (2, 2)), ((32, 32, 32), (2, 2))]
@@ -251,8 +262,8 @@ _COMPLEX_PAIR_TILES = [((128, 128, 64), (2, 4)), ((64, 64, 64), (2, 2)), ((64, 6
 # the rows and columns (both planes of A, B and D)
 _PLANAR_TILES = [((128, 128, 64), (2, 4)), ((64, 64, 64), (2, 2)), ((64, 64, 32), (2, 2)), ((32, 32, 32), (2, 2))]
 
-# tiles of the vector-ALU kernel and of the bounds-checked MFMA kernel
-_FPU_TILES = [((64, 64, 32), (2, 2)), ((128, 128, 16), (2, 2)), ((32, 32, 32), (2, 2)), ((32, 32, 32), (1, 1))]
+# tiles of FPUOp and of the bounds-checked MFMA kernel
+_FPU_TILES = [((64, 64, 32), (2, 2)), ((128, 128, 16), (2, 2)), ((128, 128, 32), (2, 2)), ((32, 32, 32), (2, 2)), ((32, 32, 32), (1, 1))]
 _CHECKED_TILES = [((64, 64, 32), (2, 2))]
 
 

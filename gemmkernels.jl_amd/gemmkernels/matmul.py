@@ -403,14 +403,15 @@ def create_config(A: DType, sizeA, stridesA, transA: bool, B: DType, sizeB, stri
     # The library runs a 16-bit product on bounds-checked layouts on the aligned kernels all the same (any address
     # and leading dimension; tiles over the edge clamp their loads and mask their stores; the last K tile is
     # repaired in LDS when a 16-byte chunk reaches over the end of an operand) as long as A and B hold one whole
-    # chunk of 8 elements along their contiguous index.  Then the tile is chosen among all tiles, not only those
+    # chunk of 8 elements along their contiguous index; floating-point FPUOp takes any size and alignment on every tile.  Then the tile is chosen among all tiles, not only those
     # that divide the sizes (4096 x 4096 x 4000: the 64-deep tile with a partial last step instead of the 32-deep
     # one), and the operands it does not divide get the bounds-checked layouts, as the reference's rule says.
-    edge_ok = use_mfma and not zeroAlpha and (k if transA else m) >= 8 and (n if transB else k) >= 8
+    edge_ok = not zeroAlpha and (((k if transA else m) >= 8 and (n if transB else k) >= 8) if use_mfma
+                                 else compute_type in (Float16, Float32, Float64))
     block_shape = default_block_shape(operator, NT(M=m, N=n, K=k), tile_sized=not edge_ok, a_kmajor=transA, b_kmajor=not transB)
     global_a_layout, global_b_layout, global_c_layout, global_d_layout = layouts_for(block_shape)
     if not edge_ok and any(l.kind in (Layout.COL_MAJOR, Layout.ROW_MAJOR) for l in (global_a_layout, global_b_layout, global_c_layout, global_d_layout)):
-        # some operand needs bounds checks: the bounds-checked kernels have one tile shape
+        # some operand needs bounds checks (and C = beta C, the zero alpha): one tile shape
         block_shape = NT(M=64, N=64, K=32)
         global_a_layout, global_b_layout, global_c_layout, global_d_layout = layouts_for(block_shape)
 

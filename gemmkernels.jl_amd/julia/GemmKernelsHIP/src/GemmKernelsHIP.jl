@@ -356,7 +356,10 @@ end
 # the same table for every transpose
 const COMPLEX_PAIR_TILES = [((128, 128, 64), (2, 4)), ((64, 64, 64), (2, 2)), ((64, 64, 32), (2, 2)), ((32, 32, 32), (2, 2))]
 complex_tiles(operator::Type, a_kmajor::Bool, b_kmajor::Bool; planar::Bool = false) = COMPLEX_PAIR_TILES
-const FPU_TILES = [((64, 64, 32), (2, 2)), ((128, 128, 16), (2, 2)), ((32, 32, 32), (2, 2)), ((32, 32, 32), (1, 1))]
+const FPU_TILES = [((64, 64, 32), (2, 2)), ((128, 128, 16), (2, 2)), ((128, 128, 32), (2, 2)), ((32, 32, 32), (2, 2)), ((32, 32, 32), (1, 1))]
+# FPUOp on the FP32 / FP64 matrix instructions: microseconds per 1000 k of a tile that has a CU to itself, and of each of several
+const FPU_TILE_COST = Dict((:Float32, :Float32) => [((128, 128, 32), (65.0, 63.0)), ((64, 64, 32), (21.0, 17.8)), ((32, 32, 32), (9.0, 6.1))],
+                           (:Float64, :Float64) => [((64, 64, 32), (38.0, 33.0)), ((32, 32, 32), (14.0, 9.8))])
 
 "reference src/config.jl:84-120, unchanged (the reference-compatible answer; the launch uses the tile table)"
 function heuristic_block_shape(shared_a::Type, shared_b::Type, shared_c::Type, shared_d::Type)
@@ -378,9 +381,15 @@ end
 function default_block_shape(operator::Type, gemm_shape; tile_sized::Bool = true, a_kmajor::Bool = false, b_kmajor::Bool = true, planar::Bool = false)
     M, N, K = gemm_shape.M, gemm_shape.N, gemm_shape.K
     if Operator.is_fpu(operator)
-        small = nameof(operator) == :FPUOp && Operator.compute_type(operator) == Float32 && Operator.accum_type(operator) == Float32 &&
-                tile_sized && M % 32 == 0 && N % 32 == 0 && K % 32 == 0 && cld(M, 64) * cld(N, 64) < NUM_CUS ÷ 2
-        return small ? (M = 32, N = 32, K = 32) : (M = 64, N = 64, K = 32)
+        costs = nameof(operator) == :FPUOp ? get(FPU_TILE_COST, (nameof(Operator.compute_type(operator)), nameof(Operator.accum_type(operator))), []) : []
+        fitting = [(t, c) for (t, c) in costs if !tile_sized || (M % t[1] == 0 && N % t[2] == 0 && K % t[3] == 0)]
+        isempty(fitting) && return (M = 64, N = 64, K = 32)
+        function fpu_cost((t, c))
+            rounds = cld(cld(M, t[1]) * cld(N, t[2]), NUM_CUS)
+            rounds == 1 ? c[1] : c[2] * rounds
+        end
+        best = fitting[argmin(map(fpu_cost, fitting))][1]
+        return (M = best[1], N = best[2], K = best[3])
     elseif !Operator.is_mfma(operator)
         fitting = [t for (t, _) in complex_tiles(operator, a_kmajor, b_kmajor; planar = planar) if M % t[1] == 0 && N % t[2] == 0 && K % t[3] == 0]
         for t in fitting
@@ -742,7 +751,8 @@ function create_config(A::Type, sizeA::Dims, stridesA::Dims, transA::Bool,
     # and leading dimension, tiles over the edge, a partial last K tile) as long as A and B hold one whole chunk of
     # 8 elements along their contiguous index: then the tile is chosen among all tiles, not only those that divide
     # the sizes, and the operands it does not divide get the bounds-checked layouts, as the reference's rule says.
-    edge_ok = use_mfma && !zeroAlpha && (transA ? k : m) >= 8 && (transB ? n : k) >= 8
+    # (floating-point FPUOp takes any size and alignment on every tile)
+    edge_ok = !zeroAlpha && (use_mfma ? (transA ? k : m) >= 8 && (transB ? n : k) >= 8 : nameof(compute_type) in (:Float16, :Float32, :Float64))
     block_shape = default_block_shape(operator, (M = m, N = n, K = k); tile_sized = !edge_ok)
     ga, gb, gc, gd = layouts_for(block_shape)
     if !edge_ok && any(Layout.is_checked, (ga, gb, gc, gd))
