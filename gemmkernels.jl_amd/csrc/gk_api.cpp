@@ -115,8 +115,7 @@ bool ragged_fast_path(const gk_config* c) {
   return true;
 }
 
-// The aligned kernel has to take the last K tile out of its pipeline (see ragged_fast_path): the instances that
-// cannot (K-split) must not run such a product.
+// The aligned kernel has to take the last K tile out of its pipeline (see ragged_fast_path).
 bool needs_tail_tile(const gk_config* c) {
   const bool a_row = is_row_major(c->global_a_layout.kind), b_row = is_row_major(c->global_b_layout.kind);
   return (c->matmul_shape.K % c->block_shape.K) != 0 || (!a_row && (c->matmul_shape.M % 8) != 0) || (b_row && (c->matmul_shape.N % 8) != 0);
@@ -1057,14 +1056,15 @@ namespace {
 constexpr size_t kSplitCounterBytes = 2048;
 static_assert(kSplitCounterBytes / sizeof(unsigned) >= 2 * (size_t)gk::kNumCUs - 1, "one counter for every tile of a launch that is split");
 
-// K slices of a K-split launch, from a sweep of slice counts on 4096 x 64 x 4096, 256 x 256 x 16384 and
-// 8192 x 128 x 8192: about two workgroups per CU, and slices at least 1024 deep in K -- a slice pays for its
-// prologue, for the trip of its partial tile to memory and for the arrival counter (about 3 us on the last
-// workgroup's path), which shorter slices do not earn back (4096 x 64 x 4096: 4 slices 12.4 us, 8 slices 14.1 us,
-// 16 slices 19.4 us).
+// K slices of a K-split launch, from a sweep of 2 .. 24 slices on the 64 x 64 x 64 tile over eighteen products: no more
+// workgroups than two per CU (what a CU holds of these tiles at a time: 700 x 900 x 3001, 165 tiles, takes 18.6 us on 3 slices
+// and 21.9 on 4), and slices at least 640 deep in K -- a slice pays for its prologue, for the trip of its partial tile to
+// memory and for the arrival counter (about 3 us on the last workgroup's path), which shorter slices do not earn back.
+// 4096 x 64 x 4096: 2 slices 17.2 us, 4 14.1, 6 14.6, 8 15.7, 16 20.5; 300 x 500 x 4000: 3 14.5, 4 13.6, 6 13.0, 8 14.0;
+// 64 x 64 x 8000: 8 12.2, 12 11.4, 16 12.0, 24 12.2; 256 x 256 x 1024: 1 7.1, 2 8.9.
 int split_k_slices(int tiles, int k_tiles, int block_k) {
-  int slices = (2 * gk::kNumCUs + tiles - 1) / tiles;
-  const int min_tiles = (1024 + block_k - 1) / block_k;
+  int slices = tiles > 0 ? 2 * gk::kNumCUs / tiles : 1;
+  const int min_tiles = (640 + block_k - 1) / block_k;
   if (slices > k_tiles / min_tiles) slices = k_tiles / min_tiles;
   return slices < 1 ? 1 : slices;
 }
@@ -1089,13 +1089,17 @@ int launch_split_k(const gk_config* conf, const void* a, const void* b, const vo
   int slices = split_k_slices(tiles, kt, conf->block_shape.K);
   gk::InstanceInfo sk_info;
   // K-split instances exist for the small tiles that skinny products run; anything else (a large tile,
-  // generic A / B hooks, a partial last K tile on the aligned kernel) runs unsplit.  The bounds-checked
+  // generic A / B hooks) runs unsplit.  The bounds-checked
   // kernel takes its K range from the launch arguments, the aligned kernels have instances of their own.
   gk::FamilyFn sk_fn = L.key.family == gk::FAMILY_MFMA_CHECKED ? fn : gk::family_mfma_splitk;
-  if (slices > 1 && !L.ragged && sk_fn && sk_fn(L.key, L.args, dim3(1), nullptr, 0, &sk_info, &err)) {
-    const int per = (kt + slices - 1) / slices;
-    slices = (kt + per - 1) / per;           // no empty slice: every slice arrives at its tile's counter
-    const size_t counters = kSplitCounterBytes;
+  const int per = slices > 1 ? (kt + slices - 1) / slices : kt;
+  slices = (kt + per - 1) / per;           // no empty slice: every slice arrives at its tile's counter
+  const size_t counters = kSplitCounterBytes;
+  bool split = slices > 1 && sk_fn && sk_fn(L.key, L.args, dim3(1), nullptr, 0, &sk_info, &err);
+  // a product whose last K tile runs outside the pipeline does not insist on a workspace: it is the same launch unsplit
+  if (split && L.ragged && (!workspace || workspace_bytes < counters + (size_t)tiles * slices * conf->block_shape.M * conf->block_shape.N * sizeof(float) ||
+                            ((uintptr_t)workspace & 15u) != 0)) split = false;
+  if (split) {
     if ((size_t)tiles * sizeof(unsigned) > counters)
       return fail(GK_ERR_INVALID_ARGUMENT, "a K-split launch of %d tiles has no room for its arrival counters (%zu bytes)", tiles, counters);
     const size_t need = counters + (size_t)tiles * slices * conf->block_shape.M * conf->block_shape.N * sizeof(float);

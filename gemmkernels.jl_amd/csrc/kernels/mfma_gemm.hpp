@@ -466,9 +466,9 @@ struct MfmaGemmConfig {
   // tile (the host asks for it only with 16-byte aligned columns, M or N a multiple of 8 where that index is
   // the contiguous one of A or B, and K a multiple of 8): loads are clamped, the C load and the D store
   // masked, the part of the last K tile beyond K zeroed in LDS
-  // (the K-split instances take tiles over M and N, not a partial K tile)
+  // (K-split instances as well: the tile outside the pipeline belongs to the last slice)
   static constexpr bool RAGGED_OK = !GETT_ && FIX_ == FIX_NONE && !SOLO;
-  static constexpr bool RAGGED_K_OK = RAGGED_OK && !SPLITK_;
+  static constexpr bool RAGGED_K_OK = RAGGED_OK;
   static constexpr bool SYNC_FRAGS = FUSE_ == 2 || (!SOLO && (BM_ / WAVES_M_ / 32) * (BN_ / WAVES_N_ / 32) > 8) || (GK_FORCE_SYNC_FRAGS != 0);
   static constexpr bool PLANAR = (FIX_ == FIX_PLANAR);
   static constexpr bool PAIR = (FIX_ == FIX_PAIR || FIX_ == FIX_PAIR_DUAL);     // complex / dual product as one real product (see FIX_PAIR)
@@ -805,9 +805,13 @@ __global__ void __launch_bounds__(Cfg::THREADS) mfma_gemm_kernel(const GemmArgs 
     if (tail_k == 0 && straddle && KT > 0) { KT -= 1; tail_k = BK; }
   }
   if constexpr (Cfg::SPLITK) {
+    // Slice z takes k_steps of all K tiles, the one outside the pipeline counted with them: it is the last tile of the
+    // last slice (which may hold nothing else), every other slice ends inside the pipeline.
+    const int total = KT + (tail_k > 0 ? 1 : 0);
     const int kt0 = (int)blockIdx.z * args.k_steps;
+    if (kt0 >= total) return;       // the whole workgroup leaves together, before any barrier
+    if (kt0 + args.k_steps < total) tail_k = 0;
     KT = (KT - kt0) < args.k_steps ? (KT - kt0) : args.k_steps;
-    if (KT <= 0) return;       // the whole workgroup leaves together, before any barrier
     ga += (long long)kt0 * a_step;
     gb += (long long)kt0 * b_step;
   }

@@ -28,6 +28,8 @@ int family_mfma_splitk(const InstanceKey& key, const GemmArgs& args, dim3 grid, 
   GK_SK_T(bm_, bn_, bk_, wm_, wn_, st_, __bf16, DT_BF16, 3, "_bf16_fused_cd")
   GK_SK_TILE(128, 128, 64, 2, 2, 2)
   GK_SK_TILE(64, 64, 64, 2, 2, 4)
+  // (what a scale of A in BF16 is: the tile that the BLAS-style entry points run on slices of K takes every factor)
+  GK_SK_T(64, 64, 64, 2, 2, 4, __bf16, DT_BF16, 2, "_bf16_fused_ab")
   GK_SK_TILE(64, 64, 32, 1, 1, 2)
 #undef GK_SK_TILE
 #undef GK_SK_T

@@ -220,6 +220,16 @@ def default_block_shape(operator, gemm_shape, tile_sized: bool = True, gett: boo
     return NT(M=best[0], N=best[1], K=best[2])
 
 
+def split_k_block_shape(M, N, K) -> Optional[NT]:
+    """The tile of a 16-bit product that is worth cutting into slices of K (``Kernel.matmul_split_k``), or None: few output
+    tiles, which alone leave CUs idle, and a long K.  Measured against the best tile unsplit: 4096 x 64 x 4096 14.1 us
+    against 22.2, 300 x 500 x 4000 13.0 against 23.5, 64 x 64 x 8000 11.4 against 39, 2000 x 100 x 1500 11.6 against 12.3,
+    256 x 256 x 1024 8.9 against 7.1; with more than 128 tiles, which leave two or three slices, 1024 x 1024 x 4096 22.1
+    against 23.6, 700 x 900 x 3001 18.6 against 20.9, 1000 x 1000 x 2000 17.8 against 16.2."""
+    tiles = -(-M // 64) * -(-N // 64)
+    return NT(M=64, N=64, K=64) if K >= 1280 and tiles <= 128 or K >= 3000 and tiles <= 256 else None
+
+
 # Throughput of a CU that has one tile at a time, relative to 256 x 256 x 64 on four waves; a pair: a launch with at most
 # one tile per CU, a launch with several (the small tiles are bound by latency when alone).  From timings of every tile
 # and panel height at 1024^3 ... 6144^3 and eight rectangular problems ('N','N', three interleaved passes each):

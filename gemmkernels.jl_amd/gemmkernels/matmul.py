@@ -19,7 +19,7 @@ from . import kernel as Kernel
 from . import layout as Layout
 from . import operator as Operator
 from . import transform as Transform
-from .config import Config, default_block_shape, get_config as _get_config
+from .config import Config, default_block_shape, get_config as _get_config, split_k_block_shape
 from .dtypes import BFloat16, DType, Float16, Float32, Float64, from_torch, promote_type
 from .errors import ConfigError, DimensionMismatch
 from .tiling import NT
@@ -83,6 +83,7 @@ def _current_stream() -> int:
 
 
 _workspaces = {}
+_COUNTER_BYTES = 2048       # arrival counters at the head of a workspace (kSplitCounterBytes of the library)
 
 
 def split_k_workspace(conf_c, stream: int):
@@ -91,17 +92,31 @@ def split_k_workspace(conf_c, stream: int):
     (``gk_matmul_split_k``).  One zero-initialised buffer per device and stream, grown when a launch needs
     more: launches on one stream are ordered, so they can share it, and every launch leaves the arrival
     counters at its head at zero.  (0, 0) when the product runs unsplit."""
-    import torch
+    return _workspace(_split_k_bytes(conf_c), stream)
+
+
+def _split_k_bytes(conf_c) -> int:
     need = ctypes.c_size_t()
     rc = _lib.lib().gk_split_k_workspace_size(ctypes.byref(conf_c), ctypes.byref(need))
     if rc != _lib.GK_OK:
         _raise(rc)
-    if need.value == 0:
+    return need.value
+
+
+def _workspace(need: int, stream: int):
+    if need == 0:
         return 0, 0
+    import torch
+    if torch.cuda.is_current_stream_capturing():
+        # a buffer of the graph's own, cleared by every replay: one that eager launches or other graphs use as well could be
+        # in use, replaced by a larger one or not yet cleared when this graph runs
+        buf = torch.empty(need, dtype=torch.uint8, device="cuda")
+        buf[:_COUNTER_BYTES].zero_()
+        return int(buf.data_ptr()), need
     key = (torch.cuda.current_device(), int(stream))
     buf = _workspaces.get(key)
-    if buf is None or buf.numel() < need.value:
-        size = max(need.value, 1 << 20)
+    if buf is None or buf.numel() < need:
+        size = max(need, 1 << 20)
         buf = _workspaces[key] = torch.zeros(size, dtype=torch.uint8, device="cuda")
     return int(buf.data_ptr()), int(buf.numel())
 
@@ -408,7 +423,9 @@ def create_config(A: DType, sizeA, stridesA, transA: bool, B: DType, sizeB, stri
     # one), and the operands it does not divide get the bounds-checked layouts, as the reference's rule says.
     edge_ok = not zeroAlpha and (((k if transA else m) >= 8 and (n if transB else k) >= 8) if use_mfma
                                  else compute_type in (Float16, Float32, Float64))
-    block_shape = default_block_shape(operator, NT(M=m, N=n, K=k), tile_sized=not edge_ok, a_kmajor=transA, b_kmajor=not transB)
+    block_shape = split_k_block_shape(m, n, k) if use_mfma and edge_ok else None
+    if block_shape is None:
+        block_shape = default_block_shape(operator, NT(M=m, N=n, K=k), tile_sized=not edge_ok, a_kmajor=transA, b_kmajor=not transB)
     global_a_layout, global_b_layout, global_c_layout, global_d_layout = layouts_for(block_shape)
     if not edge_ok and any(l.kind in (Layout.COL_MAJOR, Layout.ROW_MAJOR) for l in (global_a_layout, global_b_layout, global_c_layout, global_d_layout)):
         # some operand needs bounds checks (and C = beta C, the zero alpha): one tile shape
@@ -453,13 +470,13 @@ def _single_plan(C, tA: bool, tB: bool, A, B, alpha, beta, wmma=None) -> Plan:
     ta = Transform.Elementwise(ops=[] if alpha_c == 1.0 else [(Transform.SCALE, alpha_c, 0.0)])
     tc = Transform.Elementwise(ops=[] if beta_c == 1.0 or beta == 0 else [(Transform.SCALE, beta_c, 0.0)])
     if conf.operator.kind == Operator.MFMA:
-        # few output tiles and a long K loop (skinny products, the rims of a cut-up product): the K-split kind
-        # cuts K into slices so that every CU gets work (the library decides how many, and runs the product
-        # unsplit when slices would be shorter than 1024 or the tile has no K-split instance).  Its sum is
+        # few output tiles and a long K loop (skinny products): the K-split kind cuts K into slices so that every CU gets
+        # work (the library decides how many, and runs the product unsplit when slices would be too short or the tile
+        # has no K-split instance; the bounds-checked kernel takes slices too).  Its sum is
         # ordered, so the result is the same on every run, like the reference's mul!.
         bs, ms = conf.block_shape, conf.matmul_shape
         tiles = -(-ms.M // bs.M) * -(-ms.N // bs.N)
-        if tiles <= 256 and ms.K >= 2048:
+        if split_k_block_shape(ms.M, ms.N, ms.K) is not None or tiles <= 256 and ms.K >= 2048:
             kernel = Kernel.matmul_split_k
     p = plan(conf, A, B, C, C, transform_shared_to_regs_a=ta, transform_shared_to_regs_c=tc, kernel=kernel)
     p.kernel_names = (kernel_name(conf, kernel, dict(transform_shared_to_regs_a=ta, transform_shared_to_regs_c=tc)),)

@@ -247,3 +247,69 @@ def test_blas_entry_after_a_product_with_fewer_tiles(gpu):
         gk.matmatmul_(C, "N", "N", gk.colmajor(ai), gk.colmajor(bi), 1.0, 1.0)
         torch.cuda.synchronize()
         assert np.array_equal(gk.to_numpy(C).astype(np.float64), ai.astype(np.float64) @ bi.astype(np.float64) + ci), (M, N, K)
+
+
+def _inside_nan(x, rows, cols):
+    """x as a view that starts off a 16-byte boundary inside a larger matrix of NaN, with the given number of rows and columns more."""
+    big = np.full((x.shape[0] + rows, x.shape[1] + cols), np.nan, x.dtype, order="F")
+    big[1:x.shape[0] + 1, :x.shape[1]] = x
+    return gk.colmajor(big)[1:x.shape[0] + 1, :x.shape[1]]
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("dims,tile", [((70, 61, 2049), ((64, 64, 64), (2, 2))),        # 33 K tiles, a single k in the last
+                                       ((65, 72, 18501), ((64, 64, 64), (2, 2))),       # 290 K tiles on 18 slices of 17: the last slice is the partial tile alone
+                                       ((131, 67, 2048), ((64, 64, 64), (2, 2))),       # whole K tiles, chunks over the end of an operand
+                                       ((129, 130, 3007), ((128, 128, 64), (2, 2))), ((9, 8, 2050), ((128, 128, 64), (2, 2))),
+                                       ((33, 90, 2079), ((64, 64, 32), (1, 1)))])
+def test_a_partial_last_k_tile_is_the_end_of_the_last_slice(gpu, dims, tile, ta, tb):
+    """Any extents, leading dimensions and addresses are split as well.  Small-integer data (every sum is exact in FP32, so
+    the result equals the float64 product), NaN wherever an operand has no values, C read and D written in place."""
+    from gemmkernels import Float16, Float32, Layout, NT, Operator
+    M, N, K = dims
+    (bm, bn, bk), (wm, wn) = tile
+    rs = np.random.RandomState(M)
+    a = np.asfortranarray(rs.randint(-4, 5, size=(K, M) if ta else (M, K)).astype(np.float16))
+    b = np.asfortranarray(rs.randint(-4, 5, size=(N, K) if tb else (K, N)).astype(np.float16))
+    c = np.asfortranarray(rs.randint(-64, 65, size=(M, N)).astype(np.float32))
+    conf = gk.get_config(gemm_shape=NT(M=M, N=N, K=K), block_shape=NT(M=bm, N=bn, K=bk), warps_per_block=wm * wn,
+                         compute_warp=NT(M=bm // wm, N=bn // wn, K=16), operator=Operator.MFMAOp[32, 32, 16, Float16, Float32],
+                         global_a_layout=(Layout.RowMajor if ta else Layout.ColMajor)[Float16], global_b_layout=(Layout.RowMajor if tb else Layout.ColMajor)[Float16],
+                         global_c_layout=Layout.ColMajor[Float32], global_d_layout=Layout.ColMajor[Float32],
+                         shared_a_layout=Layout.Padded[(Layout.UnsafeAlignedRowMajor if ta else Layout.UnsafeAlignedColMajor)[Float16], 8],
+                         shared_b_layout=Layout.Padded[(Layout.UnsafeAlignedRowMajor if tb else Layout.UnsafeAlignedColMajor)[Float16], 8],
+                         shared_c_layout=Layout.UnsafeAlignedColMajor[Float32], shared_d_layout=Layout.UnsafeAlignedColMajor[Float32],
+                         is_a_col_major=not ta, is_b_col_major=not tb)
+    print("case", dims, tile, ta, tb, gk.kernel_name(conf, Kernel.matmul_split_k), flush=True)
+    C = _inside_nan(c, 5, 2)
+    gk.matmul(conf, _inside_nan(a, 3, 1), _inside_nan(b, 4, 1), C, C, kernel=Kernel.matmul_split_k)
+    torch.cuda.synchronize()
+    product = (a.T if ta else a).astype(np.float64) @ (b.T if tb else b).astype(np.float64)
+    assert np.array_equal(C.cpu().numpy().astype(np.float64), product + c)
+
+
+def test_captured_products_keep_a_workspace_of_their_own(gpu):
+    """Two graphs of mul! on K slices, replayed in either order with eager products (which grow the shared workspace)
+    between the replays: every replay gives the eager result."""
+    def operands_of(M, N, K, seed):
+        rs = np.random.RandomState(seed)
+        return (gk.colmajor(np.asfortranarray(rs.randint(-4, 5, size=s).astype(np.float16))) for s in ((M, K), (K, N)))
+    cases = []
+    for i, (M, N, K) in enumerate(((1024, 64, 4096), (515, 130, 4099))):
+        A, B = operands_of(M, N, K, i)
+        C, ref = gk.colmajor_empty((M, N), torch.float32), gk.colmajor_empty((M, N), torch.float32)
+        gk.mul_(ref, A, B)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            gk.mul_(C, A, B)
+        cases.append((graph, A, B, C, ref))
+    for turn in range(4):
+        for graph, A, B, C, ref in (cases if turn % 2 else cases[::-1]):
+            C.fill_(float("nan"))
+            graph.replay()
+            X, Y = operands_of(64 * (turn + 1), 64 * (turn + 1), 8192, 10 + turn)
+            Z = gk.colmajor_empty((X.shape[0], Y.shape[1]), torch.float32)
+            gk.mul_(Z, X, Y)
+            torch.cuda.synchronize()
+            assert torch.equal(C, ref) and torch.equal(Z, (X.double() @ Y.double()).float())
