@@ -271,3 +271,22 @@ def test_fpu_operator_shapes(gpu, ta, tb):
 def _lib_status_op_shape():
     from gemmkernels import _lib
     return _lib.GK_ERR_OP_SHAPE
+
+
+def test_calls_of_one_kind_share_their_descriptors_and_nothing_else(gpu):
+    """mul! keeps the lowered launch by element types, sizes, strides, alignment and factors: calls that agree in these
+    on other buffers, and calls that differ in one of them, each give their own product (small integers: exact)."""
+    rs = np.random.RandomState(11)
+    M, N, K = 96, 64, 80
+    for turn in range(3):
+        for dtype, ld, first, alpha, beta in ((torch.float16, 96, 0, 1.0, 0.0), (torch.float16, 96, 0, 2.0, 0.0), (torch.float16, 96, 0, 1, True),
+                                              (torch.float16, 104, 0, 1.0, 0.0), (torch.float16, 104, 1, 1.0, 0.0), (torch.float32, 96, 0, 1.0, 3.0),
+                                              (torch.float64, 104, 1, 0.0, 3.0)):
+            out = torch.float32 if dtype == torch.float16 else dtype
+            a = gk.colmajor(np.asfortranarray(rs.randint(-4, 5, size=(ld, K)).astype(np.float32))).to(dtype)[first:first + M]
+            b = gk.colmajor(np.asfortranarray(rs.randint(-4, 5, size=(K, N)).astype(np.float32))).to(dtype)
+            c = gk.colmajor(np.asfortranarray(rs.randint(-4, 5, size=(M, N)).astype(np.float32))).to(out)
+            ref = float(alpha) * (a.double().cpu() @ b.double().cpu()) + float(beta) * c.double().cpu()
+            gk.matmatmul_(c, "N", "N", a, b, alpha, beta)
+            torch.cuda.synchronize()
+            assert torch.equal(c.double().cpu(), ref), (turn, dtype, ld, first, alpha, beta)
