@@ -1062,11 +1062,17 @@ static_assert(kSplitCounterBytes / sizeof(unsigned) >= 2 * (size_t)gk::kNumCUs -
 // memory and for the arrival counter (about 3 us on the last workgroup's path), which shorter slices do not earn back.
 // 4096 x 64 x 4096: 2 slices 17.2 us, 4 14.1, 6 14.6, 8 15.7, 16 20.5; 300 x 500 x 4000: 3 14.5, 4 13.6, 6 13.0, 8 14.0;
 // 64 x 64 x 8000: 8 12.2, 12 11.4, 16 12.0, 24 12.2; 256 x 256 x 1024: 1 7.1, 2 8.9.
-int split_k_slices(int tiles, int k_tiles, int block_k) {
+// Where the partial tiles of that many slices would not fit the library's static workspace (512 tiles of 128 x 128 and the
+// counters are 2 KiB more than it holds) the slices are 1024 deep: what fits it at that depth is not refused.
+int split_k_slices(int tiles, int k_tiles, const gk_shape& block) {
   int slices = tiles > 0 ? 2 * gk::kNumCUs / tiles : 1;
-  const int min_tiles = (640 + block_k - 1) / block_k;
-  if (slices > k_tiles / min_tiles) slices = k_tiles / min_tiles;
-  return slices < 1 ? 1 : slices;
+  for (const int depth : {640, 1024}) {
+    const int min_tiles = (depth + block.K - 1) / block.K;
+    if (slices > k_tiles / min_tiles) slices = k_tiles / min_tiles;
+    if (slices < 2) return 1;
+    if (kSplitCounterBytes + (size_t)tiles * slices * block.M * block.N * sizeof(float) <= gk_split_k_noalloc_capacity()) break;
+  }
+  return slices;
 }
 
 }  // namespace
@@ -1086,7 +1092,7 @@ int launch_split_k(const gk_config* conf, const void* a, const void* b, const vo
   hipError_t err = hipSuccess;
   const int tiles = L.gx * L.gy;
   const int kt = (conf->matmul_shape.K + conf->block_shape.K - 1) / conf->block_shape.K;   // bounds-checked layouts: the last tile may be partial
-  int slices = split_k_slices(tiles, kt, conf->block_shape.K);
+  int slices = split_k_slices(tiles, kt, conf->block_shape);
   gk::InstanceInfo sk_info;
   // K-split instances exist for the small tiles that skinny products run; anything else (a large tile,
   // generic A / B hooks) runs unsplit.  The bounds-checked
@@ -1132,7 +1138,7 @@ int gk_split_k_workspace_size(const gk_config* conf, size_t* bytes) {
   if (g.M <= 0 || g.N <= 0 || g.K <= 0 || b.M <= 0 || b.N <= 0 || b.K <= 0) return fail(GK_ERR_INVALID_ARGUMENT, "shapes must be positive");
   const long long tiles = (long long)((g.M + b.M - 1) / b.M) * ((g.N + b.N - 1) / b.N);
   const int kt = (g.K + b.K - 1) / b.K;
-  const long long slices = split_k_slices((int)(tiles > (1 << 30) ? (1 << 30) : tiles), kt, b.K);
+  const long long slices = split_k_slices((int)(tiles > (1 << 30) ? (1 << 30) : tiles), kt, b);
   if (slices < 2) { *bytes = 0; return GK_OK; }      // runs unsplit
   *bytes = kSplitCounterBytes + (size_t)tiles * (size_t)slices * b.M * b.N * sizeof(float);
   return GK_OK;

@@ -345,3 +345,16 @@ def test_reference_shmem_size_known_answers():
     c.shared_d_layout.kind = Layout.ALIGNED_COL_MAJOR; c.shared_d_layout.eltype = 0
     # C as a 64 x 64 F16 tile (8 192 B), D the same: now A + B = 9 216 + 10 240 wins
     assert _lib.lib().gk_reference_shmem_size(ctypes.byref(c)) == 9216 + 10240
+
+
+@pytest.mark.parametrize("tiles,K", [((8, 8), 5120), ((8, 8), 8128), ((16, 8), 2560), ((16, 16), 1280), ((4, 4), 20480)])
+def test_k_slices_that_fit_the_static_workspace_at_1024_deep_fit_it(tiles, K):
+    """gk_matmul_split_k_noalloc takes every product whose slices of at least 1024 values leave partial tiles that the static
+    workspace holds, also where slices of 640 would be one too many (512 tiles of 128 x 128 and the counters)."""
+    import ctypes
+    from gemmkernels import _lib, configs
+    m, n = tiles
+    cconf = configs.mfma_config(128 * m, 128 * n, K, block_shape=(128, 128, 64)).to_c(128 * m, K, 128 * m, 128 * m)
+    need = ctypes.c_size_t()
+    assert _lib.lib().gk_split_k_workspace_size(ctypes.byref(cconf), ctypes.byref(need)) == _lib.GK_OK
+    assert need.value <= _lib.lib().gk_split_k_noalloc_capacity()
