@@ -25,6 +25,12 @@
 // Float64 1000^3 115 -> 41 us, 2048^3 -> 270 (64 TFLOP/s, 0.83).  What is left: the last round of tiles (2560^3 has 1600
 // tiles of 64 x 64 for 256 CUs: 7 rounds where 6.25 would do), and the ends of a launch.
 //
+// A K tile of 32 x 32 x 32 is a few hundred clocks of work for the matrix cores (512 in FP64, 256 in FP32), less than a load
+// takes from the last-level cache: on four waves these tiles have the loads of two K tiles in flight (DEPTH; the loop is
+// written out for a pair of tiles, so that each finds its registers): Float32 1024^3 25.7 -> 24.7 us, 300 x 700 x 1500
+// 17.2 -> 16.3, Float64 500 x 500 x 700 12.7 -> 12.1, 1024^3 44.9 -> 42.6.  Tiles of 64 x 64 gain nothing from it (Float64
+// 1024^3 41.1 -> 41.6, Float32 2048^3 142 -> 145): one in flight.
+//
 // Sizes, leading dimensions and addresses are free.  A vector load takes any address that is aligned to its elements; rows
 // beyond the edge of an operand are clamped to the last ones (their products land in outputs that are not stored):
 // where memory is contiguous along the rows the vector that reaches over the edge is fetched from 1 .. 3 elements further
@@ -55,9 +61,9 @@ template <> struct ChainBlock<double> {
 };
 
 template <int BM_, int BN_, int BK_, int WAVES_M_, int WAVES_N_, typename TIN_, bool A_KMAJOR_, bool B_KMAJOR_, typename TACC_, bool FUSED_,
-          int STAGES_, int RING_>
+          int STAGES_, int RING_, int DEPTH_>
 struct FpuMfmaConfig {
-  static constexpr int BM = BM_, BN = BN_, BK = BK_, WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, STAGES = STAGES_, RING = RING_;
+  static constexpr int BM = BM_, BN = BN_, BK = BK_, WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, STAGES = STAGES_, RING = RING_, DEPTH = DEPTH_;
   static constexpr bool A_KMAJOR = A_KMAJOR_, B_KMAJOR = B_KMAJOR_, FUSED = FUSED_;
   typedef TIN_ TIN;
   typedef TACC_ TACC;
@@ -266,7 +272,8 @@ __global__ void __launch_bounds__(Cfg::THREADS, 2) fpu_mfma_kernel(const GemmArg
   constexpr int COUNT = FM * FN * 4;
   typedef typename Block::acc_t acc_t;
   constexpr bool AHEAD = STAGES == 3;
-  constexpr int FAR = AHEAD ? 2 : 1;             // a tile goes to LDS FAR tiles before it is multiplied, one tile after its loads set out
+  constexpr int FAR = AHEAD ? 2 : 1;             // a tile goes to LDS FAR tiles before it is multiplied, DEPTH tiles after its loads set out
+  constexpr int DEPTH = Cfg::DEPTH;
   constexpr int STAGE = Cfg::A_ELEMS + Cfg::B_ELEMS, PA = Cfg::A_PER_THREAD, PB = Cfg::B_PER_THREAD;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   TACC* lds = (TACC*)smem;
@@ -375,11 +382,11 @@ __global__ void __launch_bounds__(Cfg::THREADS, 2) fpu_mfma_kernel(const GemmArg
   const int whole = K / BK, k_tail = whole * BK;
   auto pipeline = [&](auto moved_c, auto listed_c) __attribute__((always_inline)) {
     constexpr bool MOVED = decltype(moved_c)::value, LISTED = decltype(listed_c)::value;
-    typename decltype(oa)::vec ra[FAR + 1][PA], ta[PA];
-    typename decltype(ob)::vec rb[FAR + 1][PB], tb[PB];
+    typename decltype(oa)::vec ra[FAR + DEPTH][PA], ta[PA];      // (tile t of the loop waits in slot FAR + (t - FAR) % DEPTH)
+    typename decltype(ob)::vec rb[FAR + DEPTH][PB], tb[PB];
     auto k_of = [&](int t) { return (t < whole ? t : whole - 1) * BK; };      // a tile that exists
     if (whole > 0)
-      fpu_static_for<0, FAR + 1>([&](auto t_c) __attribute__((always_inline)) {
+      fpu_static_for<0, FAR + DEPTH>([&](auto t_c) __attribute__((always_inline)) {
         constexpr int t = decltype(t_c)::value;
 #pragma unroll
         for (int i = 0; i < PA; ++i) ra[t][i] = oa.template fetch<false>(i, k_of(t));
@@ -413,11 +420,12 @@ __global__ void __launch_bounds__(Cfg::THREADS, 2) fpu_mfma_kernel(const GemmArg
       if constexpr (AHEAD)
         fpu_static_for<0, LOOK>([&](auto s_c) __attribute__((always_inline)) { read(decltype(s_c)::value, lds, decltype(s_c)::value); });
     }
-    for (int kt = 0; kt < whole; ++kt) {
+    auto tile = [&](int kt, auto slot_c) __attribute__((always_inline)) {
+      constexpr int SLOT = FAR + decltype(slot_c)::value;
       const TACC* here = lds + stage * STAGE;
       const int next = stage + 1 == STAGES ? 0 : stage + 1, after = next + 1 == STAGES ? 0 : next + 1;
       TACC* into = lds + (AHEAD ? after : next) * STAGE;
-      const int k_in = k_of(kt + FAR), k_out = k_of(kt + FAR + 1);
+      const int k_in = k_of(kt + FAR), k_out = k_of(kt + FAR + DEPTH);
       if constexpr (!AHEAD) read(0, here, 0);
       fpu_static_for<0, STEPS>([&](auto s_c) __attribute__((always_inline)) {
         constexpr int s = decltype(s_c)::value;
@@ -429,11 +437,11 @@ __global__ void __launch_bounds__(Cfg::THREADS, 2) fpu_mfma_kernel(const GemmArg
         fpu_static_for<lo, hi>([&](auto v_c) __attribute__((always_inline)) {
           constexpr int v = decltype(v_c)::value;
           if constexpr (v < PA) {
-            stash_a(into, ra[FAR][v], v, k_in);
-            ra[FAR][v] = oa.template fetch<false>(v, k_out);
+            stash_a(into, ra[SLOT][v], v, k_in);
+            ra[SLOT][v] = oa.template fetch<false>(v, k_out);
           } else {
-            stash_b(into, rb[FAR][v - PA], v - PA, k_in);
-            rb[FAR][v - PA] = ob.template fetch<false>(v - PA, k_out);
+            stash_b(into, rb[SLOT][v - PA], v - PA, k_in);
+            rb[SLOT][v - PA] = ob.template fetch<false>(v - PA, k_out);
           }
         });
         interleave();
@@ -442,6 +450,16 @@ __global__ void __launch_bounds__(Cfg::THREADS, 2) fpu_mfma_kernel(const GemmArg
       wait_lds<QUIET * ((FM + FN + 1) / 2)>();
       block_barrier();
       stage = next;
+    };
+    // The accumulators that C filled have arrived when the loop begins: left open, the compiler waits for every load of the
+    // next tile in front of the first MFMA of each tile (vmcnt(0) there; with this, one vector at a time where it goes to LDS).
+    __builtin_amdgcn_s_waitcnt(0x0F70);         // vmcnt(0)
+    static_assert(DEPTH == 1 || DEPTH == 2, "the tiles in flight find their registers by the parity of the tile");
+    for (int kt = 0; kt < whole; kt += DEPTH) {
+      tile(kt, std::integral_constant<int, 0>{});
+      if constexpr (DEPTH == 2) {
+        if (kt + 1 < whole) tile(kt + 1, std::integral_constant<int, 1>{});
+      }
     }
     if (k_tail < K) {
       // (the barrier above: everyone has read the last whole tile)
