@@ -224,9 +224,9 @@ struct ChainOperand {
     return x;
   }
   // the two load hooks, each rounded to the element type of its destination (the operand's own type), then the
-  // conversion to the accumulator type for the fma.  LISTED: the hooks are lists; values beyond K stay zero whatever
-  // the lists make of them
-  template <bool LISTED>
+  // conversion to the accumulator type for the fma.  LISTED: the hooks are lists.  Values beyond K stay zero whatever the
+  // hooks make of them (TAIL: a partial K tile, which alone has such values; 0 times an infinite factor is a NaN)
+  template <bool LISTED, bool TAIL>
   __device__ __forceinline__ void store(TACC* lds, vec x, int i, int k0) const {
     typedef TACC accv __attribute__((ext_vector_type(V)));
     if constexpr (LISTED) {
@@ -246,7 +246,10 @@ struct ChainOperand {
       }
     } else if constexpr (Cfg::FUSED) {
 #pragma unroll
-      for (int e = 0; e < V; ++e) x[e] = (TIN)((TAR)x[e] * scale);
+      for (int e = 0; e < V; ++e) {
+        x[e] = (TIN)((TAR)x[e] * scale);
+        if constexpr (TAIL) x[e] = k0 + (KMAJOR ? within + e : line + i * LINES) < K ? x[e] : (TIN)0;
+      }
     }
     accv z;
 #pragma unroll
@@ -401,10 +404,10 @@ __global__ void __launch_bounds__(Cfg::THREADS, 2) fpu_mfma_kernel(const GemmArg
     }
     load_c();
     auto stash_a = [&](TACC* stage, typename decltype(oa)::vec x, int i, int k0) __attribute__((always_inline)) {
-      oa.template store<LISTED>(stage, oa.template settle<MOVED, false>(x, i, k0), i, k0);
+      oa.template store<LISTED, false>(stage, oa.template settle<MOVED, false>(x, i, k0), i, k0);
     };
     auto stash_b = [&](TACC* stage, typename decltype(ob)::vec x, int i, int k0) __attribute__((always_inline)) {
-      ob.template store<LISTED>(stage + Cfg::A_ELEMS, ob.template settle<MOVED, false>(x, i, k0), i, k0);
+      ob.template store<LISTED, false>(stage + Cfg::A_ELEMS, ob.template settle<MOVED, false>(x, i, k0), i, k0);
     };
     int stage = 0;
     if (whole > 0) {
@@ -466,9 +469,9 @@ __global__ void __launch_bounds__(Cfg::THREADS, 2) fpu_mfma_kernel(const GemmArg
       wait_lgkmcnt0();
       block_barrier();
 #pragma unroll
-      for (int i = 0; i < PA; ++i) oa.template store<LISTED>(lds, oa.template settle<MOVED, true>(ta[i], i, k_tail), i, k_tail);
+      for (int i = 0; i < PA; ++i) oa.template store<LISTED, true>(lds, oa.template settle<MOVED, true>(ta[i], i, k_tail), i, k_tail);
 #pragma unroll
-      for (int i = 0; i < PB; ++i) ob.template store<LISTED>(lds + Cfg::A_ELEMS, ob.template settle<MOVED, true>(tb[i], i, k_tail), i, k_tail);
+      for (int i = 0; i < PB; ++i) ob.template store<LISTED, true>(lds + Cfg::A_ELEMS, ob.template settle<MOVED, true>(tb[i], i, k_tail), i, k_tail);
       wait_lgkmcnt0();
       block_barrier();
       const int steps = (K - k_tail + 3) / 4;            // the steps that hold values
@@ -509,9 +512,9 @@ __global__ void __launch_bounds__(Cfg::THREADS, 2) fpu_mfma_kernel(const GemmArg
     for (int kt = 0; kt < KT; ++kt) {
       block_barrier();
 #pragma unroll
-      for (int i = 0; i < PA; ++i) oa.template store<Cfg::FUSED>(lds, xa[i], i, kt * BK);
+      for (int i = 0; i < PA; ++i) oa.template store<Cfg::FUSED, true>(lds, xa[i], i, kt * BK);
 #pragma unroll
-      for (int i = 0; i < PB; ++i) ob.template store<Cfg::FUSED>(lds + Cfg::A_ELEMS, xb[i], i, kt * BK);
+      for (int i = 0; i < PB; ++i) ob.template store<Cfg::FUSED, true>(lds + Cfg::A_ELEMS, xb[i], i, kt * BK);
       wait_lgkmcnt0();
       block_barrier();
       if (kt + 1 < KT) fetch((kt + 1) * BK);

@@ -68,6 +68,22 @@ def test_zeros_infinities_and_subnormals_go_through_as_in_an_fma_chain(gpu, ta, 
         assert np.array_equal(np.signbit(d[ref == 0]), np.signbit(ref[ref == 0]))
 
 
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, True)])
+def test_nothing_behind_k_meets_an_infinite_factor(gpu, ta, tb):
+    """A scale by infinity makes NaN of a zero: the values behind a partial K tile are none of the product's."""
+    times_inf = Transform.Elementwise(lambda x: x * float("inf"))
+    for types in TYPES:
+        _, _, np_in, np_out = TYPES[types]
+        for K in (1, 5, 34, 45, 67):
+            M, N = 66, 70
+            a, b = abs(operand((K, M) if ta else (M, K), np_in, 61)) + np_in(1), abs(operand((N, K) if tb else (K, N), np_in, 62)) + np_in(1)
+            for hooks in (dict(transform_shared_to_regs_a=times_inf), dict(transform_global_to_shared_b=times_inf)):
+                conf = config(M, N, K, ta, tb, types, TILES[types][-1], True)
+                d = helpers.run_gpu(conf, a, b, None, (M, N), d_dtype=TORCH[np_out], transforms=hooks)
+                ref = helpers.run_oracle(conf, a, b, None, (M, N), d_dtype=np_out, transforms=hooks)
+                assert np.all(np.isposinf(ref)) and np.array_equal(d, ref), (types, K, list(hooks))
+
+
 def test_operands_at_the_end_of_an_allocation_and_off_16_byte_boundaries(gpu):
     """Leading dimensions and first elements at any multiple of the element size; bias per column and per row."""
     for types in ("f32", "f64"):
