@@ -1149,6 +1149,20 @@ int gk_matmul_split_k(const gk_config* conf, const void* a, const void* b, const
   return gk_internal::launch_split_k(conf, a, b, c, d, transforms, epilogue, workspace, workspace_bytes, "the caller's workspace", stream);
 }
 
+int gk_stream_capture(void* stream, int32_t* capturing, uint64_t* id) {
+  if (!capturing || !id) return fail(GK_ERR_INVALID_ARGUMENT, "NULL argument");
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long capture = 0;
+  if (hipStreamGetCaptureInfo((hipStream_t)stream, &status, &capture) != hipSuccess) {
+    // (the default stream may not be asked while another stream is captured; it is not captured itself)
+    (void)hipGetLastError();
+    status = hipStreamCaptureStatusNone;
+  }
+  *capturing = status != hipStreamCaptureStatusNone;
+  *id = *capturing ? capture : 0;
+  return GK_OK;
+}
+
 int gk_dev_alloc(size_t bytes, void** ptr) {
   if (!ptr) return fail(GK_ERR_INVALID_ARGUMENT, "ptr is NULL");
   *ptr = nullptr;

@@ -7,6 +7,7 @@ only the owner of the memory and of the stream; every flop runs in libgemmkernel
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 from typing import Optional
 
@@ -82,16 +83,19 @@ def _current_stream() -> int:
         return torch.cuda.current_stream().cuda_stream
 
 
-_workspaces = {}
+_workspaces = {}            # (device, stream) -> buffer of eager launches
+_recorded = {}              # (device, stream) -> buffers of graphs captured without torch
+_pool_of_capture = {}       # (device, capture) -> whether torch keeps the capture's memory for the graph
 _COUNTER_BYTES = 2048       # arrival counters at the head of a workspace (kSplitCounterBytes of the library)
 
 
 def split_k_workspace(conf_c, stream: int):
-    """Device workspace for a K-split launch of ``conf_c`` on ``stream``: (pointer, bytes).  The slices of an
-    output tile leave their partial tiles there and the last one to arrive adds them up in slice order
-    (``gk_matmul_split_k``).  One zero-initialised buffer per device and stream, grown when a launch needs
-    more: launches on one stream are ordered, so they can share it, and every launch leaves the arrival
-    counters at its head at zero.  (0, 0) when the product runs unsplit."""
+    """Device workspace for a K-split launch of ``conf_c`` on ``stream``, as a byte tensor (None: the product runs
+    unsplit).  The slices of an output tile leave their partial tiles there and the last one to arrive adds them
+    up in slice order (``gk_matmul_split_k``).  One zero-initialised buffer per device and stream, grown when a
+    launch needs more: launches on one stream are ordered, so they can share it, and every launch leaves the
+    arrival counters at its head at zero.  The caller keeps the tensor until the launch is on its stream: another
+    thread may replace the buffer by a larger one meanwhile."""
     return _workspace(_split_k_bytes(conf_c), stream)
 
 
@@ -103,22 +107,74 @@ def _split_k_bytes(conf_c) -> int:
     return need.value
 
 
+def _span(buf):
+    """What the library is told of a workspace: its address and size."""
+    return (int(buf.data_ptr()), int(buf.numel())) if buf is not None else (0, 0)
+
+
+def _on(stream: int):
+    """torch's current stream set to ``stream`` (a raw handle): what is allocated and cleared under it belongs to it, so the
+    clear runs in front of a launch on it and whatever gets the memory next runs behind that launch."""
+    import torch
+    if stream == _current_stream():
+        return contextlib.nullcontext()
+    return torch.cuda.stream(torch.cuda.ExternalStream(stream) if stream else torch.cuda.default_stream())
+
+
+def _capture_of(stream: int):
+    """The id of the capture that ``stream`` is part of, or None."""
+    capturing, capture = ctypes.c_int32(), ctypes.c_uint64()
+    rc = _lib.lib().gk_stream_capture(stream, ctypes.byref(capturing), ctypes.byref(capture))
+    if rc != _lib.GK_OK:
+        _raise(rc)
+    return capture.value if capturing.value else None
+
+
+def _in_graph_pool(buf, capture: int) -> bool:
+    """Whether a buffer allocated during a capture lies in a memory pool of the graph (``torch.cuda.graph``), which keeps
+    its memory as long as the graph lives, or in the allocator's common one, which hands it out again.  One answer for all
+    of a capture."""
+    import torch
+    key = (buf.device.index, capture)
+    known = _pool_of_capture.get(key)
+    if known is None:
+        p = buf.data_ptr()
+        pools = [tuple(s["segment_pool_id"]) for s in torch.cuda.memory_snapshot()
+                 if s["device"] == buf.device.index and s["address"] <= p < s["address"] + s["total_size"]]
+        known = bool(pools) and pools[0] != (0, 0)
+        if len(_pool_of_capture) >= 64:
+            _pool_of_capture.clear()
+        _pool_of_capture[key] = known
+    return known
+
+
 def _workspace(need: int, stream: int):
     if need == 0:
-        return 0, 0
+        return None
     import torch
-    if torch.cuda.is_current_stream_capturing():
+    stream = int(stream)
+    key = (torch.cuda.current_device(), stream)
+    capture = _capture_of(stream)
+    if capture is not None:
         # a buffer of the graph's own, cleared by every replay: one that eager launches or other graphs use as well could be
         # in use, replaced by a larger one or not yet cleared when this graph runs
-        buf = torch.empty(need, dtype=torch.uint8, device="cuda")
-        buf[:_COUNTER_BYTES].zero_()
-        return int(buf.data_ptr()), need
-    key = (torch.cuda.current_device(), int(stream))
+        with _on(stream):
+            buf = torch.empty(need, dtype=torch.uint8, device="cuda")
+            if not _in_graph_pool(buf, capture):
+                # a capture that torch does not know of: nobody else keeps the memory for the graph, so it is never given
+                # back.  The graphs captured so on one stream share a buffer (as launches on one stream do: their replays
+                # must not overlap), and a larger one is at least twice as large, which bounds all of them together
+                kept = _recorded.setdefault(key, [])
+                if not kept or kept[-1].numel() < need:
+                    kept.append(buf if not kept else torch.empty(max(need, 2 * kept[-1].numel()), dtype=torch.uint8, device="cuda"))
+                buf = kept[-1]
+            buf[:_COUNTER_BYTES].zero_()
+        return buf
     buf = _workspaces.get(key)
     if buf is None or buf.numel() < need:
-        size = max(need, 1 << 20)
-        buf = _workspaces[key] = torch.zeros(size, dtype=torch.uint8, device="cuda")
-    return int(buf.data_ptr()), int(buf.numel())
+        with _on(stream):
+            buf = _workspaces[key] = torch.zeros(max(need, 1 << 20), dtype=torch.uint8, device="cuda")
+    return buf
 
 
 _IDENTITY = Transform.Elementwise()
@@ -242,7 +298,8 @@ class Plan:
     def __call__(self, stream=None):
         stream = _current_stream() if stream is None else int(stream)
         if self._split_k:
-            rc = self._fn(*self._args, *split_k_workspace(self._conf, stream), stream)
+            workspace = split_k_workspace(self._conf, stream)
+            rc = self._fn(*self._args, *_span(workspace), stream)
             if rc != _lib.GK_OK:
                 _raise(rc)
             return self.d
@@ -311,10 +368,11 @@ def matmul(conf: Config, a, b, c, d, *,
         cepi.bias = _ptr(epilogue.bias)
     stream = _current_stream() if stream is None else int(stream)
     if kernel is Kernel.matmul_split_k:
+        workspace = split_k_workspace(cconf, stream)
         rc = _lib.lib().gk_matmul_split_k(ctypes.byref(cconf), _ptr(a), _ptr(b), _ptr(c), _ptr(d),
                                           ctypes.byref(ctrans) if ctrans is not None else None,
                                           ctypes.byref(cepi) if cepi is not None else None,
-                                          *split_k_workspace(cconf, stream), stream)
+                                          *_span(workspace), stream)
     else:
         rc = _lib.lib().gk_matmul(ctypes.byref(cconf), _ptr(a), _ptr(b), _ptr(c), _ptr(d),
                                   ctypes.byref(ctrans) if ctrans is not None else None,
@@ -536,7 +594,8 @@ class _MulLaunch:
         if self._workspace is None:
             rc = self._fn(self._conf_ref, a, b, c, c, self._trans_ref, None, self._code, stream)
         else:
-            rc = self._fn(self._conf_ref, a, b, c, c, self._trans_ref, None, *_workspace(self._workspace, stream), stream)
+            workspace = _workspace(self._workspace, stream)
+            rc = self._fn(self._conf_ref, a, b, c, c, self._trans_ref, None, *_span(workspace), stream)
         if rc != _lib.GK_OK:
             _raise(rc)
 

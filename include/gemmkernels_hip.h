@@ -286,6 +286,11 @@ int gk_matmul_split_k(const gk_config* conf, const void* a, const void* b, const
                       const gk_transforms* transforms, const gk_epilogue* epilogue, void* workspace,
                       size_t workspace_bytes, void* stream);
 
+/* Whether `stream` (NULL: the default stream) is being captured into a HIP graph, and the id of that capture: a launch that is
+ * captured needs a workspace that lives as long as the graph and is not in use by launches outside of it, which only
+ * the stream that is launched on can tell. */
+int gk_stream_capture(void* stream, int32_t* capturing, uint64_t* id);
+
 /* gk_matmul_split_k for callers that cannot allocate device memory.  No counterpart in the reference; it is
  * for code under HIP graph capture, tight serving loops and harnesses that forbid hipMalloc.  Same
  * arguments and same results, bit for bit, as gk_matmul_split_k, without the workspace: the partial tiles

@@ -1,6 +1,8 @@
 """The K-split kernel kind: few output tiles, long K.  The K slices of a tile run as workgroups of one launch,
 leave their partial tiles in a workspace and the last one to arrive adds them in slice order: results are
 compared by norm against float64, bit for bit between runs, and exactly on data whose sums are exact."""
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -313,3 +315,103 @@ def test_captured_products_keep_a_workspace_of_their_own(gpu):
             gk.mul_(Z, X, Y)
             torch.cuda.synchronize()
             assert torch.equal(C, ref) and torch.equal(Z, (X.double() @ Y.double()).float())
+
+
+def _integers(rs, shape, dtype):
+    return gk.colmajor(np.asfortranarray(rs.randint(-4, 5, size=shape).astype(dtype)))
+
+
+def _kept_for_graphs():
+    """Workspaces of captures whose memory torch does not keep for the graph."""
+    return sys.modules["gemmkernels.matmul"]._recorded
+
+
+def _replayed(replay, D, ref, stream):
+    """Every replay gives the eager result, with eager products on the same stream (which grow its workspace) and fresh
+    tensors full of NaN (in whatever memory the capture gave back) between the replays."""
+    rs = np.random.RandomState(5)
+    for turn in range(4):
+        X, Y = _integers(rs, (64 * (turn + 1), 8192), np.float16), _integers(rs, (8192, 64 * (turn + 1)), np.float16)
+        Z = gk.colmajor_empty((X.shape[0], Y.shape[1]), torch.float32)
+        junk = [torch.full((n,), float("nan"), device="cuda") for n in (256, 1 << 10, 1 << 16, 1 << 18, 1 << 20, 1 << 21)]
+        D.fill_(float("nan"))
+        torch.cuda.synchronize()
+        replay()
+        gk.matmatmul_plan(Z, "N", "N", X, Y, 1.0, 0.0)(stream)
+        torch.cuda.synchronize()
+        assert torch.equal(D, ref), turn
+        assert torch.equal(Z, (X.double() @ Y.double()).float()), turn
+        assert all(bool(torch.isnan(j).all()) for j in junk), turn
+        del junk
+
+
+def test_a_captured_launch_on_a_forked_stream(gpu):
+    """The launch goes to a side stream that is part of the capture, not to torch's current one: its workspace is allocated
+    and cleared on that stream, and what the current stream allocates meanwhile is not that memory."""
+    rs = np.random.RandomState(1)
+    A, B = _integers(rs, (1024, 4096), np.float16), _integers(rs, (4096, 64), np.float16)
+    D, ref = gk.colmajor_empty((1024, 64), torch.float32), gk.colmajor_empty((1024, 64), torch.float32)
+    gk.mul_(ref, A, B)
+    torch.cuda.synchronize()
+    side, graph, busy = torch.cuda.Stream(), torch.cuda.CUDAGraph(), torch.ones(1 << 22, device="cuda")
+    p = gk.matmatmul_plan(D, "N", "N", A, B, 1.0, 0.0)
+    with torch.cuda.graph(graph):
+        main = torch.cuda.current_stream()
+        side.wait_stream(main)
+        for _ in range(3):
+            busy.mul_(1.0)                      # (the current stream is behind the side stream)
+        p(side.cuda_stream)
+        others = [torch.full((1 << 19,), 7.0, device="cuda") for _ in range(4)]
+        main.wait_stream(side)
+    assert not any(stream == side.cuda_stream for _, stream in _kept_for_graphs())
+    _replayed(graph.replay, D, ref, side.cuda_stream)
+    assert all(bool((o == 7.0).all()) for o in others)
+
+
+def test_an_eager_launch_beside_a_capture(gpu):
+    """torch's current stream is captured, the launch goes to a stream that is not: it runs at once, on that stream's own workspace."""
+    rs = np.random.RandomState(2)
+    A, B = _integers(rs, (1024, 4096), np.float16), _integers(rs, (4096, 64), np.float16)
+    D, ref = gk.colmajor_empty((1024, 64), torch.float32), gk.colmajor_empty((1024, 64), torch.float32)
+    gk.mul_(ref, A, B)
+    other, graph, x = torch.cuda.Stream(), torch.cuda.CUDAGraph(), torch.zeros(64, device="cuda")
+    p = gk.matmatmul_plan(D, "N", "N", A, B, 1.0, 0.0)
+    p(other.cuda_stream)
+    D.fill_(float("nan"))
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, capture_error_mode="relaxed"):
+        x.add_(1.0)
+        p(other.cuda_stream)
+    other.synchronize()
+    assert torch.equal(D, ref)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(D, ref) and bool((x == 1.0).all())
+
+
+def test_a_graph_captured_without_torch(gpu):
+    """hipStreamBeginCapture by hand: torch's allocator hands the memory of such a capture out again, the workspace is kept."""
+    import ctypes
+    with open("/proc/self/maps") as maps:
+        hip = ctypes.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))
+
+    def check(status):
+        assert status == 0, status
+    rs = np.random.RandomState(3)
+    A, B = _integers(rs, (1024, 4096), np.float16), _integers(rs, (4096, 64), np.float16)
+    D, ref = gk.colmajor_empty((1024, 64), torch.float32), gk.colmajor_empty((1024, 64), torch.float32)
+    gk.mul_(ref, A, B)
+    stream = torch.cuda.Stream()
+    graph, instance = ctypes.c_void_p(), ctypes.c_void_p()
+    p = gk.matmatmul_plan(D, "N", "N", A, B, 1.0, 0.0)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        check(hip.hipStreamBeginCapture(ctypes.c_void_p(stream.cuda_stream), 2))        # relaxed
+        p()
+        check(hip.hipStreamEndCapture(ctypes.c_void_p(stream.cuda_stream), ctypes.byref(graph)))
+    assert len(_kept_for_graphs()[torch.cuda.current_device(), stream.cuda_stream]) == 1
+    check(hip.hipGraphInstantiate(ctypes.byref(instance), graph, None, None, ctypes.c_size_t(0)))
+    _replayed(lambda: check(hip.hipGraphLaunch(instance, ctypes.c_void_p(stream.cuda_stream))), D, ref, stream.cuda_stream)
+    torch.cuda.synchronize()
+    check(hip.hipGraphExecDestroy(instance))
+    check(hip.hipGraphDestroy(graph))
