@@ -1075,6 +1075,22 @@ int split_k_slices(int tiles, int k_tiles, const gk_shape& block) {
   return slices;
 }
 
+// Whether a K-split launch of the configuration can be split at all, whatever its hooks: K-split instances exist for the
+// small tiles that skinny products run; a large tile runs unsplit.  The bounds-checked kernel takes its K range from the
+// launch arguments, the aligned kernels have instances of their own (FUSED levels 0 .. 3 of the kernel).
+bool has_split_k_instance(const gk_config* conf) {
+  gk::InstanceKey key;
+  if (make_key(conf, nullptr, nullptr, &key) != GK_OK) return false;
+  if (key.family == gk::FAMILY_MFMA_CHECKED) return true;
+  if (key.family != gk::FAMILY_MFMA) return false;
+  const gk::GemmArgs none{};
+  gk::InstanceInfo info;
+  hipError_t err = hipSuccess;
+  for (key.fused = 0; key.fused <= 3; ++key.fused)
+    if (gk::family_mfma_splitk(key, none, dim3(1), nullptr, 0, &info, &err)) return true;
+  return false;
+}
+
 }  // namespace
 
 namespace gk_internal {
@@ -1094,9 +1110,7 @@ int launch_split_k(const gk_config* conf, const void* a, const void* b, const vo
   const int kt = (conf->matmul_shape.K + conf->block_shape.K - 1) / conf->block_shape.K;   // bounds-checked layouts: the last tile may be partial
   int slices = split_k_slices(tiles, kt, conf->block_shape);
   gk::InstanceInfo sk_info;
-  // K-split instances exist for the small tiles that skinny products run; anything else (a large tile,
-  // generic A / B hooks) runs unsplit.  The bounds-checked
-  // kernel takes its K range from the launch arguments, the aligned kernels have instances of their own.
+  // (a tile or hooks without a K-split instance: unsplit, see has_split_k_instance)
   gk::FamilyFn sk_fn = L.key.family == gk::FAMILY_MFMA_CHECKED ? fn : gk::family_mfma_splitk;
   const int per = slices > 1 ? (kt + slices - 1) / slices : kt;
   slices = (kt + per - 1) / per;           // no empty slice: every slice arrives at its tile's counter
@@ -1139,7 +1153,7 @@ int gk_split_k_workspace_size(const gk_config* conf, size_t* bytes) {
   const long long tiles = (long long)((g.M + b.M - 1) / b.M) * ((g.N + b.N - 1) / b.N);
   const int kt = (g.K + b.K - 1) / b.K;
   const long long slices = split_k_slices((int)(tiles > (1 << 30) ? (1 << 30) : tiles), kt, b);
-  if (slices < 2) { *bytes = 0; return GK_OK; }      // runs unsplit
+  if (slices < 2 || !has_split_k_instance(conf)) { *bytes = 0; return GK_OK; }      // runs unsplit
   *bytes = kSplitCounterBytes + (size_t)tiles * (size_t)slices * b.M * b.N * sizeof(float);
   return GK_OK;
 }

@@ -358,3 +358,19 @@ def test_k_slices_that_fit_the_static_workspace_at_1024_deep_fit_it(tiles, K):
     need = ctypes.c_size_t()
     assert _lib.lib().gk_split_k_workspace_size(ctypes.byref(cconf), ctypes.byref(need)) == _lib.GK_OK
     assert need.value <= _lib.lib().gk_split_k_noalloc_capacity()
+
+
+@pytest.mark.parametrize("dims,tile,split", [((4096, 4096, 4096), (256, 256, 64), False), ((2048, 2048, 2048), (128, 128, 32), False),
+                                             ((2048, 1024, 4096), (128, 128, 64), True), ((512, 512, 4096), (64, 64, 64), True), ((512, 512, 4096), (64, 64, 32), True)])
+def test_only_a_product_that_is_split_needs_a_workspace(dims, tile, split):
+    """A tile without K-split instances runs unsplit: no workspace to allocate, or to clear in every replay of a graph."""
+    import ctypes
+    from gemmkernels import _lib, configs
+    M, N, K = dims
+    conf = configs.mfma_config(M, N, K, block_shape=tile)
+    if tile == (64, 64, 32):
+        import dataclasses
+        conf = dataclasses.replace(conf, warps_per_block=1, compute_warp=type(conf.compute_warp)(M=64, N=64, K=conf.compute_warp.K))
+    need = ctypes.c_size_t()
+    assert _lib.lib().gk_split_k_workspace_size(ctypes.byref(conf.to_c(M, K, M, M)), ctypes.byref(need)) == _lib.GK_OK
+    assert (need.value > 0) == split
