@@ -1075,6 +1075,32 @@ int split_k_slices(int tiles, int k_tiles, const gk_shape& block) {
   return slices;
 }
 
+// How a launch of the configuration is split, from the configuration alone: the workspace that a caller brings has no say in
+// the order of a sum.  A product whose last K tile runs outside the pipeline (see needs_tail_tile) takes as many slices
+// as leave partial tiles that the static workspace holds: it is refused nowhere, and gk_matmul_split_k and
+// gk_matmul_split_k_noalloc give the same bits.
+struct SplitK {
+  int slices, per;        // slices, K tiles of each
+  size_t bytes;           // counters and partial tiles (0: one slice, unsplit)
+};
+
+SplitK split_k_plan(const gk_config* conf, int tiles, bool tail_tile) {
+  const gk_shape& block = conf->block_shape;
+  const int k_tiles = (conf->matmul_shape.K + block.K - 1) / block.K;   // bounds-checked layouts: the last tile may be partial
+  const size_t slice_bytes = (size_t)tiles * block.M * block.N * sizeof(float);
+  int slices = split_k_slices(tiles, k_tiles, block);
+  if (tail_tile && slices > 1) {
+    const size_t fit = (gk_split_k_noalloc_capacity() - kSplitCounterBytes) / slice_bytes;
+    if ((size_t)slices > fit) slices = (int)fit;
+  }
+  SplitK plan{1, k_tiles, 0};
+  if (slices < 2) return plan;
+  plan.per = (k_tiles + slices - 1) / slices;
+  plan.slices = (k_tiles + plan.per - 1) / plan.per;      // no empty slice: every slice arrives at its tile's counter
+  plan.bytes = kSplitCounterBytes + (size_t)plan.slices * slice_bytes;
+  return plan;
+}
+
 // Whether a K-split launch of the configuration can be split at all, whatever its hooks: K-split instances exist for the
 // small tiles that skinny products run; a large tile runs unsplit.  The bounds-checked kernel takes its K range from the
 // launch arguments, the aligned kernels have instances of their own (FUSED levels 0 .. 3 of the kernel).
@@ -1106,32 +1132,26 @@ int launch_split_k(const gk_config* conf, const void* a, const void* b, const vo
     return fail(GK_ERR_UNSUPPORTED, "the K-split kernel runs the real MFMA operator");
   gk::FamilyFn fn = family_fn(L.key);
   hipError_t err = hipSuccess;
-  const int tiles = L.gx * L.gy;
-  const int kt = (conf->matmul_shape.K + conf->block_shape.K - 1) / conf->block_shape.K;   // bounds-checked layouts: the last tile may be partial
-  int slices = split_k_slices(tiles, kt, conf->block_shape);
+  const int tiles = L.args.nbm * L.args.nbn;      // (the grid of a tiled walk may hold more workgroups than there are tiles)
+  const SplitK plan = split_k_plan(conf, tiles, L.ragged);
   gk::InstanceInfo sk_info;
   // (a tile or hooks without a K-split instance: unsplit, see has_split_k_instance)
   gk::FamilyFn sk_fn = L.key.family == gk::FAMILY_MFMA_CHECKED ? fn : gk::family_mfma_splitk;
-  const int per = slices > 1 ? (kt + slices - 1) / slices : kt;
-  slices = (kt + per - 1) / per;           // no empty slice: every slice arrives at its tile's counter
-  const size_t counters = kSplitCounterBytes;
-  bool split = slices > 1 && sk_fn && sk_fn(L.key, L.args, dim3(1), nullptr, 0, &sk_info, &err);
-  // a product whose last K tile runs outside the pipeline does not insist on a workspace: it is the same launch unsplit
-  if (split && L.ragged && (!workspace || workspace_bytes < counters + (size_t)tiles * slices * conf->block_shape.M * conf->block_shape.N * sizeof(float) ||
-                            ((uintptr_t)workspace & 15u) != 0)) split = false;
+  bool split = plan.slices > 1 && sk_fn && sk_fn(L.key, L.args, dim3(1), nullptr, 0, &sk_info, &err);
+  // a product whose last K tile runs outside the pipeline does not insist on a workspace: without it, it is the launch unsplit
+  if (L.ragged && (!workspace || workspace_bytes < plan.bytes || ((uintptr_t)workspace & 15u) != 0)) split = false;
   if (split) {
-    if ((size_t)tiles * sizeof(unsigned) > counters)
-      return fail(GK_ERR_INVALID_ARGUMENT, "a K-split launch of %d tiles has no room for its arrival counters (%zu bytes)", tiles, counters);
-    const size_t need = counters + (size_t)tiles * slices * conf->block_shape.M * conf->block_shape.N * sizeof(float);
-    if (!workspace || workspace_bytes < need)
+    if ((size_t)tiles * sizeof(unsigned) > kSplitCounterBytes)
+      return fail(GK_ERR_INVALID_ARGUMENT, "a K-split launch of %d tiles has no room for its arrival counters (%zu bytes)", tiles, kSplitCounterBytes);
+    if (!workspace || workspace_bytes < plan.bytes)
       return fail(GK_ERR_INVALID_ARGUMENT, "the K-split launch needs a workspace of %zu bytes (%d tiles x %d slices of %d x %d floats); %s holds %zu",
-                  need, tiles, slices, conf->block_shape.M, conf->block_shape.N, whose, workspace_bytes);
+                  plan.bytes, tiles, plan.slices, conf->block_shape.M, conf->block_shape.N, whose, workspace_bytes);
     if (((uintptr_t)workspace & 15u) != 0) return fail(GK_ERR_ALIGNMENT, "the workspace is not aligned to 16 bytes");
     gk::GemmArgs sk = L.args;
-    sk.k_steps = per; sk.k_slices = slices;
+    sk.k_steps = plan.per; sk.k_slices = plan.slices;
     sk.ws_counters = (unsigned*)workspace;
-    sk.ws_partials = (char*)workspace + counters;
-    sk_fn(L.key, sk, dim3((unsigned)L.gx, (unsigned)L.gy, (unsigned)slices), (hipStream_t)stream, 1, &sk_info, &err);
+    sk.ws_partials = (char*)workspace + kSplitCounterBytes;
+    sk_fn(L.key, sk, dim3((unsigned)L.gx, (unsigned)L.gy, (unsigned)plan.slices), (hipStream_t)stream, 1, &sk_info, &err);
     if (err != hipSuccess) return fail(GK_ERR_HIP, "HIP launch of %s failed: %s", sk_info.name, hipGetErrorString(err));
     return GK_OK;
   }
@@ -1151,10 +1171,9 @@ int gk_split_k_workspace_size(const gk_config* conf, size_t* bytes) {
   const gk_shape& b = conf->block_shape;
   if (g.M <= 0 || g.N <= 0 || g.K <= 0 || b.M <= 0 || b.N <= 0 || b.K <= 0) return fail(GK_ERR_INVALID_ARGUMENT, "shapes must be positive");
   const long long tiles = (long long)((g.M + b.M - 1) / b.M) * ((g.N + b.N - 1) / b.N);
-  const int kt = (g.K + b.K - 1) / b.K;
-  const long long slices = split_k_slices((int)(tiles > (1 << 30) ? (1 << 30) : tiles), kt, b);
-  if (slices < 2 || !has_split_k_instance(conf)) { *bytes = 0; return GK_OK; }      // runs unsplit
-  *bytes = kSplitCounterBytes + (size_t)tiles * (size_t)slices * b.M * b.N * sizeof(float);
+  gk::InstanceKey key;
+  const bool tail_tile = make_key(conf, nullptr, nullptr, &key) == GK_OK && key.family == gk::FAMILY_MFMA && ragged_fast_path(conf) && needs_tail_tile(conf);
+  *bytes = has_split_k_instance(conf) ? split_k_plan(conf, (int)(tiles > (1 << 30) ? (1 << 30) : tiles), tail_tile).bytes : 0;
   return GK_OK;
 }
 

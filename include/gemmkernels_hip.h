@@ -280,7 +280,10 @@ int gk_matmul(const gk_config* conf, const void* a, const void* b, const void* c
  * so that launches of different shapes find their counters in the same place -- which every launch leaves
  * at zero again: one workspace serves any number of launches of any products one after the other; launches
  * that overlap in time (two streams) need a workspace each.  A launch that faulted or was aborted may leave
- * counters behind: zero the first 2048 bytes again before the workspace is used after such a failure. */
+ * counters behind: zero the first 2048 bytes again before the workspace is used after such a failure.  A launch that is
+ * split and finds its workspace NULL or smaller than gk_split_k_workspace_size says is refused with
+ * GK_ERR_INVALID_ARGUMENT, except a product of bounds-checked layouts whose last K tile is partial (or holds a vector that
+ * reaches over the end of an operand), which then runs unsplit: another order of its sum, so other last bits. */
 int gk_split_k_workspace_size(const gk_config* conf, size_t* bytes);
 int gk_matmul_split_k(const gk_config* conf, const void* a, const void* b, const void* c, void* d,
                       const gk_transforms* transforms, const gk_epilogue* epilogue, void* workspace,
@@ -296,7 +299,8 @@ int gk_stream_capture(void* stream, int32_t* capturing, uint64_t* id);
  * arguments and same results, bit for bit, as gk_matmul_split_k, without the workspace: the partial tiles
  * meet in a device array that is part of the library (gk_split_k_noalloc_capacity() bytes, 32 MiB, on every
  * GPU the library is used on, for the life of the process).  A launch that needs more is refused with
- * GK_ERR_INVALID_ARGUMENT and a message that names both sizes; nothing is allocated or freed by the call,
+ * GK_ERR_INVALID_ARGUMENT and a message that names both sizes (a product with a partial last K tile, see above, is cut into
+ * as many slices as fit instead, here and in gk_matmul_split_k); nothing is allocated or freed by the call,
  * on the device or through any library.  All calls on one GPU share the array: calls that overlap in time
  * (two streams, two host threads) race on it and must be serialised by the caller.  The first call on a
  * device asks the runtime for the array's address, which may load the library's device code at that moment:

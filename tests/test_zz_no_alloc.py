@@ -63,6 +63,42 @@ def test_two_calls_in_a_row_the_second_smaller(gpu):
     _both_ways(4096, 64, 4096, (64, 64, 64), 7600)
 
 
+def test_a_partial_last_k_tile_at_the_capacity_limit(gpu):
+    """64 tiles of 128 x 128 in eight slices and the counters would be 2 KiB more than the static array holds: a product with
+    a partial last K tile is cut into fewer slices by both entry points, and gives the same bits."""
+    from gemmkernels import Float16, Float32, Layout, NT, Operator
+    lib = _lib.lib()
+    M, N, K = 1024, 1016, 8200
+    conf = gk.get_config(gemm_shape=NT(M=M, N=N, K=K), block_shape=NT(M=128, N=128, K=64), warps_per_block=4, compute_warp=NT(M=64, N=64, K=16),
+                         operator=Operator.MFMAOp[32, 32, 16, Float16, Float32],
+                         global_a_layout=Layout.ColMajor[Float16], global_b_layout=Layout.ColMajor[Float16],
+                         global_c_layout=Layout.Zero[Float32], global_d_layout=Layout.ColMajor[Float32],
+                         shared_a_layout=Layout.Padded[Layout.UnsafeAlignedColMajor[Float16], 8], shared_b_layout=Layout.Padded[Layout.UnsafeAlignedColMajor[Float16], 8],
+                         shared_c_layout=Layout.Zero[Float32], shared_d_layout=Layout.UnsafeAlignedColMajor[Float32], is_a_col_major=True, is_b_col_major=True)
+    cconf = conf.to_c(M, K, M, M)
+    need = ctypes.c_size_t()
+    assert lib.gk_split_k_workspace_size(ctypes.byref(cconf), ctypes.byref(need)) == _lib.GK_OK
+    assert 0 < need.value <= lib.gk_split_k_noalloc_capacity()
+    a, b = rng.matrix("upm1_f16", 7701, (M, K)), rng.matrix("upm1_f16", 7702, (K, N))
+    A, B = gk.colmajor(a), gk.colmajor(b)
+    out = []
+    for size in (need.value, lib.gk_split_k_noalloc_capacity() + (8 << 20), None, 0):     # the bound, more than it, the static array, none
+        D = gk.colmajor_empty((M, N), torch.float32)
+        D.fill_(float("nan"))
+        args = (ctypes.byref(cconf), A.data_ptr(), B.data_ptr(), None, D.data_ptr(), None, None)
+        if size is None:
+            rc = lib.gk_matmul_split_k_noalloc(*args, None)
+        else:
+            ws = torch.zeros(max(size, 16), dtype=torch.uint8, device="cuda")
+            torch.cuda.synchronize()
+            rc = lib.gk_matmul_split_k(*args, ws.data_ptr() if size else None, size, None)
+        assert rc == _lib.GK_OK, _lib.last_error()
+        torch.cuda.synchronize()
+        out.append(gk.to_numpy(D))
+        assert oracle.rel_frobenius(out[-1], a.astype(np.float64) @ b.astype(np.float64)) <= 1e-3
+    assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32)) and np.array_equal(out[0].view(np.uint32), out[2].view(np.uint32))
+
+
 def test_a_product_beyond_the_static_workspace_is_refused(gpu):
     lib = _lib.lib()
     M, N, K = 1024, 1024, 32768          # 64 tiles of 128 x 128 in 8 slices: 32 MiB of partial tiles plus the counters
