@@ -1008,10 +1008,13 @@ int prepare_launch(const gk_config* conf, const void* a, const void* b, const vo
       return fail(GK_ERR_DIMENSION_MISMATCH, "ldb = %lld is smaller than the leading extent of B", args.ldb);
     if (conf->global_d_layout.kind != GK_LAYOUT_GETT && (args.ldd < em || (args.c_mode && args.ldc < em)))
       return fail(GK_ERR_DIMENSION_MISMATCH, "ldc/ldd is smaller than M");
-    // the kernels keep per-lane tile offsets in 32 bits
+    // the kernels keep per-lane tile offsets in 32 bits (floating-point FPUOp on the matrix instructions: in 64, of 31-bit
+    // leading dimensions, so that its larger tiles take what the 64 x 64 tile takes)
+    const bool wide_offsets = key.family == gk::FAMILY_FPU && (key.variant & ~2) == 0 && (key.acc_dtype == GK_F32 || key.acc_dtype == GK_F64);
+    if (wide_offsets && (args.lda >= (1ll << 31) || args.ldb >= (1ll << 31))) return fail(GK_ERR_UNSUPPORTED, "leading dimension of 2^31 elements or more");
     const long long span_a = (long long)(a_row ? conf->block_shape.M : conf->block_shape.K) * args.lda * 2;
     const long long span_b = (long long)(b_row ? conf->block_shape.K : conf->block_shape.N) * args.ldb * 2;
-    if (span_a + 2 * args.plane_a >= (1ll << 31) || span_b >= (1ll << 31))
+    if (!wide_offsets && (span_a + 2 * args.plane_a >= (1ll << 31) || span_b >= (1ll << 31)))
       return fail(GK_ERR_UNSUPPORTED, "leading dimension too large for 32-bit tile offsets");
   }
 

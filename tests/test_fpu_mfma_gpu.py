@@ -116,3 +116,18 @@ def test_zero_alpha_reads_neither_a_nor_b(gpu):
         gk.matmatmul_(C, "N", "N", A, B, 0.0, 2.0)
         torch.cuda.synchronize()
         assert np.array_equal(gk.to_numpy(C), 2 * c)
+
+
+def test_leading_dimensions_beyond_32_bits_of_tile_offsets(gpu):
+    """128 rows of 2^23 Float32 lie 4 GiB apart: the offsets in a tile are 64 bits wide, so the 128 x 128 tile takes every
+    leading dimension that the 64 x 64 tile takes."""
+    M, N, K, ld = 128, 70, 37, (1 << 23) + 3
+    a, b = operand((K, M), np.float32, 71), operand((K, N), np.float32, 72)
+    A = torch.empty(ld * (M - 1) + K, device="cuda").as_strided((K, M), (1, ld))
+    A.copy_(torch.from_numpy(np.ascontiguousarray(a)))
+    for tile in TILES["f32"][:3]:
+        conf = config(M, N, K, True, False, "f32", tile, True)
+        D = gk.colmajor_empty((M, N), torch.float32)
+        gk.matmul(conf, A, gk.colmajor(b), None, D)
+        torch.cuda.synchronize()
+        assert np.array_equal(gk.to_numpy(D), helpers.run_oracle(conf, a, b, None, (M, N), d_dtype=np.float32)), tile
