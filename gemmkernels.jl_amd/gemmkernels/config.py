@@ -220,12 +220,16 @@ def default_block_shape(operator, gemm_shape, tile_sized: bool = True, gett: boo
     return NT(M=best[0], N=best[1], K=best[2])
 
 
-def split_k_block_shape(M, N, K) -> Optional[NT]:
+def split_k_block_shape(M, N, K, widest_ld=0) -> Optional[NT]:
     """The tile of a 16-bit product that is worth cutting into slices of K (``Kernel.matmul_split_k``), or None: few output
     tiles, which alone leave CUs idle, and a long K.  Measured against the best tile unsplit: 4096 x 64 x 4096 14.1 us
     against 22.2, 300 x 500 x 4000 13.0 against 23.5, 64 x 64 x 8000 11.4 against 39, 2000 x 100 x 1500 11.6 against 12.3,
     256 x 256 x 1024 8.9 against 7.1; with more than 128 tiles, which leave two or three slices, 1024 x 1024 x 4096 22.1
-    against 23.6, 700 x 900 x 3001 18.6 against 20.9, 1000 x 1000 x 2000 17.8 against 16.2."""
+    against 23.6, 700 x 900 x 3001 18.6 against 20.9, 1000 x 1000 x 2000 17.8 against 16.2.  ``widest_ld``: the larger leading
+    dimension of the operands whose rows are the k of a tile; the kernel keeps the offsets in a tile in 32 bits, so 64
+    rows of 2^24 elements are left to a tile with fewer."""
+    if 64 * widest_ld * 2 >= 1 << 31:
+        return None
     tiles = -(-M // 64) * -(-N // 64)
     return NT(M=64, N=64, K=64) if K >= 1280 and tiles <= 128 or K >= 3000 and tiles <= 256 else None
 

@@ -481,7 +481,9 @@ def create_config(A: DType, sizeA, stridesA, transA: bool, B: DType, sizeB, stri
     # one), and the operands it does not divide get the bounds-checked layouts, as the reference's rule says.
     edge_ok = not zeroAlpha and (((k if transA else m) >= 8 and (n if transB else k) >= 8) if use_mfma
                                  else compute_type in (Float16, Float32, Float64))
-    block_shape = split_k_block_shape(m, n, k) if use_mfma and edge_ok else None
+    block_shape = None
+    if use_mfma and edge_ok:
+        block_shape = split_k_block_shape(m, n, k, max(0 if transA else stridesA[1], stridesB[1] if transB else 0))
     if block_shape is None:
         block_shape = default_block_shape(operator, NT(M=m, N=n, K=k), tile_sized=not edge_ok, a_kmajor=transA, b_kmajor=not transB)
     global_a_layout, global_b_layout, global_c_layout, global_d_layout = layouts_for(block_shape)
@@ -534,7 +536,7 @@ def _single_plan(C, tA: bool, tB: bool, A, B, alpha, beta, wmma=None) -> Plan:
         # ordered, so the result is the same on every run, like the reference's mul!.
         bs, ms = conf.block_shape, conf.matmul_shape
         tiles = -(-ms.M // bs.M) * -(-ms.N // bs.N)
-        if split_k_block_shape(ms.M, ms.N, ms.K) is not None or tiles <= 256 and ms.K >= 2048:
+        if bs == split_k_block_shape(ms.M, ms.N, ms.K) or tiles <= 256 and ms.K >= 2048:
             kernel = Kernel.matmul_split_k
     p = plan(conf, A, B, C, C, transform_shared_to_regs_a=ta, transform_shared_to_regs_c=tc, kernel=kernel)
     p.kernel_names = (kernel_name(conf, kernel, dict(transform_shared_to_regs_a=ta, transform_shared_to_regs_c=tc)),)

@@ -753,7 +753,8 @@ function create_config(A::Type, sizeA::Dims, stridesA::Dims, transA::Bool,
     # the sizes, and the operands it does not divide get the bounds-checked layouts, as the reference's rule says.
     # (floating-point FPUOp takes any size and alignment on every tile)
     edge_ok = !zeroAlpha && (use_mfma ? (transA ? k : m) >= 8 && (transB ? n : k) >= 8 : nameof(compute_type) in (:Float16, :Float32, :Float64))
-    block_shape = use_mfma && edge_ok && worth_splitting(m, n, k) ? (M = 64, N = 64, K = 64) :
+    widest_ld = max(transA ? 0 : stridesA[2], transB ? stridesB[2] : 0)
+    block_shape = use_mfma && edge_ok && worth_splitting(m, n, k, widest_ld) ? (M = 64, N = 64, K = 64) :
                   default_block_shape(operator, (M = m, N = n, K = k); tile_sized = !edge_ok)
     ga, gb, gc, gd = layouts_for(block_shape)
     if !edge_ok && any(Layout.is_checked, (ga, gb, gc, gd))
@@ -769,8 +770,9 @@ function create_config(A::Type, sizeA::Dims, stridesA::Dims, transA::Bool,
     (conf, compute_type, select_kernel(ga, gb))
 end
 
-# a 16-bit product with few 64 x 64 output tiles and a long K runs on slices of K (the sizes: split_k_block_shape of the Python package)
-worth_splitting(m, n, k) = (tiles = cld(m, 64) * cld(n, 64); k >= 1280 && tiles <= 128 || k >= 3000 && tiles <= 256)
+# a 16-bit product with few 64 x 64 output tiles and a long K runs on slices of K (the sizes: split_k_block_shape of the Python package),
+# unless its operands' 64 rows of k lie further apart than 32-bit offsets reach
+worth_splitting(m, n, k, widest_ld = 0) = (tiles = cld(m, 64) * cld(n, 64); 64 * widest_ld * 2 < 2^31 && (k >= 1280 && tiles <= 128 || k >= 3000 && tiles <= 256))
 
 is_aligned_16(x) = UInt(devptr(x)) % 16 == 0
 
@@ -796,7 +798,7 @@ function matmatmul!(C, transA::Char, transB::Char, A, B, alpha::Number, beta::Nu
     if Operator.is_mfma(conf.operator)
         # few output tiles and a long K loop: K slices as workgroups of one launch (ordered sum: same bits every run)
         bs, ms = conf.block_shape, conf.matmul_shape
-        if worth_splitting(ms.M, ms.N, ms.K) || cld(ms.M, bs.M) * cld(ms.N, bs.N) <= 256 && ms.K >= 2048
+        if bs == (M = 64, N = 64, K = 64) && worth_splitting(ms.M, ms.N, ms.K) || cld(ms.M, bs.M) * cld(ms.N, bs.N) <= 256 && ms.K >= 2048
             kernel = Kernel.matmul_split_k
         end
     end

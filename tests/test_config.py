@@ -374,3 +374,19 @@ def test_only_a_product_that_is_split_needs_a_workspace(dims, tile, split):
     need = ctypes.c_size_t()
     assert _lib.lib().gk_split_k_workspace_size(ctypes.byref(conf.to_c(M, K, M, M)), ctypes.byref(need)) == _lib.GK_OK
     assert (need.value > 0) == split
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+def test_wide_leading_dimensions_keep_a_tile_that_takes_them(ta, tb):
+    """The kernels keep the offsets in a tile in 32 bits: an operand whose tile rows are k runs on tiles of 32 k from 2^24
+    elements per row on, as a product with few tiles did before it was cut into slices on 64 x 64 x 64 tiles."""
+    M, N, K = 256, 64, 4096
+
+    def block(lda, ldb):
+        conf, _, _ = create_config(Float16, (K, M) if ta else (M, K), (1, lda), ta, Float16, (N, K) if tb else (K, N), (1, ldb), tb,
+                                          Float32, (M, N), (1, M), float, False, float, True)
+        return conf.block_shape
+    split, narrow = NT(M=64, N=64, K=64), NT(M=64, N=64, K=32)
+    assert block(1 << 23, 1 << 23) == split
+    assert block(1 << 24, 4096) == (split if ta else narrow)
+    assert block(4096, 1 << 24) == (narrow if tb else split)
