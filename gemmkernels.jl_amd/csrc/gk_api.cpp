@@ -247,6 +247,21 @@ int make_key_as_configured(const gk_config* c, const gk_transforms* t, const gk_
       key->fused = 2;
     if (c->global_a_layout.eltype != GK_F16) key->fused = 2;   // level 1 is compiled for FP16 only
   }
+  if (key->fused && t && key->family == gk::FAMILY_FPU) {
+    // floating-point FPUOp: level 1 is compiled for at most one scale on A, on B and on C, level 2 for any lists
+    auto one_scale = [&](int h0, int h1) {
+      int n = 0, scales = 0;
+      for (int h : {h0, h1})
+        for (int i = 0; i < t->hook[h].n_ops && i < GK_MAX_OPS; ++i) {
+          n += t->hook[h].ops[i].kind != GK_T_IDENTITY;
+          scales += t->hook[h].ops[i].kind == GK_T_SCALE;
+        }
+      return n == 0 || (n == 1 && scales == 1);
+    };
+    if (!one_scale(GK_HOOK_GLOBAL_TO_SHARED_A, GK_HOOK_SHARED_TO_REGS_A) || !one_scale(GK_HOOK_GLOBAL_TO_SHARED_B, GK_HOOK_SHARED_TO_REGS_B) ||
+        !one_scale(GK_HOOK_GLOBAL_TO_SHARED_C, GK_HOOK_SHARED_TO_REGS_C))
+      key->fused = 2;
+  }
   if (key->fused && !t && c->global_a_layout.eltype != GK_F16 && (key->family == gk::FAMILY_MFMA || key->family == gk::FAMILY_GETT))
     key->fused = 2;
   return GK_OK;
@@ -406,6 +421,14 @@ void make_args(const gk_config* c, const void* a, const void* b, const void* cc,
   };
   single_scale(GK_HOOK_GLOBAL_TO_SHARED_A, GK_HOOK_SHARED_TO_REGS_A, &args->fast_scale_a, &args->scale_a);
   single_scale(GK_HOOK_GLOBAL_TO_SHARED_B, GK_HOOK_SHARED_TO_REGS_B, &args->fast_scale_b, &args->scale_b);
+  if (c->op.kind == GK_OP_FPU) {
+    // floating-point FPUOp at hook level 1: the one scale of A, of B and of C, looked up here (in the kernel a chain of
+    // dependent loads of arguments stands in front of the first load of a tile: Float32 512^3 9.3 us, so 8.0)
+    auto scale_of = [&](int h0, int h1) { return args->t[h0].n > 0 ? args->t[h0].p0[0] : args->t[h1].n > 0 ? args->t[h1].p0[0] : 1.0f; };
+    args->scale_a = scale_of(GK_HOOK_GLOBAL_TO_SHARED_A, GK_HOOK_SHARED_TO_REGS_A);
+    args->scale_b = scale_of(GK_HOOK_GLOBAL_TO_SHARED_B, GK_HOOK_SHARED_TO_REGS_B);
+    args->acc_pre_scale = args->c_mode != 0 ? scale_of(GK_HOOK_GLOBAL_TO_SHARED_C, GK_HOOK_SHARED_TO_REGS_C) : 1.0f;
+  }
   auto copy_dim = [](const gk_gett_dim& s, gk::GettDim& d) {
     d.nmodes = s.nmodes;
     for (int i = 0; i < GK_MAX_MODES; ++i) {

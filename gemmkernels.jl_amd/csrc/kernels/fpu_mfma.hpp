@@ -37,6 +37,13 @@
 // back and moved into place.  The last K tile, when it is partial, is fetched the same way along k with zeros beyond K,
 // waits in registers for the end of the loop, and only its steps that hold values are multiplied (moved and zeroed inside
 // the loop instead: 3001 x 3003 x 2999 557 us).
+//
+// Hooks.  What a BLAS-level call asks for -- a factor on A, one on C -- is a multiplication in the loads' way to LDS and one of C
+// before the loop (level 1: the K loop of the plain kernel); lists of operations run over all vectors of a tile at once, in
+// front of its first MFMA (level 2).  One instance for both, whose lists were indexed at run time per vector, had the
+// argument block in scratch memory and up to 259 spilled registers.  From it to these: factors, Float64 1000^3 'T','N' 49.4 ->
+// 42.9 us, Float32 512^3 8.9 -> 8.0, 4096^3 1215 -> 1126 (plain 1024); lists on A, B and D, Float32 4096^3 3774 -> 1653 (on the
+// vector ALUs 1975), 512^3 21.4 -> 18.6 (26.8), Float64 2048^3 668 -> 386 (567).
 #pragma once
 #include "fpu_gemm.hpp"
 
@@ -60,11 +67,13 @@ template <> struct ChainBlock<double> {
   static __device__ __forceinline__ int col(int lane, int r) { return 4 * r + (lane >> 4); }
 };
 
-template <int BM_, int BN_, int BK_, int WAVES_M_, int WAVES_N_, typename TIN_, bool A_KMAJOR_, bool B_KMAJOR_, typename TACC_, bool FUSED_,
+template <int BM_, int BN_, int BK_, int WAVES_M_, int WAVES_N_, typename TIN_, bool A_KMAJOR_, bool B_KMAJOR_, typename TACC_, int FUSED_,
           int STAGES_, int RING_, int DEPTH_>
 struct FpuMfmaConfig {
   static constexpr int BM = BM_, BN = BN_, BK = BK_, WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, STAGES = STAGES_, RING = RING_, DEPTH = DEPTH_;
-  static constexpr bool A_KMAJOR = A_KMAJOR_, B_KMAJOR = B_KMAJOR_, FUSED = FUSED_;
+  static constexpr bool A_KMAJOR = A_KMAJOR_, B_KMAJOR = B_KMAJOR_;
+  // hooks: 0 none (no bias either); 1 at most one scale on A, on B and on C, any on D; 2 any
+  static constexpr int FUSED = FUSED_;
   typedef TIN_ TIN;
   typedef TACC_ TACC;
   static constexpr int THREADS = WAVES_M * WAVES_N * kWaveSize;
@@ -78,24 +87,44 @@ struct FpuMfmaConfig {
   static constexpr int A_ELEMS = (A_KMAJOR ? BM : BK) * PA, B_ELEMS = (B_KMAJOR ? BN : BK) * PB;
   static constexpr int LDS_BYTES = STAGES * (A_ELEMS + B_ELEMS) * (int)sizeof(TACC);
   static constexpr int A_PER_THREAD = BM * BK / V / THREADS, B_PER_THREAD = BN * BK / V / THREADS;
+  // Hooks take registers: a wave may have all 512 of its SIMD where LDS leaves room for one workgroup of a tile anyway, and
+  // where lists meet 64 accumulators (256 registers spill there).
+  static constexpr int WAVES_PER_SIMD = FUSED != 0 && THREADS == 256 && (LDS_BYTES > 80 * 1024 || (FUSED == 2 && BM * BN >= 64 * THREADS)) ? 1 : 2;
   static_assert(BM % (16 * WAVES_M) == 0 && BN % (16 * WAVES_N) == 0 && BM % 32 == 0 && BN % 32 == 0 && BK % 8 == 0, "wave tiles are made of 16 x 16 blocks");
   static_assert(A_PER_THREAD * V * THREADS == BM * BK && B_PER_THREAD * V * THREADS == BN * BK, "tile loads divide evenly over the threads");
   static_assert(STAGES == 3 || (STAGES == 2 && RING == 2), "two stages, or three with the first fragments read ahead of the barrier");
   static_assert((RING & (RING - 1)) == 0 && STEPS % RING == 0, "a step finds its fragments in buffer s % RING in every tile");
 };
 
+// A list of operations in scalar registers, loaded from the kernel arguments where it is used.  (The address goes through a
+// statement that the compiler cannot see through: loaded once, the lists would hold half of the scalar registers all
+// through the K loop.  The arguments themselves, indexed at run time, would be copied to scratch memory as a whole.)
+struct ListRegs {
+  int n, kind[kMaxOps];
+  float p0[kMaxOps], p1[kMaxOps];
+  __device__ __forceinline__ explicit ListRegs(int hook) {
+    typedef const __attribute__((address_space(4))) char* bytes;
+    typedef const __attribute__((address_space(4))) OpList* list;
+    bytes arguments = (bytes)__builtin_amdgcn_kernarg_segment_ptr();      // (GemmArgs is the kernel's only argument)
+    asm volatile("" : "+s"(arguments));
+    list t = (list)(arguments + __builtin_offsetof(GemmArgs, t) + hook * (int)sizeof(OpList));
+    n = t->n;
+#pragma unroll
+    for (int i = 0; i < kMaxOps; ++i) { kind[i] = t->kind[i]; p0[i] = t->p0[i]; p1[i] = t->p1[i]; }
+  }
+};
+
 // A list applied to COUNT values in registers, slot after slot in a loop that is not unrolled: with up to 64 accumulators the
-// code of every op stands once per hook, not once per slot.  (The slot is picked by comparisons, so that the list stays
-// in the kernel arguments; see apply_list_regs_t.)
+// code of every op stands once per hook, not once per slot, and the switch is paid once per slot, not once per value.
+// The loop always takes the first slot and moves the others up.
 template <typename X, int COUNT>
-__device__ __forceinline__ void apply_list_looped(const OpList& t, X (&x)[COUNT]) {
+__device__ __forceinline__ void apply_list_looped(ListRegs t, X (&x)[COUNT]) {
 #pragma clang loop unroll(disable)
   for (int i = 0; i < t.n; ++i) {
-    int kind = t.kind[0];
-    float p0 = t.p0[0], p1 = t.p1[0];
+    const int kind = t.kind[0];
+    const float p0 = t.p0[0], p1 = t.p1[0];
 #pragma unroll
-    for (int j = 1; j < kMaxOps; ++j)
-      if (i == j) { kind = t.kind[j]; p0 = t.p0[j]; p1 = t.p1[j]; }
+    for (int j = 1; j < kMaxOps; ++j) { t.kind[j - 1] = t.kind[j]; t.p0[j - 1] = t.p0[j]; t.p1[j - 1] = t.p1[j]; }
     auto each = [&](auto kind_c) __attribute__((always_inline)) {
 #pragma unroll
       for (int e = 0; e < COUNT; ++e) x[e] = apply_op_t<X>(decltype(kind_c)::value, p0, p1, x[e]);
@@ -133,14 +162,10 @@ struct ChainOperand {
   int line, within;       // LDS row of the thread's first vector, element in it
   int shift;              // rows by which the thread's vectors are fetched too early (memory contiguous along the rows)
   int r0, limit, K;
-  TAR scale;              // the hooks of the operand are one multiplication (1: there are none) ...
-  bool listed;            // ... or a list of operations
-  const OpList* t0;
-  const OpList* t1;
+  TAR scale;              // FUSED == 1: the hooks of the operand are one multiplication (1: there are none)
 
-  __device__ __forceinline__ void init(const void* p, long long ld_, int r0_, int limit_, int K_, int tid, const OpList& h0, const OpList& h1) {
+  __device__ __forceinline__ void init(const void* p, long long ld_, int r0_, int limit_, int K_, int tid, float scale_) {
     base = (const TIN*)p; ld = ld_; r0 = r0_; limit = limit_; K = K_;
-    t0 = &h0; t1 = &h1;
     line = tid / PER_LINE;
     within = (tid % PER_LINE) * V;
     shift = 0;
@@ -156,13 +181,7 @@ struct ChainOperand {
       if (r > last) { shift = r - last; r = last; }
       off[0] = r;
     }
-    scale = (TAR)1;
-    listed = false;
-    if constexpr (Cfg::FUSED) {
-      // (x * 1 is x: a multiplication in the K loop costs no branch)
-      if (h0.n + h1.n == 1 && (h0.n ? h0.kind[0] : h1.kind[0]) == T_SCALE) scale = (TAR)(h0.n ? h0.p0[0] : h1.p0[0]);
-      else listed = h0.n + h1.n > 0;
-    }
+    scale = (TAR)scale_;        // (x * 1 is x: a multiplication in the K loop costs no branch)
   }
   // no row or K is short of a whole vector (else every fetch of this workgroup is element by element)
   __device__ __forceinline__ bool vectors_fit() const { return (KMAJOR ? K : limit) >= V; }
@@ -204,12 +223,11 @@ struct ChainOperand {
     if constexpr (TAIL) {
       const int k = k0 + (KMAJOR ? within : line + i * LINES), early = k - (K - V);
       if constexpr (KMAJOR) x = moved(x, early > 0 ? early : 0);
-#pragma unroll
-      for (int e = 0; e < V; ++e) x[e] = k + (KMAJOR ? e : 0) < K ? x[e] : (TIN)0;
+      x = cut(x, i, k0);
     }
     return x;
   }
-  // a vector element by element
+  // a vector element by element (beyond K: the last values)
   __device__ __forceinline__ vec fetch_slow(int i, int k0) const {
     vec x;
 #pragma unroll
@@ -218,39 +236,43 @@ struct ChainOperand {
       const int k = k0 + (KMAJOR ? within + e : line + i * LINES);
       r = r < limit ? r : limit - 1;
       const int kk = k < K ? k : K - 1;
-      const TIN y = base[KMAJOR ? (long long)r * ld + kk : (long long)kk * ld + r];
-      x[e] = k < K ? y : (TIN)0;
+      x[e] = base[KMAJOR ? (long long)r * ld + kk : (long long)kk * ld + r];
     }
     return x;
   }
-  // the two load hooks, each rounded to the element type of its destination (the operand's own type), then the
-  // conversion to the accumulator type for the fma.  LISTED: the hooks are lists.  Values beyond K stay zero whatever the
-  // hooks make of them (TAIL: a partial K tile, which alone has such values; 0 times an infinite factor is a NaN)
-  template <bool LISTED, bool TAIL>
-  __device__ __forceinline__ void store(TACC* lds, vec x, int i, int k0) const {
-    typedef TACC accv __attribute__((ext_vector_type(V)));
-    if constexpr (LISTED) {
-      TAR w[V];
+  // The two load hooks, each rounded to the element type of its destination (the operand's own type): a scale of one
+  // vector, or the lists over all vectors of a tile at once.  They come before settle: 0 times an infinite factor, or a
+  // list, makes something of the zeros behind K.
+  __device__ __forceinline__ vec scaled(vec x) const {
+    if constexpr (Cfg::FUSED == 1) {
 #pragma unroll
-      for (int e = 0; e < V; ++e) w[e] = (TAR)x[e];
-      if (t0->n > 0) {
-        apply_list_looped<TAR, V>(*t0, w);
-#pragma unroll
-        for (int e = 0; e < V; ++e) w[e] = (TAR)(TIN)w[e];
-      }
-      apply_list_looped<TAR, V>(*t1, w);
-#pragma unroll
-      for (int e = 0; e < V; ++e) {
-        const int k = k0 + (KMAJOR ? within + e : line + i * LINES);
-        x[e] = k < K ? (TIN)w[e] : (TIN)0;
-      }
-    } else if constexpr (Cfg::FUSED) {
-#pragma unroll
-      for (int e = 0; e < V; ++e) {
-        x[e] = (TIN)((TAR)x[e] * scale);
-        if constexpr (TAIL) x[e] = k0 + (KMAJOR ? within + e : line + i * LINES) < K ? x[e] : (TIN)0;
-      }
+      for (int e = 0; e < V; ++e) x[e] = (TIN)((TAR)x[e] * scale);
     }
+    return x;
+  }
+  static __device__ __forceinline__ void listed(vec (&x)[PER], int hook0, int hook1) {
+    const ListRegs t0(hook0), t1(hook1);
+    TAR w[PER * V];
+#pragma unroll
+    for (int i = 0; i < PER * V; ++i) w[i] = (TAR)x[i / V][i % V];
+    if (t0.n > 0) {
+      apply_list_looped<TAR, PER * V>(t0, w);
+#pragma unroll
+      for (int i = 0; i < PER * V; ++i) w[i] = (TAR)(TIN)w[i];
+    }
+    apply_list_looped<TAR, PER * V>(t1, w);
+#pragma unroll
+    for (int i = 0; i < PER * V; ++i) x[i / V][i % V] = (TIN)w[i];
+  }
+  // values beyond K are zero
+  __device__ __forceinline__ vec cut(vec x, int i, int k0) const {
+#pragma unroll
+    for (int e = 0; e < V; ++e) x[e] = k0 + (KMAJOR ? within + e : line + i * LINES) < K ? x[e] : (TIN)0;
+    return x;
+  }
+  // converted to the accumulator type for the fma
+  __device__ __forceinline__ void store(TACC* lds, vec x, int i) const {
+    typedef TACC accv __attribute__((ext_vector_type(V)));
     accv z;
 #pragma unroll
     for (int e = 0; e < V; ++e) z[e] = (TACC)x[e];
@@ -267,7 +289,7 @@ template <int N>
 __device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N < 15 ? N : 15) : "memory"); }
 
 template <class Cfg>
-__global__ void __launch_bounds__(Cfg::THREADS, 2) fpu_mfma_kernel(const GemmArgs args) {
+__global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES_PER_SIMD) fpu_mfma_kernel(const GemmArgs args) {
   typedef typename Cfg::TIN TIN;
   typedef typename Cfg::TACC TACC;
   constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, FM = Cfg::FM, FN = Cfg::FN, STEPS = Cfg::STEPS, STAGES = Cfg::STAGES;
@@ -294,8 +316,8 @@ __global__ void __launch_bounds__(Cfg::THREADS, 2) fpu_mfma_kernel(const GemmArg
 
   ChainOperand<Cfg, BM, Cfg::A_KMAJOR, Cfg::PA, PA> oa;
   ChainOperand<Cfg, BN, Cfg::B_KMAJOR, Cfg::PB, PB> ob;
-  oa.init(args.a, args.lda, m0, args.M, K, tid, args.t[H_GL2SH_A], args.t[H_SH2RF_A]);
-  ob.init(args.b, args.ldb, n0, args.N, K, tid, args.t[H_GL2SH_B], args.t[H_SH2RF_B]);
+  oa.init(args.a, args.lda, m0, args.M, K, tid, Cfg::FUSED == 1 ? args.scale_a : 1.0f);
+  ob.init(args.b, args.ldb, n0, args.N, K, tid, Cfg::FUSED == 1 ? args.scale_b : 1.0f);
 
   acc_t acc[FM][FN];
   auto row_of = [&](int fi, int r) { return m0 + wm * Cfg::WTM + fi * 16 + Block::row(lane, r); };
@@ -303,7 +325,9 @@ __global__ void __launch_bounds__(Cfg::THREADS, 2) fpu_mfma_kernel(const GemmArg
   constexpr bool WIDE = sizeof(TACC) == 4;            // a lane's four outputs of a block are consecutive rows
   struct __attribute__((packed, aligned(sizeof(TACC)))) loose_acc { acc_t v; };
   // one hook over all accumulators of the lane
-  [[maybe_unused]] auto hook_acc = [&](const OpList& t) __attribute__((always_inline)) {
+  [[maybe_unused]] auto hook_acc = [&](int hook) __attribute__((always_inline)) {
+    if (args.t[hook].n == 0) return;
+    const ListRegs t(hook);
     TACC flat[COUNT];
 #pragma unroll
     for (int x = 0; x < COUNT; ++x) flat[x] = acc[x / 4 % FM][x / 4 / FM][x % 4];
@@ -335,10 +359,16 @@ __global__ void __launch_bounds__(Cfg::THREADS, 2) fpu_mfma_kernel(const GemmArg
         }
         acc[fi][fj] = c;
       }
-    if constexpr (Cfg::FUSED) {
+    if constexpr (Cfg::FUSED == 1) {
+#pragma unroll
+      for (int fi = 0; fi < FM; ++fi)
+#pragma unroll
+        for (int fj = 0; fj < FN; ++fj) acc[fi][fj] *= (TACC)args.acc_pre_scale;
+    }
+    if constexpr (Cfg::FUSED == 2) {
       if (args.c_mode != 0) {
-        hook_acc(args.t[H_GL2SH_C]);
-        hook_acc(args.t[H_SH2RF_C]);
+        hook_acc(H_GL2SH_C);
+        hook_acc(H_SH2RF_C);
       }
     }
   };
@@ -377,17 +407,26 @@ __global__ void __launch_bounds__(Cfg::THREADS, 2) fpu_mfma_kernel(const GemmArg
   // or two fragments: at least (FM + FN) / 2 of them a step).
   constexpr int SHARE = (PA + PB + STEPS - 2) / (STEPS - 1), QUIET = STEPS - (PA + PB + SHARE - 1) / SHARE;
 
+  // FUSED == 2: the lists of both operands over the vectors of a tile
+  auto lists = [&](auto& xa, auto& xb) __attribute__((always_inline)) {
+    if constexpr (Cfg::FUSED == 2) {
+      if (args.t[H_GL2SH_A].n + args.t[H_SH2RF_A].n > 0) decltype(oa)::listed(xa, H_GL2SH_A, H_SH2RF_A);
+      if (args.t[H_GL2SH_B].n + args.t[H_SH2RF_B].n > 0) decltype(ob)::listed(xb, H_GL2SH_B, H_SH2RF_B);
+    }
+  };
+
   // The K loop over the whole tiles, written without a branch inside a tile: tiles beyond the last one are fetched and
   // stored like any other (from the addresses of the last, into stages that nobody reads), so that the loads, the moves and
   // the LDS writes of a later tile stand between the MFMAs of this one.  A partial last tile sets out before the loop
   // and waits in registers of its own for the end of it.  MOVED: the rows of an operand that is contiguous along them
-  // reach over its edge; LISTED: hooks other than one scale.
+  // reach over its edge.
   const int whole = K / BK, k_tail = whole * BK;
-  auto pipeline = [&](auto moved_c, auto listed_c) __attribute__((always_inline)) {
-    constexpr bool MOVED = decltype(moved_c)::value, LISTED = decltype(listed_c)::value;
+  auto pipeline = [&](auto moved_c) __attribute__((always_inline)) {
+    constexpr bool MOVED = decltype(moved_c)::value;
     typename decltype(oa)::vec ra[FAR + DEPTH][PA], ta[PA];      // (tile t of the loop waits in slot FAR + (t - FAR) % DEPTH)
     typename decltype(ob)::vec rb[FAR + DEPTH][PB], tb[PB];
     auto k_of = [&](int t) { return (t < whole ? t : whole - 1) * BK; };      // a tile that exists
+    if constexpr (Cfg::FUSED == 2) load_c();       // (its lists before the tiles set out: no registers for both)
     if (whole > 0)
       fpu_static_for<0, FAR + DEPTH>([&](auto t_c) __attribute__((always_inline)) {
         constexpr int t = decltype(t_c)::value;
@@ -402,17 +441,18 @@ __global__ void __launch_bounds__(Cfg::THREADS, 2) fpu_mfma_kernel(const GemmArg
 #pragma unroll
       for (int i = 0; i < PB; ++i) tb[i] = ob.template fetch<true>(i, k_tail);
     }
-    load_c();
+    if constexpr (Cfg::FUSED != 2) load_c();
     auto stash_a = [&](TACC* stage, typename decltype(oa)::vec x, int i, int k0) __attribute__((always_inline)) {
-      oa.template store<LISTED, false>(stage, oa.template settle<MOVED, false>(x, i, k0), i, k0);
+      oa.store(stage, oa.template settle<MOVED, false>(oa.scaled(x), i, k0), i);
     };
     auto stash_b = [&](TACC* stage, typename decltype(ob)::vec x, int i, int k0) __attribute__((always_inline)) {
-      ob.template store<LISTED, false>(stage + Cfg::A_ELEMS, ob.template settle<MOVED, false>(x, i, k0), i, k0);
+      ob.store(stage + Cfg::A_ELEMS, ob.template settle<MOVED, false>(ob.scaled(x), i, k0), i);
     };
     int stage = 0;
     if (whole > 0) {
       fpu_static_for<0, FAR>([&](auto t_c) __attribute__((always_inline)) {
         constexpr int t = decltype(t_c)::value;
+        lists(ra[t], rb[t]);
 #pragma unroll
         for (int i = 0; i < PA; ++i) stash_a(lds + t * STAGE, ra[t][i], i, k_of(t));
 #pragma unroll
@@ -429,6 +469,7 @@ __global__ void __launch_bounds__(Cfg::THREADS, 2) fpu_mfma_kernel(const GemmArg
       const int next = stage + 1 == STAGES ? 0 : stage + 1, after = next + 1 == STAGES ? 0 : next + 1;
       TACC* into = lds + (AHEAD ? after : next) * STAGE;
       const int k_in = k_of(kt + FAR), k_out = k_of(kt + FAR + DEPTH);
+      lists(ra[SLOT], rb[SLOT]);
       if constexpr (!AHEAD) read(0, here, 0);
       fpu_static_for<0, STEPS>([&](auto s_c) __attribute__((always_inline)) {
         constexpr int s = decltype(s_c)::value;
@@ -468,10 +509,11 @@ __global__ void __launch_bounds__(Cfg::THREADS, 2) fpu_mfma_kernel(const GemmArg
       // (the barrier above: everyone has read the last whole tile)
       wait_lgkmcnt0();
       block_barrier();
+      lists(ta, tb);
 #pragma unroll
-      for (int i = 0; i < PA; ++i) oa.template store<LISTED, true>(lds, oa.template settle<MOVED, true>(ta[i], i, k_tail), i, k_tail);
+      for (int i = 0; i < PA; ++i) oa.store(lds, oa.template settle<MOVED, true>(oa.scaled(ta[i]), i, k_tail), i);
 #pragma unroll
-      for (int i = 0; i < PB; ++i) ob.template store<LISTED, true>(lds + Cfg::A_ELEMS, ob.template settle<MOVED, true>(tb[i], i, k_tail), i, k_tail);
+      for (int i = 0; i < PB; ++i) ob.store(lds + Cfg::A_ELEMS, ob.template settle<MOVED, true>(ob.scaled(tb[i]), i, k_tail), i);
       wait_lgkmcnt0();
       block_barrier();
       const int steps = (K - k_tail + 3) / 4;            // the steps that hold values
@@ -484,13 +526,12 @@ __global__ void __launch_bounds__(Cfg::THREADS, 2) fpu_mfma_kernel(const GemmArg
 
   if (zero_ab) {
     load_c();
-    if constexpr (Cfg::FUSED) {
+    if constexpr (Cfg::FUSED != 0) {
       // zeros through the hooks, as loaded values would go
-      typename ArithOf<TIN>::type a[1] = {0}, b[1] = {0};
-      apply_list_looped<typename ArithOf<TIN>::type, 1>(args.t[H_GL2SH_A], a); a[0] = (TIN)a[0];
-      apply_list_looped<typename ArithOf<TIN>::type, 1>(args.t[H_SH2RF_A], a); a[0] = (TIN)a[0];
-      apply_list_looped<typename ArithOf<TIN>::type, 1>(args.t[H_GL2SH_B], b); b[0] = (TIN)b[0];
-      apply_list_looped<typename ArithOf<TIN>::type, 1>(args.t[H_SH2RF_B], b); b[0] = (TIN)b[0];
+      typedef typename ArithOf<TIN>::type TAR;
+      TAR a[1] = {0}, b[1] = {0};
+      for (const int h : {H_GL2SH_A, H_SH2RF_A}) { apply_list_looped<TAR, 1>(ListRegs(h), a); a[0] = (TIN)a[0]; }
+      for (const int h : {H_GL2SH_B, H_SH2RF_B}) { apply_list_looped<TAR, 1>(ListRegs(h), b); b[0] = (TIN)b[0]; }
       if (!(a[0] == 0 || b[0] == 0))
         for (int k = 0; k < K; ++k)
 #pragma unroll
@@ -511,10 +552,11 @@ __global__ void __launch_bounds__(Cfg::THREADS, 2) fpu_mfma_kernel(const GemmArg
     load_c();
     for (int kt = 0; kt < KT; ++kt) {
       block_barrier();
+      lists(xa, xb);
 #pragma unroll
-      for (int i = 0; i < PA; ++i) oa.template store<Cfg::FUSED, true>(lds, xa[i], i, kt * BK);
+      for (int i = 0; i < PA; ++i) oa.store(lds, oa.cut(oa.scaled(xa[i]), i, kt * BK), i);
 #pragma unroll
-      for (int i = 0; i < PB; ++i) ob.template store<Cfg::FUSED, true>(lds + Cfg::A_ELEMS, xb[i], i, kt * BK);
+      for (int i = 0; i < PB; ++i) ob.store(lds + Cfg::A_ELEMS, ob.cut(ob.scaled(xb[i]), i, kt * BK), i);
       wait_lgkmcnt0();
       block_barrier();
       if (kt + 1 < KT) fetch((kt + 1) * BK);
@@ -525,19 +567,18 @@ __global__ void __launch_bounds__(Cfg::THREADS, 2) fpu_mfma_kernel(const GemmArg
       }
       wait_lgkmcnt0();
     }
-  } else if (Cfg::FUSED && (oa.listed || ob.listed)) {
-    pipeline(std::true_type{}, std::integral_constant<bool, Cfg::FUSED>{});
-  } else if ((!Cfg::A_KMAJOR && edge_m) || (!Cfg::B_KMAJOR && edge_n)) {
-    pipeline(std::true_type{}, std::false_type{});
+  } else if (Cfg::FUSED == 2 || (!Cfg::A_KMAJOR && edge_m) || (!Cfg::B_KMAJOR && edge_n)) {
+    pipeline(std::true_type{});
   } else {
-    pipeline(std::false_type{}, std::false_type{});
+    pipeline(std::false_type{});
   }
 
   // epilogue: transform, bias, transform, store; the bias of Epilogue.Bias is fp32 (reference src/epilogue.jl:44-52) and
   // only offered with fp32 accumulators
   TACC* D = (TACC*)args.d;
-  if constexpr (Cfg::FUSED) {
-    hook_acc(args.t[H_RF2SH_D]);
+  // (one look at all three arguments: a wait for each, one behind another, is part of the end of every launch)
+  if (Cfg::FUSED != 0 && (args.t[H_RF2SH_D].n | args.t[H_SH2GL_D].n | args.epi_kind) != 0) {
+    hook_acc(H_RF2SH_D);
     if constexpr (std::is_same<TACC, float>::value) {
       if (args.epi_kind == 1) {
 #pragma unroll
@@ -561,7 +602,7 @@ __global__ void __launch_bounds__(Cfg::THREADS, 2) fpu_mfma_kernel(const GemmArg
           }
       }
     }
-    hook_acc(args.t[H_SH2GL_D]);
+    hook_acc(H_SH2GL_D);
   }
 #pragma unroll
   for (int fj = 0; fj < FN; ++fj)

@@ -43,6 +43,10 @@ def test_every_tile_at_its_edges(gpu, types, ta, tb):
             hooks = {}
             if n % 3 == 1:          # a scale of A in the K loop, C scaled
                 hooks = dict(transform_shared_to_regs_a=Transform.Elementwise(lambda x: x * 1.5), transform_shared_to_regs_c=Transform.Elementwise(lambda x: x * 0.5))
+            if n == 6:              # lists of four on C alone, a scale of B, lists in both hooks of D
+                steps = Transform.Elementwise(lambda x: (x * 0.5 + 1) * 3 - 2)
+                hooks = dict(transform_global_to_shared_c=steps, transform_shared_to_regs_c=steps, transform_global_to_shared_b=Transform.Elementwise(lambda x: x * -0.75),
+                             transform_regs_to_shared_d=steps, transform_shared_to_global_d=steps)
             if n % 3 == 2:          # lists in both hooks of A and one of B (x + 1 leaves no zero behind K), and of D
                 hooks = dict(transform_global_to_shared_a=Transform.Elementwise(lambda x: x + 1), transform_shared_to_regs_a=Transform.Elementwise(lambda x: x * 0.75),
                              transform_global_to_shared_b=Transform.Elementwise(lambda x: (x + 1) * 3), transform_shared_to_global_d=Transform.Elementwise(Transform.relu))
