@@ -1082,27 +1082,47 @@ namespace {
 constexpr size_t kSplitCounterBytes = 2048;
 static_assert(kSplitCounterBytes / sizeof(unsigned) >= 2 * (size_t)gk::kNumCUs - 1, "one counter for every tile of a launch that is split");
 
-// K slices of a K-split launch, from a sweep of 2 .. 24 slices on the 64 x 64 x 64 tile over eighteen products: no more
-// workgroups than two per CU (what a CU holds of these tiles at a time: 700 x 900 x 3001, 165 tiles, takes 18.6 us on 3 slices
-// and 21.9 on 4), and slices at least 640 deep in K -- a slice pays for its prologue, for the trip of its partial tile to
-// memory and for the arrival counter (about 3 us on the last workgroup's path), which shorter slices do not earn back.
-// 4096 x 64 x 4096: 2 slices 17.2 us, 4 14.1, 6 14.6, 8 15.7, 16 20.5; 300 x 500 x 4000: 3 14.5, 4 13.6, 6 13.0, 8 14.0;
-// 64 x 64 x 8000: 8 12.2, 12 11.4, 16 12.0, 24 12.2; 256 x 256 x 1024: 1 7.1, 2 8.9.
+// K slices of a K-split launch, from sweeps of 1 .. 51 slices over 80 products and their transposes.  A slice pays for its
+// prologue, for the trip of its partial tile to memory and back and for the arrival counter (about 3 us on the last
+// workgroup's path), so slices are at least 640 deep in K, and no more workgroups start than two per CU, what a CU holds of
+// these tiles at a time.
+//
+// 64 x 64 x 64 without hooks on A or B: as many slices as give every CU one workgroup, rather than some CUs two (us by slices):
+//   4096 x 64 x 4096 (64 tiles) 3 12.0, 4 12.5, 6 13.1, 8 14.3; 1024 x 256 x 16384 (64) 4 23.9, 8 27.1; 287 x 589 x 7104 (50) 5 15.0,
+//   10 16.8; 8192 x 64 x 4096 (128) 2 18.7, 4 21.0; 2560 x 128 x 5120 (80) 3 13.4, 6 14.4;
+// two per CU where one leaves a fifth of the CUs idle and two no more than a sixth:
+//   960 x 384 x 4096 (90) 2 14.1, 5 12.4; 1600 x 256 x 8192 (100) 2 21.8, 5 18.5; 3000 x 128 x 6000 (94) 2 21.9, 5 20.1;
+//   700 x 900 x 3001 (165) 1 34.4, 2 24.4, 3 20.0;
+// and with few tiles, whose slices all end at once, not many unless they are 1024 deep:
+//   1776 x 33 x 7392 (28) 7 14.4, 8 14.4, 11 16.0; 300 x 200 x 9001 (20) 9 15.4, 14 18.9; 1085 x 47 x 6136 (17) 6 15.0, 9 13.9;
+//   64 x 64 x 8000 (1) 7 10.6, 12 10.0; 64 x 64 x 32768 (1) 24 15.3, 32 15.8, 51 18.0.
+// A factor on A or B (AB_HOOKS) makes the K loop longer and what a slice costs weigh less: up to two per CU.  FP16 4096 x 64 x 4096
+//   'T','N' 4 13.8, 6 12.9; BF16 4 66.5, 6 61.6, 8 57.0; BF16 7 x 7 x 20000 (1) 19 54.2, 31 46.6.
+// 128 x 128 x 64, whose partial tiles are four times as large: 768 deep (1024 above 64 tiles), sixteen slices or 2048 deep:
+//   512 x 512 x 4096 (16) 4 22.7, 5 22.0, 6 21.8; 2048 x 512 x 4096 (64) 4 25.3, 5 25.3, 6 26.2; 1536 x 1024 x 4096 (96) 4 29.5, 5 30.6;
+//   256 x 256 x 16384 (4) 12 34.4, 16 35.5, 25 40.2.
+// Other tiles (64 x 64 x 32): 4096 x 64 x 4096 (64) 4 24.4, 6 21.1, 7 20.6, 8 21.3.
+//
 // Where the partial tiles of that many slices would not fit the library's static workspace (512 tiles of 128 x 128 and the
 // counters are 2 KiB more than it holds) the slices are 1024 deep: what fits it at that depth is not refused.
-int split_k_slices(int tiles, int k_tiles, const gk_shape& block) {
-  int slices = tiles > 0 ? 2 * gk::kNumCUs / tiles : 1;
-  for (const int depth : {640, 1024}) {
-    const int min_tiles = (depth + block.K - 1) / block.K;
-    if (slices > k_tiles / min_tiles) slices = k_tiles / min_tiles;
-    if (slices < 2) return 1;
-    if (kSplitCounterBytes + (size_t)tiles * slices * block.M * block.N * sizeof(float) <= gk_split_k_noalloc_capacity()) break;
+int split_k_slices(int tiles, int k_tiles, const gk_shape& block, bool ab_hooks) {
+  auto at_depth = [&](int depth) { return k_tiles / ((depth + block.K - 1) / block.K); };
+  const int per_cu_2 = tiles > 0 ? 2 * gk::kNumCUs / tiles : 1;
+  const bool medium = block.M * block.N == 64 * 64 && block.K == 64, large = block.M * block.N >= 128 * 128;
+  int slices = std::min(per_cu_2, at_depth(large ? (tiles <= 64 ? 768 : 1024) : 640));
+  if (medium && !ab_hooks && tiles <= gk::kNumCUs / 2) {
+    const int per_cu_1 = gk::kNumCUs / tiles, at_once = tiles <= 8 ? 12 : (tiles <= 20 ? 9 : 8);
+    const bool idle = 5 * tiles * per_cu_1 <= 4 * gk::kNumCUs && 6 * tiles * slices >= 5 * 2 * gk::kNumCUs;
+    if (!idle) slices = std::min(std::min(slices, per_cu_1), std::max(at_once, at_depth(1024)));
   }
-  return slices;
+  if (large) slices = std::min(slices, std::max(16, at_depth(2048)));
+  if (kSplitCounterBytes + (size_t)tiles * std::max(slices, 0) * block.M * block.N * sizeof(float) > gk_split_k_noalloc_capacity())
+    slices = std::min(slices, at_depth(1024));
+  return slices < 2 ? 1 : slices;
 }
 
-// How a launch of the configuration is split, from the configuration alone: the workspace that a caller brings has no say in
-// the order of a sum.  A product whose last K tile runs outside the pipeline (see needs_tail_tile) takes as many slices
+// How a launch is split, from the configuration and whether A or B have hooks (ab_hooks): the workspace that a caller brings has
+// no say in the order of a sum.  A product whose last K tile runs outside the pipeline (see needs_tail_tile) takes as many slices
 // as leave partial tiles that the static workspace holds: it is refused nowhere, and gk_matmul_split_k and
 // gk_matmul_split_k_noalloc give the same bits.
 struct SplitK {
@@ -1110,11 +1130,11 @@ struct SplitK {
   size_t bytes;           // counters and partial tiles (0: one slice, unsplit)
 };
 
-SplitK split_k_plan(const gk_config* conf, int tiles, bool tail_tile) {
+SplitK split_k_plan(const gk_config* conf, int tiles, bool tail_tile, bool ab_hooks) {
   const gk_shape& block = conf->block_shape;
   const int k_tiles = (conf->matmul_shape.K + block.K - 1) / block.K;   // bounds-checked layouts: the last tile may be partial
   const size_t slice_bytes = (size_t)tiles * block.M * block.N * sizeof(float);
-  int slices = split_k_slices(tiles, k_tiles, block);
+  int slices = split_k_slices(tiles, k_tiles, block, ab_hooks);
   if (tail_tile && slices > 1) {
     const size_t fit = (gk_split_k_noalloc_capacity() - kSplitCounterBytes) / slice_bytes;
     if ((size_t)slices > fit) slices = (int)fit;
@@ -1159,7 +1179,7 @@ int launch_split_k(const gk_config* conf, const void* a, const void* b, const vo
   gk::FamilyFn fn = family_fn(L.key);
   hipError_t err = hipSuccess;
   const int tiles = L.args.nbm * L.args.nbn;      // (the grid of a tiled walk may hold more workgroups than there are tiles)
-  const SplitK plan = split_k_plan(conf, tiles, L.ragged);
+  const SplitK plan = split_k_plan(conf, tiles, L.ragged, L.key.fused == 1 || L.key.fused == 2);
   gk::InstanceInfo sk_info;
   // (a tile or hooks without a K-split instance: unsplit, see has_split_k_instance)
   gk::FamilyFn sk_fn = L.key.family == gk::FAMILY_MFMA_CHECKED ? fn : gk::family_mfma_splitk;
@@ -1199,7 +1219,9 @@ int gk_split_k_workspace_size(const gk_config* conf, size_t* bytes) {
   const long long tiles = (long long)((g.M + b.M - 1) / b.M) * ((g.N + b.N - 1) / b.N);
   gk::InstanceKey key;
   const bool tail_tile = make_key(conf, nullptr, nullptr, &key) == GK_OK && key.family == gk::FAMILY_MFMA && ragged_fast_path(conf) && needs_tail_tile(conf);
-  *bytes = has_split_k_instance(conf) ? split_k_plan(conf, (int)(tiles > (1 << 30) ? (1 << 30) : tiles), tail_tile).bytes : 0;
+  *bytes = 0;
+  if (has_split_k_instance(conf))
+    for (const bool ab_hooks : {false, true}) *bytes = std::max(*bytes, split_k_plan(conf, (int)(tiles > (1 << 30) ? (1 << 30) : tiles), tail_tile, ab_hooks).bytes);
   return GK_OK;
 }
 

@@ -281,7 +281,7 @@ int gk_matmul(const gk_config* conf, const void* a, const void* b, const void* c
  * at zero again: one workspace serves any number of launches of any products one after the other; launches
  * that overlap in time (two streams) need a workspace each.  A launch that faulted or was aborted may leave
  * counters behind: zero the first 2048 bytes again before the workspace is used after such a failure.  A launch that is
- * split and finds its workspace NULL or smaller than gk_split_k_workspace_size says is refused with
+ * split and finds its workspace NULL or smaller than it needs is refused with
  * GK_ERR_INVALID_ARGUMENT, except a product of bounds-checked layouts whose last K tile is partial (or holds a vector that
  * reaches over the end of an operand), which then runs unsplit: another order of its sum, so other last bits. */
 int gk_split_k_workspace_size(const gk_config* conf, size_t* bytes);

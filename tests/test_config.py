@@ -390,3 +390,26 @@ def test_wide_leading_dimensions_keep_a_tile_that_takes_them(ta, tb):
     assert block(1 << 23, 1 << 23) == split
     assert block(1 << 24, 4096) == (split if ta else narrow)
     assert block(4096, 1 << 24) == (narrow if tb else split)
+
+
+@pytest.mark.parametrize("dims,tile,scale,slices", [((4096, 64, 4096), (64, 64, 64), None, 4), ((4096, 64, 4096), (64, 64, 64), 1.5, 6), ((64, 64, 8000), (64, 64, 64), None, 12),
+                                                    ((8192, 64, 4096), (64, 64, 64), None, 2), ((960, 384, 4096), (64, 64, 64), None, 5), ((1792, 64, 7168), (64, 64, 64), None, 8),
+                                                    ((832, 640, 4096), (64, 64, 64), None, 3), ((1024, 1024, 4096), (64, 64, 64), None, 2), ((320, 192, 9984), (64, 64, 64), None, 9),
+                                                    ((256, 256, 16384), (128, 128, 64), None, 16), ((2048, 512, 4096), (128, 128, 64), None, 5), ((1536, 1024, 4096), (128, 128, 64), None, 4)])
+def test_k_slices_fill_the_cus_once(dims, tile, scale, slices):
+    """As many slices of a 64 x 64 x 64 product as give every CU one workgroup (two where one leaves CUs idle, or A has a factor),
+    fewer where each would be short or their partial tiles large; read from the refusal of a workspace that is too small."""
+    from gemmkernels import Transform, configs
+    import sys
+    matmul = sys.modules["gemmkernels.matmul"]
+    M, N, K = dims
+    cconf = configs.mfma_config(M, N, K, block_shape=tile).to_c(M, K, M, M)
+    hooks = matmul._collect({name: Transform.Elementwise(lambda x: x * scale) if scale and name == "transform_shared_to_regs_a" else None for name in matmul._HOOKS})
+    trans = matmul.lower_transforms(hooks)
+    need = ctypes.c_size_t()
+    assert _lib.lib().gk_split_k_workspace_size(ctypes.byref(cconf), ctypes.byref(need)) == _lib.GK_OK
+    # (nothing is launched: the workspace of 16 bytes is refused whatever the addresses are)
+    rc = _lib.lib().gk_matmul_split_k(ctypes.byref(cconf), 256, 256, 256, 256, ctypes.byref(trans) if trans else None, None, 256, 16, None)
+    assert rc == _lib.GK_ERR_INVALID_ARGUMENT
+    assert f"needs a workspace of {2048 + slices * 4 * M * N} bytes ({-(-M // tile[0]) * -(-N // tile[1])} tiles x {slices} slices" in _lib.last_error()
+    assert need.value >= 2048 + slices * 4 * M * N
