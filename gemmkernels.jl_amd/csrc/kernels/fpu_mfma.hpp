@@ -403,9 +403,12 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES_PER_SIMD) fpu_mfma_ke
   };
 
   // The vectors of a tile go to LDS in the first steps of a tile.  The LDS answers in order, so the barrier that
-  // publishes them need not wait for the fragment reads of the QUIET steps behind the last write (an instruction reads one
-  // or two fragments: at least (FM + FN) / 2 of them a step).
+  // publishes them need not wait for the fragment reads behind the last write: those of the QUIET steps that write nothing,
+  // less the last step of two stages, which has no later step of its tile to read for.  (An instruction reads one or two
+  // fragments: at least (FM + FN) / 2 of them a step.)
   constexpr int SHARE = (PA + PB + STEPS - 2) / (STEPS - 1), QUIET = STEPS - (PA + PB + SHARE - 1) / SHARE;
+  constexpr int READS_BEHIND = (AHEAD ? QUIET : QUIET - 1) * ((FM + FN + 1) / 2);
+  static_assert(QUIET >= 1, "the last step writes nothing");
 
   // FUSED == 2: the lists of both operands over the vectors of a tile
   auto lists = [&](auto& xa, auto& xb) __attribute__((always_inline)) {
@@ -491,7 +494,7 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES_PER_SIMD) fpu_mfma_ke
         interleave();
         __builtin_amdgcn_sched_barrier(0);
       });
-      wait_lds<QUIET * ((FM + FN + 1) / 2)>();
+      wait_lds<READS_BEHIND>();
       block_barrier();
       stage = next;
     };
