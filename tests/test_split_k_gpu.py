@@ -290,6 +290,28 @@ def test_a_partial_last_k_tile_is_the_end_of_the_last_slice(gpu, dims, tile, ta,
     assert np.array_equal(C.cpu().numpy().astype(np.float64), product + c)
 
 
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("ab,cd", [(torch.float16, torch.float32), (torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
+def test_slices_with_factors_and_16_bit_outputs(gpu, ab, cd, ta, tb):
+    """mul! on slices with factors on A and C (an exact FP16 scale, and the per-element path of BF16), a power of two, and FP16 C and
+    D, with whole and partial last K tiles.  A and B in {-1, 0, 1} and C in multiples of 1/2 below 8: every result is a
+    multiple of 1/4 below 512 (asserted), exact in FP16 as well as in every partial sum."""
+    rs = np.random.RandomState(21)
+    for M, N, K in ((70, 61, 2049), (131, 67, 1290), (64, 128, 4096), (9, 300, 2560)):
+        for alpha, beta in ((1.5, 0.5), (1.5, 0.0), (1.0, 1.0), (-2.0, 1.0)):
+            a, b = rs.randint(-1, 2, size=(K, M) if ta else (M, K)), rs.randint(-1, 2, size=(N, K) if tb else (K, N))
+            c = rs.randint(-15, 16, size=(M, N)) / 2.0
+            A, B, C = (gk.colmajor(np.asfortranarray(x.astype(np.float32))).to(t) for x, t in ((a, ab), (b, ab), (c, cd)))
+            p = gk.matmatmul_plan(C, "NT"[ta], "NT"[tb], A, B, alpha, beta)
+            print("case", ab, cd, (M, N, K), ta, tb, alpha, beta, p.kernel_names, flush=True)
+            assert p._split_k
+            ref = alpha * ((a.T if ta else a).astype(np.float64) @ (b.T if tb else b).astype(np.float64)) + beta * c
+            assert np.abs(ref).max() < 512
+            p()
+            torch.cuda.synchronize()
+            assert np.array_equal(C.double().cpu().numpy(), ref), ((M, N, K), alpha, beta)
+
+
 def test_captured_products_keep_a_workspace_of_their_own(gpu):
     """Two graphs of mul! on K slices, replayed in either order with eager products (which grow the shared workspace)
     between the replays: every replay gives the eager result."""
