@@ -6,7 +6,8 @@
 // device against fmaf / fma on 12 800 outputs per distribution (values spread over [-1, 1), over 40 binary orders of
 // magnitude, sums in the subnormal range, subnormal factors) with no bit different, where the descending chain differs
 // in a third to a half of them and a single rounding of the whole sum in as many.  A product on these instructions is
-// therefore bit-identical to the vector-ALU kernel (fpu_gemm.hpp) and to a sequential loop on the host, at a higher rate:
+// therefore bit-identical to the vector-ALU kernel (fpu_gemm.hpp) and to a sequential loop on the host -- but for the sign of a
+// zero where K is no multiple of four: the zeros behind K make +0 of a sum that underflowed to -0 -- at a higher rate:
 // 148 TFLOP/s in FP32 from registers (v_fma_f32: 64), 77 in FP64 (v_fma_f64: 63; the packed FP32 fma that would
 // double the vector ALUs' FP32 rate is not used in this library).
 //
@@ -16,9 +17,9 @@
 // values in a place where they are converted, scaled, moved and zeroed on their way.  What matters is that every SIMD has
 // an MFMA to issue all the time.  An MFMA leaves room for seven other instructions of its wave, and an LDS read takes about
 // four MFMAs to answer, so the instructions of a step are placed one behind each MFMA and the fragments are read LOOK
-// steps ahead (1024^3, one 64 x 64 tile per CU: 27 us with reads in a group one step ahead, 23 so).  Tiles of 64 x 64 use two
-// LDS stages and leave the CU to several workgroups; those of 128 x 128 and 32 x 32 three, with the first fragments of the
-// next tile read in front of the barrier, because they often have a CU to themselves.
+// steps ahead (1024^3, one 64 x 64 tile per CU: 27 us with reads in a group one step ahead, 23 so).  Most tiles use two
+// LDS stages and leave the CU to several workgroups; the Float32 tiles of 128 x 128, and of 32 x 32 on four waves, three, with
+// the first fragments of the next tile read in front of the barrier, because they often have a CU to themselves.
 //
 // Measured (beta = 0, one box; before, on the vector ALUs): Float32 256^3 12.2 -> 4.7 us, 1024^3 71 -> 23, 2048^3
 // 293 -> 134, 3001 x 3003 x 2999 -> 461 (0.79 of the instruction's rate), 4096^3 1900 -> 1028 us (134 TFLOP/s, 0.90);

@@ -1,6 +1,7 @@
 // K-split instances of the MFMA GEMM (kernel kind GK_KERNEL_SPLIT_K): the small tiles that skinny
 // products run, all four transposes, FP16 with no hooks, with C / D hooks and bias, or with those and one exact
-// FP16 scale on A and B (what the BLAS-style entry points produce), BF16 with no hooks or C / D hooks and bias.
+// FP16 scale on A and B (what the BLAS-style entry points produce); BF16 with no hooks, with C / D hooks and bias and, on
+// the 64 x 64 x 64 tile, with any hooks.
 #include "mfma_gemm.hpp"
 #include "registry.hpp"
 

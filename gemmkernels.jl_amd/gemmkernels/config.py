@@ -220,18 +220,28 @@ def default_block_shape(operator, gemm_shape, tile_sized: bool = True, gett: boo
     return NT(M=best[0], N=best[1], K=best[2])
 
 
-def split_k_block_shape(M, N, K, widest_ld=0) -> Optional[NT]:
+def split_k_block_shape(M, N, K, widest_ld=0, factor=None) -> Optional[NT]:
     """The tile of a 16-bit product that is worth cutting into slices of K (``Kernel.matmul_split_k``), or None: few output
-    tiles, which alone leave CUs idle, and a long K.  Measured against the best tile unsplit: 4096 x 64 x 4096 14.1 us
-    against 22.2, 300 x 500 x 4000 13.0 against 23.5, 64 x 64 x 8000 11.4 against 39, 2000 x 100 x 1500 11.6 against 12.3,
-    256 x 256 x 1024 8.9 against 7.1; with more than 128 tiles, which leave two or three slices, 1024 x 1024 x 4096 22.1
-    against 23.6, 700 x 900 x 3001 18.6 against 20.9, 1000 x 1000 x 2000 17.8 against 16.2.  ``widest_ld``: the larger leading
-    dimension of the operands whose rows are the k of a tile; the kernel keeps the offsets in a tile in 32 bits, so 64
-    rows of 2^24 elements are left to a tile with fewer."""
+    tiles, which alone leave CUs idle, and a long K.  Measured against the best tile unsplit: 4096 x 64 x 4096 12.6 us
+    against 22.0, 300 x 500 x 4000 13.0 against 23.6, 64 x 64 x 8000 9.8 against 38.9, 2000 x 100 x 1500 12.3 against 17.5,
+    256 x 256 x 1280 7.6 against 8.3 (x 1024 8.9 against 7.1); three slices of 129 .. 170 tiles 700 x 900 x 3001 19.7
+    against 23.3.  More tiles leave two slices, which pay where K or the output is whole tiles (1024 x 1024 x 4096 20.6
+    against 22.7, 1001 x 704 x 3328 20.9 against 22.5, 1024 x 768 x 4004 21.7 against 23.8; but 1001 x 700 x 3333 26.6 against
+    24.6, 1000 x 1000 x 4000 25.4 against 24.6), or where A has a factor that stays in the loop (``factor``): "packed",
+    FP16, 1001 x 700 x 3333 27.4 against 31.9; "per element", BF16, keeps the vector ALUs of every CU that has a tile busy,
+    so only where the slices still spread (768 x 1024 x 4096 105 against 113; 1001 x 1001 x 5001 161 against 141, 70 x 7000
+    x 3500 116 against 101, 12000 x 64 x 4096 122 against 114).  ``widest_ld``: the larger leading dimension of the operands whose rows are the k of a tile; the
+    kernel keeps the offsets in a tile in 32 bits, so 64 rows of 2^24 elements are left to a tile with fewer."""
     if 64 * widest_ld * 2 >= 1 << 31:
         return None
     tiles = -(-M // 64) * -(-N // 64)
-    return NT(M=64, N=64, K=64) if K >= 1280 and tiles <= 128 or K >= 3000 and tiles <= 256 else None
+    if tiles <= 128:
+        worth = K >= 1280
+    else:
+        whole = K % 64 == 0 or M % 64 == 0 and N % 64 == 0
+        two = {None: whole, "packed": True, "per element": tiles <= 225 and min(M, N) > 128}[factor]
+        worth = K >= 3000 and (tiles <= 170 or tiles <= 256 and two)
+    return NT(M=64, N=64, K=64) if worth else None
 
 
 # Throughput of a CU that has one tile at a time, relative to 256 x 256 x 64 on four waves; a pair: a launch with at most

@@ -164,7 +164,7 @@ def _config1() -> Workload:
 
     return Workload(
         name="config 1",
-        description="config 1: C = A*B through mul!, FP32, M=N=K=256, column-major NN, A,B ~ U[0,1), beta = 0 (FPUOp on the vector ALUs)",
+        description="config 1: C = A*B through mul!, FP32, M=N=K=256, column-major NN, A,B ~ U[0,1), beta = 0 (FPUOp on the FP32 matrix instructions)",
         flops=2 * M * N * K, bytes=3 * M * N * 4, bound="latency", make_host=host, make_launch=launch,
         kernel_name=kernel_name(conf, kern))
 

@@ -425,11 +425,12 @@ def get_config(*args):
 
 def create_config(A: DType, sizeA, stridesA, transA: bool, B: DType, sizeB, stridesB, transB: bool,
                   C: DType, sizeC, stridesC, alpha: type, zeroAlpha: bool, beta: type, zeroBeta: bool, wmma=None,
-                  aligned_pointers=(True, True, True)):
+                  aligned_pointers=(True, True, True), factor: Optional[str] = None):
     """reference src/matmul.jl:66-183, with the MI355X operator and block-shape choices.  ``aligned_pointers``
     says whether A, B and C start on 16-byte boundaries: the reference decides on the aligned layouts from the
     strides alone (a misaligned view then traps on the device, src/layout.jl:22-25); here such an operand gets
-    the bounds-checked layout, which takes any address."""
+    the bounds-checked layout, which takes any address.  ``factor``: how alpha is applied to A
+    in the K loop, see ``split_k_block_shape``."""
     m = sizeA[1 if transA else 0]
     k = sizeA[0 if transA else 1]
     n = sizeB[0 if transB else 1]
@@ -483,7 +484,7 @@ def create_config(A: DType, sizeA, stridesA, transA: bool, B: DType, sizeB, stri
                                  else compute_type in (Float16, Float32, Float64))
     block_shape = None
     if use_mfma and edge_ok:
-        block_shape = split_k_block_shape(m, n, k, max(0 if transA else stridesA[1], stridesB[1] if transB else 0))
+        block_shape = split_k_block_shape(m, n, k, max(0 if transA else stridesA[1], stridesB[1] if transB else 0), factor)
     if block_shape is None:
         block_shape = default_block_shape(operator, NT(M=m, N=n, K=k), tile_sized=not edge_ok, a_kmajor=transA, b_kmajor=not transB)
     global_a_layout, global_b_layout, global_c_layout, global_d_layout = layouts_for(block_shape)
@@ -512,13 +513,18 @@ def _round_to(dtype: DType, x: float) -> float:
     return float(x)
 
 
+_FOLDED = frozenset(2.0 ** e for e in range(-4, 5))
+
+
 def _single_plan(C, tA: bool, tB: bool, A, B, alpha, beta, wmma=None) -> Plan:
     """One launch for C = alpha * op(A) * op(B) + beta * C: the configuration ``create_config`` picks."""
+    # (a power of two within 2^-4 .. 2^4 leaves the K loop, see the folded scales of the library)
+    factor = None if abs(float(alpha)) in _FOLDED else ("per element" if BFloat16 in (from_torch(A.dtype), from_torch(B.dtype)) else "packed")
     conf, compute_type, kernel = get_config(
         from_torch(A.dtype), tuple(A.shape), tuple(A.stride()), tA,
         from_torch(B.dtype), tuple(B.shape), tuple(B.stride()), tB,
         from_torch(C.dtype), tuple(C.shape), tuple(C.stride()),
-        type(alpha), alpha == 0, type(beta), beta == 0, wmma, tuple(x.data_ptr() % 16 == 0 for x in (A, B, C)))
+        type(alpha), alpha == 0, type(beta), beta == 0, wmma, tuple(x.data_ptr() % 16 == 0 for x in (A, B, C)), factor)
     alpha_c = _round_to(compute_type, float(alpha))          # convert(compute_type, alpha), :196
     beta_c = _round_to(from_torch(C.dtype), float(beta))     # convert(eltype(C), beta), :197
     for name, value in (("alpha", alpha_c), ("beta", beta_c)):
@@ -536,7 +542,7 @@ def _single_plan(C, tA: bool, tB: bool, A, B, alpha, beta, wmma=None) -> Plan:
         # ordered, so the result is the same on every run, like the reference's mul!.
         bs, ms = conf.block_shape, conf.matmul_shape
         tiles = -(-ms.M // bs.M) * -(-ms.N // bs.N)
-        if bs == split_k_block_shape(ms.M, ms.N, ms.K) or tiles <= 256 and ms.K >= 2048:
+        if bs == split_k_block_shape(ms.M, ms.N, ms.K, 0, factor) or tiles <= 256 and ms.K >= 2048:
             kernel = Kernel.matmul_split_k
     p = plan(conf, A, B, C, C, transform_shared_to_regs_a=ta, transform_shared_to_regs_c=tc, kernel=kernel)
     p.kernel_names = (kernel_name(conf, kernel, dict(transform_shared_to_regs_a=ta, transform_shared_to_regs_c=tc)),)

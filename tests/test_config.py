@@ -413,3 +413,19 @@ def test_k_slices_fill_the_cus_once(dims, tile, scale, slices):
     assert rc == _lib.GK_ERR_INVALID_ARGUMENT
     assert f"needs a workspace of {2048 + slices * 4 * M * N} bytes ({-(-M // tile[0]) * -(-N // tile[1])} tiles x {slices} slices" in _lib.last_error()
     assert need.value >= 2048 + slices * 4 * M * N
+
+
+def test_two_slices_of_more_than_170_tiles_only_where_they_pay():
+    """11 x 16 tiles of 64 x 64: cut in two where K, or else the output, is whole tiles, or where an FP16 alpha stays in the K loop;
+    three slices of 165 tiles, and few tiles, are worth it in any case."""
+    def block(M, N, K, factor=None):
+        conf, _, _ = create_config(Float16, (M, K), (1, M), False, Float16, (K, N), (1, K), False,
+                                   Float32, (M, N), (1, M), float, False, float, True, factor=factor)
+        return conf.block_shape
+    split, narrow = NT(M=64, N=64, K=64), NT(M=64, N=64, K=32)
+    assert block(1001, 700, 3328) == split and block(1024, 704, 3336) == split
+    assert block(1001, 700, 3333) == narrow and block(1024, 704, 3333) == split and block(1000, 704, 3336) == narrow
+    assert block(1001, 700, 3333, "packed") == split and block(1001, 700, 3333, "per element") == split
+    assert block(768, 1024, 4096, "per element") == split and block(1024, 1024, 4096, "per element") == narrow
+    assert block(12032, 64, 4096, "per element") != split and block(12032, 64, 4096) == split
+    assert block(700, 900, 3001) == split and block(300, 200, 1301) == split
