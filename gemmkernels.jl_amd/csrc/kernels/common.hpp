@@ -134,12 +134,13 @@ struct GemmArgs {
   int cd_gett;                    // 1: C and D are addressed through gett.m / gett.n stride1
   OpList t[8];
   // set by the host when the two load hooks of A (resp. B) amount to one multiplication by a
-  // constant that is exact in the operand's 16-bit type: done as a packed 16-bit multiply
+  // constant that is exact in the operand's 16-bit type: done as a packed 16-bit multiply (FPUOp: the multiplication
+  // itself, any constant, without the flags)
   int fast_scale_a, fast_scale_b;
   float scale_a, scale_b;
   // a multiplication of A or B by a power of two commutes with every rounding of the sum: the host takes such
   // a hook out of the K loop, the accumulators start from acc_pre_scale * T_c(C) and are multiplied by
-  // acc_post_scale = 1 / acc_pre_scale before the hooks of D (both 1 otherwise)
+  // acc_post_scale = 1 / acc_pre_scale before the hooks of D (both 1 otherwise; FPUOp: acc_pre_scale is the one scale of C)
   float acc_pre_scale, acc_post_scale;
   GettDim gm, gn, gk;
   // How a K tile lies in the K modes of a contraction: it covers the modes below gk_mode whole (their extents

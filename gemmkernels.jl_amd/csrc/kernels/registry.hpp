@@ -14,7 +14,7 @@ struct InstanceKey {
   int a_kmajor, b_kmajor;   // 1: the K index is contiguous in the operand's memory
   int dtype;         // element type of A and B
   int acc_dtype;     // element type of C / D and of the accumulators (vector-ALU kernels)
-  int fused;         // 1: transforms / bias present
+  int fused;         // 0: no transforms, no bias; other levels are the family's (MfmaGemmConfig, FpuMfmaConfig)
   int variant;       // family specific
 };
 

@@ -85,7 +85,7 @@ def _current_stream() -> int:
 
 _workspaces = {}            # (device, stream) -> buffer of eager launches
 _recorded = {}              # (device, stream) -> buffers of graphs captured without torch
-_pool_of_capture = {}       # (device, capture) -> whether torch keeps the capture's memory for the graph
+_pool_of_capture = {}       # (device, stream, capture) -> whether torch keeps the capture's memory for the graph
 _COUNTER_BYTES = 2048       # arrival counters at the head of a workspace (kSplitCounterBytes of the library)
 
 
@@ -130,12 +130,12 @@ def _capture_of(stream: int):
     return capture.value if capturing.value else None
 
 
-def _in_graph_pool(buf, capture: int) -> bool:
+def _in_graph_pool(buf, stream: int, capture: int) -> bool:
     """Whether a buffer allocated during a capture lies in a memory pool of the graph (``torch.cuda.graph``), which keeps
     its memory as long as the graph lives, or in the allocator's common one, which hands it out again.  One answer for all
-    of a capture."""
+    of a stream's part in a capture."""
     import torch
-    key = (buf.device.index, capture)
+    key = (buf.device.index, stream, capture)
     known = _pool_of_capture.get(key)
     if known is None:
         p = buf.data_ptr()
@@ -160,7 +160,7 @@ def _workspace(need: int, stream: int):
         # in use, replaced by a larger one or not yet cleared when this graph runs
         with _on(stream):
             buf = torch.empty(need, dtype=torch.uint8, device="cuda")
-            if not _in_graph_pool(buf, capture):
+            if not _in_graph_pool(buf, stream, capture):
                 # a capture that torch does not know of: nobody else keeps the memory for the graph, so it is never given
                 # back.  The graphs captured so on one stream share a buffer (as launches on one stream do: their replays
                 # must not overlap), and a larger one is at least twice as large, which bounds all of them together
