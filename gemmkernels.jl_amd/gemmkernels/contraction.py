@@ -17,9 +17,11 @@ or permuted: a contraction either maps onto one launch of the GEMM kernel or is 
 """
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass
 from typing import Dict, List, Optional, Sequence, Tuple
 
+from . import _lib
 from . import kernel as Kernel
 from . import layout as Layout
 from . import operator as Operator
@@ -171,5 +173,40 @@ def plan(spec: str, a, b, d, c=None, ab_type: Optional[DType] = None, cd_type: O
 
 def contract(spec: str, a, b, d, c=None, stream=None):
     """``D[...] = sum A[...] * B[...] (+ C[...])`` in one launch on the current stream; returns ``d``."""
-    plan(spec, a, b, d, c)(stream)
+    from .matmul import _current_stream
+    key = (spec, a.dtype, a.shape, a.stride(), b.dtype, b.shape, b.stride(), d.dtype, d.shape, d.stride(),
+           None if c is None else (c.shape, c.stride()))
+    launch = _launches.get(key)
+    if launch is None:
+        launch = _Launch(plan(spec, a, b, d, c))
+        if len(_launches) >= _LAUNCHES_MAX:
+            _launches.clear()
+        _launches[key] = launch
+    launch(a.data_ptr(), b.data_ptr(), None if c is None else c.data_ptr(), d.data_ptr(), _current_stream() if stream is None else int(stream))
     return d
+
+
+class _Launch:
+    """What ``contract`` hands to the library for operands of one kind (mode string, element types, extents, strides): the descriptor
+    the planner arrived at, no address and no tensor; nothing in it is written after it is made, and the library checks
+    the addresses at every launch.  Planning again took 70 us of interpreter time a call, several times the kernel of a small contraction."""
+
+    __slots__ = ("_conf", "_conf_ref", "_swapped", "_fn", "_code")
+
+    def __init__(self, p: ContractionPlan):
+        self._conf = p._launch._conf                      # (owns the memory that the reference points to)
+        self._conf_ref = ctypes.byref(self._conf)
+        self._swapped = p.swapped
+        self._fn, self._code = p._launch._fn, p._launch._args[-1]
+
+    def __call__(self, a: int, b: int, c: Optional[int], d: int, stream: int) -> None:
+        x, y = (b, a) if self._swapped else (a, b)
+        rc = self._fn(self._conf_ref, x, y, c, d, None, None, self._code, stream)
+        if rc != _lib.GK_OK:
+            from .matmul import _raise
+            _raise(rc)
+
+
+# launches by kind of operands; a program has few kinds, one that has more pays for planning again
+_launches: Dict[tuple, _Launch] = {}
+_LAUNCHES_MAX = 256
