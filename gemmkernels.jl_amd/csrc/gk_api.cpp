@@ -451,6 +451,36 @@ void make_args(const gk_config* c, const void* a, const void* b, const void* cc,
   }
 }
 
+// Whether a launch runs its 128 x 128 or 64 x 64 tiles on four LDS stages of 64 k (mfma_deep_instances.inc): where every
+// workgroup has a CU to itself (128 KiB of LDS), or half of one (64 KiB).  Beyond that more workgroups of two stages fit a CU and
+// win: 576 tiles of 64 x 64 (1536^3) 17.5 us on two stages, 19.0 on four; 512 (2048 x 1024 x 1024) 11.9, 10.1; 400 tiles of
+// 128 x 128 (2560^3) 41.2, 46.2; 256 (2048^3) 28.8, 22.3.  BLOCK_K = 32 joins, two K tiles to a stage, where K is whole tiles of 64
+// (2048^3 on its own four stages of 32 k 24.5; 1024 x 1024 x 4096 on 64 x 64 x 32 22.1, 18.1), or long on 64 x 64 (a partial last tile of 64
+// costs more than one of 32, 1001 x 1003 x 1005 12.3, 11.6, and than none, 136 x 5124 x 6560 36.5, 35.5), and the rows of 64 k are addressed in 31 bits like those of 32.
+bool deep_instance(const gk::InstanceKey& key, const gk::GemmArgs& args) {
+  if (key.waves_m != 2 || key.waves_n != 2 || (key.variant & gk::kShallow) != 0) return false;
+  const long long tiles = (long long)((args.M + key.BM - 1) / key.BM) * ((args.N + key.BN - 1) / key.BN);
+  const bool rows_fit = 64 * std::max(args.lda, args.ldb) * 2 < (1ll << 31);
+  if (key.BM == 64 && key.BN == 64) return tiles <= 2 * gk::kNumCUs && (key.BK == 64 || (key.BK == 32 && rows_fit && (args.K % 64 == 0 || (args.K % 32 != 0 && args.K >= 1536))));
+  if (key.BM != 128 || key.BN != 128 || tiles > gk::kNumCUs) return false;
+  return key.BK == 64 || (key.BK == 32 && args.K % 64 == 0 && rows_fit);
+}
+
+int family_mfma(const gk::InstanceKey& as_asked, const gk::GemmArgs& args, dim3 grid, hipStream_t stream, int mode, gk::InstanceInfo* info, hipError_t* err) {
+  gk::InstanceKey key = as_asked;
+  key.variant &= ~gk::kShallow;
+  const bool deep = deep_instance(as_asked, args);
+  // (contractions on 64 x 64 x 64 are compiled with the deep instances, for many tiles as well)
+  if (deep || (key.family == gk::FAMILY_GETT && key.BM == 64 && key.BN == 64 && key.BK == 64)) {
+    const auto fn = key.a_kmajor ? (key.b_kmajor ? gk::family_mfma_deep_tn : gk::family_mfma_deep_tt)
+                                 : (key.b_kmajor ? gk::family_mfma_deep_nn : gk::family_mfma_deep_nt);
+    if (fn(key, args, grid, stream, mode, info, err, deep)) return 1;      // (op lists on A and B have none)
+  }
+  const gk::FamilyFn any = key.a_kmajor ? (key.b_kmajor ? gk::family_mfma_tn : gk::family_mfma_tt)
+                                        : (key.b_kmajor ? gk::family_mfma_nn : gk::family_mfma_nt);
+  return any(key, args, grid, stream, mode, info, err);
+}
+
 gk::FamilyFn family_fn(const gk::InstanceKey& key) {
   switch (key.family) {
     case gk::FAMILY_MFMA:
@@ -461,8 +491,7 @@ gk::FamilyFn family_fn(const gk::InstanceKey& key) {
       }
       [[fallthrough]];
     case gk::FAMILY_GETT:
-      if (key.a_kmajor) return key.b_kmajor ? gk::family_mfma_tn : gk::family_mfma_tt;
-      return key.b_kmajor ? gk::family_mfma_nn : gk::family_mfma_nt;
+      return family_mfma;
     case gk::FAMILY_FPU:
       return gk::family_fpu;
     case gk::FAMILY_DIAGONAL:
@@ -483,7 +512,8 @@ int find_instance(const gk_config* c, const gk_transforms* t, const gk_epilogue*
   gk::FamilyFn fn = family_fn(*key);
   gk::GemmArgs dummy;
   memset(&dummy, 0, sizeof(dummy));
-  dummy.M = c->matmul_shape.M; dummy.N = c->matmul_shape.N; dummy.K = c->matmul_shape.K;     // (instances that depend on the extents: tiles over the edges)
+  const int parts = key->family == gk::FAMILY_COMPLEX ? 2 : 1;      // (as make_args counts them)
+  dummy.M = parts * c->matmul_shape.M; dummy.N = parts * c->matmul_shape.N; dummy.K = c->matmul_shape.K;     // (instances that depend on the extents: tiles over the edges)
   hipError_t err = hipSuccess;
   if (key->family == gk::FAMILY_MFMA && allow_ragged_fast && ragged_fast_path(c) && (!fn || !fn(*key, dummy, dim3(1), nullptr, 0, info, &err))) {
     // no aligned instance of this tile: the bounds-checked kernel after all
@@ -496,6 +526,12 @@ int find_instance(const gk_config* c, const gk_transforms* t, const gk_epilogue*
                 "no compiled kernel instance for operator %d, block (%d, %d, %d), warps %d x %d, A/B layouts %d/%d, eltype %d",
                 c->op.kind, key->BM, key->BN, key->BK, key->waves_m, key->waves_n, c->global_a_layout.kind,
                 c->global_b_layout.kind, key->dtype);
+  }
+  // (the instance with more LDS stages that few tiles run on: not under a limit set by the caller that is too small for it)
+  const long long lds_max = g_lds_override.load();
+  if (lds_max > 0 && info->lds_bytes > lds_max && (key->family == gk::FAMILY_MFMA || key->family == gk::FAMILY_GETT || key->family == gk::FAMILY_COMPLEX)) {
+    key->variant |= gk::kShallow;
+    fn(*key, dummy, dim3(1), nullptr, 0, info, &err);
   }
   return GK_OK;
 }

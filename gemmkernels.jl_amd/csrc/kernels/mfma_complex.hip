@@ -13,7 +13,7 @@ namespace gk {
 
 int family_complex(const InstanceKey& key, const GemmArgs& args, dim3 grid, hipStream_t stream, int mode, InstanceInfo* info,
                    hipError_t* err) {
-  if (key.variant == 2) return family_complex_planar(key, args, grid, stream, mode, info, err);
+  if ((key.variant & ~kShallow) == 2) return family_complex_planar(key, args, grid, stream, mode, info, err);
   return family_complex_pair(key, args, grid, stream, mode, info, err);
 }
 

@@ -15,10 +15,15 @@
 
 namespace gk {
 
-int family_complex_pair(const InstanceKey& key, const GemmArgs& args, dim3 grid, hipStream_t stream, int mode, InstanceInfo* info,
+int family_complex_pair(const InstanceKey& as_asked, const GemmArgs& args, dim3 grid, hipStream_t stream, int mode, InstanceInfo* info,
                         hipError_t* err) {
+  InstanceKey key = as_asked;
+  key.variant &= ~kShallow;
   if (key.dtype != DT_F16 || (key.fused != 0 && key.fused != 3) || key.variant > 1) return 0;
   // every instance carries the hooks of C and D and the bias (FUSE level 3: they cost nothing when absent)
+  // 64 x 64 x 64 (a real tile of 128 x 128 x 64) with four LDS stages where every workgroup has a CU to itself, as
+  // the plain product (mfma_deep_instances.inc); the extents are those of the real product
+  const bool few = (as_asked.variant & kShallow) == 0 && (long long)((args.M + 127) / 128) * ((args.N + 127) / 128) <= kNumCUs;
 #define GK_PAIR(bm_, bn_, bk_, wm_, wn_, st_, akm_, bkm_, dual_, NAME)                                                     \
   if (key.BM == bm_ && key.BN == bn_ && key.BK == bk_ && key.waves_m == wm_ && key.waves_n == wn_ &&                      \
       key.a_kmajor == akm_ && key.b_kmajor == bkm_ && key.variant == dual_) {                                             \
@@ -46,12 +51,20 @@ int family_complex_pair(const InstanceKey& key, const GemmArgs& args, dim3 grid,
   GK_PAIR_SOLO(1, "mfma_dual_pair_nn_128x128x64_w2x2")
 #undef GK_PAIR_SOLO
   GK_PAIR_T(128, 128, 64, 2, 4, 2, 0, "complex_pair")
+  if (few) {
+    GK_PAIR_T(64, 64, 64, 2, 2, 4, 0, "complex_pair")
+  }
   GK_PAIR_T(64, 64, 64, 2, 2, 2, 0, "complex_pair")
   GK_PAIR_T(64, 64, 32, 2, 2, 4, 0, "complex_pair")
+  GK_PAIR_T(32, 32, 64, 2, 2, 4, 0, "complex_pair")
   GK_PAIR_T(32, 32, 32, 2, 2, 4, 0, "complex_pair")
   GK_PAIR_T(128, 128, 64, 2, 4, 2, 1, "dual_pair")
+  if (few) {
+    GK_PAIR_T(64, 64, 64, 2, 2, 4, 1, "dual_pair")
+  }
   GK_PAIR_T(64, 64, 64, 2, 2, 2, 1, "dual_pair")
   GK_PAIR_T(64, 64, 32, 2, 2, 4, 1, "dual_pair")
+  GK_PAIR_T(32, 32, 64, 2, 2, 4, 1, "dual_pair")
   GK_PAIR_T(32, 32, 32, 2, 2, 4, 1, "dual_pair")
 #undef GK_PAIR_T
 #undef GK_PAIR

@@ -15,9 +15,14 @@
 
 namespace gk {
 
-int family_complex_planar(const InstanceKey& key, const GemmArgs& args, dim3 grid, hipStream_t stream, int mode, InstanceInfo* info,
+int family_complex_planar(const InstanceKey& as_asked, const GemmArgs& args, dim3 grid, hipStream_t stream, int mode, InstanceInfo* info,
                           hipError_t* err) {
+  InstanceKey key = as_asked;
+  key.variant &= ~kShallow;
   if (key.dtype != DT_F16 || (key.fused != 0 && key.fused != 3) || key.variant != 2) return 0;
+  // 64 x 64 x 64 (a real tile of 128 x 128 x 64) with four LDS stages where every workgroup has a CU to itself, as
+  // the plain product (mfma_deep_instances.inc); the extents are those of the real product
+  const bool few = (as_asked.variant & kShallow) == 0 && (long long)((args.M + 127) / 128) * ((args.N + 127) / 128) <= kNumCUs;
 #define GK_PLANAR(bm_, bn_, bk_, wm_, wn_, st_, akm_, bkm_, NAME)                                                          \
   if (key.BM == bm_ && key.BN == bn_ && key.BK == bk_ && key.waves_m == wm_ && key.waves_n == wn_ &&                      \
       key.a_kmajor == akm_ && key.b_kmajor == bkm_) {                                                                     \
@@ -47,8 +52,12 @@ int family_complex_planar(const InstanceKey& key, const GemmArgs& args, dim3 gri
   GK_PLANAR_SOLO(1, 0, "mfma_complex_planar_tt_128x128x64_w2x2")
 #undef GK_PLANAR_SOLO
   GK_PLANAR_T(128, 128, 64, 2, 4, 2)
+  if (few) {
+    GK_PLANAR_T(64, 64, 64, 2, 2, 4)
+  }
   GK_PLANAR_T(64, 64, 64, 2, 2, 2)
   GK_PLANAR_T(64, 64, 32, 2, 2, 4)
+  GK_PLANAR_T(32, 32, 64, 2, 2, 4)
   GK_PLANAR_T(32, 32, 32, 2, 2, 4)
 #undef GK_PLANAR_T
 #undef GK_PLANAR

@@ -18,6 +18,10 @@ struct InstanceKey {
   int variant;       // family specific
 };
 
+// Bit of InstanceKey::variant (matrix-core families): the instance with the fewest LDS stages, whatever the tiles of the launch
+// (set by the host where the one with more stages asks for more LDS than the device limit in force allows).
+constexpr int kShallow = 0x100;
+
 enum : int { FAMILY_MFMA = 0, FAMILY_MFMA_CHECKED = 1, FAMILY_FPU = 2, FAMILY_COMPLEX = 3, FAMILY_DIAGONAL = 4, FAMILY_GETT = 5 };
 
 struct InstanceInfo {
@@ -65,6 +69,11 @@ int family_mfma_tn(const InstanceKey&, const GemmArgs&, dim3, hipStream_t, int, 
 int family_mfma_nn(const InstanceKey&, const GemmArgs&, dim3, hipStream_t, int, InstanceInfo*, hipError_t*);
 int family_mfma_nt(const InstanceKey&, const GemmArgs&, dim3, hipStream_t, int, InstanceInfo*, hipError_t*);
 int family_mfma_tt(const InstanceKey&, const GemmArgs&, dim3, hipStream_t, int, InstanceInfo*, hipError_t*);
+// (four LDS stages where `deep`; 64 x 64 x 64 contractions with two otherwise)
+int family_mfma_deep_tn(const InstanceKey&, const GemmArgs&, dim3, hipStream_t, int, InstanceInfo*, hipError_t*, bool deep);
+int family_mfma_deep_nn(const InstanceKey&, const GemmArgs&, dim3, hipStream_t, int, InstanceInfo*, hipError_t*, bool deep);
+int family_mfma_deep_nt(const InstanceKey&, const GemmArgs&, dim3, hipStream_t, int, InstanceInfo*, hipError_t*, bool deep);
+int family_mfma_deep_tt(const InstanceKey&, const GemmArgs&, dim3, hipStream_t, int, InstanceInfo*, hipError_t*, bool deep);
 int family_mfma_wide_tn(const InstanceKey&, const GemmArgs&, dim3, hipStream_t, int, InstanceInfo*, hipError_t*);
 int family_mfma_wide_tn_192x256(const InstanceKey&, const GemmArgs&, dim3, hipStream_t, int, InstanceInfo*, hipError_t*);
 int family_mfma_wide_nn(const InstanceKey&, const GemmArgs&, dim3, hipStream_t, int, InstanceInfo*, hipError_t*);

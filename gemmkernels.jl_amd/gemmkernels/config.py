@@ -164,7 +164,7 @@ TUNED = {}
 
 
 # tiles compiled with tensor-contraction addressing
-_GETT_TILES = [(256, 256, 64), (128, 128, 64), (64, 64, 32)]
+_GETT_TILES = [(256, 256, 64), (128, 128, 64), (64, 64, 64), (64, 64, 32)]
 
 
 def default_block_shape(operator, gemm_shape, tile_sized: bool = True, gett: bool = False, planar: bool = False,
@@ -188,11 +188,12 @@ def default_block_shape(operator, gemm_shape, tile_sized: bool = True, gett: boo
         # complex tiles, in complex elements
         table = _complex_tiles(operator, planar, a_kmajor, b_kmajor)
         fitting = [t for t, _ in table if M % t[0] == 0 and N % t[1] == 0 and K % t[2] == 0]
-        for t in fitting:
-            if (M // t[0]) * (N // t[1]) >= NUM_CUS:
-                return NT(M=t[0], N=t[1], K=t[2])
-        t = fitting[-1] if fitting else (64, 64, 32)
-        return NT(M=t[0], N=t[1], K=t[2])
+        if not fitting:
+            return NT(M=64, N=64, K=32)
+        # (one real product of twice the rows and columns; 32 x 32 x 64 has four LDS stages, of which a CU holds two tiles)
+        fitting = [t for t in fitting if t != (32, 32, 64) or (M // 32) * (N // 32) <= 2 * NUM_CUS] or fitting
+        best = min(fitting, key=lambda t: (_mfma_cost((2 * t[0], 2 * t[1], t[2]), 2 * M, 2 * N, K, False), fitting.index(t)))
+        return NT(M=best[0], N=best[1], K=best[2])
     # sizes need not be whole tiles when the layouts are the bounds-checked ones (the aligned kernels mask the
     # last tile row / column and zero the end of the last K tile)
     table = [t for t, _ in _MFMA_TILES] + [t for t, _, has in _MFMA_TILES_192 if has(a_kmajor, b_kmajor)]
@@ -201,37 +202,16 @@ def default_block_shape(operator, gemm_shape, tile_sized: bool = True, gett: boo
         fitting = [t for t in fitting if t in _GETT_TILES]
     if not fitting:
         return NT(M=64, N=64, K=32)
-    # time of the launch in units of "one CU multiplying at the rate of the 256 x 256 x 64 tile": a tile costs its area
-    # over the rate of its kernel when it has a CU to itself (_MFMA_TILE_RATE), and a CU works through its share of the
-    # tiles in rounds (_rounds: whole rounds for the tiles of which a CU holds one at a time, overlapping ones for the
-    # smaller tiles).  Ties go to the tile listed first.
-    def cost(t):
-        tiles = -(-M // t[0]) * -(-N // t[1])
-        per_cu = tiles / NUM_CUS
-        rate = _MFMA_TILE_RATE.get(t, 0.3)
-        if isinstance(rate, tuple):
-            rate = rate[0] if per_cu <= 1 else rate[1]
-        if t == (256, 192, 64) and not a_kmajor and not b_kmajor and (M % t[0] or N % t[1] or K % t[2]):
-            rate = 0.70      # 'N','T' on eight waves (tiles over the edges): the 192 side is read with transposing LDS reads
-        if t == (64, 64, 32) and per_cu <= 1 and K >= 2048:
-            rate = 0.24      # a lone workgroup on a long K: four stages in flight instead of two (1024 x 1024 x 4096: 23.4 us, 64 x 64 x 64: 34.1)
-        return _rounds(t, tiles) * t[0] * t[1] / rate
-    best = min(fitting, key=lambda t: (cost(t), fitting.index(t)))
+    # the shortest estimated launch (_MFMA_TILE_COST); ties go to the tile listed first
+    best = min(fitting, key=lambda t: (_mfma_cost(t, M, N, K), fitting.index(t)))
     return NT(M=best[0], N=best[1], K=best[2])
 
 
 def split_k_block_shape(M, N, K, widest_ld=0, factor=None) -> Optional[NT]:
-    """The tile of a 16-bit product that is worth cutting into slices of K (``Kernel.matmul_split_k``), or None: few output
-    tiles, which alone leave CUs idle, and a long K.  Measured against the best tile unsplit: 4096 x 64 x 4096 12.6 us
-    against 22.0, 300 x 500 x 4000 13.0 against 23.6, 64 x 64 x 8000 9.8 against 38.9, 2000 x 100 x 1500 12.3 against 17.5,
-    256 x 256 x 1280 7.6 against 8.3 (x 1024 8.9 against 7.1); three slices of 129 .. 170 tiles 700 x 900 x 3001 19.7
-    against 23.3.  More tiles leave two slices, which pay where K or the output is whole tiles (1024 x 1024 x 4096 20.6
-    against 22.7, 1001 x 704 x 3328 20.9 against 22.5, 1024 x 768 x 4004 21.7 against 23.8; but 1001 x 700 x 3333 26.6 against
-    24.6, 1000 x 1000 x 4000 25.4 against 24.6), or where A has a factor that stays in the loop (``factor``): "packed",
-    FP16, 1001 x 700 x 3333 27.4 against 31.9; "per element", BF16, keeps the vector ALUs of every CU that has a tile busy,
-    so only where the slices still spread (768 x 1024 x 4096 105 against 113; 1001 x 1001 x 5001 161 against 141, 70 x 7000
-    x 3500 116 against 101, 12000 x 64 x 4096 122 against 114).  ``widest_ld``: the larger leading dimension of the operands whose rows are the k of a tile; the
-    kernel keeps the offsets in a tile in 32 bits, so 64 rows of 2^24 elements are left to a tile with fewer."""
+    """The tile of a 16-bit product with few output tiles and a long K, or None (the default tile).  ``factor``: how alpha is applied to A
+    in the K loop ("packed", FP16; "per element", BF16).  ``widest_ld``: the larger leading dimension of the operands whose rows are the k
+    of a tile; the kernel keeps the offsets in a tile in 32 bits, so 64 rows of 2^24 elements are left to a tile with fewer.  Whether the
+    product is cut into slices of K as well: ``slices_pay``."""
     if 64 * widest_ld * 2 >= 1 << 31:
         return None
     tiles = -(-M // 64) * -(-N // 64)
@@ -244,30 +224,55 @@ def split_k_block_shape(M, N, K, widest_ld=0, factor=None) -> Optional[NT]:
     return NT(M=64, N=64, K=64) if worth else None
 
 
-# Throughput of a CU that has one tile at a time, relative to 256 x 256 x 64 on four waves; a pair: a launch with at most
-# one tile per CU, a launch with several (the small tiles are bound by latency when alone).  From timings of every tile
-# and panel height at 1024^3 ... 6144^3 and eight rectangular problems ('N','N', three interleaved passes each):
-# e.g. 4096^3 takes 99 us on 256 x 256 x 64, 131 on 128 x 128 x 64, 134 on 128 x 256 x 64, 194 on 64 x 64 x 64;
-# 2560^3 42.2 us on 128 x 128 x 64 (400 tiles), 45.5 on 128 x 256 x 64 (200), 53.1 on 256 x 256 x 64 (100).
-_MFMA_TILE_RATE = {(256, 256, 64): 1.0, (256, 256, 32): 0.68, (256, 128, 64): (0.61, 0.70), (128, 256, 64): (0.62, 0.72),
-                   (128, 128, 32): (0.415, 0.345), (128, 128, 64): 0.39, (64, 64, 64): 0.169, (64, 64, 32): (0.163, 0.13),
-                   (256, 192, 64): 0.86, (192, 256, 64): 0.86}
+def slices_pay(M, N, K, factor=None) -> bool:
+    """Whether a product on the tile of ``split_k_block_shape`` is worth cutting into slices of K (``Kernel.matmul_split_k``), next to the four
+    LDS stages that carry a lone workgroup through K at 0.22 us per 64 k.  In us, slices against unsplit: 64 tiles K = 1280 7.5 and 7.5,
+    2048 8.7 and 10.5, 4096 11.1 and 17.6; 128 tiles K = 1280 8.6 and 7.9, 2048 9.8 and 10.7; three slices of 165 tiles 3072 13.0 and 14.7, 4096
+    14.3 and 18.1; two slices of 180 .. 256 tiles gain nothing (180 tiles K = 4096 17.7 and 18.0, 256 tiles 19.1 and 18.4).  A factor that stays
+    in the K loop makes it longer: FP16 111 x 2629 x 1477 (84 tiles) 15.7 and 19.9, BF16 768 x 1024 x 4096 (192) 105 and 113."""
+    return factor is not None or -(-M // 64) * -(-N // 64) <= 170
+
+
+# Estimated launch time of a tile, in microseconds: what a launch costs whatever its size, per 1000 k and round, per further tile of
+# a CU, for a partial last K tile (times the square root of the rounds), for tiles over the edges.  Fitted, weighted towards the tiles near the
+# best, to timings of every tile at 61 sizes from 1000 x 1000 x 64 to 4416 x 4416 x 1024 ('N','N' and 'T','N'; whole tiles, multiples of 64 and odd ones; inputs
+# that rotate through 200 MB and more): the tile the estimate picks is 1.5 % behind the best one on average, 11 % at most.  E.g. 1024^3 7.6 us on 64 x 64 x 64,
+# 12.6 on 128 x 128 x 64, 25.8 on 256 x 256 x 64; 2048^3 26.6, 23.5 and 41.1; 4096 x 2048 x 4096 92, 64.5 and 71.9; 3072^3 51.8 on
+# 256 x 192 x 64, 58.8 on 256 x 256 x 64; 5913 x 6229 x 20 39.0 on 64 x 64 x 32, 53.4 on 64 x 64 x 64, 66.6 on 256 x 256 x 64.
+_MFMA_TILE_COST = {(256, 256, 64): (12.0, 16.4, 39.0, 21.0, 1.2), (256, 256, 32): (12.2, 29.2, 20.7, 5.7, 6.8),
+                   (256, 128, 64): (8.8, 13.5, 7.8, 15.5, 7.9), (128, 256, 64): (8.9, 12.9, 7.4, 17.4, 7.4),
+                   (128, 128, 32): (6.7, 7.5, 1.9, 4.9, 3.6), (128, 128, 64): (6.7, 7.5, 1.9, 8.5, 3.6),
+                   (64, 64, 64): (3.5, 3.5, 0.4, 3.7, 1.6), (64, 64, 32): (3.3, 4.6, 0.4, 2.0, 1.6),
+                   (256, 192, 64): (5.4, 17.1, 19.3, 9.1, 7.9), (192, 256, 64): (5.0, 17.1, 15.3, 10.4, 7.9)}
 
 
 def _rounds(t, tiles):
     """How many tile times a launch of ``tiles`` tiles of shape ``t`` takes.  A CU holds one workgroup of the tiles with
-    144 or 128 KiB of LDS at a time: whole rounds.  Of the 128 x 128 tiles it holds two, which run side by side in 1.15
-    times the time of one (2560^3, 400 tiles: 1.17; 4096^3, 1024 tiles: 2.27 = two such rounds); of the 64 x 64 tiles
-    four and more, whose time grows by about a third of a tile time per further tile of a CU (1536^3, 2.25 per CU: 1.43;
-    3072^3, 9 per CU: 3.8)."""
+    144 or 128 KiB of LDS at a time: whole rounds.  The 128 x 128 tiles run one per CU on four LDS stages where every tile has a CU,
+    and two per CU on two stages beyond that (tiles per CU and tile times: 1.1 1.55, 1.27 1.6, 1.56 1.77, 2.0 1.9; 2.25 3.7, 3.5 3.9, 4.8 6.7).  The 64 x 64
+    tiles: two of four stages side by side take 1.8 times one (2048 x 1024 x 4096 29.5 us, 1024 x 1024 x 4096 18.7), more of two stages share a CU
+    at one tile time each."""
     per_cu = tiles / NUM_CUS
     if t[0] * t[1] >= 128 * 256:
         return -(-tiles // NUM_CUS)
     if per_cu <= 1:
         return 1.0
     if t[0] * t[1] >= 128 * 128:
-        return 1.15 * -(-tiles // (2 * NUM_CUS))
-    return 1.0 + 0.36 * (per_cu - 1.0)
+        rounds = 1.3 + 0.28 * per_cu if per_cu <= 2 else 1.85 * -(-tiles // (2 * NUM_CUS))
+        return rounds if t[2] >= 64 else 1.15 * rounds
+    return 1.0 + 0.82 * (per_cu - 1.0) if per_cu <= 2 else 0.95 * per_cu
+
+
+def _mfma_cost(t, M, N, K, pairs=True):
+    """Estimated microseconds of a product in real tiles of shape ``t`` (``pairs``: a plain one)."""
+    tiles = -(-M // t[0]) * -(-N // t[1])
+    if pairs and t == (64, 64, 32) and tiles <= 2 * NUM_CUS and (K % 64 == 0 or K >= 1536):
+        # the library runs these on 64 x 64 x 64 with four stages; a lone workgroup on a long K is named 64 x 64 x 32 (any leading dimension)
+        return _mfma_cost((64, 64, 64), M, N, K) - (0.01 if tiles <= NUM_CUS and K >= 2048 else 0.0)
+    fixed, per_k, further, tail, edges = _MFMA_TILE_COST[t]
+    rounds = _rounds(t, tiles)
+    return (fixed + rounds * per_k * K * 1e-3 + further * max(tiles / NUM_CUS - 1.0, 0.0) + (tail * rounds ** 0.5 if K % t[2] else 0.0)
+            + (edges if M % t[0] or N % t[1] else 0.0))
 
 
 # FPUOp on the FP32 / FP64 matrix instructions: time of a tile per 1000 k, in microseconds, when every CU has one tile at most
@@ -280,11 +285,11 @@ _FPU_TILE_COST = {("Float32", "Float32"): {(128, 128, 32): (65.0, 63.0), (64, 64
 
 # complex / dual tiles (complex elements) -> waves: one real product of the real views of A and B, whose real tile
 # has twice the rows and columns; the same table for every transpose
-_COMPLEX_PAIR_TILES = [((128, 128, 64), (2, 4)), ((64, 64, 64), (2, 2)), ((64, 64, 32), (2, 2)), ((32, 32, 32), (2, 2))]
+_COMPLEX_PAIR_TILES = [((128, 128, 64), (2, 4)), ((64, 64, 64), (2, 2)), ((64, 64, 32), (2, 2)), ((32, 32, 64), (2, 2)), ((32, 32, 32), (2, 2))]
 
 # complex tiles (complex elements) of the kernel for planar global matrices -> waves; the real tile has twice
 # the rows and columns (both planes of A, B and D)
-_PLANAR_TILES = [((128, 128, 64), (2, 4)), ((64, 64, 64), (2, 2)), ((64, 64, 32), (2, 2)), ((32, 32, 32), (2, 2))]
+_PLANAR_TILES = [((128, 128, 64), (2, 4)), ((64, 64, 64), (2, 2)), ((64, 64, 32), (2, 2)), ((32, 32, 64), (2, 2)), ((32, 32, 32), (2, 2))]
 
 # tiles of FPUOp and of the bounds-checked MFMA kernel
 _FPU_TILES = [((64, 64, 32), (2, 2)), ((128, 128, 16), (2, 2)), ((128, 128, 32), (2, 2)), ((32, 32, 32), (2, 2)), ((32, 32, 32), (1, 1))]

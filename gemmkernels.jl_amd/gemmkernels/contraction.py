@@ -25,7 +25,7 @@ from . import _lib
 from . import kernel as Kernel
 from . import layout as Layout
 from . import operator as Operator
-from .config import _GETT_TILES, NUM_CUS, get_config
+from .config import _GETT_TILES, _mfma_cost, get_config
 from .dtypes import BFloat16, DType, Float16, Float32
 from .errors import ConfigError
 from .tiling import NT
@@ -122,13 +122,13 @@ def candidates(spec: str, extents: Dict[str, int], ab_type: DType = Float16, cd_
         am, bm = (b2, a2) if swapped else (a2, b2)
         gmap = Layout.gett_map(am, bm, d2, ext)
         M, N, K = gmap.extent("m"), gmap.extent("n"), gmap.extent("k")
-        tiles = [t for t in _GETT_TILES if M % t[0] == 0 and N % t[1] == 0 and gmap.k[0][0] % t[2] == 0]
+        tiles = [t for t in _GETT_TILES if M % t[0] == 0 and N % t[1] == 0 and K % t[2] == 0]
         if not tiles:
-            yield swapped, groups, None, (f"no tile divides M = {M}, N = {N} and the first K mode of {gmap.k[0][0]} "
+            yield swapped, groups, None, (f"no tile divides M = {M}, N = {N} and K = {K} "
                                           f"(tiles {_GETT_TILES})")
             continue
-        filling = [t for t in tiles if (M // t[0]) * (N // t[1]) >= NUM_CUS]
-        for t in (filling[:1] or tiles[-1:]) + [u for u in tiles if u not in (filling[:1] or tiles[-1:])]:
+        # the tile with the shortest estimated launch first; the library says which of them tile the K modes
+        for t in sorted(tiles, key=lambda t: _mfma_cost(t, M, N, K, False)):
             try:
                 conf = get_config(gemm_shape=NT(M=M, N=N, K=K), operator=Operator.MFMAOp[32, 32, 16, ab_type, Float32],
                                   global_a_layout=Layout.GETT[ab_type, gmap], global_b_layout=Layout.GETT[ab_type, gmap],

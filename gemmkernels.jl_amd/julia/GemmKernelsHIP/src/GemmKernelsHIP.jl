@@ -338,23 +338,37 @@ end
 # block shape -> waves (M x N) of the instances compiled into the library
 const MFMA_TILES = [((256, 256, 64), (2, 4)), ((256, 256, 32), (2, 4)), ((256, 128, 64), (2, 2)), ((128, 256, 64), (2, 2)),
                     ((128, 128, 32), (2, 2)), ((128, 128, 64), (2, 2)), ((64, 64, 64), (2, 2)), ((64, 64, 32), (2, 2))]
-# throughput of a CU that has one tile at a time, relative to 256 x 256 x 64 on four waves, measured; a pair: a launch with
-# at most one tile per CU, a launch with several (the small tiles are bound by latency when alone)
-const MFMA_TILE_RATE = Dict((256, 256, 64) => (1.0, 1.0), (256, 256, 32) => (0.68, 0.68), (256, 128, 64) => (0.61, 0.70),
-                            (128, 256, 64) => (0.62, 0.72), (128, 128, 32) => (0.415, 0.345), (128, 128, 64) => (0.39, 0.39),
-                            (64, 64, 64) => (0.169, 0.169), (64, 64, 32) => (0.163, 0.13))
-# tile times of a launch: whole rounds for the tiles of which a CU holds one at a time; two 128 x 128 tiles run side by side
-# in 1.15 times the time of one; the time of 64 x 64 tiles grows by about a third of a tile time per further tile of a CU
+# estimated launch time of a tile in microseconds: whatever the size, per 1000 k and round, per further tile of a CU, for a partial
+# last K tile, for tiles over the edges (fitted to measured launches, see _MFMA_TILE_COST of the Python package)
+const MFMA_TILE_COST = Dict((256, 256, 64) => (12.0, 16.4, 39.0, 21.0, 1.2), (256, 256, 32) => (12.2, 29.2, 20.7, 5.7, 6.8),
+                            (256, 128, 64) => (8.8, 13.5, 7.8, 15.5, 7.9), (128, 256, 64) => (8.9, 12.9, 7.4, 17.4, 7.4),
+                            (128, 128, 32) => (6.7, 7.5, 1.9, 4.9, 3.6), (128, 128, 64) => (6.7, 7.5, 1.9, 8.5, 3.6),
+                            (64, 64, 64) => (3.5, 3.5, 0.4, 3.7, 1.6), (64, 64, 32) => (3.3, 4.6, 0.4, 2.0, 1.6))
+# tile times of a launch: whole rounds for the tiles of which a CU holds one at a time; 128 x 128 tiles two to a CU beyond one
+# each; 64 x 64 tiles share a CU at about one tile time each
 function tile_rounds(t, tiles)
     per_cu = tiles / NUM_CUS
     t[1] * t[2] >= 128 * 256 && return Float64(cld(tiles, NUM_CUS))
     per_cu <= 1 && return 1.0
-    t[1] * t[2] >= 128 * 128 && return 1.15 * cld(tiles, 2 * NUM_CUS)
-    1.0 + 0.36 * (per_cu - 1.0)
+    if t[1] * t[2] >= 128 * 128
+        rounds = per_cu <= 2 ? 1.3 + 0.28 * per_cu : 1.85 * cld(tiles, 2 * NUM_CUS)
+        return t[3] >= 64 ? rounds : 1.15 * rounds
+    end
+    per_cu <= 2 ? 1.0 + 0.82 * (per_cu - 1.0) : 0.95 * per_cu
+end
+function tile_cost(t, M, N, K; pairs = true)
+    tiles = cld(M, t[1]) * cld(N, t[2])
+    if pairs && t == (64, 64, 32) && tiles <= 2 * NUM_CUS && (K % 64 == 0 || K >= 1536)      # runs on 64 x 64 x 64 with four stages
+        return tile_cost((64, 64, 64), M, N, K) - (tiles <= NUM_CUS && K >= 2048 ? 0.01 : 0.0)
+    end
+    fixed, per_k, further, tail, edges = MFMA_TILE_COST[t]
+    rounds = tile_rounds(t, tiles)
+    fixed + rounds * per_k * K * 1e-3 + further * max(tiles / NUM_CUS - 1.0, 0.0) + (K % t[3] != 0 ? tail * sqrt(rounds) : 0.0) +
+        (M % t[1] != 0 || N % t[2] != 0 ? edges : 0.0)
 end
 # complex / dual tiles (complex elements): one real product of the real views of A and B (interleaved or planar),
 # the same table for every transpose
-const COMPLEX_PAIR_TILES = [((128, 128, 64), (2, 4)), ((64, 64, 64), (2, 2)), ((64, 64, 32), (2, 2)), ((32, 32, 32), (2, 2))]
+const COMPLEX_PAIR_TILES = [((128, 128, 64), (2, 4)), ((64, 64, 64), (2, 2)), ((64, 64, 32), (2, 2)), ((32, 32, 64), (2, 2)), ((32, 32, 32), (2, 2))]
 complex_tiles(operator::Type, a_kmajor::Bool, b_kmajor::Bool; planar::Bool = false) = COMPLEX_PAIR_TILES
 const FPU_TILES = [((64, 64, 32), (2, 2)), ((128, 128, 16), (2, 2)), ((128, 128, 32), (2, 2)), ((32, 32, 32), (2, 2)), ((32, 32, 32), (1, 1))]
 # FPUOp on the FP32 / FP64 matrix instructions: microseconds per 1000 k of a tile that has a CU to itself, and of each of several
@@ -392,21 +406,15 @@ function default_block_shape(operator::Type, gemm_shape; tile_sized::Bool = true
         return (M = best[1], N = best[2], K = best[3])
     elseif !Operator.is_mfma(operator)
         fitting = [t for (t, _) in complex_tiles(operator, a_kmajor, b_kmajor; planar = planar) if M % t[1] == 0 && N % t[2] == 0 && K % t[3] == 0]
-        for t in fitting
-            (M ÷ t[1]) * (N ÷ t[2]) >= NUM_CUS && return (M = t[1], N = t[2], K = t[3])
-        end
-        t = isempty(fitting) ? (64, 64, 32) : fitting[end]
+        isempty(fitting) && return (M = 64, N = 64, K = 32)
+        few = [t for t in fitting if t != (32, 32, 64) || (M ÷ 32) * (N ÷ 32) <= 2 * NUM_CUS]
+        isempty(few) || (fitting = few)
+        t = fitting[argmin(map(t -> tile_cost((2 * t[1], 2 * t[2], t[3]), 2M, 2N, K; pairs = false), fitting))]      # one real product of twice the rows and columns
         return (M = t[1], N = t[2], K = t[3])
     end
     fitting = [t for (t, _) in MFMA_TILES if !tile_sized || (M % t[1] == 0 && N % t[2] == 0 && K % t[3] == 0)]
     isempty(fitting) && return (M = 64, N = 64, K = 32)
-    function cost(t)
-        tiles = cld(M, t[1]) * cld(N, t[2])
-        rate = MFMA_TILE_RATE[t][tiles <= NUM_CUS ? 1 : 2]
-        t == (64, 64, 32) && tiles <= NUM_CUS && K >= 2048 && (rate = 0.24)      # a lone workgroup on a long K: four stages in flight
-        tile_rounds(t, tiles) * t[1] * t[2] / rate
-    end
-    best = fitting[argmin(map(cost, fitting))]
+    best = fitting[argmin(map(t -> tile_cost(t, M, N, K), fitting))]
     (M = best[1], N = best[2], K = best[3])
 end
 
@@ -769,7 +777,7 @@ function create_config(A::Type, sizeA::Dims, stridesA::Dims, transA::Bool,
     (conf, compute_type, select_kernel(ga, gb))
 end
 
-# a 16-bit product with few 64 x 64 output tiles and a long K runs on slices of K (the sizes: split_k_block_shape of the Python package),
+# a 16-bit product with few 64 x 64 output tiles and a long K runs on tiles of 64 x 64 x 64 (the sizes: split_k_block_shape of the Python package),
 # unless its operands' 64 rows of k lie further apart than 32-bit offsets reach
 function worth_splitting(m, n, k, widest_ld, factor)
     64 * widest_ld * 2 < 2^31 || return false
@@ -779,6 +787,8 @@ function worth_splitting(m, n, k, widest_ld, factor)
     two = factor === :none ? whole : factor === :packed || (tiles <= 225 && min(m, n) > 128)
     k >= 3000 && (tiles <= 170 || (tiles <= 256 && two))
 end
+# ... and these are the ones that slices make faster than four LDS stages do (slices_pay of the Python package)
+slices_pay(m, n, k, factor) = factor !== :none || cld(m, 64) * cld(n, 64) <= 170
 # alpha stays in the K loop unless it is a power of two that the library folds into the accumulators
 factor_of(alpha, A, B) = abs(Float64(alpha)) in (2.0 .^ (-4:4)) ? :none : (:BFloat16 in (nameof(eltype(A)), nameof(eltype(B))) ? :per_element : :packed)
 
@@ -806,7 +816,9 @@ function matmatmul!(C, transA::Char, transB::Char, A, B, alpha::Number, beta::Nu
     if Operator.is_mfma(conf.operator)
         # few output tiles and a long K loop: K slices as workgroups of one launch (ordered sum: same bits every run)
         bs, ms = conf.block_shape, conf.matmul_shape
-        if bs == (M = 64, N = 64, K = 64) && worth_splitting(ms.M, ms.N, ms.K, 0, factor_of(alpha, A, B)) || cld(ms.M, bs.M) * cld(ms.N, bs.N) <= 256 && ms.K >= 2048
+        factor = factor_of(alpha, A, B)
+        few = bs == (M = 64, N = 64, K = 64) && worth_splitting(ms.M, ms.N, ms.K, 0, factor)
+        if few ? slices_pay(ms.M, ms.N, ms.K, factor) : cld(ms.M, bs.M) * cld(ms.N, bs.N) <= 128 && ms.K >= 2048
             kernel = Kernel.matmul_split_k
         end
     end
