@@ -230,8 +230,9 @@ int make_key_as_configured(const gk_config* c, const gk_transforms* t, const gk_
     return GK_OK;
   }
   if (key->fused && t && (key->family == gk::FAMILY_MFMA || key->family == gk::FAMILY_GETT)) {
-    // level 1 covers A / B hooks that are one exact 16-bit scale (or nothing); anything else needs
+    // level 1 covers A / B hooks that are one exact FP16 scale (or nothing), and for BF16 one scale of A; anything else needs
     // the generic per-element path of level 2
+    const bool bf16 = c->global_a_layout.eltype == GK_BF16 && key->family == gk::FAMILY_MFMA;
     auto simple = [&](int h0, int h1) {
       const gk_transform& a0 = t->hook[h0];
       const gk_transform& a1 = t->hook[h1];
@@ -240,12 +241,13 @@ int make_key_as_configured(const gk_config* c, const gk_transforms* t, const gk_
       for (int i = 0; i < a0.n_ops && i < GK_MAX_OPS; ++i) if (a0.ops[i].kind != GK_T_IDENTITY) { ++n; one = &a0.ops[i]; }
       for (int i = 0; i < a1.n_ops && i < GK_MAX_OPS; ++i) if (a1.ops[i].kind != GK_T_IDENTITY) { ++n; one = &a1.ops[i]; }
       if (n == 0) return true;
-      if (n != 1 || one->kind != GK_T_SCALE || c->global_a_layout.eltype != GK_F16) return false;
-      return (float)(_Float16)one->p0 == one->p0;
+      if (n != 1 || one->kind != GK_T_SCALE) return false;
+      if (bf16) return h0 == GK_HOOK_GLOBAL_TO_SHARED_A;
+      return c->global_a_layout.eltype == GK_F16 && (float)(_Float16)one->p0 == one->p0;
     };
     if (!simple(GK_HOOK_GLOBAL_TO_SHARED_A, GK_HOOK_SHARED_TO_REGS_A) || !simple(GK_HOOK_GLOBAL_TO_SHARED_B, GK_HOOK_SHARED_TO_REGS_B))
       key->fused = 2;
-    if (c->global_a_layout.eltype != GK_F16) key->fused = 2;   // level 1 is compiled for FP16 only
+    if (c->global_a_layout.eltype != GK_F16 && !bf16) key->fused = 2;   // (level 1 is not compiled for other types)
   }
   if (key->fused && t && key->family == gk::FAMILY_FPU) {
     // floating-point FPUOp: level 1 is compiled for at most one scale on A, on B and on C, level 2 for any lists
@@ -405,7 +407,7 @@ void make_args(const gk_config* c, const void* a, const void* b, const void* cc,
       dst.n = out;
     }
   }
-  // one exact FP16 scale over the two load hooks of an operand -> packed multiply in the kernel
+  // one exact FP16 scale (BF16: any) over the two load hooks of an operand -> a multiply per fragment in the kernel
   auto single_scale = [&](int h0, int h1, int* fast, float* scale) {
     const gk::OpList& a0 = args->t[h0];
     const gk::OpList& a1 = args->t[h1];
@@ -415,7 +417,7 @@ void make_args(const gk_config* c, const void* a, const void* b, const void* cc,
     const gk::OpList& one = a0.n ? a0 : a1;
     if (one.kind[0] != GK_T_SCALE) return;
     const float v = one.p0[0];
-    if ((float)(_Float16)v != v) return;
+    if (c->global_a_layout.eltype != GK_BF16 && (float)(_Float16)v != v) return;      // (BF16: multiplied in fp32)
     *fast = 1;
     *scale = v;
   };
@@ -475,6 +477,11 @@ int family_mfma(const gk::InstanceKey& as_asked, const gk::GemmArgs& args, dim3 
     const auto fn = key.a_kmajor ? (key.b_kmajor ? gk::family_mfma_deep_tn : gk::family_mfma_deep_tt)
                                  : (key.b_kmajor ? gk::family_mfma_deep_nn : gk::family_mfma_deep_nt);
     if (fn(key, args, grid, stream, mode, info, err, deep)) return 1;      // (op lists on A and B have none)
+  }
+  if (key.dtype == gk::DT_BF16 && key.fused == 1 && key.family == gk::FAMILY_MFMA) {
+    const gk::FamilyFn scaled = key.a_kmajor ? (key.b_kmajor ? gk::family_mfma_bf16_scaled_tn : gk::family_mfma_bf16_scaled_tt)
+                                             : (key.b_kmajor ? gk::family_mfma_bf16_scaled_nn : gk::family_mfma_bf16_scaled_nt);
+    return scaled(key, args, grid, stream, mode, info, err);
   }
   const gk::FamilyFn any = key.a_kmajor ? (key.b_kmajor ? gk::family_mfma_tn : gk::family_mfma_tt)
                                         : (key.b_kmajor ? gk::family_mfma_nn : gk::family_mfma_nt);
@@ -1133,7 +1140,7 @@ static_assert(kSplitCounterBytes / sizeof(unsigned) >= 2 * (size_t)gk::kNumCUs -
 //   1776 x 33 x 7392 (28) 7 14.4, 8 14.4, 11 16.0; 300 x 200 x 9001 (20) 9 15.4, 14 18.9; 1085 x 47 x 6136 (17) 6 15.0, 9 13.9;
 //   64 x 64 x 8000 (1) 7 10.6, 12 10.0; 64 x 64 x 32768 (1) 24 15.3, 32 15.8, 51 18.0.
 // A factor on A or B (AB_HOOKS) makes the K loop longer and what a slice costs weigh less: up to two per CU.  FP16 4096 x 64 x 4096
-//   'T','N' 4 13.8, 6 12.9; BF16 4 66.5, 6 61.6, 8 57.0; BF16 7 x 7 x 20000 (1) 19 54.2, 31 46.6.
+//   'T','N' 4 13.8, 6 12.9; BF16 with op lists on A (level 2) 4 66.5, 6 61.6, 8 57.0, 7 x 7 x 20000 (1) 19 54.2, 31 46.6.
 // 128 x 128 x 64, whose partial tiles are four times as large: 768 deep (1024 above 64 tiles), sixteen slices or 2048 deep:
 //   512 x 512 x 4096 (16) 4 22.7, 5 22.0, 6 21.8; 2048 x 512 x 4096 (64) 4 25.3, 5 25.3, 6 26.2; 1536 x 1024 x 4096 (96) 4 29.5, 5 30.6;
 //   256 x 256 x 16384 (4) 12 34.4, 16 35.5, 25 40.2.

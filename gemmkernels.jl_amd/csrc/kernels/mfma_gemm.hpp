@@ -428,6 +428,27 @@ __device__ __forceinline__ int4v scale_fragment_f16(int4v f, float scale) {
   return __builtin_bit_cast(int4v, v);
 }
 
+// The same for BF16 and any constant: widened (a shift or a mask, exact), multiplied in fp32 and rounded once to nearest even, two
+// values per conversion -- five vector instructions per two values, the bits of transform_fragment without its walk over an op list.
+__device__ __forceinline__ int4v scale_fragment_bf16(int4v f, float scale) {
+  typedef float float2v_ __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2_ __attribute__((ext_vector_type(2)));
+  int4v out;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float2v_ x;
+    x[0] = __builtin_bit_cast(float, f[i] << 16) * scale;
+    x[1] = __builtin_bit_cast(float, (int)((unsigned)f[i] & 0xFFFF0000u)) * scale;
+    out[i] = __builtin_bit_cast(int, __builtin_convertvector(x, bf16x2_));
+  }
+  return out;
+}
+template <typename T>
+__device__ __forceinline__ int4v scale_fragment(int4v f, float scale) {
+  if constexpr (std::is_same<T, __bf16>::value) return scale_fragment_bf16(f, scale);
+  else return scale_fragment_f16(f, scale);
+}
+
 #ifndef GK_FORCE_SYNC_FRAGS
 #define GK_FORCE_SYNC_FRAGS 0     // set by the run-time compiler for a tile that turned out to spill registers
 #endif
@@ -439,8 +460,8 @@ struct MfmaGemmConfig {
   static constexpr int KSTEP_K = MI_ == 32 ? 16 : 32;    // k-values per MFMA
   static constexpr int BM = BM_, BN = BN_, BK = BK_, WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, STAGES = STAGES_;
   static constexpr int A_KIND = A_KIND_, B_KIND = B_KIND_, FIX = FIX_;
-  // 0: no transform and no bias; 1: C / D hooks, bias and at most one exact 16-bit scale on A and on B
-  // (a packed multiply per fragment); 2: arbitrary op lists on A and B as well (evaluated in fp32 per
+  // 0: no transform and no bias; 1: C / D hooks, bias and at most one exact FP16 scale on A and on B
+  // (a packed multiply per fragment), or for BF16 one scale on A by any factor (scale_fragment_bf16); 2: arbitrary op lists on A and B as well (evaluated in fp32 per
   // element inside the K loop: complete, and markedly slower); 3: C / D hooks and bias only, the K loop of
   // level 0 (also what a power-of-two scale of A or B runs on: the host folds it into the accumulators);
   // 4 (one-wave-per-SIMD instances only): level 3 narrowed to what the host can name in closed form -- no hook on C, at
@@ -1270,17 +1291,17 @@ __global__ void __launch_bounds__(Cfg::THREADS) mfma_gemm_kernel(const GemmArgs 
       if constexpr ((MODE & 2) != 0 && half <= 0) {
 #pragma unroll
         for (int fj = 0; fj < FN; ++fj) {
-          vb[fj] = scale_fragment_f16(vb[fj], scale_b);
+          vb[fj] = scale_fragment<T>(vb[fj], scale_b);
           if constexpr (half == 0) RB::store(fb[ks & 1][fj], vb[fj]);
         }
       }
-      if constexpr ((MODE & 1) != 0) va[0] = scale_fragment_f16(va[0], scale_a);
+      if constexpr ((MODE & 1) != 0) va[0] = scale_fragment<T>(va[0], scale_a);
 #pragma unroll
       for (int fi = 0; fi < NA; ++fi) {
 #pragma unroll
         for (int fj = 0; fj < FN; ++fj) acc[FI0 + fi][fj] = Mfma<T, MI>::run(vb[fj], va[fi], acc[FI0 + fi][fj]);
         if constexpr ((MODE & 1) != 0) {
-          if (fi + 1 < NA) va[fi + 1] = scale_fragment_f16(va[fi + 1], scale_a);
+          if (fi + 1 < NA) va[fi + 1] = scale_fragment<T>(va[fi + 1], scale_a);
         }
       }
       return;
@@ -1919,8 +1940,8 @@ __global__ void __launch_bounds__(Cfg::THREADS) mfma_gemm_kernel(const GemmArgs 
     // FP16 operands whose hooks are at most one multiplication by a factor that is exact in FP16 (the host
     // passes 1 for an operand without one): both multiplications always run.  Separate copies of the loop
     // per combination cost more than the multiplications save (the accumulators of the copies meet in
-    // registers the compiler then has to spill).
-    k_loop(std::integral_constant<int, 3>{});
+    // registers the compiler then has to spill).  BF16: one factor, on A.
+    k_loop(std::integral_constant<int, std::is_same<T, __bf16>::value ? 1 : 3>{});
   } else {
     k_loop(std::integral_constant<int, -1>{});
   }

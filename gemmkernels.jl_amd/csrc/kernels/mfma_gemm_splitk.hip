@@ -1,7 +1,7 @@
 // K-split instances of the MFMA GEMM (kernel kind GK_KERNEL_SPLIT_K): the small tiles that skinny
 // products run, all four transposes, FP16 with no hooks, with C / D hooks and bias, or with those and one exact
-// FP16 scale on A and B (what the BLAS-style entry points produce); BF16 with no hooks, with C / D hooks and bias and, on
-// the 64 x 64 x 64 tile, with any hooks.
+// FP16 scale on A and B (what the BLAS-style entry points produce); BF16 with no hooks, with C / D hooks and bias, with those
+// and one scale on A and, on the 64 x 64 x 64 tile, with any hooks.
 #include "mfma_gemm.hpp"
 #include "registry.hpp"
 
@@ -26,10 +26,11 @@ int family_mfma_splitk(const InstanceKey& key, const GemmArgs& args, dim3 grid, 
   GK_SK_T(bm_, bn_, bk_, wm_, wn_, st_, _Float16, DT_F16, 1, "_f16_fused")  \
   GK_SK_T(bm_, bn_, bk_, wm_, wn_, st_, _Float16, DT_F16, 3, "_f16_fused_cd")  \
   GK_SK_T(bm_, bn_, bk_, wm_, wn_, st_, __bf16, DT_BF16, 0, "_bf16")  \
+  GK_SK_T(bm_, bn_, bk_, wm_, wn_, st_, __bf16, DT_BF16, 1, "_bf16_fused")  \
   GK_SK_T(bm_, bn_, bk_, wm_, wn_, st_, __bf16, DT_BF16, 3, "_bf16_fused_cd")
   GK_SK_TILE(128, 128, 64, 2, 2, 2)
   GK_SK_TILE(64, 64, 64, 2, 2, 4)
-  // (what a scale of A in BF16 is: the tile that the BLAS-style entry points run on slices of K takes every factor)
+  // (op lists on A and B)
   GK_SK_T(64, 64, 64, 2, 2, 4, __bf16, DT_BF16, 2, "_bf16_fused_ab")
   GK_SK_TILE(64, 64, 32, 1, 1, 2)
 #undef GK_SK_TILE

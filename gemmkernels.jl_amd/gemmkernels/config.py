@@ -229,7 +229,7 @@ def slices_pay(M, N, K, factor=None) -> bool:
     LDS stages that carry a lone workgroup through K at 0.22 us per 64 k.  In us, slices against unsplit: 64 tiles K = 1280 7.5 and 7.5,
     2048 8.7 and 10.5, 4096 11.1 and 17.6; 128 tiles K = 1280 8.6 and 7.9, 2048 9.8 and 10.7; three slices of 165 tiles 3072 13.0 and 14.7, 4096
     14.3 and 18.1; two slices of 180 .. 256 tiles gain nothing (180 tiles K = 4096 17.7 and 18.0, 256 tiles 19.1 and 18.4).  A factor that stays
-    in the K loop makes it longer: FP16 111 x 2629 x 1477 (84 tiles) 15.7 and 19.9, BF16 768 x 1024 x 4096 (192) 105 and 113."""
+    in the K loop makes it longer: FP16 111 x 2629 x 1477 (84 tiles) 15.7 and 19.9; 1024 x 1024 x 4096 (256) FP16 21.4 in two slices, BF16 unsplit 33.9."""
     return factor is not None or -(-M // 64) * -(-N // 64) <= 170
 
 
