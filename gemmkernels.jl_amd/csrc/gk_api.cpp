@@ -536,7 +536,7 @@ int find_instance(const gk_config* c, const gk_transforms* t, const gk_epilogue*
   }
   // (the instance with more LDS stages that few tiles run on: not under a limit set by the caller that is too small for it)
   const long long lds_max = g_lds_override.load();
-  if (lds_max > 0 && info->lds_bytes > lds_max && (key->family == gk::FAMILY_MFMA || key->family == gk::FAMILY_GETT || key->family == gk::FAMILY_COMPLEX)) {
+  if (lds_max > 0 && info->lds_bytes > lds_max && (key->family == gk::FAMILY_MFMA || key->family == gk::FAMILY_GETT || key->family == gk::FAMILY_COMPLEX || key->family == gk::FAMILY_FPU)) {
     key->variant |= gk::kShallow;
     fn(*key, dummy, dim3(1), nullptr, 0, info, &err);
   }
@@ -1076,7 +1076,7 @@ int prepare_launch(const gk_config* conf, const void* a, const void* b, const vo
       return fail(GK_ERR_DIMENSION_MISMATCH, "ldc/ldd is smaller than M");
     // the kernels keep per-lane tile offsets in 32 bits (floating-point FPUOp on the matrix instructions: in 64, of 31-bit
     // leading dimensions, so that its larger tiles take what the 64 x 64 tile takes)
-    const bool wide_offsets = key.family == gk::FAMILY_FPU && (key.variant & ~2) == 0 && (key.acc_dtype == GK_F32 || key.acc_dtype == GK_F64);
+    const bool wide_offsets = key.family == gk::FAMILY_FPU && (key.variant & ~(2 | gk::kShallow)) == 0 && (key.acc_dtype == GK_F32 || key.acc_dtype == GK_F64);
     if (wide_offsets && (args.lda >= (1ll << 31) || args.ldb >= (1ll << 31))) return fail(GK_ERR_UNSUPPORTED, "leading dimension of 2^31 elements or more");
     const long long span_a = (long long)(a_row ? conf->block_shape.M : conf->block_shape.K) * args.lda * 2;
     const long long span_b = (long long)(b_row ? conf->block_shape.K : conf->block_shape.N) * args.ldb * 2;

@@ -29,8 +29,10 @@
 // A K tile of 32 x 32 x 32 is a few hundred clocks of work for the matrix cores (512 in FP64, 256 in FP32), less than a load
 // takes from the last-level cache: on four waves these tiles have the loads of two K tiles in flight (DEPTH; the loop is
 // written out for a pair of tiles, so that each finds its registers): Float32 1024^3 25.7 -> 24.7 us, 300 x 700 x 1500
-// 17.2 -> 16.3, Float64 500 x 500 x 700 12.7 -> 12.1, 1024^3 44.9 -> 42.6.  Tiles of 64 x 64 gain nothing from it (Float64
+// 17.2 -> 16.3, Float64 500 x 500 x 700 12.7 -> 12.1, 1024^3 44.9 -> 42.6.  Tiles of 64 x 64 that share a CU gain nothing from it (Float64
 // 1024^3 41.1 -> 41.6, Float32 2048^3 142 -> 145): one in flight.
+//
+// Launches that have at most one workgroup per CU run instances of their own (fpu_mfma_deep.hip).
 //
 // Sizes, leading dimensions and addresses are free.  A vector load takes any address that is aligned to its elements; rows
 // beyond the edge of an operand are clamped to the last ones (their products land in outputs that are not stored):
@@ -502,12 +504,12 @@ __global__ void __launch_bounds__(Cfg::THREADS, Cfg::WAVES_PER_SIMD) fpu_mfma_ke
     // The accumulators that C filled have arrived when the loop begins: left open, the compiler waits for every load of the
     // next tile in front of the first MFMA of each tile (vmcnt(0) there; with this, one vector at a time where it goes to LDS).
     __builtin_amdgcn_s_waitcnt(0x0F70);         // vmcnt(0)
-    static_assert(DEPTH == 1 || DEPTH == 2, "the tiles in flight find their registers by the parity of the tile");
     for (int kt = 0; kt < whole; kt += DEPTH) {
-      tile(kt, std::integral_constant<int, 0>{});
-      if constexpr (DEPTH == 2) {
-        if (kt + 1 < whole) tile(kt + 1, std::integral_constant<int, 1>{});
-      }
+      // (written out for DEPTH tiles: each finds the registers of its loads)
+      fpu_static_for<0, DEPTH>([&](auto d_c) __attribute__((always_inline)) {
+        constexpr int d = decltype(d_c)::value;
+        if (d == 0 || kt + d < whole) tile(kt + d, d_c);
+      });
     }
     if (k_tail < K) {
       // (the barrier above: everyone has read the last whole tile)

@@ -18,7 +18,7 @@ struct InstanceKey {
   int variant;       // family specific
 };
 
-// Bit of InstanceKey::variant (matrix-core families): the instance with the fewest LDS stages, whatever the tiles of the launch
+// Bit of InstanceKey::variant (products on the matrix instructions): the instance with the fewest LDS stages, whatever the tiles of the launch
 // (set by the host where the one with more stages asks for more LDS than the device limit in force allows).
 constexpr int kShallow = 0x100;
 
@@ -92,6 +92,7 @@ int family_mfma_stream_tt(const InstanceKey&, const GemmArgs&, dim3, hipStream_t
 int family_fpu(const InstanceKey&, const GemmArgs&, dim3, hipStream_t, int, InstanceInfo*, hipError_t*);
 int family_fpu_mfma_f32_large(const InstanceKey&, const GemmArgs&, dim3, hipStream_t, int, InstanceInfo*, hipError_t*);
 int family_fpu_mfma_f32_small(const InstanceKey&, const GemmArgs&, dim3, hipStream_t, int, InstanceInfo*, hipError_t*);
+int family_fpu_mfma_deep(const InstanceKey&, const GemmArgs&, dim3, hipStream_t, int, InstanceInfo*, hipError_t*);
 int family_fpu_mfma_f64(const InstanceKey&, const GemmArgs&, dim3, hipStream_t, int, InstanceInfo*, hipError_t*);
 int family_fpu_mfma_mixed(const InstanceKey&, const GemmArgs&, dim3, hipStream_t, int, InstanceInfo*, hipError_t*);
 int family_fpu_integers(const InstanceKey&, const GemmArgs&, dim3, hipStream_t, int, InstanceInfo*, hipError_t*);

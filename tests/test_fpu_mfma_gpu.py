@@ -135,3 +135,25 @@ def test_leading_dimensions_beyond_32_bits_of_tile_offsets(gpu):
         gk.matmul(conf, A, gk.colmajor(b), None, D)
         torch.cuda.synchronize()
         assert np.array_equal(gk.to_numpy(D), helpers.run_oracle(conf, a, b, None, (M, N), d_dtype=np.float32)), tile
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, True)])
+@pytest.mark.parametrize("types", ["f32", "f64"])
+def test_instances_for_one_workgroup_per_cu_and_for_more(gpu, types, ta, tb):
+    """At most 256 tiles run on instances of their own (32 x 32 x 32 in pairs of K tiles from K = 512 on), more on the others: the same fma
+    chains either way, with factors on A and C, at tile counts on both sides and K around a pair."""
+    _, _, np_in, np_out = TYPES[types]
+    half = dict(transform_shared_to_regs_a=Transform.Elementwise(lambda x: x * 1.5), transform_shared_to_regs_c=Transform.Elementwise(lambda x: x * 0.5))
+    for tile, (M, N), Ks in ((((32, 32, 32), (2, 2)), (37, 61), (511, 512, 543, 577, 640)), (((32, 32, 32), (2, 2)), (512, 512), (512,)), (((32, 32, 32), (2, 2)), (545, 512), (66, 520)),
+                             (((64, 64, 32), (2, 2)), (65, 130), (31, 64, 101)), (((64, 64, 32), (2, 2)), (1030, 1021), (70,))):
+        for K in Ks:
+            a, b = operand((K, M) if ta else (M, K), np_in, K), operand((N, K) if tb else (K, N), np_in, K + 1)
+            for hooks in ({}, half):
+                c = operand((M, N), np_out, K + 2) if hooks else None
+                conf = config(M, N, K, ta, tb, types, tile, c is None)
+                name = gk.kernel_name(conf, Kernel.matmul_singlestage, hooks)
+                few = -(-M // tile[0][0]) * -(-N // tile[0][1]) <= 256
+                assert ("_s3_" in name or "_pairs_" in name) == (few and (tile[0][0] == 64 or K >= 512)), name
+                print("case", types, tile, (M, N, K), ta, tb, name, flush=True)
+                d = helpers.run_gpu(conf, a, b, c, (M, N), d_dtype=TORCH[np_out], transforms=hooks)
+                assert np.array_equal(d, helpers.run_oracle(conf, a, b, c, (M, N), d_dtype=np_out, transforms=hooks)), (tile, (M, N, K))
