@@ -570,7 +570,8 @@ def matmatmul_(C, transA: str, transB: str, A, B, alpha, beta, *, wmma=None):
         if hit is not None:
             hit(a, b, c, _current_stream())
             return C
-    launch = _MulLaunch(_single_plan(C, tA, tB, A, B, alpha, beta, wmma))
+    p = _single_plan(C, tA, tB, A, B, alpha, beta, wmma)
+    launch = _MulLaunch(p, None if p._split_k else packed_leading_dims(p._conf, a, b))
     if key is not None:
         if len(_mul_launches) >= _MUL_LAUNCHES_MAX:
             _mul_launches.clear()
@@ -582,23 +583,108 @@ def matmatmul_(C, transA: str, transB: str, A, B, alpha, beta, *, wmma=None):
 _PLAIN_NUMBERS = (float, int, bool)
 
 
+def _stored(which: int, kind: int, extent: int, k: int):
+    """Rows (contiguous) and columns of operand A (0) or B (1) as it lies in memory."""
+    row_major = kind in (Layout.ROW_MAJOR, Layout.ALIGNED_ROW_MAJOR)
+    return (k, extent) if row_major == (which == 0) else (extent, k)
+
+
+_PACK_MIN_WORK, _PACK_MIN_WORK_ONE = 24 * 10 ** 9, 50 * 10 ** 9      # M N K with both operands, with one of them
+_PACK_MAX_BYTES = 512 << 20
+
+
+def packed_leading_dims(conf_c, a: int, b: int):
+    """Leading dimensions of copies of A and of B (None: the operand stays as it is) on which a product runs faster, the
+    copying included, or None.
+
+    An operand whose columns start off 16-byte boundaries costs a launch more lines of memory and of L2 than its bytes:
+    every 128-byte row of a tile lies on two lines.  Copies with columns on 128-byte lines cost 24 us for two operands of 32 MB
+    (5.3 TB/s) and leave the operands in the memory-side cache.  Inputs that rotate through more than that cache holds, BF16,
+    both operands odd, 'N','N' / 'T','N': 4001 x 4003 x 4005 172 -> 155 / 182 -> 160 us, 3001 x 3003 x 3005 105 -> 87 / 113 -> 88,
+    8001 x 8003 x 2005 459 -> 333 / 469 -> 337, 6001 x 5003 x 7005 488 -> 402 / 497 -> 405, 801 x 5003 x 6005 134 -> 108 / 133 -> 108; on
+    the same inputs over and over they win from some 4e10 products on and are level below (4001 x 4003 x 4005 132 -> 138, 8001 x 8003
+    x 2005 376 -> 330).  Below 2.4e10 the copies take what they save (2001 x 2003 x 4005 57 -> 65, 3001 x 3003 x 1505 55 -> 57,
+    8001 x 503 x 3005 63 -> 63).  One odd operand, contiguous along k: 4000 x 4000 x 4001 'N','N' 140 -> 126, 3000 x 3000 x 3001 100 -> 92
+    and 73 -> 77 on the same inputs; along m or n: 4001 x 4000 x 4000 160 -> 155, 123 -> 125, not worth a copy."""
+    shape, layouts = conf_c.matmul_shape, (conf_c.global_a_layout, conf_c.global_b_layout)
+    work = shape.M * shape.N * shape.K
+    if conf_c.op.kind != Operator.MFMA or work < _PACK_MIN_WORK or min(shape.M, shape.N) < 512 or shape.K < 1000:
+        return None
+    if any(layout.kind == Layout.ZERO for layout in layouts):        # (alpha = 0)
+        return None
+    odd = tuple(layout.ld % 8 != 0 or address % 16 != 0 for layout, address in zip(layouts, (a, b)))
+    stored = tuple(_stored(which, layouts[which].kind, (shape.M, shape.N)[which], shape.K) for which in (0, 1))
+    if not all(odd):
+        k_major = tuple(layouts[which].kind in ((Layout.ROW_MAJOR, Layout.ALIGNED_ROW_MAJOR) if which == 0 else (Layout.COL_MAJOR, Layout.ALIGNED_COL_MAJOR))
+                        for which in (0, 1))
+        if work < _PACK_MIN_WORK_ONE or not any(o and k for o, k in zip(odd, k_major)):
+            return None
+    packed = tuple(-(-rows // 64) * 64 if o else None for o, (rows, _) in zip(odd, stored))
+    total = sum(2 * ld * cols for ld, (_, cols) in zip(packed, stored) if ld is not None)
+    if total > _PACK_MAX_BYTES or max(rows for rows, _ in stored) > _PACK_MAX_ROWS:
+        return None
+    return packed
+
+
+_PACK_MAX_ROWS = 255 * 512          # of one launch of gk_pack_columns
+
+
 class _MulLaunch:
     """What ``matmatmul_`` hands to the library for operands of one kind (element types, sizes, strides, alignment) and one
     pair of factors: descriptors only, no address and no tensor, so any operands of that kind can use it, on any
     stream and from any thread (nothing in it is written after it is made).  Lowering the same call again took 22 us of
     interpreter time, the whole of a small product: mul! at 256^3 in Float32 takes 5 us on the device."""
 
-    __slots__ = ("_fn", "_conf", "_trans", "_conf_ref", "_trans_ref", "_code", "_workspace")
+    __slots__ = ("_fn", "_conf", "_trans", "_conf_ref", "_trans_ref", "_code", "_workspace", "_packed", "_packed_ref", "_copies", "_copy_bytes")
 
-    def __init__(self, p: Plan):
+    def __init__(self, p: Plan, packed):
         self._conf, self._trans = p._conf, p._trans         # (own the memory that the references point to)
         self._conf_ref = ctypes.byref(self._conf)
         self._trans_ref = ctypes.byref(self._trans) if self._trans is not None else None
         self._fn = p._fn
         self._workspace = _split_k_bytes(self._conf) if p._split_k else None
         self._code = None if p._split_k else p._args[-1]
+        self._packed = self._packed_ref = None
+        if packed is not None:
+            self._packed = _lib.gk_config.from_buffer_copy(self._conf)
+            self._packed_ref = ctypes.byref(self._packed)
+            shape, self._copies, at = self._conf.matmul_shape, [], 0
+            for which, (layout, mine, ld, extent) in enumerate(((self._packed.global_a_layout, self._conf.global_a_layout, packed[0], shape.M),
+                                                                (self._packed.global_b_layout, self._conf.global_b_layout, packed[1], shape.N))):
+                if ld is None:
+                    continue
+                rows, cols = _stored(which, mine.kind, extent, shape.K)
+                self._copies.append((which, rows, cols, mine.ld, at, ld))
+                layout.ld = ld
+                at += 2 * ld * cols
+            self._copy_bytes = at
+
+    def _on_copies(self, a: int, b: int, c: int, stream: int) -> bool:
+        """The product on copies of the operands whose columns start off a 16-byte boundary (the same launch, the same bits).
+        False: not here -- no memory for the copies, or a capture, whose graph would have to keep them."""
+        import torch
+        if _capture_of(stream) is not None:
+            return False
+        # memory of this call alone, in the order of the stream: what gets it next on this stream runs behind the product
+        with _on(stream):
+            try:
+                copies = torch.empty(self._copy_bytes, dtype=torch.uint8, device="cuda")
+            except torch.OutOfMemoryError:
+                return False
+        base, operands, jobs = copies.data_ptr(), [a, b], []
+        for which, rows, cols, ld, at, ld_packed in self._copies:
+            jobs += [operands[which], rows, cols, ld, base + at, ld_packed]
+            operands[which] = base + at
+        rc = _lib.lib().gk_pack_columns(*jobs, *((None, 0, 0, 0, None, 0) if len(jobs) == 6 else ()), stream)
+        if rc == _lib.GK_OK:
+            rc = self._fn(self._packed_ref, *operands, c, c, self._trans_ref, None, self._code, stream)
+        if rc != _lib.GK_OK:
+            _raise(rc)
+        return True
 
     def __call__(self, a: int, b: int, c: int, stream: int) -> None:
+        if self._packed is not None and self._on_copies(a, b, c, stream):
+            return
         if self._workspace is None:
             rc = self._fn(self._conf_ref, a, b, c, c, self._trans_ref, None, self._code, stream)
         else:

@@ -310,6 +310,14 @@ size_t gk_split_k_noalloc_capacity(void);
 int gk_matmul_split_k_noalloc(const gk_config* conf, const void* a, const void* b, const void* c, void* d,
                               const gk_transforms* transforms, const gk_epilogue* epilogue, void* stream);
 
+/* One or two matrices of 16-bit elements (rows x cols, column-major, leading dimension ld, any 2-byte aligned address; cols1 == 0:
+ * one matrix) copied to the leading dimension ld_dst (at least rows, a multiple of 8) at the 16-byte aligned address dst, in one
+ * launch on `stream`.  At most 130560 rows.  No counterpart in the reference: a large product whose columns start off a 16-byte
+ * boundary runs faster on copies whose columns start on 128-byte lines (ld_dst a multiple of 64), to the same bits.  What
+ * lies between rows and ld_dst is neither read nor written. */
+int gk_pack_columns(const void* src0, int64_t rows0, int64_t cols0, int64_t ld0, void* dst0, int64_t ld_dst0, const void* src1,
+                    int64_t rows1, int64_t cols1, int64_t ld1, void* dst1, int64_t ld_dst1, void* stream);
+
 /* A measurement aid with no counterpart in the reference (its benchmarks quote fractions of a data-sheet peak): the
  * rate, in TFLOP/s, of a register-only loop of the MFMA instruction the GEMM kernels use (v_mfma_f32_16x16x32_f16,
  * one wave per SIMD, 64 accumulator blocks per wave, operands that change every 64 MFMAs), over `launches` launches

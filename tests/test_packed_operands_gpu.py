@@ -1,0 +1,124 @@
+"""Large 16-bit products whose columns start off 16-byte boundaries: ``mul_`` copies such operands to columns on 128-byte lines
+first.  The launch is the same one, so the result is that of the product on the operands as they lie, bit for bit."""
+import itertools
+
+import pytest
+import torch
+
+import gemmkernels as gk
+from gemmkernels import _lib
+from gemmkernels.matmul import matmatmul_plan, packed_leading_dims
+
+
+class _Layouts:
+    """The fields of a lowered configuration that the rule looks at, of op(A) op(B) on matrices with the leading dimensions given."""
+
+    def __new__(cls, M, N, K, ta, tb, lda, ldb):
+        conf = _lib.gk_config()
+        conf.op.kind = gk.Operator.MFMA
+        conf.matmul_shape.M, conf.matmul_shape.N, conf.matmul_shape.K = M, N, K
+        conf.global_a_layout.kind, conf.global_b_layout.kind = 1 + ta, 1 + tb        # ColMajor, RowMajor
+        conf.global_a_layout.ld, conf.global_b_layout.ld = lda, ldb
+        return conf
+
+
+def test_the_rule():
+    """No GPU: which products are worth the copies."""
+    dims = lambda M, N, K, ta, tb, a=0, b=0: packed_leading_dims(_Layouts(M, N, K, ta, tb, K if ta else M, N if tb else K), a, b)
+    assert dims(4001, 4003, 4005, True, False) == (4032, 4032)
+    assert dims(4001, 4003, 4005, False, True) == (4032, 4032)
+    assert dims(4001, 4003, 8100, False, False) == (4032, 8128)
+    assert dims(4000, 4000, 4000, True, False) is None and dims(4096, 4096, 4096, False, False) is None
+    assert dims(4096, 4096, 4096, False, False, 2, 6) == (4096, 4096)             # misaligned addresses
+    assert dims(4000, 4000, 4001, False, False) == (None, 4032)                   # one operand, contiguous along k
+    assert dims(4001, 4000, 4000, False, False) is None                           # one operand, contiguous along m
+    assert dims(2001, 2003, 4005, True, False) is None                            # too little work
+    assert dims(131, 8191, 31111, True, False) is None                            # too few rows
+    assert dims(16001, 16001, 16001, True, False) is None                         # copies of more than 512 MiB
+
+
+def _odd(rows, cols, ld, dtype, gen, offset=0):
+    buffer = (torch.rand(ld * (cols - 1) + rows + offset, generator=gen, device="cuda") * 2 - 1).to(dtype)      # ends with the last column
+    return torch.as_strided(buffer, (rows, cols), (1, ld), offset)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols,ld,offset", [(1, 1, 1, 0), (7, 17, 9, 1), (8, 16, 8, 0), (511, 33, 513, 3), (512, 5, 515, 1), (515, 20, 515, 0), (1029, 3, 2001, 7)])
+def test_pack_columns(rows, cols, ld, offset):
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    x, y = _odd(rows, cols, ld, torch.float16, gen, offset), _odd(rows + 1, cols + 2, ld + 1, torch.float16, gen)
+    dims = [(-(-r // 8) * 8) for r in (rows, rows + 1)]
+    copies = [torch.full((c, d), -2.0, dtype=torch.float16, device="cuda") for c, d in zip((cols, cols + 2), dims)]
+    job = lambda m, copy, d: (m.data_ptr(), m.shape[0], m.shape[1], m.stride(1) if m.shape[1] > 1 else m.shape[0], copy.data_ptr(), d)
+    stream = torch.cuda.current_stream().cuda_stream
+    assert _lib.lib().gk_pack_columns(*job(x, copies[0], dims[0]), *job(y, copies[1], dims[1]), stream) == _lib.GK_OK, _lib.last_error()
+    for m, copy in zip((x, y), copies):
+        assert torch.equal(copy[:, :m.shape[0]].t(), m) and bool((copy[:, m.shape[0]:] == -2.0).all())
+    copies[0].fill_(-2.0)
+    assert _lib.lib().gk_pack_columns(*job(x, copies[0], dims[0]), None, 0, 0, 0, None, 0, stream) == _lib.GK_OK, _lib.last_error()
+    assert torch.equal(copies[0][:, :rows].t(), x) and bool((copies[0][:, rows:] == -2.0).all())
+
+
+def test_pack_columns_refuses():
+    """No GPU: nothing is launched."""
+    pack = _lib.lib().gk_pack_columns
+    none = (None, 0, 0, 0, None, 0, None)
+    assert pack(None, 8, 8, 8, 256, 8, *none) == _lib.GK_ERR_INVALID_ARGUMENT
+    assert pack(256, 8, 8, 7, 256, 8, *none) == _lib.GK_ERR_INVALID_ARGUMENT
+    assert pack(256, 9, 8, 9, 256, 9, *none) == _lib.GK_ERR_INVALID_ARGUMENT
+    assert pack(257, 8, 8, 8, 256, 8, *none) == _lib.GK_ERR_ALIGNMENT
+    assert pack(256, 8, 8, 8, 264, 8, *none) == _lib.GK_ERR_ALIGNMENT
+    assert pack(256, 8, 8, 8, 256, 8, 256, 8, -1, 8, 256, 8, None) == _lib.GK_ERR_INVALID_ARGUMENT
+    assert pack(256, 1 << 20, 8, 1 << 20, 256, 1 << 20, *none) == _lib.GK_ERR_INVALID_ARGUMENT
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ab,cd", [(torch.bfloat16, torch.float32), (torch.float16, torch.float32), (torch.float16, torch.float16)])
+@pytest.mark.parametrize("ta,tb", list(itertools.product((False, True), repeat=2)))
+def test_product_on_copies(ta, tb, ab, cd):
+    """Against the plan of the same product, which launches on the operands as they lie; a call under capture does so too."""
+    M, N, K = 3001, 2999, 3003
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    a = _odd(K, M, K, ab, gen, 1) if ta else _odd(M, K, M + 2, ab, gen)
+    b = _odd(N, K, N, ab, gen) if tb else _odd(K, N, K, ab, gen, 3)
+    c = (torch.rand(N, M, generator=gen, device="cuda") * 2 - 1).to(cd).t()
+    for alpha, beta in ((1.0, 0.0), (1.5, 0.5)):
+        ref, out, captured = (c.clone(memory_format=torch.preserve_format) for _ in range(3))
+        matmatmul_plan(ref, 'T' if ta else 'N', 'T' if tb else 'N', a, b, alpha, beta)()
+        call = lambda d: gk.mul_(d, gk.Transpose(a) if ta else a, gk.Transpose(b) if tb else b, alpha, beta)
+        call(out)
+        assert torch.equal(out, ref)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            call(captured)
+        for _ in range(2):
+            captured.copy_(c)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(captured, ref)
+
+
+@pytest.mark.gpu
+def test_streams_and_no_memory(monkeypatch):
+    """On a stream of its own, beside the default one, and where the copies find no memory: the same bits."""
+    M = N = K = 3001
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    a, b = _odd(M, K, M, torch.bfloat16, gen), _odd(K, N, K, torch.bfloat16, gen)
+    ref, out, other = (gk.colmajor_empty((M, N), torch.float32) for _ in range(3))
+    matmatmul_plan(ref, 'N', 'N', a, b, 1.0, 0.0)()
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    for _ in range(3):
+        gk.mul_(out, a, b)
+        with torch.cuda.stream(stream):
+            gk.mul_(other, a, b)
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref) and torch.equal(other, ref)
+    out.zero_()
+
+    def none(*args, **kwargs):
+        raise torch.OutOfMemoryError("no memory")
+    monkeypatch.setattr(torch, "empty", none)
+    gk.mul_(out, a, b)
+    monkeypatch.undo()
+    assert torch.equal(out, ref)
