@@ -109,15 +109,21 @@ __device__ __forceinline__ void pin_scalar(const char*& p) {
 }
 
 // Tensor-contraction index maps: walks the K index of a contraction tile by tile.  A tile covers the K modes below
-// `mode` whole and `step` indices of mode `mode` (see GemmArgs::gk_mode); the modes above are the digits of a counter.
+// `mode` whole and `step` indices of mode `mode` (see GemmArgs::gk_mode); the modes from `mode` on are the digits of a counter.
+// On a tile that is alone on its CU a wave issues nothing else meanwhile, so a step is two 64-bit additions, the lowest
+// digit and one branch; all that a carry needs stands behind the branch.  Tests of every digit and of its mode at every tile, and
+// a walk with a loop over the modes for every DMA chunk in front of the first one, cost contractions on the small tiles
+// 3 to 10 us over the plain product: M x N x K = 1536 x 256 x 2048 18.1 -> 13.6 us, 3840 x 1088 x 2048 37.0 -> 31.9,
+// 640 x 640 x 4096 28.4 -> 23.9, 960 x 3968 x 4096 62.0 -> 54.3 (plain products on the same tile 11.1, 29.9, 18.2 and 46.6).
 struct KWalker {
-  int d0, d1, d2;           // digits of the K modes 0 .. 2 at the first k of the tile (modes below `mode` stay 0)
-  long long oa, ob;         // element offsets of the tile's first k in A and in B, kept up to date by advance()
+  int d0, d1, d2;           // digits of the K modes mode .. mode + 2 at the first k of the tile
+  long long oa, ob;         // byte offsets of the tile's first k in A and in B, kept up to date by advance()
   // copies of the mode table, held in scalar registers for the whole K loop: read from the kernel arguments inside the
-  // loop they would be scalar loads, and the wait for a scalar load also waits for every LDS read in flight.  Only
-  // additions are left in the loop: step_a / step_b move the offsets by one tile along `mode`, wrap_a[i] / wrap_b[i]
-  // are what a carry out of mode i adds (one stride of mode i + 1 minus the whole extent of mode i).
-  int nmodes, mode, step, e0, e1, e2;
+  // loop they would be scalar loads, and the wait for a scalar load also waits for every LDS read in flight.
+  // e0 .. e2: extents of the modes mode .. mode + 2 (the last K mode never wraps inside K: no extent that a digit reaches);
+  // step_a / step_b move the offsets by one tile along `mode`, wa_i / wb_i are what a carry out of mode + i adds (one
+  // stride of the next mode minus the whole extent of this one).
+  int step, e0, e1, e2;
   long long step_a, step_b, wa0, wa1, wa2, wb0, wb1, wb2;
   // (the values are the same in every lane; readfirstlane says so to the compiler where it has loaded the kernel
   // arguments with vector instructions)
@@ -127,45 +133,43 @@ struct KWalker {
     asm volatile("" : "+s"(lo), "+s"(hi));
     x = (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
   }
-  __device__ __forceinline__ void init(const GettDim& gk, int mode_, int step_) {
+  __device__ __forceinline__ void init(const GettDim& gk, int mode, int step_) {
     d0 = d1 = d2 = 0;
     oa = ob = 0;
-    nmodes = gk.nmodes; mode = mode_; step = step_;
-    e0 = gk.extent[0]; e1 = gk.extent[1]; e2 = gk.extent[2];
-    step_a = (long long)step_ * gk.stride0[mode_];
-    step_b = (long long)step_ * gk.stride1[mode_];
-    wa0 = gk.stride0[1] - (long long)e0 * gk.stride0[0]; wb0 = gk.stride1[1] - (long long)e0 * gk.stride1[0];
-    wa1 = gk.stride0[2] - (long long)e1 * gk.stride0[1]; wb1 = gk.stride1[2] - (long long)e1 * gk.stride1[1];
-    wa2 = gk.stride0[3] - (long long)e2 * gk.stride0[2]; wb2 = gk.stride1[3] - (long long)e2 * gk.stride1[2];
-    keep(nmodes); keep(mode); keep(step); keep(e0); keep(e1); keep(e2);
+    step = step_;
+    step_a = 2 * (long long)step_ * gk.stride0[mode];
+    step_b = 2 * (long long)step_ * gk.stride1[mode];
+    auto carry = [&](int i, int& e, long long& wa, long long& wb) __attribute__((always_inline)) {
+      const bool on = i + 1 < gk.nmodes;
+      const int m = on ? i : 0, next = on ? i + 1 : 0;
+      e = on ? gk.extent[m] : 0x7fffffff;
+      wa = 2 * (gk.stride0[next] - (long long)gk.extent[m] * gk.stride0[m]);
+      wb = 2 * (gk.stride1[next] - (long long)gk.extent[m] * gk.stride1[m]);
+    };
+    carry(mode, e0, wa0, wb0);
+    carry(mode + 1, e1, wa1, wb1);
+    carry(mode + 2, e2, wa2, wb2);
+    keep(step); keep(e0); keep(e1); keep(e2);
     keep(step_a); keep(step_b); keep(wa0); keep(wa1); keep(wa2); keep(wb0); keep(wb1); keep(wb2);
   }
   __device__ __forceinline__ void advance() {
-    // the digit of `mode` moves on by step; a digit that reaches its extent goes back to 0 and carries (the digit
-    // of the last mode never wraps inside K and is not kept)
-    if (mode == 0) d0 += step; else if (mode == 1) d1 += step; else if (mode == 2) d2 += step;
+    d0 += step;
     oa += step_a; ob += step_b;
-    if (nmodes > 1 && d0 >= e0) { d0 = 0; ++d1; oa += wa0; ob += wb0; }
-    if (nmodes > 2 && d1 >= e1) { d1 = 0; ++d2; oa += wa1; ob += wb1; }
-    if (nmodes > 3 && d2 >= e2) { d2 = 0; oa += wa2; ob += wb2; }
+    if (__builtin_expect(d0 >= e0, 0)) {
+      d0 = 0; ++d1; oa += wa0; ob += wb0;
+      if (d1 >= e1) {
+        d1 = 0; ++d2; oa += wa1; ob += wb1;
+        if (d2 >= e2) { d2 = 0; oa += wa2; ob += wb2; }
+      }
+    }
   }
-  // element offsets of the tile's first k in A and in B
+  // byte offsets of the tile's first k in A and in B
   __device__ __forceinline__ long long offset_a() const { return oa; }
   __device__ __forceinline__ long long offset_b() const { return ob; }
 };
-// element offset of k-value k (< BLOCK_K) of a tile from the tile's first k: digits of the modes the tile covers whole,
-// the rest along mode `mode`
-__device__ __forceinline__ long long gett_k_local(const GettDim& gk, int mode, int k, const long long* stride) {
-  long long o = 0;
-  for (int i = 0; i < mode; ++i) {
-    const int q = gett_div(k, gk.magic[i], gk.shift[i]);
-    o += (long long)(k - q * gk.extent[i]) * stride[i];
-    k = q;
-  }
-  return o + (long long)k * stride[mode];
-}
-// (the same modulo 2^32 and written out over all modes like gett_offsets32_flat: a mode below `mode` gives a digit, mode
-// `mode` takes what is left of k, the modes above it nothing)
+// Element offset, modulo 2^32, of k-value k (< BLOCK_K) of a tile from the tile's first k: digits of the modes the tile covers
+// whole, the rest along mode `mode`.  Written out over all modes like gett_offsets32_flat: a mode below `mode` gives a digit,
+// mode `mode` takes what is left of k, the modes above it nothing.
 __device__ __forceinline__ unsigned gett_k_local_flat(const GettDim& gk, int mode, int k, const long long* stride) {
   unsigned o = 0;
 #pragma unroll
@@ -178,6 +182,30 @@ __device__ __forceinline__ unsigned gett_k_local_flat(const GettDim& gk, int mod
     o += (unsigned)digit * (unsigned)(unsigned long long)stride[i];
   }
   return o;
+}
+
+// The same walks, modulo 2^32, for N indices of a GEMM dimension (N k-values of a tile) at once, mode by mode: one branch per
+// mode for all of them, no division for the last mode, and the steps of the N walks overlap.  off[] is added to.
+template <int N>
+__device__ __forceinline__ void gett_add_offsets32(const GettDim& d, int nmodes, const long long* stride, int (&idx)[N], unsigned (&off)[N]) {
+#pragma unroll
+  for (int i = 0; i < kMaxModes; ++i) {
+    if (i < nmodes) {
+      const unsigned s = (unsigned)(unsigned long long)stride[i];
+      if (i + 1 == nmodes) {
+#pragma unroll
+        for (int n = 0; n < N; ++n) off[n] += (unsigned)idx[n] * s;
+      } else if (const unsigned magic = d.magic[i]) {         // (an extent of 1 has no digit)
+        const int shift = d.shift[i], extent = d.extent[i];
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+          const int q = (int)((unsigned)(((unsigned long long)(unsigned)idx[n] * magic) >> 32) >> shift);
+          off[n] += (unsigned)(idx[n] - q * extent) * s;
+          idx[n] = q;
+        }
+      }
+    }
+  }
 }
 
 // Makes every later use of x depend on the point where pin() stands (no instruction is emitted).
@@ -721,24 +749,25 @@ __global__ void __launch_bounds__(Cfg::THREADS) mfma_gemm_kernel(const GemmArgs 
         offb[i] = (tab_b[r] + tab_kb[k]) * 2u;
       }
     } else {
+    auto chunk_offsets = [&](auto kind_c, auto ndma_c, auto geom, const GettDim& dim, int origin, const long long* k_stride, unsigned* off) __attribute__((always_inline)) {
+      constexpr int KIND = decltype(kind_c)::value, NDMA = decltype(ndma_c)::value;
+      int r[NDMA], k[NDMA];
+      unsigned o[NDMA];
 #pragma unroll
-    for (int i = 0; i < DMA_A; ++i) {
-      int row, col;
-      dma_lane_coords<GA, Cfg::A_KIND>(dma_chunk(i, DMA_A), lane, row, col);
-      const int r = Cfg::A_KIND == OPK_KMAJOR ? row : col, k = Cfg::A_KIND == OPK_KMAJOR ? col : row;
-      long long o0, o1;
-      gett_offsets32(args.gm, m0 + r, o0, o1);
-      offa[i] = (unsigned)((o0 + gett_k_local(args.gk, args.gk_mode, k, args.gk.stride0)) * 2);
-    }
+      for (int i = 0; i < NDMA; ++i) {
+        int row, col;
+        dma_lane_coords<decltype(geom), KIND>(dma_chunk(i, NDMA), lane, row, col);
+        r[i] = origin + (KIND == OPK_KMAJOR ? row : col);
+        k[i] = KIND == OPK_KMAJOR ? col : row;
+        o[i] = 0;
+      }
+      gett_add_offsets32(dim, dim.nmodes, dim.stride0, r, o);
+      gett_add_offsets32(args.gk, args.gk_mode + 1, k_stride, k, o);       // (k inside a tile: the modes below gk_mode whole, the rest along it)
 #pragma unroll
-    for (int i = 0; i < DMA_B; ++i) {
-      int row, col;
-      dma_lane_coords<GB, Cfg::B_KIND>(dma_chunk(i, DMA_B), lane, row, col);
-      const int r = Cfg::B_KIND == OPK_KMAJOR ? row : col, k = Cfg::B_KIND == OPK_KMAJOR ? col : row;
-      long long o0, o1;
-      gett_offsets32(args.gn, n0 + r, o0, o1);
-      offb[i] = (unsigned)((o0 + gett_k_local(args.gk, args.gk_mode, k, args.gk.stride1)) * 2);
-    }
+      for (int i = 0; i < NDMA; ++i) off[i] = o[i] * 2u;
+    };
+    chunk_offsets(std::integral_constant<int, Cfg::A_KIND>{}, std::integral_constant<int, DMA_A>{}, GA{}, args.gm, m0, args.gk.stride0, offa);
+    chunk_offsets(std::integral_constant<int, Cfg::B_KIND>{}, std::integral_constant<int, DMA_B>{}, GB{}, args.gn, n0, args.gk.stride1, offb);
     }
   }
 
@@ -757,8 +786,8 @@ __global__ void __launch_bounds__(Cfg::THREADS) mfma_gemm_kernel(const GemmArgs 
     const char* pa = ga;
     const char* pb = gb;
     if constexpr (Cfg::GETT) {
-      pa = ga + walk.offset_a() * 2;
-      pb = gb + walk.offset_b() * 2;
+      pa = ga + walk.offset_a();
+      pb = gb + walk.offset_b();
       walk.advance();
     }
     static_for<0, DMA_A>([&](auto i_c) {
@@ -784,8 +813,8 @@ __global__ void __launch_bounds__(Cfg::THREADS) mfma_gemm_kernel(const GemmArgs 
     char* sb = sa + GA::BYTES;
     if constexpr (Cfg::GETT && P == 0) {
       // tile base of the tensor walk, the same for every part of this tile
-      part_a = ga + walk.offset_a() * 2;
-      part_b = gb + walk.offset_b() * 2;
+      part_a = ga + walk.offset_a();
+      part_b = gb + walk.offset_b();
       walk.advance();
     }
     const char* pa = Cfg::GETT ? part_a : ga;
