@@ -571,7 +571,8 @@ def matmatmul_(C, transA: str, transB: str, A, B, alpha, beta, *, wmma=None):
             hit(a, b, c, _current_stream())
             return C
     p = _single_plan(C, tA, tB, A, B, alpha, beta, wmma)
-    launch = _MulLaunch(p, None if p._split_k else packed_leading_dims(p._conf, a, b))
+    packed = None if p._split_k else packed_leading_dims(p._conf, a, b)
+    launch = _MulLaunch(p) if packed is None else _MulLaunchOnCopies(p, packed)
     if key is not None:
         if len(_mul_launches) >= _MUL_LAUNCHES_MAX:
             _mul_launches.clear()
@@ -635,29 +636,45 @@ class _MulLaunch:
     stream and from any thread (nothing in it is written after it is made).  Lowering the same call again took 22 us of
     interpreter time, the whole of a small product: mul! at 256^3 in Float32 takes 5 us on the device."""
 
-    __slots__ = ("_fn", "_conf", "_trans", "_conf_ref", "_trans_ref", "_code", "_workspace", "_packed", "_packed_ref", "_copies", "_copy_bytes")
+    __slots__ = ("_fn", "_conf", "_trans", "_conf_ref", "_trans_ref", "_code", "_workspace")
 
-    def __init__(self, p: Plan, packed):
+    def __init__(self, p: Plan):
         self._conf, self._trans = p._conf, p._trans         # (own the memory that the references point to)
         self._conf_ref = ctypes.byref(self._conf)
         self._trans_ref = ctypes.byref(self._trans) if self._trans is not None else None
         self._fn = p._fn
         self._workspace = _split_k_bytes(self._conf) if p._split_k else None
         self._code = None if p._split_k else p._args[-1]
-        self._packed = self._packed_ref = None
-        if packed is not None:
-            self._packed = _lib.gk_config.from_buffer_copy(self._conf)
-            self._packed_ref = ctypes.byref(self._packed)
-            shape, self._copies, at = self._conf.matmul_shape, [], 0
-            for which, (layout, mine, ld, extent) in enumerate(((self._packed.global_a_layout, self._conf.global_a_layout, packed[0], shape.M),
-                                                                (self._packed.global_b_layout, self._conf.global_b_layout, packed[1], shape.N))):
-                if ld is None:
-                    continue
-                rows, cols = _stored(which, mine.kind, extent, shape.K)
-                self._copies.append((which, rows, cols, mine.ld, at, ld))
-                layout.ld = ld
-                at += 2 * ld * cols
-            self._copy_bytes = at
+
+    def __call__(self, a: int, b: int, c: int, stream: int) -> None:
+        if self._workspace is None:
+            rc = self._fn(self._conf_ref, a, b, c, c, self._trans_ref, None, self._code, stream)
+        else:
+            workspace = _workspace(self._workspace, stream)
+            rc = self._fn(self._conf_ref, a, b, c, c, self._trans_ref, None, *_span(workspace), stream)
+        if rc != _lib.GK_OK:
+            _raise(rc)
+
+
+class _MulLaunchOnCopies(_MulLaunch):
+    """The same on copies of the operands whose columns start off a 16-byte boundary (``packed_leading_dims``)."""
+
+    __slots__ = ("_packed", "_packed_ref", "_copies", "_copy_bytes")
+
+    def __init__(self, p: Plan, packed):
+        super().__init__(p)
+        self._packed = _lib.gk_config.from_buffer_copy(self._conf)
+        self._packed_ref = ctypes.byref(self._packed)
+        shape, self._copies, at = self._conf.matmul_shape, [], 0
+        for which, (layout, mine, ld, extent) in enumerate(((self._packed.global_a_layout, self._conf.global_a_layout, packed[0], shape.M),
+                                                            (self._packed.global_b_layout, self._conf.global_b_layout, packed[1], shape.N))):
+            if ld is None:
+                continue
+            rows, cols = _stored(which, mine.kind, extent, shape.K)
+            self._copies.append((which, rows, cols, mine.ld, at, ld))
+            layout.ld = ld
+            at += 2 * ld * cols
+        self._copy_bytes = at
 
     def _on_copies(self, a: int, b: int, c: int, stream: int) -> bool:
         """The product on copies of the operands whose columns start off a 16-byte boundary (the same launch, the same bits).
@@ -683,15 +700,8 @@ class _MulLaunch:
         return True
 
     def __call__(self, a: int, b: int, c: int, stream: int) -> None:
-        if self._packed is not None and self._on_copies(a, b, c, stream):
-            return
-        if self._workspace is None:
-            rc = self._fn(self._conf_ref, a, b, c, c, self._trans_ref, None, self._code, stream)
-        else:
-            workspace = _workspace(self._workspace, stream)
-            rc = self._fn(self._conf_ref, a, b, c, c, self._trans_ref, None, *_span(workspace), stream)
-        if rc != _lib.GK_OK:
-            _raise(rc)
+        if not self._on_copies(a, b, c, stream):
+            super().__call__(a, b, c, stream)
 
 
 # launches by kind of operands and factors; a program has few kinds, one that has more pays for lowering again
