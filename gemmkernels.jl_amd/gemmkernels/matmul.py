@@ -600,7 +600,7 @@ def packed_leading_dims(conf_c, a: int, b: int):
 
     An operand whose columns start off 16-byte boundaries costs a launch more lines of memory and of L2 than its bytes:
     every 128-byte row of a tile lies on two lines.  Copies with columns on 128-byte lines cost 24 us for two operands of 32 MB
-    (5.3 TB/s) and leave the operands in the memory-side cache.  Inputs that rotate through more than that cache holds, BF16,
+    (5.3 TB/s; 33 us from inputs that left the caches) and leave the operands in the memory-side cache.  Inputs that rotate through more than that cache holds, BF16,
     both operands odd, 'N','N' / 'T','N': 4001 x 4003 x 4005 172 -> 155 / 182 -> 160 us, 3001 x 3003 x 3005 105 -> 87 / 113 -> 88,
     8001 x 8003 x 2005 459 -> 333 / 469 -> 337, 6001 x 5003 x 7005 488 -> 402 / 497 -> 405, 801 x 5003 x 6005 134 -> 108 / 133 -> 108; on
     the same inputs over and over they win from some 4e10 products on and are level below (4001 x 4003 x 4005 132 -> 138, 8001 x 8003
