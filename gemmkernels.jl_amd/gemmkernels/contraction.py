@@ -155,6 +155,8 @@ def plan(spec: str, a, b, d, c=None, ab_type: Optional[DType] = None, cd_type: O
     _shape_extents(dm, d, extents, "D")
     if c is not None:
         _shape_extents(dm, c, extents, "C")
+        if c.dtype != d.dtype:         # (the kernel reads C as it writes D: elements of another size lie elsewhere, also behind the end of C)
+            raise ConfigError(f"C must have the element type of D: {c.dtype} and {d.dtype}")
     ab_type = ab_type or from_torch(a.dtype)
     cd_type = cd_type or from_torch(d.dtype)
     if ab_type not in (Float16, BFloat16) or from_torch(b.dtype) != ab_type:
@@ -175,7 +177,7 @@ def contract(spec: str, a, b, d, c=None, stream=None):
     """``D[...] = sum A[...] * B[...] (+ C[...])`` in one launch on the current stream; returns ``d``."""
     from .matmul import _current_stream
     key = (spec, a.dtype, a.shape, a.stride(), b.dtype, b.shape, b.stride(), d.dtype, d.shape, d.stride(),
-           None if c is None else (c.shape, c.stride()))
+           None if c is None else (c.dtype, c.shape, c.stride()))
     launch = _launches.get(key)
     if launch is None:
         launch = _Launch(plan(spec, a, b, d, c))

@@ -110,6 +110,35 @@ def test_refused_contraction_names_the_reasons(gpu):
         contraction.plan("ab-ac-cb", a, gk.colmajor(np.zeros((32, 64), np.float16, order="F")), d)
 
 
+def test_c_of_another_type_than_d_is_refused(monkeypatch):
+    """The kernel reads C in D's element type: an FP16 C beside an FP32 D would be read behind its end.  Refused when the
+    contraction is planned and when its kind has been launched before (host memory: nothing is launched)."""
+    import torch
+    launched = []
+
+    class Recorder:
+        def __init__(self, p):
+            pass
+
+        def __call__(self, *args):
+            launched.append(args)
+    monkeypatch.setattr(contraction, "_Launch", Recorder)
+    monkeypatch.setattr(contraction, "_launches", {})
+    host = lambda shape, dtype: torch.zeros(tuple(reversed(shape)), dtype=dtype).permute(*reversed(range(len(shape))))
+    a, b = host((64, 32), torch.float16), host((32, 64), torch.float16)
+    for d_type, wrong in ((torch.float32, torch.float16), (torch.float16, torch.float32)):
+        d, c, bad = host((64, 64), d_type), host((64, 64), d_type), host((64, 64), wrong)
+        with pytest.raises(gk.ConfigError):
+            contraction.plan("ab-ac-cb", a, b, d, bad)
+        with pytest.raises(gk.ConfigError):
+            gk.contract("ab-ac-cb", a, b, d, bad, stream=0)
+        before = len(launched)
+        assert gk.contract("ab-ac-cb", a, b, d, c, stream=0) is d and len(launched) == before + 1
+        with pytest.raises(gk.ConfigError):
+            gk.contract("ab-ac-cb", a, b, d, bad, stream=0)
+        assert len(launched) == before + 1
+
+
 def test_division_by_multiplication_is_exact():
     """The kernels divide mode indices by the extents through a multiplication by a 32-bit reciprocal (s = ceil(log2 e),
     magic = floor(2^(31+s) / e) + 1, quotient = (n * magic) >> (31 + s)): exact for every n < 2^31.  Checked here on the
