@@ -167,11 +167,25 @@ TUNED = {}
 _GETT_TILES = [(256, 256, 64), (128, 128, 64), (64, 64, 64), (64, 64, 32)]
 
 
+def _tiles_k_modes(extents, block_k) -> bool:
+    """Whether a K tile of a contraction is a whole number of leading K modes times a divisor of the next one."""
+    whole = 1
+    for extent in extents:
+        if block_k % whole != 0:
+            return False
+        need = block_k // whole
+        if need <= extent:
+            return extent % need == 0
+        whole *= extent
+    return False
+
+
 def default_block_shape(operator, gemm_shape, tile_sized: bool = True, gett: bool = False, planar: bool = False,
-                        a_kmajor: bool = False, b_kmajor: bool = True) -> NT:
+                        a_kmajor: bool = False, b_kmajor: bool = True, k_modes=None) -> NT:
     """MI355X block shape: of the tiles of the table that divide the problem, the one with the shortest
     estimated launch (tiles per CU times the cost of a tile).  ``a_kmajor``: A is stored K x M ('T');
-    ``b_kmajor``: B is stored K x N ('N'); they admit the tiles with a side of 192."""
+    ``b_kmajor``: B is stored K x N ('N'); they admit the tiles with a side of 192.  ``k_modes``: extents of the K modes of a
+    contraction, which a K tile has to divide evenly as well."""
     M, N, K = gemm_shape["M"], gemm_shape["N"], gemm_shape["K"]
     if operator.kind in (Operator.FPU, Operator.FPU_TROPICAL):
         costs = _FPU_TILE_COST.get((operator.CT.name, operator.AT.name), {}) if operator.kind == Operator.FPU else {}
@@ -199,7 +213,7 @@ def default_block_shape(operator, gemm_shape, tile_sized: bool = True, gett: boo
     table = [t for t, _ in _MFMA_TILES] + [t for t, _, has in _MFMA_TILES_192 if has(a_kmajor, b_kmajor)]
     fitting = [t for t in table if not tile_sized or (M % t[0] == 0 and N % t[1] == 0 and K % t[2] == 0)]
     if gett:
-        fitting = [t for t in fitting if t in _GETT_TILES]
+        fitting = [t for t in fitting if t in _GETT_TILES and (k_modes is None or _tiles_k_modes(k_modes, t[2]))]
     if not fitting:
         return NT(M=64, N=64, K=32)
     # the shortest estimated launch (_MFMA_TILE_COST); ties go to the tile listed first
@@ -389,8 +403,10 @@ def get_config(*, gemm_shape, operator, global_a_layout, global_c_layout, **para
     planar = global_a_layout.kind in (Layout.SPLIT_COL_MAJOR, Layout.SPLIT_ROW_MAJOR)
     a_kmajor = global_a_layout.kind in (Layout.ROW_MAJOR, Layout.ALIGNED_ROW_MAJOR, Layout.INTERLEAVED_ROW_MAJOR, Layout.SPLIT_ROW_MAJOR)
     b_kmajor = global_b_layout.kind in (Layout.COL_MAJOR, Layout.ALIGNED_COL_MAJOR, Layout.INTERLEAVED_COL_MAJOR, Layout.SPLIT_COL_MAJOR)
-    block_shape = (default_block_shape(operator, gemm_shape, tile_sized, is_gett, planar, a_kmajor=a_kmajor, b_kmajor=b_kmajor)
-                   if block_shape is None else NT(block_shape))
+    if block_shape is None:
+        k_modes = [mode[0] for mode in global_a_layout.gett.k] if global_a_layout.kind == Layout.GETT_KIND else None
+        block_shape = default_block_shape(operator, gemm_shape, tile_sized, is_gett, planar, a_kmajor=a_kmajor, b_kmajor=b_kmajor, k_modes=k_modes)
+    block_shape = NT(block_shape)
     op_shape = Operator.shape(operator)
 
     checked = any(l.kind in (Layout.COL_MAJOR, Layout.ROW_MAJOR) for l in (global_a_layout, global_b_layout, global_c_layout, global_d_layout))

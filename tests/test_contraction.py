@@ -110,6 +110,18 @@ def test_refused_contraction_names_the_reasons(gpu):
         contraction.plan("ab-ac-cb", a, gk.colmajor(np.zeros((32, 64), np.float16, order="F")), d)
 
 
+@pytest.mark.parametrize("e,f", [(96, 2), (64, 2), (32, 2), (16, 6), (96, 4), (32, 3), (8, 24), (160, 2)])
+@pytest.mark.parametrize("a", [64, 128, 1024])
+def test_default_tile_of_a_configuration_tiles_the_k_modes(a, e, f):
+    """A contraction configured without a block shape gets a tile that the library takes: 64 divides K = 96 x 2 but tiles
+    neither mode.  (No GPU.)"""
+    from gemmkernels import Kernel, configs
+    conf, _ = configs.gett_config("aef", "bfe", "ab", dict(a=a, b=a, e=e, f=f))
+    assert gk.kernel_name(conf, Kernel.matmul_pipelined).endswith("_gett")
+    if (e, f) == (96, 2):
+        assert conf.block_shape.K == 32
+
+
 def test_c_of_another_type_than_d_is_refused(monkeypatch):
     """The kernel reads C in D's element type: an FP16 C beside an FP32 D would be read behind its end.  Refused when the
     contraction is planned and when its kind has been launched before (host memory: nothing is launched)."""
