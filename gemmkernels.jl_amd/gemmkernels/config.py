@@ -217,7 +217,7 @@ def default_block_shape(operator, gemm_shape, tile_sized: bool = True, gett: boo
     if not fitting:
         return NT(M=64, N=64, K=32)
     # the shortest estimated launch (_MFMA_TILE_COST); ties go to the tile listed first
-    best = min(fitting, key=lambda t: (_mfma_cost(t, M, N, K), fitting.index(t)))
+    best = min(fitting, key=lambda t: (_mfma_cost(t, M, N, K, not gett), fitting.index(t)))
     return NT(M=best[0], N=best[1], K=best[2])
 
 

@@ -122,6 +122,15 @@ def test_default_tile_of_a_configuration_tiles_the_k_modes(a, e, f):
         assert conf.block_shape.K == 32
 
 
+@pytest.mark.parametrize("ext", [dict(a=640, b=640, e=64, f=64), dict(a=1024, b=1024, e=64, f=32), dict(a=64, b=64, e=64, f=64)])
+def test_default_tile_of_a_contraction_with_few_tiles_and_a_long_k(ext):
+    """64 x 64 x 64 on four LDS stages: the plain product of these sizes named 64 x 64 x 32 runs there too, two K tiles to a
+    stage, but the contraction of that tile is one wave on two stages.  (No GPU.)"""
+    from gemmkernels import Kernel, configs
+    conf, _ = configs.gett_config("aef", "bfe", "ab", ext)
+    assert gk.kernel_name(conf, Kernel.matmul_pipelined) == "mfma_gemm_nt_64x64x64_w2x2_s4__Float16_gett"
+
+
 def test_c_of_another_type_than_d_is_refused(monkeypatch):
     """The kernel reads C in D's element type: an FP16 C beside an FP32 D would be read behind its end.  Refused when the
     contraction is planned and when its kind has been launched before (host memory: nothing is launched)."""
