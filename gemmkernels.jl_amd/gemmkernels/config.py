@@ -222,10 +222,20 @@ def default_block_shape(operator, gemm_shape, tile_sized: bool = True, gett: boo
 
 
 def split_k_block_shape(M, N, K, widest_ld=0, factor=None) -> Optional[NT]:
-    """The tile of a 16-bit product with few output tiles and a long K, or None (the default tile).  ``factor``: how alpha is applied to A
-    in the K loop ("packed", FP16; "per element", BF16).  ``widest_ld``: the larger leading dimension of the operands whose rows are the k
-    of a tile; the kernel keeps the offsets in a tile in 32 bits, so 64 rows of 2^24 elements are left to a tile with fewer.  Whether the
-    product is cut into slices of K as well: ``slices_pay``."""
+    """The tile of a 16-bit product with few output tiles and a long K, which is cut into slices of K (``Kernel.matmul_split_k``), or None (the
+    default tile, and one chain over K).  In us, slices against unsplit with four LDS stages: 64 tiles K = 1280 7.5 and 7.5, 2048 8.7 and 10.5, 4096
+    11.1 and 17.6; 128 tiles K = 1280 8.6 and 7.9, 2048 9.8 and 10.7; three slices of 165 tiles K = 3072 13.0 and 14.7, 4096 14.3 and 18.1.
+
+    171 to 256 tiles leave two slices, which are there for the error as well: half the chain has 2.9e-7 of the norm where the whole has 4.1e-7 (K = 4096,
+    FP16 uniform in [-1, 1); 1.5e-7 and 3e-7 on values of one sign; 4.1 and 5.7e-7, 2.2 and 4.3e-7 at K = 8192).  Their time, 'N','N' / 'T','N':
+    K = 8192 180 tiles 29.5 and 32.1 / 28.1 and 31.1, 210 tiles 30.0 and 32.3 / 28.4 and 31.3, 256 tiles 32.3 and 32.4 / 28.2 and 31.8; K = 16384 256 tiles
+    80.0 and 86.1 / 67.5 and 72.6; K = 4096 180 tiles 18.0 and 18.1 / 17.0 and 17.6, 256 tiles 19.2 and 18.1 / 17.6 and 17.8; 256 tiles K = 3072 16.2 and 14.7
+    / 15.4 and 14.4; 1001 x 704 x 3328 20.9 and 18.1 / 15.7 and 16.0; 1024 x 768 x 4004 21.5 and 22.4 / 25.3 and 24.3.  Not where K and the output are both
+    ragged (1001 x 700 x 3333, 1000 x 1000 x 4000).
+
+    ``factor``: how alpha is applied to A in the K loop, which makes it longer ("packed", FP16; "per element", BF16): FP16 111 x 2629 x 1477 (84 tiles) 15.7
+    and 19.9.  ``widest_ld``: the larger leading dimension of the operands whose rows are the k of a tile; the kernel keeps the offsets in a tile
+    in 32 bits, so 64 rows of 2^24 elements are left to a tile with fewer."""
     if 64 * widest_ld * 2 >= 1 << 31:
         return None
     tiles = -(-M // 64) * -(-N // 64)
@@ -236,15 +246,6 @@ def split_k_block_shape(M, N, K, widest_ld=0, factor=None) -> Optional[NT]:
         two = {None: whole, "packed": True, "per element": tiles <= 225 and min(M, N) > 128}[factor]
         worth = K >= 3000 and (tiles <= 170 or tiles <= 256 and two)
     return NT(M=64, N=64, K=64) if worth else None
-
-
-def slices_pay(M, N, K, factor=None) -> bool:
-    """Whether a product on the tile of ``split_k_block_shape`` is worth cutting into slices of K (``Kernel.matmul_split_k``), next to the four
-    LDS stages that carry a lone workgroup through K at 0.22 us per 64 k.  In us, slices against unsplit: 64 tiles K = 1280 7.5 and 7.5,
-    2048 8.7 and 10.5, 4096 11.1 and 17.6; 128 tiles K = 1280 8.6 and 7.9, 2048 9.8 and 10.7; three slices of 165 tiles 3072 13.0 and 14.7, 4096
-    14.3 and 18.1; two slices of 180 .. 256 tiles gain nothing (180 tiles K = 4096 17.7 and 18.0, 256 tiles 19.1 and 18.4).  A factor that stays
-    in the K loop makes it longer: FP16 111 x 2629 x 1477 (84 tiles) 15.7 and 19.9; 1024 x 1024 x 4096 (256) FP16 21.4 in two slices, BF16 unsplit 33.9."""
-    return factor is not None or -(-M // 64) * -(-N // 64) <= 170
 
 
 # Estimated launch time of a tile, in microseconds: what a launch costs whatever its size, per 1000 k and round, per further tile of

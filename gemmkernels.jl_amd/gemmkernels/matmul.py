@@ -20,7 +20,7 @@ from . import kernel as Kernel
 from . import layout as Layout
 from . import operator as Operator
 from . import transform as Transform
-from .config import Config, default_block_shape, get_config as _get_config, slices_pay, split_k_block_shape
+from .config import Config, default_block_shape, get_config as _get_config, split_k_block_shape
 from .dtypes import BFloat16, DType, Float16, Float32, Float64, from_torch, promote_type
 from .errors import ConfigError, DimensionMismatch
 from .tiling import NT
@@ -542,7 +542,7 @@ def _single_plan(C, tA: bool, tB: bool, A, B, alpha, beta, wmma=None) -> Plan:
         # ordered, so the result is the same on every run, like the reference's mul!.
         bs, ms = conf.block_shape, conf.matmul_shape
         tiles = -(-ms.M // bs.M) * -(-ms.N // bs.N)
-        if slices_pay(ms.M, ms.N, ms.K, factor) if bs == split_k_block_shape(ms.M, ms.N, ms.K, 0, factor) else (tiles <= 128 and ms.K >= 2048):
+        if bs == split_k_block_shape(ms.M, ms.N, ms.K, 0, factor) or tiles <= 128 and ms.K >= 2048:
             kernel = Kernel.matmul_split_k
     p = plan(conf, A, B, C, C, transform_shared_to_regs_a=ta, transform_shared_to_regs_c=tc, kernel=kernel)
     p.kernel_names = (kernel_name(conf, kernel, dict(transform_shared_to_regs_a=ta, transform_shared_to_regs_c=tc)),)

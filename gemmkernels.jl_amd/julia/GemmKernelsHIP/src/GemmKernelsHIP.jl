@@ -777,7 +777,7 @@ function create_config(A::Type, sizeA::Dims, stridesA::Dims, transA::Bool,
     (conf, compute_type, select_kernel(ga, gb))
 end
 
-# a 16-bit product with few 64 x 64 output tiles and a long K runs on tiles of 64 x 64 x 64 (the sizes: split_k_block_shape of the Python package),
+# a 16-bit product with few 64 x 64 output tiles and a long K runs on slices of K (the sizes: split_k_block_shape of the Python package),
 # unless its operands' 64 rows of k lie further apart than 32-bit offsets reach
 function worth_splitting(m, n, k, widest_ld, factor)
     64 * widest_ld * 2 < 2^31 || return false
@@ -787,8 +787,6 @@ function worth_splitting(m, n, k, widest_ld, factor)
     two = factor === :none ? whole : factor === :packed || (tiles <= 225 && min(m, n) > 128)
     k >= 3000 && (tiles <= 170 || (tiles <= 256 && two))
 end
-# ... and these are the ones that slices make faster than four LDS stages do (slices_pay of the Python package)
-slices_pay(m, n, k, factor) = factor !== :none || cld(m, 64) * cld(n, 64) <= 170
 # alpha stays in the K loop unless it is a power of two that the library folds into the accumulators
 factor_of(alpha, A, B) = abs(Float64(alpha)) in (2.0 .^ (-4:4)) ? :none : (:BFloat16 in (nameof(eltype(A)), nameof(eltype(B))) ? :per_element : :packed)
 
@@ -816,9 +814,7 @@ function matmatmul!(C, transA::Char, transB::Char, A, B, alpha::Number, beta::Nu
     if Operator.is_mfma(conf.operator)
         # few output tiles and a long K loop: K slices as workgroups of one launch (ordered sum: same bits every run)
         bs, ms = conf.block_shape, conf.matmul_shape
-        factor = factor_of(alpha, A, B)
-        few = bs == (M = 64, N = 64, K = 64) && worth_splitting(ms.M, ms.N, ms.K, 0, factor)
-        if few ? slices_pay(ms.M, ms.N, ms.K, factor) : cld(ms.M, bs.M) * cld(ms.N, bs.N) <= 128 && ms.K >= 2048
+        if bs == (M = 64, N = 64, K = 64) && worth_splitting(ms.M, ms.N, ms.K, 0, factor_of(alpha, A, B)) || cld(ms.M, bs.M) * cld(ms.N, bs.N) <= 128 && ms.K >= 2048
             kernel = Kernel.matmul_split_k
         end
     end

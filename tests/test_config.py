@@ -429,3 +429,26 @@ def test_two_slices_of_more_than_170_tiles_only_where_they_pay():
     assert block(768, 1024, 4096, "per element") == split and block(1024, 1024, 4096, "per element") == narrow
     assert block(12032, 64, 4096, "per element") != split and block(12032, 64, 4096) == split
     assert block(700, 900, 3001) == split and block(300, 200, 1301) == split
+
+
+@pytest.mark.parametrize("dims,dtype,alpha,slices", [((700, 900, 3001), "float16", 1.0, 3), ((1001, 704, 3328), "float16", 1.0, 2), ((1024, 704, 3333), "bfloat16", 1.0, 2), ((1024, 1024, 4096), "float16", 1.0, 2),
+                                                     ((1024, 1024, 16384), "bfloat16", 2.0, 2), ((201, 4096, 8064), "float16", 1.0, 2), ((3722, 192, 7232), "bfloat16", 1.0, 2), ((1001, 700, 3333), "float16", 1.0, 1),
+                                                     ((1001, 700, 3333), "float16", 1.5, 2), ((1024, 1088, 4096), "float16", 1.0, 1), ((1024, 1024, 2944), "float16", 1.0, 1), ((4096, 64, 4096), "float16", 1.0, 4)])
+def test_the_slices_a_product_is_launched_in(dims, dtype, alpha, slices):
+    """What mul! launches on both sides of 170 and of 256 tiles, read from the plan and the workspace it asks for (no GPU: the operands
+    are on the host, nothing is launched).  Two slices halve the chain of a sum: products of 171 to 256 tiles have 0.7 of the error."""
+    import torch
+    import sys
+    matmul = sys.modules["gemmkernels.matmul"]
+    M, N, K = dims
+    host = lambda rows, cols, t: torch.empty((cols, rows), dtype=t).t()
+    a, b, c = host(M, K, getattr(torch, dtype)), host(K, N, getattr(torch, dtype)), host(M, N, torch.float32)
+    p = matmul.matmatmul_plan(c, 'N', 'N', a, b, alpha, 0.0)
+    need = matmul._split_k_bytes(p._conf) if p._split_k else 0
+    bs = p._conf.block_shape
+    tiles = -(-M // bs.M) * -(-N // bs.N)
+    # (the query answers for the launch with hooks on A and B too, which takes more slices of few tiles)
+    assert p._split_k == (slices > 1)
+    if slices > 1:
+        most = (need - 2048) // (tiles * bs.M * bs.N * 4)
+        assert most == slices or tiles <= 128 and most > slices
