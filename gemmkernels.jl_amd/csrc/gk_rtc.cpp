@@ -122,15 +122,15 @@ int gk_rtc_compile(const gk_config* conf, const char* const hooks[8], int32_t ke
   const int b_kmajor = is_row_major(c->global_b_layout.kind) ? 0 : 1;     // 'N' B: stored K x N, K contiguous
   if ((!a_kmajor && (b.M & (b.M - 1))) || (!b_kmajor && (b.N & (b.N - 1))))
     return fail(GK_ERR_BLOCK_SHAPE, "an operand that is contiguous along M (N) needs a power-of-two BLOCK_M (BLOCK_N)");
-  bool any_ab = false, any = false;
+  bool any_ab = false;
   for (int h = 0; h < 8; ++h)
     if (hooks && hooks[h] && hooks[h][0]) {
-      any = true;
       if (h == GK_HOOK_GLOBAL_TO_SHARED_A || h == GK_HOOK_GLOBAL_TO_SHARED_B || h == GK_HOOK_SHARED_TO_REGS_A || h == GK_HOOK_SHARED_TO_REGS_B) any_ab = true;
       if (strlen(hooks[h]) > 1024) return fail(GK_ERR_INVALID_ARGUMENT, "hook expression longer than 1024 characters");
     }
-  (void)any;
-  const int fuse = any_ab ? 2 : 1;      // level 1 also carries the bias epilogue, chosen at launch time
+  // level 3: C / D hooks and the bias epilogue, chosen at launch time, on the K loop without hooks (level 1 multiplies every fragment of A,
+  // by 1 here: five instructions per two values in BF16)
+  const int fuse = any_ab ? 2 : 3;
   // operand kinds of the kernel template: 0 K-major, 1 M-major
   const std::string src = build_source(c, hooks, stages, fuse, a_kmajor ? 0 : 1, b_kmajor ? 0 : 1, dt == GK_F16 ? "_Float16" : "__bf16");
 
@@ -253,7 +253,7 @@ int gk_rtc_matmul(gk_rtc_kernel* k, const gk_config* conf, const void* a, const 
   const int kind = conf->block_shape.K < 2 * conf->compute_op_shape.K ? GK_KERNEL_SINGLESTAGE : GK_KERNEL_PIPELINED;
   int rc = gk_internal::prepare_launch(conf, a, b, c, d, nullptr, epilogue, kind, &k->info, &L);
   if (rc != GK_OK) return rc;
-  L.args.fast_scale_a = L.args.fast_scale_b = 0;
+  L.args.fast_scale_a = L.args.fast_scale_b = 0;        // (hooks on A and B are compiled in)
   if (k->info.lds_bytes > 64 * 1024 && !k->lds_raised) {
     // module functions take the attribute through the same call as host-side kernel symbols; a
     // runtime that does not accept it for them reports the LDS request at the launch below instead

@@ -68,6 +68,16 @@ def test_no_packed_fp32_instructions(tmp_path, hooks, dtype):
     assert not [line for line in text.splitlines() if "v_pk_" in line and "_f32" in line]
 
 
+@pytest.mark.parametrize("dtype", ["BFloat16", "Float16"])
+def test_without_hooks_on_a_and_b_the_k_loop_has_no_vector_arithmetic_on_fragments(tmp_path, dtype):
+    """Only a hook on D: between the first and the last matrix instruction nothing multiplies or converts values of A and B."""
+    lines = assembly(tmp_path, dict(transform_shared_to_global_d=LEAKY), dtype).splitlines()
+    mfma = [i for i, line in enumerate(lines) if "v_mfma_f32_16x16x32" in line]
+    assert len(mfma) >= 64
+    loop = lines[mfma[0]:mfma[-1]]
+    assert not [line for line in loop if any(op in line for op in ("v_mul_f32", "v_pk_mul_f16", "v_cvt_pk_bf16_f32"))]
+
+
 def reference(a, b, c, bias, leaky=True, scale_a=1.0):
     acc = (a.astype(np.float64) * scale_a) @ b.astype(np.float64)
     if c is not None:
@@ -117,6 +127,31 @@ def test_closed_vocabulary_hooks_give_the_same_bits_as_the_compiled_kernels(gpu,
     gk.specialize(conf, **hooks)(A, B, C, D2)
     torch.cuda.synchronize()
     assert np.array_equal(gk.to_numpy(D1), gk.to_numpy(D2))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+def test_a_hook_on_d_alone_gives_the_same_bits_as_the_compiled_kernel(gpu, dtype):
+    """With C and a bias, over partial magnitudes and signs; the K loop is that of a product without hooks."""
+    import torch
+    M, N, K = 256, 384, 320
+    T = gk.BFloat16 if dtype == "bfloat16" else Float16
+    conf = gk.get_config(gemm_shape=NT(M=M, N=N, K=K), operator=Operator.MFMAOp[32, 32, 16, T, Float32],
+                         global_a_layout=Layout.UnsafeAlignedColMajor[T], global_b_layout=Layout.UnsafeAlignedColMajor[T],
+                         global_c_layout=Layout.UnsafeAlignedColMajor[Float32], global_d_layout=Layout.UnsafeAlignedColMajor[Float32],
+                         block_shape=NT(M=128, N=128, K=64))
+    gen = torch.Generator(device="cuda").manual_seed(17)
+    draw = lambda rows, cols, t: (torch.rand(cols, rows, generator=gen, device="cuda") * 2 - 1).to(t).t()
+    a, b, c = draw(M, K, getattr(torch, dtype)), draw(K, N, getattr(torch, dtype)), draw(M, N, torch.float32)
+    bias = torch.randn(N, generator=gen, device="cuda")
+    d1, d2 = gk.colmajor_empty((M, N), torch.float32), gk.colmajor_empty((M, N), torch.float32)
+    relu = Transform.Elementwise(Transform.relu)
+    gk.matmul(conf, a, b, c, d1, kernel=Kernel.matmul_pipelined, transform_shared_to_global_d=relu, epilogue=Epilogue.Bias(bias))
+    gk.specialize(conf, transform_shared_to_global_d=relu)(a, b, c, d2, epilogue=Epilogue.Bias(bias))
+    torch.cuda.synchronize()
+    assert torch.equal(d1, d2)
+    want = torch.relu(a.double() @ b.double() + c.double() + bias.double())
+    assert float((d2.double() - want).norm() / want.norm()) <= 1e-6          # (fp32 sums of exact products, K = 320)
 
 
 @pytest.mark.gpu
