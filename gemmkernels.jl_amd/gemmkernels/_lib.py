@@ -117,6 +117,8 @@ _SIGNATURES = {
                                                  ctypes.POINTER(gk_transforms), ctypes.POINTER(gk_epilogue), ctypes.c_void_p]),
     "gk_pack_columns": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64,
                                        ctypes.c_void_p, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]),
+    "gk_pack_columns_padded": (ctypes.c_int, 2 * [ctypes.c_void_p, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int64,
+                                                  ctypes.c_int64] + [ctypes.c_void_p]),
     "gk_probe_matrix_rate": (ctypes.c_int, [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.POINTER(ctypes.c_double)]),
     "gk_rtc_compile": (ctypes.c_int, [ctypes.POINTER(gk_config), ctypes.POINTER(ctypes.c_char_p), ctypes.c_int32,
                                       ctypes.POINTER(ctypes.c_void_p)]),

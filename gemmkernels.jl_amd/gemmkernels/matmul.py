@@ -20,7 +20,7 @@ from . import kernel as Kernel
 from . import layout as Layout
 from . import operator as Operator
 from . import transform as Transform
-from .config import Config, default_block_shape, get_config as _get_config, split_k_block_shape
+from .config import _MFMA_TILE_COST, Config, _mfma_cost, default_block_shape, get_config as _get_config, split_k_block_shape
 from .dtypes import BFloat16, DType, Float16, Float32, Float64, from_torch, promote_type
 from .errors import ConfigError, DimensionMismatch
 from .tiling import NT
@@ -590,41 +590,52 @@ def _stored(which: int, kind: int, extent: int, k: int):
     return (k, extent) if row_major == (which == 0) else (extent, k)
 
 
-_PACK_MIN_WORK, _PACK_MIN_WORK_ONE = 24 * 10 ** 9, 50 * 10 ** 9      # M N K with both operands, with one of them
+_PACK_MIN_WORK, _PACK_MIN_WORK_ONE = 24 * 10 ** 9, 80 * 10 ** 9      # M N K with both operands, with one of them
 _PACK_MAX_BYTES = 512 << 20
+_PACK_SHARE, _PACK_SHARE_ONE = (0.29, 0.325, 0.36), 0.13             # of the product's time; both operands: by how many are contiguous along k
 
 
 def packed_leading_dims(conf_c, a: int, b: int):
     """Leading dimensions of copies of A and of B (None: the operand stays as it is) on which a product runs faster, the
     copying included, or None.
 
-    An operand whose columns start off 16-byte boundaries costs a launch more lines of memory and of L2 than its bytes:
-    every 128-byte row of a tile lies on two lines.  Copies with columns on 128-byte lines cost 24 us for two operands of 32 MB
-    (5.3 TB/s; 33 us from inputs that left the caches) and leave the operands in the memory-side cache.  Inputs that rotate through more than that cache holds, BF16,
-    both operands odd, 'N','N' / 'T','N': 4001 x 4003 x 4005 172 -> 155 / 182 -> 160 us, 3001 x 3003 x 3005 105 -> 87 / 113 -> 88,
-    8001 x 8003 x 2005 459 -> 333 / 469 -> 337, 6001 x 5003 x 7005 488 -> 402 / 497 -> 405, 801 x 5003 x 6005 134 -> 108 / 133 -> 108; on
-    the same inputs over and over they win from some 4e10 products on and are level below (4001 x 4003 x 4005 132 -> 138, 8001 x 8003
-    x 2005 376 -> 330).  Below 2.4e10 the copies take what they save (2001 x 2003 x 4005 57 -> 65, 3001 x 3003 x 1505 55 -> 57,
-    8001 x 503 x 3005 63 -> 63).  One odd operand, contiguous along k: 4000 x 4000 x 4001 'N','N' 140 -> 126, 3000 x 3000 x 3001 100 -> 92
-    and 73 -> 77 on the same inputs; along m or n: 4001 x 4000 x 4000 160 -> 155, 123 -> 125, not worth a copy."""
+    An operand whose columns start off 16-byte boundaries costs a launch more lines of memory and of L2 than its bytes: a 128-byte row of a
+    tile lies on two lines where k is contiguous, one of 512 bytes on five.  Copies with columns on 128-byte lines are read and written at 5.3 TB/s while
+    they and the operands fit the memory-side cache (4 TB/s beyond), and they pay where that is a small enough share of the product
+    (_mfma_cost); copies of both operands end in whole K tiles as well (_MulLaunchOnCopies).  BF16, us without and with copies, each on the same inputs over
+    and over / on inputs that rotate through 600 MB / alone on new ones, by that share:
+      0.08 8001 x 8003 x 2005 'N','T' 366 307 / 441 309 / 450 328, 'T','N' 396 292 / 468 292 / 483 311;
+      0.18 3001 x 3003 x 3005 'N','T' 82 83 / 105 86 / 100 104, 'T','N' 83 76 / 113 80 / 101 99; 2501 x 8003 x 4005 'N','N' 202 190 / 268 197 / 288 225;
+      0.24 4001 x 4003 x 4005 'N','N' 133 126 / 171 143 / 153 151, 'N','T' 129 129 / 168 144 / 145 147, 'T','N' 137 126 / 178 143 / 155 149;
+      0.28 801 x 5003 x 6005 'N','N' 117 99 / 134 102 / 131 117; 0.30 2001 x 2003 x 6005 'N','T' 71 78 / 88 81 / 89 101, 'N','N' 78 73 / 105 78 / 97 94;
+      0.27 2501 x 8003 x 8005 'N','T' 4 % slower / 22 % faster / 12 % faster; 0.34 1001 x 8003 x 4005 'N','N' 90 91 / 122 93 / 148 124, 'N','T' 86 91 / 108 94 / 120 131,
+      'T','N' 94 88 / 125 91 / 148 122; 0.39 4001 x 4003 x 8100 6 to 9 % slower / 13 to 20 % faster / between;
+      0.48 1501 x 8003 x 8005 'N','N' 193 233 / 249 233 / 270 287.
+    Below 2.4e10 products the copies take what they save (2001 x 2003 x 4005, 3001 x 3003 x 1505).  One odd operand, contiguous along k:
+      4000 x 4000 x 4001 'N','N' 111 114 / 139 125 / 125 128 (6.4e10, not copied), 5000 x 5000 x 5001 258 239 / 337 281 / 342 296, 6000 x 6000 x 6001 'N','N' 387 389 / 440 417 /
+      466 443 and 'T','T' 408 439 / 509 441 / 526 466, 8000 x 8000 x 8001 915 796 / 929 795 / 944 794; a share of 0.3 2000 x 8000 x 8001 210 242 / 255 243 / 253 264;
+      along m or n: not worth a copy (4001 x 4000 x 4000 'N','N' 123 125 / 160 155)."""
     shape, layouts = conf_c.matmul_shape, (conf_c.global_a_layout, conf_c.global_b_layout)
     work = shape.M * shape.N * shape.K
-    if conf_c.op.kind != Operator.MFMA or work < _PACK_MIN_WORK or min(shape.M, shape.N) < 512 or shape.K < 1000:
+    tile = (conf_c.block_shape.M, conf_c.block_shape.N, conf_c.block_shape.K)
+    if conf_c.op.kind != Operator.MFMA or work < _PACK_MIN_WORK or min(shape.M, shape.N) < 512 or shape.K < 1000 or tile not in _MFMA_TILE_COST:
         return None
     if any(layout.kind == Layout.ZERO for layout in layouts):        # (alpha = 0)
         return None
     odd = tuple(layout.ld % 8 != 0 or address % 16 != 0 for layout, address in zip(layouts, (a, b)))
-    stored = tuple(_stored(which, layouts[which].kind, (shape.M, shape.N)[which], shape.K) for which in (0, 1))
-    if not all(odd):
-        k_major = tuple(layouts[which].kind in ((Layout.ROW_MAJOR, Layout.ALIGNED_ROW_MAJOR) if which == 0 else (Layout.COL_MAJOR, Layout.ALIGNED_COL_MAJOR))
-                        for which in (0, 1))
-        if work < _PACK_MIN_WORK_ONE or not any(o and k for o, k in zip(odd, k_major)):
-            return None
+    k_major = tuple(layouts[which].kind in ((Layout.ROW_MAJOR, Layout.ALIGNED_ROW_MAJOR) if which == 0 else (Layout.COL_MAJOR, Layout.ALIGNED_COL_MAJOR))
+                    for which in (0, 1))
+    if not all(odd) and (work < _PACK_MIN_WORK_ONE or not any(o and k for o, k in zip(odd, k_major))):
+        return None
+    k = -(-shape.K // 64) * 64 if all(odd) else shape.K
+    stored = tuple(_stored(which, layouts[which].kind, (shape.M, shape.N)[which], k) for which in (0, 1))
     packed = tuple(-(-rows // 64) * 64 if o else None for o, (rows, _) in zip(odd, stored))
     total = sum(2 * ld * cols for ld, (_, cols) in zip(packed, stored) if ld is not None)
     if total > _PACK_MAX_BYTES or max(rows for rows, _ in stored) > _PACK_MAX_ROWS:
         return None
-    return packed
+    copying = 2 * total / (5.3e6 if total < 100e6 else 4.0e6)
+    share = _PACK_SHARE[sum(k_major)] if all(odd) else _PACK_SHARE_ONE
+    return packed if copying <= share * _mfma_cost(tile, shape.M, shape.N, shape.K) else None
 
 
 _PACK_MAX_ROWS = 255 * 512          # of one launch of gk_pack_columns
@@ -657,7 +668,9 @@ class _MulLaunch:
 
 
 class _MulLaunchOnCopies(_MulLaunch):
-    """The same on copies of the operands whose columns start off a 16-byte boundary (``packed_leading_dims``)."""
+    """The same on copies of the operands whose columns start off a 16-byte boundary (``packed_leading_dims``).  Copies of both operands
+    are filled up with zeros to whole K tiles of 64: the partial one, which the kernels run outside their pipeline, takes some 10 us per
+    round of tiles (the product on copies 4001 x 4003 x 4005 110 -> 100 us, from memory 136 -> 127), and sums of zeros change no bit."""
 
     __slots__ = ("_packed", "_packed_ref", "_copies", "_copy_bytes")
 
@@ -666,33 +679,35 @@ class _MulLaunchOnCopies(_MulLaunch):
         self._packed = _lib.gk_config.from_buffer_copy(self._conf)
         self._packed_ref = ctypes.byref(self._packed)
         shape, self._copies, at = self._conf.matmul_shape, [], 0
+        k = shape.K if None in packed else -(-shape.K // 64) * 64
+        self._packed.matmul_shape.K = k
         for which, (layout, mine, ld, extent) in enumerate(((self._packed.global_a_layout, self._conf.global_a_layout, packed[0], shape.M),
                                                             (self._packed.global_b_layout, self._conf.global_b_layout, packed[1], shape.N))):
             if ld is None:
                 continue
-            rows, cols = _stored(which, mine.kind, extent, shape.K)
-            self._copies.append((which, rows, cols, mine.ld, at, ld))
+            (rows, cols), (rows_copy, cols_copy) = _stored(which, mine.kind, extent, shape.K), _stored(which, mine.kind, extent, k)
+            self._copies.append((which, at, (rows, cols, mine.ld), (ld, rows_copy, cols_copy)))
             layout.ld = ld
-            at += 2 * ld * cols
+            at += 2 * ld * cols_copy
         self._copy_bytes = at
 
     def _on_copies(self, a: int, b: int, c: int, stream: int) -> bool:
         """The product on copies of the operands whose columns start off a 16-byte boundary (the same launch, the same bits).
         False: not here -- no memory for the copies, or a capture, whose graph would have to keep them."""
         import torch
-        if _capture_of(stream) is not None:
+        # (`stream` is torch's current one: what torch says of captures and allocates is that stream's)
+        if torch.cuda.is_current_stream_capturing():
             return False
         # memory of this call alone, in the order of the stream: what gets it next on this stream runs behind the product
-        with _on(stream):
-            try:
-                copies = torch.empty(self._copy_bytes, dtype=torch.uint8, device="cuda")
-            except torch.OutOfMemoryError:
-                return False
+        try:
+            copies = torch.empty(self._copy_bytes, dtype=torch.uint8, device="cuda")
+        except torch.OutOfMemoryError:
+            return False
         base, operands, jobs = copies.data_ptr(), [a, b], []
-        for which, rows, cols, ld, at, ld_packed in self._copies:
-            jobs += [operands[which], rows, cols, ld, base + at, ld_packed]
+        for which, at, source, copy in self._copies:
+            jobs += (operands[which], *source, base + at, *copy)
             operands[which] = base + at
-        rc = _lib.lib().gk_pack_columns(*jobs, *((None, 0, 0, 0, None, 0) if len(jobs) == 6 else ()), stream)
+        rc = _lib.lib().gk_pack_columns_padded(*jobs, *((None, 0, 0, 0, None, 0, 0, 0) if len(jobs) == 8 else ()), stream)
         if rc == _lib.GK_OK:
             rc = self._fn(self._packed_ref, *operands, c, c, self._trans_ref, None, self._code, stream)
         if rc != _lib.GK_OK:

@@ -318,6 +318,12 @@ int gk_matmul_split_k_noalloc(const gk_config* conf, const void* a, const void* 
 int gk_pack_columns(const void* src0, int64_t rows0, int64_t cols0, int64_t ld0, void* dst0, int64_t ld_dst0, const void* src1,
                     int64_t rows1, int64_t cols1, int64_t ld1, void* dst1, int64_t ld_dst1, void* stream);
 
+/* The same with copies of rows_dst x cols_dst elements each (at least rows x cols, ld_dst at least rows_dst), zero outside the
+ * matrix: a product whose K is no whole number of K tiles runs on whole ones. */
+int gk_pack_columns_padded(const void* src0, int64_t rows0, int64_t cols0, int64_t ld0, void* dst0, int64_t ld_dst0, int64_t rows_dst0, int64_t cols_dst0,
+                           const void* src1, int64_t rows1, int64_t cols1, int64_t ld1, void* dst1, int64_t ld_dst1, int64_t rows_dst1,
+                           int64_t cols_dst1, void* stream);
+
 /* A measurement aid with no counterpart in the reference (its benchmarks quote fractions of a data-sheet peak): the
  * rate, in TFLOP/s, of a register-only loop of the MFMA instruction the GEMM kernels use (v_mfma_f32_16x16x32_f16,
  * one wave per SIMD, 64 accumulator blocks per wave, operands that change every 64 MFMAs), over `launches` launches

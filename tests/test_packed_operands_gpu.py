@@ -19,6 +19,8 @@ class _Layouts:
         conf.matmul_shape.M, conf.matmul_shape.N, conf.matmul_shape.K = M, N, K
         conf.global_a_layout.kind, conf.global_b_layout.kind = 1 + ta, 1 + tb        # ColMajor, RowMajor
         conf.global_a_layout.ld, conf.global_b_layout.ld = lda, ldb
+        tile = gk.default_block_shape(gk.Operator.MFMAOp[32, 32, 16, gk.BFloat16, gk.Float32], gk.NT(M=M, N=N, K=K), tile_sized=False, a_kmajor=ta, b_kmajor=not tb)
+        conf.block_shape.M, conf.block_shape.N, conf.block_shape.K = tile.M, tile.N, tile.K
         return conf
 
 
@@ -27,10 +29,18 @@ def test_the_rule():
     dims = lambda M, N, K, ta, tb, a=0, b=0: packed_leading_dims(_Layouts(M, N, K, ta, tb, K if ta else M, N if tb else K), a, b)
     assert dims(4001, 4003, 4005, True, False) == (4032, 4032)
     assert dims(4001, 4003, 4005, False, True) == (4032, 4032)
-    assert dims(4001, 4003, 8100, False, False) == (4032, 8128)
+    assert dims(6001, 5003, 7100, False, False) == (6016, 7104)
+    assert dims(4001, 4003, 8100, False, False) is None                           # (copies and operands outgrow the memory-side cache)
     assert dims(4000, 4000, 4000, True, False) is None and dims(4096, 4096, 4096, False, False) is None
     assert dims(4096, 4096, 4096, False, False, 2, 6) == (4096, 4096)             # misaligned addresses
-    assert dims(4000, 4000, 4001, False, False) == (None, 4032)                   # one operand, contiguous along k
+    assert dims(5000, 5000, 5001, False, False) == (None, 5056)                   # one operand, contiguous along k
+    assert dims(4000, 4000, 4001, False, False) is None                           # (less work: level or slower but for rotating inputs)
+    assert dims(2000, 8000, 8001, False, False) is None                           # (a copy of most of what is read)
+    # both operands: by the share of the product's time that copying them takes, more where they are contiguous along k
+    assert all(dims(1501, 8003, 8005, ta, tb) is None for ta, tb in itertools.product((False, True), repeat=2))
+    assert [dims(1001, 8003, 4005, ta, tb) is not None for ta, tb in ((False, False), (False, True), (True, False), (True, True))] == [False, False, True, False]
+    assert [dims(2001, 2003, 6005, ta, tb) is not None for ta, tb in ((False, False), (False, True), (True, False), (True, True))] == [True, False, True, True]
+    assert all(dims(3001, 3003, 3005, ta, tb) is not None for ta, tb in itertools.product((False, True), repeat=2))
     assert dims(4001, 4000, 4000, False, False) is None                           # one operand, contiguous along m
     assert dims(2001, 2003, 4005, True, False) is None                            # too little work
     assert dims(131, 8191, 31111, True, False) is None                            # too few rows
@@ -59,6 +69,27 @@ def test_pack_columns(rows, cols, ld, offset):
     assert torch.equal(copies[0][:, :rows].t(), x) and bool((copies[0][:, rows:] == -2.0).all())
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols,ld,offset", [(1, 1, 1, 0), (7, 17, 9, 1), (8, 16, 8, 0), (9, 4, 9, 2), (511, 33, 513, 3), (512, 5, 515, 1), (519, 20, 519, 0), (1029, 3, 2001, 7)])
+@pytest.mark.parametrize("more_rows,more_cols", [(0, 0), (1, 0), (9, 3), (63, 16), (520, 1)])
+def test_pack_columns_padded(rows, cols, ld, offset, more_rows, more_cols):
+    """Zeros behind the rows and the columns of the matrix, what lies behind the rows of the copy left alone; NaN in the source behind its columns."""
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    x = _odd(rows, cols, ld, torch.float16, gen, offset)
+    if cols > 1:
+        torch.as_strided(x, (ld - rows, cols - 1), (1, ld), offset + rows).fill_(float("nan"))
+    rows_copy, cols_copy = rows + more_rows, cols + more_cols
+    ld_copy = -(-rows_copy // 8) * 8 + 8
+    copies = [torch.full((cols_copy + 1, ld_copy), -2.0, dtype=torch.float16, device="cuda") for _ in range(2)]
+    job = lambda copy: (x.data_ptr(), rows, cols, ld, copy.data_ptr(), ld_copy, rows_copy, cols_copy)
+    stream = torch.cuda.current_stream().cuda_stream
+    assert _lib.lib().gk_pack_columns_padded(*job(copies[0]), *job(copies[1]), stream) == _lib.GK_OK, _lib.last_error()
+    want = torch.full((cols_copy + 1, ld_copy), -2.0, dtype=torch.float16, device="cuda")
+    want[:cols_copy, :rows_copy] = 0
+    want[:cols, :rows] = x.t()
+    assert torch.equal(copies[0].view(torch.int16), want.view(torch.int16)) and torch.equal(copies[1].view(torch.int16), want.view(torch.int16))
+
+
 def test_pack_columns_refuses():
     """No GPU: nothing is launched."""
     pack = _lib.lib().gk_pack_columns
@@ -70,6 +101,11 @@ def test_pack_columns_refuses():
     assert pack(256, 8, 8, 8, 264, 8, *none) == _lib.GK_ERR_ALIGNMENT
     assert pack(256, 8, 8, 8, 256, 8, 256, 8, -1, 8, 256, 8, None) == _lib.GK_ERR_INVALID_ARGUMENT
     assert pack(256, 1 << 20, 8, 1 << 20, 256, 1 << 20, *none) == _lib.GK_ERR_INVALID_ARGUMENT
+    padded = _lib.lib().gk_pack_columns_padded
+    none = (None, 0, 0, 0, None, 0, 0, 0, None)
+    assert padded(256, 8, 8, 8, 256, 16, 7, 8, *none) == _lib.GK_ERR_INVALID_ARGUMENT
+    assert padded(256, 8, 8, 8, 256, 16, 8, 7, *none) == _lib.GK_ERR_INVALID_ARGUMENT
+    assert padded(256, 8, 8, 8, 256, 16, 17, 8, *none) == _lib.GK_ERR_INVALID_ARGUMENT
 
 
 @pytest.mark.gpu
