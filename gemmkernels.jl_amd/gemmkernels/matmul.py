@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import math
 from typing import Optional
 
 import numpy as np
@@ -571,7 +572,8 @@ def matmatmul_(C, transA: str, transB: str, A, B, alpha, beta, *, wmma=None):
             hit(a, b, c, _current_stream())
             return C
     p = _single_plan(C, tA, tB, A, B, alpha, beta, wmma)
-    packed = None if p._split_k else packed_leading_dims(p._conf, a, b)
+    # (an alpha that is infinite in A's type would make NaN of the zeros that fill a copy up)
+    packed = packed_leading_dims(p._conf, a, b) if not p._split_k and math.isfinite(_round_to(from_torch(A.dtype), float(alpha))) else None
     launch = _MulLaunch(p) if packed is None else _MulLaunchOnCopies(p, packed)
     if key is not None:
         if len(_mul_launches) >= _MUL_LAUNCHES_MAX:

@@ -158,3 +158,24 @@ def test_streams_and_no_memory(monkeypatch):
     gk.mul_(out, a, b)
     monkeypatch.undo()
     assert torch.equal(out, ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ab", [torch.float16, torch.bfloat16])
+def test_an_infinite_factor_and_infinite_values(ab):
+    """K = 6048 is whole tiles of 32, on which the product runs, and 94.5 of 64: zeros behind it must not meet an infinite alpha (values of one
+    sign: every output is infinite), nor change what infinities and NaN in A and B give."""
+    M, N, K = 2001, 2003, 6048
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    a, b = _odd(K, M, K + 3, ab, gen).abs_(), _odd(K, N, K + 1, ab, gen).abs_()
+    for spoil in (False, True):
+        if spoil:
+            a[K - 1, 5], a[0, M - 1], b[K - 1, 7] = float("inf"), float("nan"), float("-inf")
+        for alpha in (float("inf"), 1e6, 1.5, 1.0):                 # (1e6 is infinite in FP16)
+            ref, out = (gk.colmajor_empty((M, N), torch.float32) for _ in range(2))
+            p = matmatmul_plan(ref, 'T', 'N', a, b, alpha, 0.0)
+            assert packed_leading_dims(p._conf, a.data_ptr(), b.data_ptr()) is not None and p._conf.block_shape.K == 32
+            p()
+            gk.mul_(out, gk.Transpose(a), b, alpha, 0.0)
+            assert torch.equal(out.isnan(), ref.isnan()) and torch.equal(out.nan_to_num(), ref.nan_to_num())
+            assert spoil or bool((out == float("inf")).all() if alpha == float("inf") or alpha == 1e6 and ab is torch.float16 else out.isfinite().all())
