@@ -672,9 +672,15 @@ class _MulLaunch:
 class _MulLaunchOnCopies(_MulLaunch):
     """The same on copies of the operands whose columns start off a 16-byte boundary (``packed_leading_dims``).  Copies of both operands
     are filled up with zeros to whole K tiles of 64: the partial one, which the kernels run outside their pipeline, takes some 10 us per
-    round of tiles (the product on copies 4001 x 4003 x 4005 110 -> 100 us, from memory 136 -> 127), and sums of zeros change no bit."""
+    round of tiles (the product on copies 4001 x 4003 x 4005 110 -> 100 us, from memory 136 -> 127), and sums of zeros change no bit.
 
-    __slots__ = ("_packed", "_packed_ref", "_copies", "_copy_bytes")
+    A call that finds no memory for the copies costs milliseconds (the allocator gives its cache back and waits for the device before it
+    says so), so the calls behind it run on the operands as they lie and only every 256th tries again.  (The count is the one thing written
+    after the launch is made: threads that meet on it try once more or less.)"""
+
+    __slots__ = ("_packed", "_packed_ref", "_copies", "_copy_bytes", "_calls_without")
+
+    _RETRY_AFTER = 256
 
     def __init__(self, p: Plan, packed):
         super().__init__(p)
@@ -691,7 +697,7 @@ class _MulLaunchOnCopies(_MulLaunch):
             self._copies.append((which, at, (rows, cols, mine.ld), (ld, rows_copy, cols_copy)))
             layout.ld = ld
             at += 2 * ld * cols_copy
-        self._copy_bytes = at
+        self._copy_bytes, self._calls_without = at, 0
 
     def _on_copies(self, a: int, b: int, c: int, stream: int) -> bool:
         """The product on copies of the operands whose columns start off a 16-byte boundary (the same launch, the same bits).
@@ -700,10 +706,14 @@ class _MulLaunchOnCopies(_MulLaunch):
         # (`stream` is torch's current one: what torch says of captures and allocates is that stream's)
         if torch.cuda.is_current_stream_capturing():
             return False
+        if self._calls_without > 0:
+            self._calls_without -= 1
+            return False
         # memory of this call alone, in the order of the stream: what gets it next on this stream runs behind the product
         try:
             copies = torch.empty(self._copy_bytes, dtype=torch.uint8, device="cuda")
         except torch.OutOfMemoryError:
+            self._calls_without = self._RETRY_AFTER - 1
             return False
         base, operands, jobs = copies.data_ptr(), [a, b], []
         for which, at, source, copy in self._copies:

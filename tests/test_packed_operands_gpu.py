@@ -47,6 +47,26 @@ def test_the_rule():
     assert dims(16001, 16001, 16001, True, False) is None                         # copies of more than 512 MiB
 
 
+def test_a_launch_without_memory_for_copies_seldom_asks_again(monkeypatch):
+    """No GPU: the launches are recorded, the allocation fails."""
+    import sys
+    matmul = sys.modules["gemmkernels.matmul"]
+    host = lambda rows, cols, dtype: torch.empty((cols, rows), dtype=dtype).t()
+    p = matmatmul_plan(host(3001, 2999, torch.float32), 'N', 'N', host(3001, 3003, torch.float16), host(3003, 2999, torch.float16), 1.0, 0.0)
+    launch = matmul._MulLaunchOnCopies(p, packed_leading_dims(p._conf, 0, 0))
+    plain, asked = [], []
+    launch._fn = lambda conf, a, b, c, d, *rest: plain.append((a, b, c)) or _lib.GK_OK
+
+    def none(*args, **kwargs):
+        asked.append(len(plain))
+        raise torch.OutOfMemoryError("no memory")
+    monkeypatch.setattr(torch, "empty", none)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    for _ in range(600):
+        launch(2, 4, 6, 0)
+    assert plain == [(2, 4, 6)] * 600 and asked == [0, 256, 512]
+
+
 def _odd(rows, cols, ld, dtype, gen, offset=0):
     buffer = (torch.rand(ld * (cols - 1) + rows + offset, generator=gen, device="cuda") * 2 - 1).to(dtype)      # ends with the last column
     return torch.as_strided(buffer, (rows, cols), (1, ld), offset)
