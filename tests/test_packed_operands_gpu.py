@@ -128,12 +128,29 @@ def test_pack_columns_refuses():
     assert padded(256, 8, 8, 8, 256, 16, 17, 8, *none) == _lib.GK_ERR_INVALID_ARGUMENT
 
 
+class _Poisoned:
+    """Buffers of bytes that ``torch.empty`` makes are full of NaN (0xFF), whatever the allocator had left there; counts them."""
+
+    def __init__(self, monkeypatch):
+        self.made, empty = 0, torch.empty
+
+        def poisoned(*args, **kwargs):
+            out = empty(*args, **kwargs)
+            if kwargs.get("dtype") is torch.uint8:
+                self.made += 1
+                out.fill_(255)
+            return out
+        monkeypatch.setattr(torch, "empty", poisoned)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("ab,cd", [(torch.bfloat16, torch.float32), (torch.float16, torch.float32), (torch.float16, torch.float16)])
 @pytest.mark.parametrize("ta,tb", list(itertools.product((False, True), repeat=2)))
-def test_product_on_copies(ta, tb, ab, cd):
-    """Against the plan of the same product, which launches on the operands as they lie; a call under capture does so too."""
+def test_product_on_copies(ta, tb, ab, cd, monkeypatch):
+    """Against the plan of the same product, which launches on the operands as they lie; a call under capture does so too.  What
+    the copies do not fill is NaN."""
     M, N, K = 3001, 2999, 3003
+    poisoned = _Poisoned(monkeypatch)
     gen = torch.Generator(device="cuda").manual_seed(5)
     a = _odd(K, M, K, ab, gen, 1) if ta else _odd(M, K, M + 2, ab, gen)
     b = _odd(N, K, N, ab, gen) if tb else _odd(K, N, K, ab, gen, 3)
@@ -142,16 +159,37 @@ def test_product_on_copies(ta, tb, ab, cd):
         ref, out, captured = (c.clone(memory_format=torch.preserve_format) for _ in range(3))
         matmatmul_plan(ref, 'T' if ta else 'N', 'T' if tb else 'N', a, b, alpha, beta)()
         call = lambda d: gk.mul_(d, gk.Transpose(a) if ta else a, gk.Transpose(b) if tb else b, alpha, beta)
+        before = poisoned.made
         call(out)
+        assert poisoned.made == before + 1
         assert torch.equal(out, ref)
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph):
             call(captured)
+        assert poisoned.made == before + 1
         for _ in range(2):
             captured.copy_(c)
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(captured, ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, True)])
+def test_one_operand_on_a_copy(ta, tb, monkeypatch):
+    """The operand that is contiguous along an odd K is copied, the other stays: the partial K tile runs as it does on the operands
+    as they lie, next to NaN behind the rows of the copy."""
+    M, N, K = 4800, 4992, 3501
+    poisoned = _Poisoned(monkeypatch)
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    a = _odd(K, M, K, torch.float16, gen) if ta else _odd(M, K, M, torch.float16, gen)
+    b = _odd(N, K, N, torch.float16, gen) if tb else _odd(K, N, K, torch.float16, gen)
+    ref, out = (gk.colmajor_empty((M, N), torch.float32) for _ in range(2))
+    p = matmatmul_plan(ref, 'T' if ta else 'N', 'T' if tb else 'N', a, b, 1.0, 0.0)
+    assert packed_leading_dims(p._conf, a.data_ptr(), b.data_ptr()) == ((3520, None) if ta else (None, 3520))
+    p()
+    gk.mul_(out, gk.Transpose(a) if ta else a, gk.Transpose(b) if tb else b)
+    assert poisoned.made == 1 and torch.equal(out, ref)
 
 
 @pytest.mark.gpu
@@ -161,7 +199,9 @@ def test_streams_and_no_memory(monkeypatch):
     gen = torch.Generator(device="cuda").manual_seed(6)
     a, b = _odd(M, K, M, torch.bfloat16, gen), _odd(K, N, K, torch.bfloat16, gen)
     ref, out, other = (gk.colmajor_empty((M, N), torch.float32) for _ in range(3))
-    matmatmul_plan(ref, 'N', 'N', a, b, 1.0, 0.0)()
+    p = matmatmul_plan(ref, 'N', 'N', a, b, 1.0, 0.0)
+    assert packed_leading_dims(p._conf, a.data_ptr(), b.data_ptr()) is not None
+    p()
     torch.cuda.synchronize()
     stream = torch.cuda.Stream()
     for _ in range(3):
@@ -172,12 +212,15 @@ def test_streams_and_no_memory(monkeypatch):
     assert torch.equal(out, ref) and torch.equal(other, ref)
     out.zero_()
 
+    asked = []
+
     def none(*args, **kwargs):
+        asked.append(args)
         raise torch.OutOfMemoryError("no memory")
     monkeypatch.setattr(torch, "empty", none)
     gk.mul_(out, a, b)
     monkeypatch.undo()
-    assert torch.equal(out, ref)
+    assert len(asked) == 1 and torch.equal(out, ref)
 
 
 @pytest.mark.gpu
