@@ -1140,7 +1140,9 @@ static_assert(kSplitCounterBytes / sizeof(unsigned) >= 2 * (size_t)gk::kNumCUs -
 //   1776 x 33 x 7392 (28) 7 14.4, 8 14.4, 11 16.0; 300 x 200 x 9001 (20) 9 15.4, 14 18.9; 1085 x 47 x 6136 (17) 6 15.0, 9 13.9;
 //   64 x 64 x 8000 (1) 7 10.6, 12 10.0; 64 x 64 x 32768 (1) 24 15.3, 32 15.8, 51 18.0.
 // A factor on A or B (AB_HOOKS) makes the K loop longer and what a slice costs weigh less: up to two per CU.  FP16 4096 x 64 x 4096
-//   'T','N' 4 13.8, 6 12.9; BF16 with op lists on A (level 2) 4 66.5, 6 61.6, 8 57.0, 7 x 7 x 20000 (1) 19 54.2, 31 46.6.
+//   'T','N' 4 13.8, 6 12.9; BF16 with op lists on A (level 2) 4 66.5, 6 61.6, 8 57.0, 7 x 7 x 20000 (1) 19 54.2, 31 46.6.  BF16 with one factor (level 1),
+//   whose loop is little longer, lies within 5 % of its best on the same slices: 4096 x 64 x 4096 'N','N' 4 15.9, 6 16.1, 8 16.3; 7 x 7 x 20000 19 17.1, 31 16.2;
+//   512 x 512 x 4096 (64) 4 15.2, 6 14.1, 8 13.7; 2048 x 128 x 8192 (64) 6 20.5, 8 18.2, 10 23.6; 960 x 384 x 4096 (90) 3 18.0, 5 15.6, 6 19.2; 8192 x 64 x 4096 (128) 2 23.3, 4 24.2.
 // 128 x 128 x 64, whose partial tiles are four times as large: 768 deep (1024 above 64 tiles), sixteen slices or 2048 deep:
 //   512 x 512 x 4096 (16) 4 22.7, 5 22.0, 6 21.8; 2048 x 512 x 4096 (64) 4 25.3, 5 25.3, 6 26.2; 1536 x 1024 x 4096 (96) 4 29.5, 5 30.6;
 //   256 x 256 x 16384 (4) 12 34.4, 16 35.5, 25 40.2.

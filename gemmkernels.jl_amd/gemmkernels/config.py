@@ -233,8 +233,9 @@ def split_k_block_shape(M, N, K, widest_ld=0, factor=None) -> Optional[NT]:
     / 15.4 and 14.4; 1001 x 704 x 3328 20.9 and 18.1 / 15.7 and 16.0; 1024 x 768 x 4004 21.5 and 22.4 / 25.3 and 24.3.  Not where K and the output are both
     ragged (1001 x 700 x 3333, 1000 x 1000 x 4000).
 
-    ``factor``: how alpha is applied to A in the K loop, which makes it longer ("packed", FP16; "per element", BF16): FP16 111 x 2629 x 1477 (84 tiles) 15.7
-    and 19.9.  ``widest_ld``: the larger leading dimension of the operands whose rows are the k of a tile; the kernel keeps the offsets in a tile
+    ``factor``: alpha stays in the K loop (None: it does not), which makes it longer, and two slices pay whatever the extents: FP16 111 x 2629 x 1477 (84 tiles) 15.7
+    and 19.9; two slices, BF16, 1024 x 1024 x 4096 24.4 and 32.9, 768 x 1024 x 4096 23.8 and 32.5, 1001 x 1001 x 5001 37.6 and 43.5, 960 x 896 x 8192 41.2 and 61.5, 1000 x 900 x 3001
+    25.0 and 29.0, 70 x 7000 x 3500 31.0 and 32.3, 12000 x 64 x 4096 33.1 and 34.3 ('T','N' 33.6 and 33.4).  ``widest_ld``: the larger leading dimension of the operands whose rows are the k of a tile; the kernel keeps the offsets in a tile
     in 32 bits, so 64 rows of 2^24 elements are left to a tile with fewer."""
     if 64 * widest_ld * 2 >= 1 << 31:
         return None
@@ -242,8 +243,7 @@ def split_k_block_shape(M, N, K, widest_ld=0, factor=None) -> Optional[NT]:
     if tiles <= 128:
         worth = K >= 1280
     else:
-        whole = K % 64 == 0 or M % 64 == 0 and N % 64 == 0
-        two = {None: whole, "packed": True, "per element": tiles <= 225 and min(M, N) > 128}[factor]
+        two = factor is not None or K % 64 == 0 or M % 64 == 0 and N % 64 == 0
         worth = K >= 3000 and (tiles <= 170 or tiles <= 256 and two)
     return NT(M=64, N=64, K=64) if worth else None
 

@@ -431,7 +431,7 @@ def create_config(A: DType, sizeA, stridesA, transA: bool, B: DType, sizeB, stri
     says whether A, B and C start on 16-byte boundaries: the reference decides on the aligned layouts from the
     strides alone (a misaligned view then traps on the device, src/layout.jl:22-25); here such an operand gets
     the bounds-checked layout, which takes any address.  ``factor``: how alpha is applied to A
-    in the K loop, see ``split_k_block_shape``."""
+    in the K loop (None: not there), see ``split_k_block_shape``."""
     m = sizeA[1 if transA else 0]
     k = sizeA[0 if transA else 1]
     n = sizeB[0 if transB else 1]
@@ -520,7 +520,7 @@ _FOLDED = frozenset(2.0 ** e for e in range(-4, 5))
 def _single_plan(C, tA: bool, tB: bool, A, B, alpha, beta, wmma=None) -> Plan:
     """One launch for C = alpha * op(A) * op(B) + beta * C: the configuration ``create_config`` picks."""
     # (a power of two within 2^-4 .. 2^4 leaves the K loop, see the folded scales of the library)
-    factor = None if abs(float(alpha)) in _FOLDED else ("per element" if BFloat16 in (from_torch(A.dtype), from_torch(B.dtype)) else "packed")
+    factor = None if abs(float(alpha)) in _FOLDED else "per fragment"
     conf, compute_type, kernel = get_config(
         from_torch(A.dtype), tuple(A.shape), tuple(A.stride()), tA,
         from_torch(B.dtype), tuple(B.shape), tuple(B.stride()), tB,

@@ -711,7 +711,7 @@ function create_config(A::Type, sizeA::Dims, stridesA::Dims, transA::Bool,
                        B::Type, sizeB::Dims, stridesB::Dims, transB::Bool,
                        C::Type, sizeC::Dims, stridesC::Dims,
                        alpha::Type, zeroAlpha::Bool, beta::Type, zeroBeta::Bool,
-                       wmma::Union{Bool,Nothing} = nothing, aligned_pointers::NTuple{3,Bool} = (true, true, true), factor::Symbol = :none)
+                       wmma::Union{Bool,Nothing} = nothing, aligned_pointers::NTuple{3,Bool} = (true, true, true), factor::Bool = false)
     m = sizeA[transA ? 2 : 1]
     k = sizeA[transA ? 1 : 2]
     n = sizeB[transB ? 1 : 2]
@@ -783,12 +783,11 @@ function worth_splitting(m, n, k, widest_ld, factor)
     64 * widest_ld * 2 < 2^31 || return false
     tiles = cld(m, 64) * cld(n, 64)
     tiles <= 128 && return k >= 1280
-    whole = k % 64 == 0 || (m % 64 == 0 && n % 64 == 0)
-    two = factor === :none ? whole : factor === :packed || (tiles <= 225 && min(m, n) > 128)
+    two = factor || k % 64 == 0 || (m % 64 == 0 && n % 64 == 0)
     k >= 3000 && (tiles <= 170 || (tiles <= 256 && two))
 end
 # alpha stays in the K loop unless it is a power of two that the library folds into the accumulators
-factor_of(alpha, A, B) = abs(Float64(alpha)) in (2.0 .^ (-4:4)) ? :none : (:BFloat16 in (nameof(eltype(A)), nameof(eltype(B))) ? :per_element : :packed)
+stays_in_the_loop(alpha) = !(abs(Float64(alpha)) in (2.0 .^ (-4:4)))
 
 is_aligned_16(x) = UInt(devptr(x)) % 16 == 0
 
@@ -803,7 +802,7 @@ function matmatmul!(C, transA::Char, transB::Char, A, B, alpha::Number, beta::Nu
     conf, compute_type, kernel = get_cached_config(
         eltype(A), size(A), strides(A), tA, eltype(B), size(B), strides(B), tB,
         eltype(C), size(C), strides(C), typeof(alpha), iszero(alpha), typeof(beta), iszero(beta), wmma,
-        (is_aligned_16(A), is_aligned_16(B), is_aligned_16(C)), factor_of(alpha, A, B))
+        (is_aligned_16(A), is_aligned_16(B), is_aligned_16(C)), stays_in_the_loop(alpha))
     alpha_c = convert(compute_type === BFloat16 ? Float32 : compute_type, alpha)       # :196
     beta_c = convert(eltype(C) === BFloat16 ? Float32 : eltype(C), beta)               # :197
     for (name, v) in (("alpha", alpha_c), ("beta", beta_c))
@@ -814,7 +813,7 @@ function matmatmul!(C, transA::Char, transB::Char, A, B, alpha::Number, beta::Nu
     if Operator.is_mfma(conf.operator)
         # few output tiles and a long K loop: K slices as workgroups of one launch (ordered sum: same bits every run)
         bs, ms = conf.block_shape, conf.matmul_shape
-        if bs == (M = 64, N = 64, K = 64) && worth_splitting(ms.M, ms.N, ms.K, 0, factor_of(alpha, A, B)) || cld(ms.M, bs.M) * cld(ms.N, bs.N) <= 128 && ms.K >= 2048
+        if bs == (M = 64, N = 64, K = 64) && worth_splitting(ms.M, ms.N, ms.K, 0, stays_in_the_loop(alpha)) || cld(ms.M, bs.M) * cld(ms.N, bs.N) <= 128 && ms.K >= 2048
             kernel = Kernel.matmul_split_k
         end
     end

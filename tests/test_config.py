@@ -416,8 +416,9 @@ def test_k_slices_fill_the_cus_once(dims, tile, scale, slices):
 
 
 def test_two_slices_of_more_than_170_tiles_only_where_they_pay():
-    """11 x 16 tiles of 64 x 64: cut in two where K, or else the output, is whole tiles, or where an FP16 alpha stays in the K loop;
+    """11 x 16 tiles of 64 x 64: cut in two where K, or else the output, is whole tiles, or where alpha stays in the K loop;
     three slices of 165 tiles, and few tiles, are worth it in any case."""
+    from gemmkernels.config import split_k_block_shape
     def block(M, N, K, factor=None):
         conf, _, _ = create_config(Float16, (M, K), (1, M), False, Float16, (K, N), (1, K), False,
                                    Float32, (M, N), (1, M), float, False, float, True, factor=factor)
@@ -425,15 +426,15 @@ def test_two_slices_of_more_than_170_tiles_only_where_they_pay():
     split, narrow = NT(M=64, N=64, K=64), NT(M=64, N=64, K=32)
     assert block(1001, 700, 3328) == split and block(1024, 704, 3336) == split
     assert block(1001, 700, 3333) == narrow and block(1024, 704, 3333) == split and block(1000, 704, 3336) == narrow
-    assert block(1001, 700, 3333, "packed") == split and block(1001, 700, 3333, "per element") == split
-    assert block(768, 1024, 4096, "per element") == split and block(1024, 1024, 4096, "per element") == narrow
-    assert block(12032, 64, 4096, "per element") != split and block(12032, 64, 4096) == split
+    assert block(1001, 700, 3333, "per fragment") == split and block(1001, 1001, 5001, "per fragment") == split
+    assert block(12032, 64, 4097, "per fragment") == split and split_k_block_shape(12032, 65, 4097, 0, "per fragment") is None      # (188 and 376 tiles)
+    assert block(12032, 64, 4096) == split
     assert block(700, 900, 3001) == split and block(300, 200, 1301) == split
 
 
 @pytest.mark.parametrize("dims,dtype,alpha,slices", [((700, 900, 3001), "float16", 1.0, 3), ((1001, 704, 3328), "float16", 1.0, 2), ((1024, 704, 3333), "bfloat16", 1.0, 2), ((1024, 1024, 4096), "float16", 1.0, 2),
                                                      ((1024, 1024, 16384), "bfloat16", 2.0, 2), ((201, 4096, 8064), "float16", 1.0, 2), ((3722, 192, 7232), "bfloat16", 1.0, 2), ((1001, 700, 3333), "float16", 1.0, 1),
-                                                     ((1001, 700, 3333), "float16", 1.5, 2), ((1024, 1088, 4096), "float16", 1.0, 1), ((1024, 1024, 2944), "float16", 1.0, 1), ((4096, 64, 4096), "float16", 1.0, 4)])
+                                                     ((1001, 700, 3333), "float16", 1.5, 2), ((1024, 1024, 4096), "bfloat16", 1.5, 2), ((12000, 64, 4096), "bfloat16", 1.5, 2), ((1024, 1088, 4096), "float16", 1.0, 1), ((1024, 1024, 2944), "float16", 1.0, 1), ((4096, 64, 4096), "float16", 1.0, 4)])
 def test_the_slices_a_product_is_launched_in(dims, dtype, alpha, slices):
     """What mul! launches on both sides of 170 and of 256 tiles, read from the plan and the workspace it asks for (no GPU: the operands
     are on the host, nothing is launched).  Two slices halve the chain of a sum: products of 171 to 256 tiles have 0.7 of the error."""

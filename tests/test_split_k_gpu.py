@@ -293,7 +293,7 @@ def test_a_partial_last_k_tile_is_the_end_of_the_last_slice(gpu, dims, tile, ta,
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("ab,cd", [(torch.float16, torch.float32), (torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
 def test_slices_with_factors_and_16_bit_outputs(gpu, ab, cd, ta, tb):
-    """mul! on slices with factors on A and C (an exact FP16 scale, and the per-element path of BF16), a power of two, and FP16 C and
+    """mul! on slices with factors on A and C (one FP16 or BF16 scale per fragment), a power of two, and FP16 C and
     D, with whole and partial last K tiles.  A and B in {-1, 0, 1} and C in multiples of 1/2 below 8: every result is a
     multiple of 1/4 below 512 (asserted), exact in FP16 as well as in every partial sum."""
     rs = np.random.RandomState(21)
