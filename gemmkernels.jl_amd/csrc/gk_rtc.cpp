@@ -128,8 +128,9 @@ int gk_rtc_compile(const gk_config* conf, const char* const hooks[8], int32_t ke
       if (h == GK_HOOK_GLOBAL_TO_SHARED_A || h == GK_HOOK_GLOBAL_TO_SHARED_B || h == GK_HOOK_SHARED_TO_REGS_A || h == GK_HOOK_SHARED_TO_REGS_B) any_ab = true;
       if (strlen(hooks[h]) > 1024) return fail(GK_ERR_INVALID_ARGUMENT, "hook expression longer than 1024 characters");
     }
-  // level 3: C / D hooks and the bias epilogue, chosen at launch time, on the K loop without hooks (level 1 multiplies every fragment of A,
-  // by 1 here: five instructions per two values in BF16)
+  // level 3: C / D hooks and the bias epilogue, chosen at launch time, on the K loop without hooks.  Level 1 multiplies every fragment of A,
+  // by 1 here (BF16: five instructions per two values): with a hook on D 4096^3 on 256 x 128 x 64 BF16 189.5 -> 142.1 us, FP16 167.7 -> 147.8;
+  // 2048^3 on 128 x 128 x 64 37.9 -> 27.5 and 34.4 -> 28.4
   const int fuse = any_ab ? 2 : 3;
   // operand kinds of the kernel template: 0 K-major, 1 M-major
   const std::string src = build_source(c, hooks, stages, fuse, a_kmajor ? 0 : 1, b_kmajor ? 0 : 1, dt == GK_F16 ? "_Float16" : "__bf16");
