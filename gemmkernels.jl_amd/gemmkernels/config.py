@@ -3,6 +3,7 @@
 from __future__ import annotations
 
 import ctypes
+import math
 from dataclasses import dataclass, fields
 from typing import Optional
 
@@ -180,6 +181,10 @@ def _tiles_k_modes(extents, block_k) -> bool:
     return False
 
 
+def _mfma_tiles(a_kmajor: bool, b_kmajor: bool):
+    return [t for t, _ in _MFMA_TILES] + [t for t, _, has in _MFMA_TILES_192 if has(a_kmajor, b_kmajor)]
+
+
 def default_block_shape(operator, gemm_shape, tile_sized: bool = True, gett: bool = False, planar: bool = False,
                         a_kmajor: bool = False, b_kmajor: bool = True, k_modes=None) -> NT:
     """MI355X block shape: of the tiles of the table that divide the problem, the one with the shortest
@@ -210,7 +215,7 @@ def default_block_shape(operator, gemm_shape, tile_sized: bool = True, gett: boo
         return NT(M=best[0], N=best[1], K=best[2])
     # sizes need not be whole tiles when the layouts are the bounds-checked ones (the aligned kernels mask the
     # last tile row / column and zero the end of the last K tile)
-    table = [t for t, _ in _MFMA_TILES] + [t for t, _, has in _MFMA_TILES_192 if has(a_kmajor, b_kmajor)]
+    table = _mfma_tiles(a_kmajor, b_kmajor)
     fitting = [t for t in table if not tile_sized or (M % t[0] == 0 and N % t[1] == 0 and K % t[2] == 0)]
     if gett:
         fitting = [t for t in fitting if t in _GETT_TILES and (k_modes is None or _tiles_k_modes(k_modes, t[2]))]
@@ -467,7 +472,55 @@ def get_config(*, gemm_shape, operator, global_a_layout, global_c_layout, **para
         # will be compiled at run time (gemmkernels.specialize); that compilation and every launch run
         # the same checks, minus the table lookup
         check_config(conf, params.get("kernel"))
+        conf.__dict__["_tile_left_open"] = not any(k in params for k in _TILE_CHOICES)
     return conf
+
+
+_TILE_CHOICES = ("block_shape", "warps_per_block", "compute_warp", "mem_a_warp", "mem_b_warp", "mem_cd_warp", "mem_a_thread", "mem_b_thread",
+                 "mem_cd_thread", "cta_swizzle")
+_ANY_SIZE = {Layout.ALIGNED_COL_MAJOR: Layout.ColMajor, Layout.ALIGNED_ROW_MAJOR: Layout.RowMajor}
+
+
+def larger_tile(conf: Config, hooks: bool) -> Optional[Config]:
+    """The configuration that a launch of ``conf`` runs on where the tile was left to the default and one that does not divide the sizes is faster, or None.
+
+    Aligned layouts ask for sizes in whole tiles (reference src/config.jl:268-275), so most multiples of 64 leave only the 64 x 64 tiles, which bring every
+    operand into the CUs four times as often as 256 x 256 ones do.  The kernels take tiles over the edges on any layout (one
+    launch, the same bits: every output is summed in the same order), so the launch is that of the bounds-checked layouts on the tile with the shortest
+    estimate, once the operands have passed for what the aligned ones ask (``matmul``).  us on the tile that divides and on the larger one, and the ratio of the
+    estimates, inputs that rotate: 2240 x 5568 x 2304 'N','N' with C 100.0 and 69.9 (0.52), 4544 x 2048 x 2368 'T','N' 70.8 and 47.9 (0.68), 1344 x 2880 x 5696 'T','T' 64.7 and 58.3 (0.71),
+    1600 x 4480 x 2048 'N','T' with C 54.9 and 47.5 (0.75), 5632 x 2240 x 384 24.2 and 20.7 (0.84), 5120 x 4224 x 5888 with C 285.8 and 269.4 (0.84); beyond the line 1920 x 1856 x 2368 27.9 and 29.2 (0.90),
+    2368 x 3072 x 896 with C 28.4 and 30.0 (0.90).  ``hooks``: transforms or a bias, which tiles of 256 x 256 over the edges run on eight waves (5376 x 2176 x 768 with C 47.5 and 53.0,
+    3520 x 2432 x 2048 72.4 and 76.1, so not those) and which the estimates leave out: 5696 x 5760 x 4160 with C 440 and 320 on 128 x 128 (0.57), 4992 x 1344 x 4416 99.6 and 73.7 (0.70), 4608 x 832 x 6080 75.5
+    and 61.6 (0.71); beyond the line 5056 x 768 x 2176 29.1 and 31.0 (0.85)."""
+    if not conf.__dict__.get("_tile_left_open"):
+        return None
+    key = "_larger_tile_with_hooks" if hooks else "_larger_tile"
+    if key not in conf.__dict__:
+        conf.__dict__[key] = _find_larger_tile(conf, hooks)
+    return conf.__dict__[key]
+
+
+def _find_larger_tile(conf: Config, hooks: bool) -> Optional[Config]:
+    layouts = (conf.global_a_layout, conf.global_b_layout, conf.global_c_layout, conf.global_d_layout)
+    if conf.operator.kind != Operator.MFMA or any(l.kind not in _ANY_SIZE and not (i == 2 and l.kind == Layout.ZERO) for i, l in enumerate(layouts)):
+        return None
+    M, N, K = (conf.matmul_shape[x] for x in "MNK")
+    own = tuple(conf.block_shape[x] for x in "MNK")
+    if own not in _MFMA_TILE_COST:
+        return None
+    a_kmajor, b_kmajor = layouts[0].kind == Layout.ALIGNED_ROW_MAJOR, layouts[1].kind == Layout.ALIGNED_COL_MAJOR
+    best = min(_mfma_tiles(a_kmajor, b_kmajor), key=lambda t: math.inf if hooks and t[:2] == (256, 256) else _mfma_cost(t, M, N, K))
+    if best == own or _mfma_cost(best, M, N, K) > (0.8 if hooks else 0.86) * _mfma_cost(own, M, N, K):
+        return None
+    a, b, c, d = (_ANY_SIZE[l.kind][l.T] if l.kind in _ANY_SIZE else l for l in layouts)
+    try:
+        return get_config(gemm_shape=conf.matmul_shape, operator=conf.operator, block_shape=NT(M=best[0], N=best[1], K=best[2]),
+                          global_a_layout=a, global_b_layout=b, global_c_layout=c, global_d_layout=d,
+                          shared_a_layout=conf.shared_a_layout, shared_b_layout=conf.shared_b_layout, shared_c_layout=conf.shared_c_layout,
+                          shared_d_layout=conf.shared_d_layout, is_a_col_major=conf.is_a_col_major, is_b_col_major=conf.is_b_col_major)
+    except ConfigError:
+        return None
 
 
 def check_config(conf: Config, kernel=None) -> None:

@@ -21,7 +21,7 @@ from . import kernel as Kernel
 from . import layout as Layout
 from . import operator as Operator
 from . import transform as Transform
-from .config import _MFMA_TILE_COST, Config, _mfma_cost, default_block_shape, get_config as _get_config, split_k_block_shape
+from .config import _MFMA_TILE_COST, Config, _mfma_cost, default_block_shape, get_config as _get_config, larger_tile, split_k_block_shape
 from .dtypes import BFloat16, DType, Float16, Float32, Float64, from_torch, promote_type
 from .errors import ConfigError, DimensionMismatch
 from .tiling import NT
@@ -256,6 +256,21 @@ def specialize(conf: Config, *,
     return SpecializedKernel(conf, {k: (Transform.Elementwise(expr=v) if isinstance(v, str) else v) for k, v in given.items()})
 
 
+def _launched_as(conf: Config, a, b, c, d, hooks: bool) -> Optional[Config]:
+    """``larger_tile`` of ``conf`` where the operands are what the aligned layouts of ``conf`` ask for (the library refuses others, and is left to), or None."""
+    larger = larger_tile(conf, hooks)
+    if larger is None:
+        return None
+    for x, layout in ((a, conf.global_a_layout), (b, conf.global_b_layout), (c, conf.global_c_layout), (d, conf.global_d_layout)):
+        if layout.kind == Layout.ZERO:
+            continue
+        ld = _leading_dim(x, layout)
+        # (the offsets in a tile are kept in 32 bits: 256 columns of 2^22 elements are left to a tile with fewer)
+        if x is None or _ptr(x) % 16 != 0 or ld * layout.T.size % 16 != 0 or ld >= 1 << 21:
+            return None
+    return larger
+
+
 class Plan:
     """One launch with everything but the stream lowered ahead of time: the descriptors of the
     configuration, the transforms and the epilogue, and the operand addresses.  Calling the plan is
@@ -264,15 +279,20 @@ class Plan:
     other means while it is in use.  For loops that launch the same GEMM many times, where the
     microseconds a general ``matmul`` call spends on lowering would rival the kernel itself."""
 
-    __slots__ = ("_fn", "_conf", "_trans", "_epi", "_args", "_keep", "_split_k", "d", "kernel_names")
+    __slots__ = ("_fn", "_conf", "_trans", "_epi", "_args", "_keep", "_split_k", "_as_given", "d", "kernel_names")
 
     def __init__(self, conf: Config, a, b, c, d, transforms: dict, epilogue, kernel, specialized=None):
         if specialized is None and any(t.expr is not None for t in transforms.values()):
             specialized = SpecializedKernel(conf, transforms)       # expression hooks: a run-time compiled kernel
-        cconf = conf.to_c(_leading_dim(a, conf.global_a_layout), _leading_dim(b, conf.global_b_layout),
-                          _leading_dim(c, conf.global_c_layout), _leading_dim(d, conf.global_d_layout))
-        self._conf = _lib.gk_config.from_buffer_copy(cconf)        # to_c hands out a cached, shared descriptor
+        lds = (_leading_dim(a, conf.global_a_layout), _leading_dim(b, conf.global_b_layout),
+               _leading_dim(c, conf.global_c_layout), _leading_dim(d, conf.global_d_layout))
+        self._conf = _lib.gk_config.from_buffer_copy(conf.to_c(*lds))        # to_c hands out a cached, shared descriptor
         self._trans = None if specialized is not None else lower_transforms(transforms)
+        self._as_given = None                                      # (what is launched where the library refuses the larger tile)
+        hooks = self._trans is not None or epilogue.kind != Epilogue.DEFAULT
+        larger = _launched_as(conf, a, b, c, d, hooks) if specialized is None and kernel is not Kernel.matmul_split_k else None
+        if larger is not None:
+            self._as_given, self._conf = self._conf, _lib.gk_config.from_buffer_copy(larger.to_c(*lds))
         self._epi = None
         self._split_k = False
         if epilogue.kind != Epilogue.DEFAULT:
@@ -305,6 +325,8 @@ class Plan:
                 _raise(rc)
             return self.d
         rc = self._fn(*self._args, stream)
+        if rc != _lib.GK_OK and self._as_given is not None:
+            rc = self._fn(ctypes.byref(self._as_given), *self._args[1:], stream)
         if rc != _lib.GK_OK:
             _raise(rc)
         return self.d
@@ -360,8 +382,9 @@ def matmul(conf: Config, a, b, c, d, *,
             return Plan(conf, a, b, c, d, collected, _DEFAULT_EPILOGUE if epilogue is None else epilogue, kernel)(stream)
         ctrans = lower_transforms(collected)
 
-    cconf = conf.to_c(_leading_dim(a, conf.global_a_layout), _leading_dim(b, conf.global_b_layout),
-                      _leading_dim(c, conf.global_c_layout), _leading_dim(d, conf.global_d_layout))
+    lds = (_leading_dim(a, conf.global_a_layout), _leading_dim(b, conf.global_b_layout),
+           _leading_dim(c, conf.global_c_layout), _leading_dim(d, conf.global_d_layout))
+    cconf = conf.to_c(*lds)
     cepi = None
     if epilogue is not None and epilogue.kind != Epilogue.DEFAULT:
         cepi = _lib.gk_epilogue()
@@ -375,9 +398,12 @@ def matmul(conf: Config, a, b, c, d, *,
                                           ctypes.byref(cepi) if cepi is not None else None,
                                           *_span(workspace), stream)
     else:
-        rc = _lib.lib().gk_matmul(ctypes.byref(cconf), _ptr(a), _ptr(b), _ptr(c), _ptr(d),
-                                  ctypes.byref(ctrans) if ctrans is not None else None,
-                                  ctypes.byref(cepi) if cepi is not None else None, kernel.code, stream)
+        args = (_ptr(a), _ptr(b), _ptr(c), _ptr(d), ctypes.byref(ctrans) if ctrans is not None else None,
+                ctypes.byref(cepi) if cepi is not None else None, kernel.code, stream)
+        larger = _launched_as(conf, a, b, c, d, ctrans is not None or cepi is not None)
+        rc = _lib.lib().gk_matmul(ctypes.byref(larger.to_c(*lds)), *args) if larger is not None else _lib.GK_ERR_UNSUPPORTED
+        if rc != _lib.GK_OK:
+            rc = _lib.lib().gk_matmul(ctypes.byref(cconf), *args)
     if rc != _lib.GK_OK:
         _raise(rc)
     return d
