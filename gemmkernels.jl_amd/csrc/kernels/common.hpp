@@ -339,7 +339,7 @@ __device__ __forceinline__ void store_cd(void* base, int dtype, long long idx, f
 // false in every workgroup but the last to arrive at the tile; in that one acc2 comes back as
 // partial(0) + partial(1) + ... + partial(k_slices - 1), added in this order whatever the order of arrival,
 // so the result does not change from run to run.  The partial tiles lie in the workspace in the lane order
-// of the accumulators: a store or load instruction of a wave moves 256 consecutive bytes.
+// of the accumulators: a store or load instruction of a wave moves 1024 consecutive bytes.
 //
 // The workgroups of a tile run on different XCDs, whose L2 caches are not coherent with each other.  The
 // partial tiles are therefore written and read with device-scope accesses (they go through to memory,
@@ -350,51 +350,61 @@ __device__ __forceinline__ void store_cd(void* base, int dtype, long long idx, f
 // workgroup, which made the launch five times longer (measured: 70 us against 13 us for 4096 x 64 x 4096).
 // No workgroup waits for another.
 // ---------------------------------------------------------------------------------------------
-template <int THREADS, int ROWS, int COLS, class V>
+//
+// What it costs is a chain of trips behind the L2 -- stores, the counter, loads -- so the accesses are 16 bytes wide (a quarter of the
+// instructions of 4-byte ones) and the partial tiles of as many slices as the registers hold travel together.  (Buffer accesses with the
+// sc1 bit: the same scope as an agent-scope atomic access, which the compiler emits 4 bytes wide only; nobody reads a value before
+// the counter says that all of them are there, so none of them has to be atomic.)
+template <int THREADS, typename E = float, int ROWS, int COLS, class V>
 __device__ __forceinline__ bool splitk_reduce(V (&acc2)[ROWS][COLS], const GemmArgs& args, int tile_id, unsigned* lds_word) {
   constexpr int COUNT = ROWS * COLS;
-  constexpr int NV = (int)(sizeof(V) / sizeof(float));   // floats per accumulator block and lane
-  auto blk = [&](int i) -> V& { return acc2[i / COLS][i % COLS]; };
+  constexpr int NV = (int)(sizeof(V) / sizeof(E));         // values per accumulator block and lane
+  constexpr int PB = (int)(sizeof(V) / 16), PIECES = COUNT * PB;       // 16-byte pieces per block and per lane
+  static_assert(sizeof(V) % 16 == 0, "accumulator blocks are whole 16-byte pieces");
+  typedef unsigned uint4v __attribute__((ext_vector_type(4)));
+  struct Pieces { uint4v p[PB]; };
+  constexpr int kScope = 16;                               // sc1
+  constexpr unsigned TILE_BYTES = (unsigned)(PIECES * 16 * THREADS);
   const int S = args.k_slices, z = (int)blockIdx.z, tid = (int)threadIdx.x;
-  constexpr size_t TILE_FLOATS = (size_t)COUNT * NV * THREADS;
-  float* tile_ws = (float*)args.ws_partials + (size_t)tile_id * S * TILE_FLOATS;
-  float* mine = tile_ws + (size_t)z * TILE_FLOATS;
+  char* tile_ws = (char*)args.ws_partials + (size_t)tile_id * S * TILE_BYTES;
+  const auto ws = __builtin_amdgcn_make_buffer_rsrc(tile_ws, 0, (int)(S * TILE_BYTES), 0x00020000);
 #pragma unroll
-  for (int i = 0; i < COUNT; ++i)
+  for (int i = 0; i < COUNT; ++i) {
+    const Pieces b = __builtin_bit_cast(Pieces, acc2[i / COLS][i % COLS]);
 #pragma unroll
-    for (int e = 0; e < NV; ++e)
-      __hip_atomic_store(&mine[(size_t)(i * NV + e) * THREADS + tid], blk(i)[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int e = 0; e < PB; ++e)
+      __builtin_amdgcn_raw_buffer_store_b128(b.p[e], ws, ((i * PB + e) * THREADS + tid) * 16, z * (int)TILE_BYTES, kScope);
+  }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // this lane's part of the tile has reached memory ...
   __syncthreads();                                     // ... and so has every other lane's, before the arrival is counted
   if (tid == 0) *lds_word = __hip_atomic_fetch_add(&args.ws_counters[tile_id], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
   const unsigned before_me = *lds_word;
   if (before_me != (unsigned)(S - 1)) return false;
+  asm volatile("" ::: "memory");
 #pragma unroll
-  for (int i = 0; i < COUNT; ++i)
-#pragma unroll
-    for (int e = 0; e < NV; ++e) blk(i)[e] = 0.0f;
-  // The partial tiles of U slices travel together (one slice at a time the loop would pay the latency of the
-  // memory behind the L2 once per slice); they are added in slice order all the same.
-  constexpr int PER = COUNT * NV;                            // floats per lane and slice
-  constexpr int U = PER >= 32 ? 1 : (PER >= 16 ? 3 : 4);     // at most 63 loads can be outstanding per wave
+  for (int i = 0; i < COUNT; ++i) acc2[i / COLS][i % COLS] = (E)0;
+  // (a tile holds at most 16 pieces of a lane at a time; slices beyond the last one re-read the last, and are not added)
+  constexpr int U = PIECES >= 16 ? 1 : (16 / PIECES > 8 ? 8 : 16 / PIECES);
   for (int s0 = 0; s0 < S; s0 += U) {
-    float x[U][PER];
+    Pieces x[U][COUNT];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      // a slice beyond the last one re-reads the last (its values are not added)
-      const float* part = tile_ws + (size_t)(s0 + u < S ? s0 + u : S - 1) * TILE_FLOATS;
+      const int from = (s0 + u < S ? s0 + u : S - 1) * (int)TILE_BYTES;
 #pragma unroll
-      for (int q = 0; q < PER; ++q)
-        x[u][q] = __hip_atomic_load(&part[(size_t)q * THREADS + tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (int i = 0; i < COUNT; ++i)
+#pragma unroll
+        for (int e = 0; e < PB; ++e) x[u][i].p[e] = __builtin_amdgcn_raw_buffer_load_b128(ws, ((i * PB + e) * THREADS + tid) * 16, from, kScope);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
       if (s0 + u < S) {
 #pragma unroll
-        for (int i = 0; i < COUNT; ++i)
+        for (int i = 0; i < COUNT; ++i) {
+          const V part = __builtin_bit_cast(V, x[u][i]);
 #pragma unroll
-          for (int e = 0; e < NV; ++e) blk(i)[e] += x[u][i * NV + e];
+          for (int e = 0; e < NV; ++e) acc2[i / COLS][i % COLS][e] += part[e];
+        }
       }
   }
   // the next launch on this workspace finds the counter at zero
