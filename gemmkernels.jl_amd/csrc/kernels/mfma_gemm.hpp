@@ -2170,23 +2170,33 @@ __global__ void __launch_bounds__(Cfg::THREADS) mfma_gemm_kernel(const GemmArgs 
     if constexpr (CPATH == 3) {
       // (what lies outside D is left out: columns, groups of four rows, and the last rows of the group that reaches over
       // the last row of a D whose M is not in fours)
+      auto store_edges = [&](auto through_c) __attribute__((always_inline)) {
 #pragma unroll
-      for (int fj = 0; fj < FN; ++fj)
+        for (int fj = 0; fj < FN; ++fj)
 #pragma unroll
-        for (int fi = 0; fi < FM; ++fi) {
-          const int r = solo_row + MI * fi, cc = solo_col + MI * fj;
-          if (r < args.M && cc < args.N) {
-            float* dp = (float*)args.d + ((long long)r + (long long)cc * args.ldd);
-            if (r + 4 <= args.M) {
-              asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" :: "v"(dp), "a"(acc[fi][fj]) : "memory");
-            } else {
-              const int left = args.M - r;     // 1 .. 3
-              asm volatile("global_store_dword %0, %1, off" :: "v"(dp), "a"(acc[fi][fj][0]) : "memory");
-              if (left > 1) asm volatile("global_store_dword %0, %1, off offset:4" :: "v"(dp), "a"(acc[fi][fj][1]) : "memory");
-              if (left > 2) asm volatile("global_store_dword %0, %1, off offset:8" :: "v"(dp), "a"(acc[fi][fj][2]) : "memory");
+          for (int fi = 0; fi < FM; ++fi) {
+            const int r = solo_row + MI * fi, cc = solo_col + MI * fj;
+            if (r < args.M && cc < args.N) {
+              float* dp = (float*)args.d + ((long long)r + (long long)cc * args.ldd);
+              AccV& blk = acc[fi][fj];
+              if (r + 4 <= args.M) {
+                if constexpr (decltype(through_c)::value) asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" :: "v"(dp), "a"(blk) : "memory");
+                else asm volatile("global_store_dwordx4 %0, %1, off" :: "v"(dp), "a"(blk) : "memory");
+              } else {
+                const int left = args.M - r;     // 1 .. 3
+                asm volatile("global_store_dword %0, %1, off" :: "v"(dp), "a"(blk[0]) : "memory");
+                if (left > 1) asm volatile("global_store_dword %0, %1, off offset:4" :: "v"(dp), "a"(blk[1]) : "memory");
+                if (left > 2) asm volatile("global_store_dword %0, %1, off offset:8" :: "v"(dp), "a"(blk[2]) : "memory");
+              }
             }
           }
-        }
+      };
+      // Write-through stores (see path 4) where the 64 bytes that a column gets from an instruction are 64 bytes of memory; where columns start
+      // elsewhere the pieces share lines with their neighbours, which the L2 puts together before they leave it.  BF16 4001 x 4003 x 4032 on inputs
+      // that rotate, us with write-through and with plain stores: ldd = 4001 129.5 and 108.8, 4004 124.0 and 107.4, 4008 117.0 and 107.2, 4016 105.7 and
+      // 106.4, 4032 105.8 and 106.6; on the same inputs over and over 106.3 and 97.2, 101.9 and 95.4, 97.9 and 94.4, 93.8 and 94.2, 93.6 and 94.9.
+      if (((((uintptr_t)args.d) | ((uintptr_t)args.ldd << 2)) & 63u) == 0) store_edges(std::true_type{});
+      else store_edges(std::false_type{});
     } else if constexpr (STREAM_C) {
       // from the accumulation registers the kernel manages itself: the wave tile's origin in D from scalar registers, the
       // lane's offset in it from a vector register, the row block as an immediate.  The stores write through to memory
