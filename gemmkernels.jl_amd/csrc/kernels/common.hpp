@@ -194,19 +194,18 @@ __host__ __device__ inline void cta_swizzle(int kind, int param, int bx, int by,
       tj = (int)extract_even_bits((unsigned)bx >> 1);
       break;
     case SWZ_XCD: {
-      const int total = nbm * nbn;
+      const unsigned m = (unsigned)nbm, n = (unsigned)nbn, total = m * n, id = (unsigned)bx;
       // ids x, x + 8, x + 16, ... run on XCD x: XCD x holds total / 8 of them, one more when x < total % 8;
       // the ids of one XCD become consecutive
-      const int x = bx % 8, q = total / 8, rem = total % 8;
-      const int r = x * q + (x < rem ? x : rem) + bx / 8;
-      const int g = param > 0 ? param : 1;
-      const int width = g * nbn;
-      const int group = r / width;
-      const int first = group * g;
-      const int gsz = (nbm - first) < g ? (nbm - first) : g;
-      const int in_group = r % width;
-      ti = first + in_group % gsz;
-      tj = in_group / gsz;
+      const unsigned x = id % 8, q = total / 8, rem = total % 8;
+      const unsigned r = x * q + (x < rem ? x : rem) + id / 8;
+      const unsigned g = param > 0 ? (unsigned)param : 1u;
+      // (one panel: a division less in front of the first load of a launch with few tiles)
+      const unsigned group = m <= g ? 0u : r / (g * n);
+      const unsigned first = group * g, in_group = r - group * (g * n);
+      const unsigned gsz = m - first < g ? m - first : g;
+      tj = (int)(in_group / gsz);
+      ti = (int)(first + (in_group - (unsigned)tj * gsz));
       break;
     }
     default:

@@ -619,6 +619,14 @@ __global__ void __launch_bounds__(Cfg::THREADS) mfma_gemm_kernel(const GemmArgs 
 
   extern __shared__ __attribute__((aligned(1024))) char smem[];
 
+  // What stands in front of the first DMA, read in one go: each group of arguments on its own is another trip to a line of memory
+  // that no cache holds (0.2 us), and the compiler reads them where they are first used, behind the walk of the tiles.
+  if constexpr (!Cfg::GETT)
+    asm volatile("" ::"s"(args.a), "s"(args.b), "s"(args.lda), "s"(args.ldb), "s"(args.M), "s"(args.N), "s"(args.K), "s"(args.nbm), "s"(args.nbn), "s"(args.swz_kind), "s"(args.swz_param));
+  if constexpr (Cfg::SPLITK) asm volatile("" ::"s"(args.k_steps), "s"(args.k_slices));
+  if constexpr (Cfg::GETT)          // (one word of each line of the mode tables)
+    asm volatile("" ::"s"(args.a), "s"(args.b), "s"(args.nbm), "s"(args.swz_param), "s"(args.gm.nmodes), "s"(args.gm.stride0[3]), "s"(args.gn.nmodes), "s"(args.gn.stride0[3]), "s"(args.gk.nmodes),
+                 "s"(args.gk.stride0[3]), "s"(args.gk.shift[3]), "s"(args.gk_mode));
   int ti, tj;
   cta_swizzle(args.swz_kind, args.swz_param, (int)blockIdx.x, (int)blockIdx.y, args.nbm, args.nbn, ti, tj);
   if (ti >= args.nbm || tj >= args.nbn) return;   // whole block leaves together
@@ -889,6 +897,11 @@ __global__ void __launch_bounds__(Cfg::THREADS) mfma_gemm_kernel(const GemmArgs 
       table[2 * t + 1] = (long long)(gb + ob * 2);
     }
   }
+
+  // (what hooks and epilogue look up later, each in a line of its own: on their way with the first tiles)
+  if constexpr (Cfg::FUSED && !Cfg::SOLO)
+    asm volatile("" ::"s"(args.t[H_GL2SH_C].n), "s"(args.t[H_SH2GL_D].n), "s"(args.t[H_SH2RF_C].n), "s"(args.t[H_RF2SH_D].n), "s"(args.scale_a), "s"(args.acc_pre_scale),
+                 "s"(args.acc_post_scale), "s"(args.epi_kind));
 
   // --- accumulators: C tile (two transforms) or zeros -------------------------------------------
   // 32x32 blocks: lane l owns row m = 32*fi + l%32 and columns n = 32*fj + 8*(v/4) + 4*(l/32) + v%4, v < 16;
