@@ -152,6 +152,28 @@ struct KWalker {
     keep(step); keep(e0); keep(e1); keep(e2);
     keep(step_a); keep(step_b); keep(wa0); keep(wa1); keep(wa2); keep(wb0); keep(wb1); keep(wb2);
   }
+  // Starts at k-value k instead of 0 (a whole number of tiles): a slice of a K-split launch.
+  __device__ __forceinline__ void start_at(const GettDim& gk, int mode, int k) {
+    long long a, b;
+    gett_offsets32(gk, k, a, b);
+    oa = 2 * a; ob = 2 * b;
+    int q = k;
+    for (int i = 0; i < mode; ++i) q = gett_div(q, gk.magic[i], gk.shift[i]);
+    auto digit = [&](int i, int& d) __attribute__((always_inline)) {
+      if (i + 1 < gk.nmodes) {
+        const int next = gett_div(q, gk.magic[i], gk.shift[i]);
+        d = q - next * gk.extent[i];
+        q = next;
+      } else {
+        d = q;            // (the last mode takes what is left; none behind it)
+        q = 0;
+      }
+    };
+    digit(mode, d0);
+    digit(mode + 1, d1);
+    digit(mode + 2, d2);
+    keep(d0); keep(d1); keep(d2); keep(oa); keep(ob);
+  }
   __device__ __forceinline__ void advance() {
     d0 += step;
     oa += step_a; ob += step_b;
@@ -542,6 +564,13 @@ struct MfmaGemmConfig {
   // outstanding (the wait counter holds 15)
   static constexpr bool SPLIT_A = MI_ == 16 && ((BM_ / WAVES_M_ / MI_) % 2 == 0);
   static constexpr bool PREFETCH = !SPLIT_A && (STAGES_ >= 3) && ((BK_ / KSTEP_K) % 2 == 0);   // cross-step fragment prefetch
+  // The last K tile, when it is partial (or has a chunk over the end of an operand), sets out behind the others like one more tile
+  // of the pipeline and is repaired and multiplied behind the loop; fetched behind the loop it stands there for the whole latency of
+  // memory with nothing else to do.  (Larger tiles would hold the repairs' registers through the loop.)  With offsets in 32 bits and a repair by shifts instead of 64
+  // selections per chunk: 704 x 27 x 869 10.3 -> 8.9 us, 16 x 56 x 2016 10.9 -> 9.4, 256 x 512 x 435 7.3 -> 5.6.
+  // (PEELED: the K loop without branches, for the tiles that run alone, or nearly alone, on a SIMD)
+  static constexpr bool PEELED = SPLIT_A && !PREFETCH;
+  static constexpr bool TAIL_AHEAD = RAGGED_K_OK && PEELED && BM_ * BN_ <= 256 * 128;
   // The DMA instructions of a tile are issued a few per k-step instead of all at once: a wave whose
   // DMA instruction waits for room in the memory pipeline cannot issue its MFMAs either, and a burst
   // from every wave right after the barrier makes all of them wait together (measured on 4096^3:
@@ -870,9 +899,85 @@ __global__ void __launch_bounds__(Cfg::THREADS) mfma_gemm_kernel(const GemmArgs 
     if (kt0 >= total) return;       // the whole workgroup leaves together, before any barrier
     if (kt0 + args.k_steps < total) tail_k = 0;
     KT = (KT - kt0) < args.k_steps ? (KT - kt0) : args.k_steps;
-    ga += (long long)kt0 * a_step;
-    gb += (long long)kt0 * b_step;
+    if constexpr (Cfg::GETT) {
+      walk.start_at(args.gk, args.gk_mode, kt0 * BK);
+    } else {
+      ga += (long long)kt0 * a_step;
+      gb += (long long)kt0 * b_step;
+    }
   }
+
+  // The last K tile when it stands outside the pipeline (tail_k): every lane fetches its 16-byte chunks with coordinates clamped to
+  // valid ones -- a chunk that would reach past the last element of the operand is fetched from 1 .. 7 elements further back -- and
+  // repairs its own chunks in LDS once they have landed: shifted into place, values whose k is beyond K set to zero.  Offsets in a tile
+  // fit 32 bits (the host refuses others).
+  // per chunk: elements it was fetched too far back (0 .. 7), leading elements that keep their value (0 .. 8)
+  [[maybe_unused]] int tail_shift[RAGGED_K ? DPT : 1], tail_keep[RAGGED_K ? DPT : 1];
+  [[maybe_unused]] auto issue_tail = [&](int stage, auto gta, auto gtb) __attribute__((always_inline)) {
+    char* sa = smem + stage * Cfg::STAGE_BYTES;
+    char* sb = sa + GA::BYTES;
+    int l = lane;
+    asm volatile("" : "+v"(l));                          // (computed here, not ahead of the branch around it)
+    auto fetch = [&](auto kind_c, auto geom, int q, const char* g, int ld, int rows_valid, char* dst, int& shift, int& keep) __attribute__((always_inline)) {
+      constexpr int KIND = decltype(kind_c)::value;
+      typedef decltype(geom) G;
+      int row, col;
+      dma_lane_coords<G, KIND>(q, l, row, col);
+      int& r = KIND == OPK_KMAJOR ? row : col;           // index along M (A) or N (B), from the tile origin
+      int& k = KIND == OPK_KMAJOR ? col : row;
+      const int last_r = KIND == OPK_KMAJOR ? rows_valid - 1 : ((rows_valid - 1) >> 3) << 3;
+      r = r > last_r ? last_r : r;
+      if (KIND == OPK_KMAJOR) {                          // the chunk runs along k
+        keep = tail_k - k;
+        keep = keep < 0 ? 0 : (keep > 8 ? 8 : keep);
+        const int last_k = ((tail_k - 1) >> 3) << 3;
+        k = k > last_k ? last_k : k;
+      } else {
+        keep = k < tail_k ? 8 : 0;
+        k = k < tail_k ? k : tail_k - 1;
+      }
+      const int e = row * ld + col;
+      // one past the last element of the operand, counted from the tile origin
+      const int end = KIND == OPK_KMAJOR ? (rows_valid - 1) * ld + tail_k : (tail_k - 1) * ld + rows_valid;
+      shift = e + 8 - end;
+      shift = shift < 0 ? 0 : shift;
+      __builtin_amdgcn_global_load_lds(GK_GLOBAL_PTR(g + (long long)(e - shift) * 2), GK_LDS_PTR(void, dst + q * 1024), 16, 0, 0);
+    };
+#pragma unroll
+    for (int i = 0; i < DMA_A; ++i)
+      fetch(std::integral_constant<int, Cfg::A_KIND>{}, GA{}, wave + i * NWAVES, gta, (int)args.lda, args.M - m0, sa, tail_shift[i], tail_keep[i]);
+#pragma unroll
+    for (int i = 0; i < DMA_B; ++i)
+      fetch(std::integral_constant<int, Cfg::B_KIND>{}, GB{}, wave + i * NWAVES, gtb, (int)args.ldb, args.N - n0, sb, tail_shift[DMA_A + i], tail_keep[DMA_A + i]);
+  };
+  [[maybe_unused]] auto repair_tail = [&](int stage) __attribute__((always_inline)) {
+    char* sa = smem + stage * Cfg::STAGE_BYTES;
+    char* sb = sa + GA::BYTES;
+    wait_vmcnt<0>();                                     // this lane's own slots have landed
+    auto repair = [&](char* slot, int shift, int keep) __attribute__((always_inline)) {
+      if (shift == 0 && keep == 8) return;
+      int4v v = *(const int4v*)slot;
+      // element e was fetched into place e + shift: four elements, two, one
+      const bool by4 = (shift & 4) != 0, by2 = (shift & 2) != 0;
+      v[0] = by4 ? v[2] : v[0];
+      v[1] = by4 ? v[3] : v[1];
+      v[0] = by2 ? v[1] : v[0];
+      v[1] = by2 ? v[2] : v[1];
+      v[2] = by2 ? v[3] : v[2];
+      const int by1 = (shift & 1) * 16;
+#pragma unroll
+      for (int w = 0; w < 3; ++w) v[w] = (int)__builtin_amdgcn_alignbit((unsigned)v[w + 1], (unsigned)v[w], (unsigned)by1);
+      v[3] = (int)((unsigned)v[3] >> by1);
+      // (what a shift leaves behind the end of the operand is beyond `keep`, or belongs to rows that are not stored)
+#pragma unroll
+      for (int w = 0; w < 4; ++w) v[w] = keep >= 2 * w + 2 ? v[w] : (keep == 2 * w + 1 ? v[w] & 0xffff : 0);
+      *(int4v*)slot = v;
+    };
+#pragma unroll
+    for (int i = 0; i < DMA_A; ++i) repair(sa + (wave + i * NWAVES) * 1024 + lane * 16, tail_shift[i], tail_keep[i]);
+#pragma unroll
+    for (int i = 0; i < DMA_B; ++i) repair(sb + (wave + i * NWAVES) * 1024 + lane * 16, tail_shift[DMA_A + i], tail_keep[DMA_A + i]);
+  };
 
   // (SOLO: the loop leaves ga / gb at the last tile it fetched, so the tile behind the loop is kept here)
   [[maybe_unused]] const char* ga_tail = ga + kDmaBias;
@@ -883,9 +988,15 @@ __global__ void __launch_bounds__(Cfg::THREADS) mfma_gemm_kernel(const GemmArgs 
   }
 
   // --- prologue: start the first STAGES-1 tiles on their way ---
+  // (TAIL_AHEAD: the tile outside the pipeline travels as one more tile behind the others)
+  constexpr bool TAIL_AHEAD = Cfg::TAIL_AHEAD;
+  [[maybe_unused]] const int KTI = TAIL_AHEAD && tail_k > 0 ? KT + 1 : KT;
 #pragma unroll
   for (int s = 0; s < (Cfg::SOLO ? STAGES : STAGES - 1); ++s)
     if (s < KT) issue_tile(s);      // (SOLO: both stages are free and the loop issues tile kt + 2 from tile kt)
+  if constexpr (TAIL_AHEAD) {
+    if (KT < STAGES - 1 && tail_k > 0) issue_tail(KT, ga, gb);
+  }
   if constexpr (Cfg::SOLO && Cfg::GETT) {
     // where K tile t starts in A and in B: the pointers that the DMA of the tile takes as its scalar base (published by the
     // barrier in front of the K loop)
@@ -1393,58 +1504,11 @@ __global__ void __launch_bounds__(Cfg::THREADS) mfma_gemm_kernel(const GemmArgs 
     }
   };
   // The last K tile of a product whose K is not a whole number of tiles (or that has a chunk over the end of an operand,
-  // see tail_k): fetched into the first stage from gta / gtb with clamped coordinates and repaired there, outside the pipeline.
+  // see tail_k), outside the pipeline: fetched into the first stage from gta / gtb and repaired there.
   [[maybe_unused]] auto fetch_tail_tile = [&](auto gta, auto gtb) __attribute__((always_inline)) {
     block_barrier();                                     // every wave is done with the stages of the loop
-    char* sa = smem;
-    char* sb = sa + GA::BYTES;
-    // per chunk: elements it was fetched too far back (0 .. 7), leading elements that keep their value (0 .. 8)
-    int shift_a[DMA_A], keep_a[DMA_A], shift_b[DMA_B], keep_b[DMA_B];
-    auto fetch = [&](auto kind_c, auto geom, int q, const char* g, long long ld, int rows_valid, char* dst, int& shift, int& keep)
-        __attribute__((always_inline)) {
-      constexpr int KIND = decltype(kind_c)::value;
-      typedef decltype(geom) G;
-      int row, col;
-      dma_lane_coords<G, KIND>(q, lane, row, col);
-      int& r = KIND == OPK_KMAJOR ? row : col;           // index along M (A) or N (B), from the tile origin
-      int& k = KIND == OPK_KMAJOR ? col : row;
-      const int last_r = KIND == OPK_KMAJOR ? rows_valid - 1 : ((rows_valid - 1) >> 3) << 3;
-      r = r > last_r ? last_r : r;
-      keep = 8;
-      if (KIND == OPK_KMAJOR) {                          // the chunk runs along k
-        if (k >= tail_k) { keep = 0; k = ((tail_k - 1) >> 3) << 3; }
-        else if (k + 8 > tail_k) keep = tail_k - k;
-      } else if (k >= tail_k) { keep = 0; k = tail_k - 1; }
-      long long e = (long long)row * ld + col;
-      // one past the last element of the operand, counted from the tile origin
-      const long long end = KIND == OPK_KMAJOR ? (long long)(rows_valid - 1) * ld + tail_k : (long long)(tail_k - 1) * ld + rows_valid;
-      shift = 0;
-      if (e + 8 > end) { shift = (int)(e + 8 - end); e -= shift; }
-      __builtin_amdgcn_global_load_lds(GK_GLOBAL_PTR(g + e * 2), GK_LDS_PTR(void, dst + q * 1024), 16, 0, 0);
-    };
-#pragma unroll
-    for (int i = 0; i < DMA_A; ++i)
-      fetch(std::integral_constant<int, Cfg::A_KIND>{}, GA{}, wave + i * NWAVES, gta, args.lda, args.M - m0, sa, shift_a[i], keep_a[i]);
-#pragma unroll
-    for (int i = 0; i < DMA_B; ++i)
-      fetch(std::integral_constant<int, Cfg::B_KIND>{}, GB{}, wave + i * NWAVES, gtb, args.ldb, args.N - n0, sb, shift_b[i], keep_b[i]);
-    wait_vmcnt<0>();                                     // this lane's own slots have landed
-    auto repair = [&](char* slot, int shift, int keep) __attribute__((always_inline)) {
-      if (shift == 0 && keep == 8) return;
-      short8v v = *(const short8v*)slot, out;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        short x = 0;
-#pragma unroll
-        for (int f = 0; f < 8; ++f) x = (f == e + shift) ? v[f] : x;      // element e was fetched into place e + shift
-        out[e] = e < keep ? x : (short)0;
-      }
-      *(short8v*)slot = out;
-    };
-#pragma unroll
-    for (int i = 0; i < DMA_A; ++i) repair(sa + (wave + i * NWAVES) * 1024 + lane * 16, shift_a[i], keep_a[i]);
-#pragma unroll
-    for (int i = 0; i < DMA_B; ++i) repair(sb + (wave + i * NWAVES) * 1024 + lane * 16, shift_b[i], keep_b[i]);
+    issue_tail(0, gta, gtb);
+    repair_tail(0);
     __syncthreads();                                     // waits for the LDS writes as well
     ra.set_stage(lds_base);
     rb.set_stage(lds_base + GA::BYTES);
@@ -1766,128 +1830,163 @@ __global__ void __launch_bounds__(Cfg::THREADS) mfma_gemm_kernel(const GemmArgs 
   } else if constexpr (!Cfg::PREFETCH) {
     // Two LDS stages: the DMA of tile kt+1 runs while tile kt is consumed; the first fragments of a
     // tile are read after the barrier that publishes it.
-    for (int kt = 0; kt < KT; ++kt) {
-      // tile kt has landed once at most the DMA of the STAGES-2 younger tiles is outstanding
-      if (kt + STAGES - 2 < KT) wait_vmcnt<(STAGES - 2) * DPT>(); else wait_vmcnt<0>();
-      block_barrier();   // every wave's share of tile kt is in LDS; every wave is done with tile kt-1
-      const unsigned stage_addr = lds_base + (unsigned)(kt % STAGES) * Cfg::STAGE_BYTES;
+    auto enter_stage = [&](int stage) __attribute__((always_inline)) {
+      const unsigned stage_addr = lds_base + (unsigned)stage * Cfg::STAGE_BYTES;
       ra.set_stage(stage_addr);
       rb.set_stage(stage_addr + GA::BYTES);
-      const bool issue = (kt + STAGES - 1 < KT);
+    };
+    // the k-steps of tile kt (Cfg::SPLIT_A); issue: tile kt + STAGES - 1 sets out meanwhile
+    [[maybe_unused]] auto multiply_tile = [&](int kt, auto issue) __attribute__((always_inline)) {
       if constexpr (Cfg::SPLIT_A) {
-        constexpr int HF = FM / 2;
-        constexpr int OPS_AH = HF * RA::OPS, OPS_B = RB::NREAD * RB::OPS;
-        // reads of A half H of k-step KS into fa[H], of B of k-step KS into fb[KS & 1]
-        auto load_a_half = [&](auto ks2_c, auto h_c) __attribute__((always_inline)) {
-          constexpr int KS2 = decltype(ks2_c)::value, H = decltype(h_c)::value;
+      constexpr int HF = FM / 2;
+      constexpr int OPS_AH = HF * RA::OPS, OPS_B = RB::NREAD * RB::OPS;
+      // reads of A half H of k-step KS into fa[H], of B of k-step KS into fb[KS & 1]
+      auto load_a_half = [&](auto ks2_c, auto h_c) __attribute__((always_inline)) {
+        constexpr int KS2 = decltype(ks2_c)::value, H = decltype(h_c)::value;
+        static_for<0, HF>([&](auto i_c) {
+          constexpr int I = decltype(i_c)::value;
+          ra.template read<H * HF + I, KS2, Cfg::SYNC_FRAGS>(fa[H][I]);
+        });
+      };
+      auto load_b = [&](auto ks2_c) __attribute__((always_inline)) {
+        constexpr int KS2 = decltype(ks2_c)::value;
+        static_for<0, RB::NREAD>([&](auto j_c) {
+          constexpr int J = decltype(j_c)::value;
+          rb.template read<J, KS2, Cfg::SYNC_FRAGS>(fb[KS2 & 1][J]);
+        });
+      };
+      if constexpr (Cfg::A_KIND == OPK_KSPLIT) {
+        // One set of reads per k-step serves both halves: once it has arrived, the real and the imaginary fragments
+        // of A (and the fragments of B) are made from it and kept, which frees the registers of the reads for those
+        // of the next k-step; they are in flight under the MFMAs of both halves.  One buffer each for A and B.
+        auto load_both = [&](auto ks2_c) __attribute__((always_inline)) {
+          constexpr int KS2 = decltype(ks2_c)::value;
           static_for<0, HF>([&](auto i_c) {
             constexpr int I = decltype(i_c)::value;
-            ra.template read<H * HF + I, KS2, Cfg::SYNC_FRAGS>(fa[H][I]);
+            ra.template read<I, KS2, Cfg::SYNC_FRAGS>(fa[0][I]);
           });
-        };
-        auto load_b = [&](auto ks2_c) __attribute__((always_inline)) {
-          constexpr int KS2 = decltype(ks2_c)::value;
           static_for<0, RB::NREAD>([&](auto j_c) {
             constexpr int J = decltype(j_c)::value;
-            rb.template read<J, KS2, Cfg::SYNC_FRAGS>(fb[KS2 & 1][J]);
+            rb.template read<J, KS2, Cfg::SYNC_FRAGS>(fb[0][J]);
           });
         };
-        if constexpr (Cfg::A_KIND == OPK_KSPLIT) {
-          // One set of reads per k-step serves both halves: once it has arrived, the real and the imaginary fragments
-          // of A (and the fragments of B) are made from it and kept, which frees the registers of the reads for those
-          // of the next k-step; they are in flight under the MFMAs of both halves.  One buffer each for A and B.
-          auto load_both = [&](auto ks2_c) __attribute__((always_inline)) {
-            constexpr int KS2 = decltype(ks2_c)::value;
-            static_for<0, HF>([&](auto i_c) {
-              constexpr int I = decltype(i_c)::value;
-              ra.template read<I, KS2, Cfg::SYNC_FRAGS>(fa[0][I]);
-            });
-            static_for<0, RB::NREAD>([&](auto j_c) {
-              constexpr int J = decltype(j_c)::value;
-              rb.template read<J, KS2, Cfg::SYNC_FRAGS>(fb[0][J]);
-            });
-          };
-          load_both(std::integral_constant<int, 0>{});
-          static_for<0, 2 * Cfg::KSTEPS>([&](auto u_c) {
-            constexpr int u = decltype(u_c)::value;
-            constexpr int ks = u / 2, h = u % 2;
-            if (issue) issue_part(u_c, std::integral_constant<int, 2 * Cfg::KSTEPS>{}, (kt + STAGES - 1) % STAGES);
-            if constexpr (h == 0) {
-              wait_lgkmcnt<0>();                          // the reads of this k-step have arrived
-              // Program order = the order the instructions should issue in (the scheduling groups below pin it): the
-              // byte permutes that make a fragment stand right before the MFMAs that first need it, those of the
-              // imaginary fragments of A (needed by the second half) between the MFMA groups of the first half, so
-              // that all but the first eight run in the shadow of MFMAs; the reads of the next k-step follow the
-              // last permute (they reuse the registers the permutes read) and have the whole second half to land.
-              constexpr bool B_BOTH = Cfg::B_KIND == OPK_KSPLIT;
-              int4v va[HF];
-#pragma unroll
-              for (int i = 0; i < HF; ++i) RA::pin_raw(fa[0][i]);
-#pragma unroll
-              for (int fj = 0; fj < RB::NREAD; ++fj) RB::pin_raw(fb[0][fj]);
-              va[0] = RA::finish(fa[0][0], lane, false);
-#pragma unroll
-              for (int fj = 0; fj < FN; ++fj) {
-                vb_keep[fj] = RB::finish(fb[0][fj % RB::NREAD], lane, fj >= RB::NREAD);
-                acc[0][fj] = Mfma<T, MI>::run(vb_keep[fj], va[0], acc[0][fj]);
-              }
-#pragma unroll
-              for (int i = 1; i < HF; ++i) {
-                va[i] = RA::finish(fa[0][i], lane, false);
-                va_keep[i - 1] = RA::finish(fa[0][i - 1], lane, true);
-                pin(va_keep[i - 1]);          // made here, not where the second half uses it
-#pragma unroll
-                for (int fj = 0; fj < FN; ++fj) acc[i][fj] = Mfma<T, MI>::run(vb_keep[fj], va[i], acc[i][fj]);
-              }
-              va_keep[HF - 1] = RA::finish(fa[0][HF - 1], lane, true);
-              pin(va_keep[HF - 1]);
-              if constexpr (B_BOTH) {
-                __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);
-                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-#pragma unroll
-                for (int fj = 1; fj < FN; ++fj) {
-                  __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
-                  __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-                }
-              } else {
-                __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
-                __builtin_amdgcn_sched_group_barrier(0x8, FN, 0);
-              }
-#pragma unroll
-              for (int i = 1; i < HF; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);
-                __builtin_amdgcn_sched_group_barrier(0x8, FN, 0);
-              }
-              __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
-              if constexpr (ks + 1 < Cfg::KSTEPS) load_both(std::integral_constant<int, ks + 1>{});
-            } else {
-#pragma unroll
-              for (int i = 0; i < HF; ++i)
-#pragma unroll
-                for (int fj = 0; fj < FN; ++fj) acc[HF + i][fj] = Mfma<T, MI>::run(vb_keep[fj], va_keep[i], acc[HF + i][fj]);
-            }
-          });
-          // (the last reads of the stage were waited for before its last MFMAs: complete before the next barrier)
-          continue;
-        }
-        load_a_half(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
-        load_b(std::integral_constant<int, 0>{});
+        load_both(std::integral_constant<int, 0>{});
         static_for<0, 2 * Cfg::KSTEPS>([&](auto u_c) {
           constexpr int u = decltype(u_c)::value;
           constexpr int ks = u / 2, h = u % 2;
           if (issue) issue_part(u_c, std::integral_constant<int, 2 * Cfg::KSTEPS>{}, (kt + STAGES - 1) % STAGES);
           if constexpr (h == 0) {
-            load_a_half(std::integral_constant<int, ks>{}, std::integral_constant<int, 1>{});
-            wait_lgkmcnt<OPS_AH>();                     // half 0 and B of this k-step have arrived
-          } else if constexpr (ks + 1 < Cfg::KSTEPS) {
-            load_a_half(std::integral_constant<int, ks + 1>{}, std::integral_constant<int, 0>{});
-            load_b(std::integral_constant<int, ks + 1>{});
-            wait_lgkmcnt<OPS_AH + OPS_B>();             // half 1 of this k-step has arrived
+            wait_lgkmcnt<0>();                          // the reads of this k-step have arrived
+            // Program order = the order the instructions should issue in (the scheduling groups below pin it): the
+            // byte permutes that make a fragment stand right before the MFMAs that first need it, those of the
+            // imaginary fragments of A (needed by the second half) between the MFMA groups of the first half, so
+            // that all but the first eight run in the shadow of MFMAs; the reads of the next k-step follow the
+            // last permute (they reuse the registers the permutes read) and have the whole second half to land.
+            constexpr bool B_BOTH = Cfg::B_KIND == OPK_KSPLIT;
+            int4v va[HF];
+#pragma unroll
+            for (int i = 0; i < HF; ++i) RA::pin_raw(fa[0][i]);
+#pragma unroll
+            for (int fj = 0; fj < RB::NREAD; ++fj) RB::pin_raw(fb[0][fj]);
+            va[0] = RA::finish(fa[0][0], lane, false);
+#pragma unroll
+            for (int fj = 0; fj < FN; ++fj) {
+              vb_keep[fj] = RB::finish(fb[0][fj % RB::NREAD], lane, fj >= RB::NREAD);
+              acc[0][fj] = Mfma<T, MI>::run(vb_keep[fj], va[0], acc[0][fj]);
+            }
+#pragma unroll
+            for (int i = 1; i < HF; ++i) {
+              va[i] = RA::finish(fa[0][i], lane, false);
+              va_keep[i - 1] = RA::finish(fa[0][i - 1], lane, true);
+              pin(va_keep[i - 1]);          // made here, not where the second half uses it
+#pragma unroll
+              for (int fj = 0; fj < FN; ++fj) acc[i][fj] = Mfma<T, MI>::run(vb_keep[fj], va[i], acc[i][fj]);
+            }
+            va_keep[HF - 1] = RA::finish(fa[0][HF - 1], lane, true);
+            pin(va_keep[HF - 1]);
+            if constexpr (B_BOTH) {
+              __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);
+              __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+#pragma unroll
+              for (int fj = 1; fj < FN; ++fj) {
+                __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+              }
+            } else {
+              __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
+              __builtin_amdgcn_sched_group_barrier(0x8, FN, 0);
+            }
+#pragma unroll
+            for (int i = 1; i < HF; ++i) {
+              __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);
+              __builtin_amdgcn_sched_group_barrier(0x8, FN, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
+            if constexpr (ks + 1 < Cfg::KSTEPS) load_both(std::integral_constant<int, ks + 1>{});
           } else {
-            wait_lgkmcnt<0>();                          // all LDS reads of this stage are complete before the next barrier
+#pragma unroll
+            for (int i = 0; i < HF; ++i)
+#pragma unroll
+              for (int fj = 0; fj < FN; ++fj) acc[HF + i][fj] = Mfma<T, MI>::run(vb_keep[fj], va_keep[i], acc[HF + i][fj]);
           }
-          compute(std::integral_constant<int, ks>{}, std::integral_constant<int, h>{});
         });
+        // (the last reads of the stage were waited for before its last MFMAs: complete before the next barrier)
+        return;
+      }
+      load_a_half(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
+      load_b(std::integral_constant<int, 0>{});
+      static_for<0, 2 * Cfg::KSTEPS>([&](auto u_c) {
+        constexpr int u = decltype(u_c)::value;
+        constexpr int ks = u / 2, h = u % 2;
+        if (issue) issue_part(u_c, std::integral_constant<int, 2 * Cfg::KSTEPS>{}, (kt + STAGES - 1) % STAGES);
+        if constexpr (h == 0) {
+          load_a_half(std::integral_constant<int, ks>{}, std::integral_constant<int, 1>{});
+          wait_lgkmcnt<OPS_AH>();                     // half 0 and B of this k-step have arrived
+        } else if constexpr (ks + 1 < Cfg::KSTEPS) {
+          load_a_half(std::integral_constant<int, ks + 1>{}, std::integral_constant<int, 0>{});
+          load_b(std::integral_constant<int, ks + 1>{});
+          wait_lgkmcnt<OPS_AH + OPS_B>();             // half 1 of this k-step has arrived
+        } else {
+          wait_lgkmcnt<0>();                          // all LDS reads of this stage are complete before the next barrier
+        }
+        compute(std::integral_constant<int, ks>{}, std::integral_constant<int, h>{});
+      });
+      }
+    };
+    if constexpr (Cfg::PEELED) {
+      // The tiles behind which another one sets out, without a branch but the loop's own; the last STAGES - 1 (and the one outside the
+      // pipeline, which sets out where the tile behind the last one would) in a loop of their own.  A wave that is alone on its
+      // SIMD pays some twenty clocks for a branch, and the loop over all tiles had one for each part of the DMA, two for the wait and two at its end.
+      // us, 'T','T': 64 x 64 x 1984 on one 64 x 64 tile 9.6 -> 8.0, 4096 x 64 x 4096 unsplit 17.8 -> 14.2, 1024^3 7.4 -> 6.9, 256 x 256 x 16384 on 128 x 128 tiles
+      // 118 -> 94; with two waves on a SIMD 3072^3 on 256 x 192 57.5 -> 53.3, 4096 x 4096 x 2048 on 256 x 256 66.1 -> 63.9.
+      int kt = 0;
+      for (; kt < KT - (STAGES - 1); ++kt) {
+        enter_stage(kt % STAGES);
+        wait_vmcnt<(STAGES - 2) * DPT>();      // tile kt has landed: at most the DMA of the STAGES-2 younger tiles is outstanding
+        block_barrier();                       // every wave's share of tile kt is in LDS; every wave is done with tile kt-1
+        multiply_tile(kt, std::true_type{});
+      }
+      for (const int first = kt; kt < KT; ++kt) {
+        enter_stage(kt % STAGES);
+        const int younger = KTI - 1 - kt;
+        if (STAGES > 2 && younger >= STAGES - 2) wait_vmcnt<(STAGES > 2 ? STAGES - 2 : 0) * DPT>();
+        else if (STAGES > 3 && younger >= STAGES - 3) wait_vmcnt<(STAGES > 3 ? STAGES - 3 : 0) * DPT>();
+        else wait_vmcnt<0>();
+        block_barrier();
+        if constexpr (TAIL_AHEAD) {
+          if (kt == first && KT >= STAGES - 1 && tail_k > 0) issue_tail(KT % STAGES, ga, gb);
+        }
+        multiply_tile(kt, std::false_type{});
+      }
+    } else
+    for (int kt = 0; kt < KT; ++kt) {
+      // tile kt has landed once at most the DMA of the STAGES-2 younger tiles is outstanding
+      if (kt + STAGES - 2 < KT) wait_vmcnt<(STAGES - 2) * DPT>(); else wait_vmcnt<0>();
+      block_barrier();   // every wave's share of tile kt is in LDS; every wave is done with tile kt-1
+      enter_stage(kt % STAGES);
+      const bool issue = (kt + STAGES - 1 < KT);
+      if constexpr (Cfg::SPLIT_A) {
+        multiply_tile(kt, issue);
         continue;
       }
       load_frags<0, Cfg::SYNC_FRAGS>(ra, rb, fa[0], fb[0]);
@@ -1951,12 +2050,18 @@ __global__ void __launch_bounds__(Cfg::THREADS) mfma_gemm_kernel(const GemmArgs 
   }
   if constexpr (Cfg::RAGGED_K_OK) {
     // --- the last K tile, when it is partial or has a chunk over the end of an operand (see tail_k above) ---------
-    // Outside the pipeline: every lane fetches its 16-byte chunks with coordinates clamped to valid ones -- a chunk
-    // that would reach past the last element of the operand is fetched from 1 .. 7 elements further back -- and
-    // then repairs its own chunks in LDS: shifted into place, values whose k is beyond K set to zero.  Then the
-    // k-steps that hold valid values are multiplied.  ga / gb stand at this tile: every earlier tile has been issued.
+    // Its k-steps that hold valid values.  ga / gb stand at this tile: every earlier tile has been issued.  (TAIL_AHEAD: in
+    // the stage behind the last tile of the loop, which was free when that tile's successor set out.)
     if (tail_k > 0) {
-      fetch_tail_tile(ga, gb);
+      if constexpr (TAIL_AHEAD) {
+        const int stage = KT % STAGES;
+        repair_tail(stage);
+        __syncthreads();
+        ra.set_stage(lds_base + (unsigned)stage * Cfg::STAGE_BYTES);
+        rb.set_stage(lds_base + (unsigned)stage * Cfg::STAGE_BYTES + GA::BYTES);
+      } else {
+        fetch_tail_tile(ga, gb);
+      }
       static_for<0, Cfg::KSTEPS>([&](auto ks_c) {
         constexpr int ks = decltype(ks_c)::value;
         if (ks * Cfg::KSTEP_K < tail_k) {
