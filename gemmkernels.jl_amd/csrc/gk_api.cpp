@@ -1275,6 +1275,105 @@ int gk_matmul_split_k(const gk_config* conf, const void* a, const void* b, const
   return gk_internal::launch_split_k(conf, a, b, c, d, transforms, epilogue, workspace, workspace_bytes, "the caller's workspace", stream);
 }
 
+}  // extern "C"
+
+namespace {
+
+// Slices of K of a Float32 / Float64 product: the number with the shortest estimated launch, in us per 1000 k by the workgroups of a CU, plus what
+// the slices cost (workspace and counter; measured in fpu_mfma_splitk.hip).  `chain`: what one chain takes on the instances that such a launch runs on unsplit.
+// Slices are taken where they are estimated a tenth faster than one chain.
+int fpu_slices(const gk::InstanceKey& key, int tiles, int K) {
+  const bool f64 = key.dtype == gk::DT_F64, large = key.BM == 64;
+  if ((large && f64) || tiles > (int)(kSplitCounterBytes / sizeof(unsigned))) return 1;
+  const double k = K * 1e-3;
+  auto per_cu = [&](int n) {
+    if (large) return n == 1 ? 23.5 : 18.3 * n;
+    return f64 ? (n == 1 ? 11.6 : 10.4 * n) : (n == 1 ? 9.0 : (n == 2 ? 14.5 : (n == 3 ? 20.0 : 6.2 * n)));
+  };
+  auto workgroups = [&](int slices) { return (tiles * slices + gk::kNumCUs - 1) / gk::kNumCUs; };
+  const int n1 = workgroups(1);
+  const double chain = k * (n1 > 1 ? per_cu(n1) : (large ? 22.0 : (f64 ? 11.2 : (K >= 512 ? 6.9 : 8.5))));
+  const int k_tiles = (K + 31) / 32;
+  int best = 1;
+  double least = 0.9 * chain;
+  for (int slices = 2; slices <= 32 && k_tiles >= 2 * slices; ++slices) {
+    const int n = workgroups(slices);
+    if (n > 8) break;
+    const double t = k / slices * per_cu(n) + 1.2 + 0.12 * slices + 0.35 * n + (large ? 1.5 : 0.0);
+    if (t < least) { least = t; best = slices; }
+  }
+  return best;
+}
+
+// How gk_matmul_sliced cuts the K of a launch (slices < 2: not at all), from its configuration, hooks and sizes alone.
+struct Sliced {
+  gk::FamilyFn fn = nullptr;
+  int slices = 1, per = 0;
+  size_t bytes = 0;
+};
+
+Sliced sliced_route(const gk::InstanceKey& key, const gk::GemmArgs& args) {
+  Sliced r;
+  if (args.a_kind == GK_LAYOUT_ZERO || args.b_kind == GK_LAYOUT_ZERO || args.K <= 0) return r;
+  const long long all = (long long)args.nbm * args.nbn;
+  if (all > (long long)(kSplitCounterBytes / sizeof(unsigned))) return r;
+  const int tiles = (int)all;
+  if (key.family == gk::FAMILY_FPU) {
+    if ((key.variant & ~2) != 0 || key.dtype != key.acc_dtype || (key.dtype != gk::DT_F32 && key.dtype != gk::DT_F64)) return r;
+    r.fn = gk::family_fpu_mfma_splitk;
+    r.slices = fpu_slices(key, tiles, args.K);
+  }
+  if (r.slices < 2) return r;
+  const int k_tiles = (args.K + key.BK - 1) / key.BK;
+  r.per = (k_tiles + r.slices - 1) / r.slices;
+  r.slices = (k_tiles + r.per - 1) / r.per;        // no empty slice: every slice arrives at its tile's counter
+  r.bytes = kSplitCounterBytes + (size_t)tiles * r.slices * key.BM * key.BN * (key.acc_dtype == gk::DT_F64 ? 8 : 4);
+  gk::InstanceInfo info;
+  hipError_t err = hipSuccess;
+  const long long lds_max = g_lds_override.load();
+  if (r.slices < 2 || !r.fn(key, args, dim3(1), nullptr, 0, &info, &err) || (lds_max > 0 && info.lds_bytes > lds_max)) r = Sliced();
+  return r;
+}
+
+}  // namespace
+
+extern "C" {
+
+int gk_sliced_workspace_size(const gk_config* conf, const gk_transforms* transforms, const gk_epilogue* epilogue, size_t* bytes) {
+  if (!conf || !bytes) return fail(GK_ERR_INVALID_ARGUMENT, "NULL argument");
+  *bytes = 0;
+  gk::InstanceKey key;
+  gk::InstanceInfo info;
+  // (what the launch refuses, or what no kernel is compiled for, the launch says)
+  if (validate_config(conf, GK_KERNEL_SINGLESTAGE, transforms, epilogue, &key, &info) != GK_OK) return GK_OK;
+  gk::GemmArgs args;
+  make_args(conf, nullptr, nullptr, nullptr, nullptr, transforms, epilogue, &args);
+  *bytes = sliced_route(key, args).bytes;
+  return GK_OK;
+}
+
+int gk_matmul_sliced(const gk_config* conf, const void* a, const void* b, const void* c, void* d, const gk_transforms* transforms,
+                     const gk_epilogue* epilogue, int32_t kernel, void* workspace, size_t workspace_bytes, void* stream) {
+  if (kernel == GK_KERNEL_SPLIT_K) return fail(GK_ERR_INVALID_ARGUMENT, "the K-split kernel has an entry point of its own: gk_matmul_split_k");
+  gk_internal::Launch L;
+  int rc = gk_internal::prepare_launch(conf, a, b, c, d, transforms, epilogue, kernel, nullptr, &L);
+  if (rc != GK_OK) return rc;
+  gk::FamilyFn fn = family_fn(L.key);
+  dim3 grid((unsigned)L.gx, (unsigned)L.gy);
+  const Sliced route = sliced_route(L.key, L.args);
+  if (route.slices > 1 && workspace && workspace_bytes >= route.bytes && ((uintptr_t)workspace & 15u) == 0) {
+    L.args.k_steps = route.per; L.args.k_slices = route.slices;
+    L.args.ws_counters = (unsigned*)workspace;
+    L.args.ws_partials = (char*)workspace + kSplitCounterBytes;
+    grid.z = (unsigned)route.slices;
+    fn = route.fn;
+  }
+  hipError_t err = hipSuccess;
+  if (!fn || !fn(L.key, L.args, grid, (hipStream_t)stream, 1, &L.info, &err)) return fail(GK_ERR_UNSUPPORTED, "no compiled kernel instance");
+  if (err != hipSuccess) return fail(GK_ERR_HIP, "HIP launch of %s failed: %s", L.info.name, hipGetErrorString(err));
+  return GK_OK;
+}
+
 int gk_stream_capture(void* stream, int32_t* capturing, uint64_t* id) {
   if (!capturing || !id) return fail(GK_ERR_INVALID_ARGUMENT, "NULL argument");
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;

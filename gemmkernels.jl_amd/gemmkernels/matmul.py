@@ -108,6 +108,16 @@ def _split_k_bytes(conf_c) -> int:
     return need.value
 
 
+def _sliced_bytes(conf_c, trans, epi) -> int:
+    """Workspace of a launch that runs in slices of K (``gk_matmul_sliced``), 0 of any other."""
+    need = ctypes.c_size_t()
+    rc = _lib.lib().gk_sliced_workspace_size(ctypes.byref(conf_c), ctypes.byref(trans) if trans is not None else None,
+                                             ctypes.byref(epi) if epi is not None else None, ctypes.byref(need))
+    if rc != _lib.GK_OK:
+        _raise(rc)
+    return need.value
+
+
 def _span(buf):
     """What the library is told of a workspace: its address and size."""
     return (int(buf.data_ptr()), int(buf.numel())) if buf is not None else (0, 0)
@@ -279,9 +289,9 @@ class Plan:
     other means while it is in use.  For loops that launch the same GEMM many times, where the
     microseconds a general ``matmul`` call spends on lowering would rival the kernel itself."""
 
-    __slots__ = ("_fn", "_conf", "_trans", "_epi", "_args", "_keep", "_split_k", "_as_given", "d", "kernel_names")
+    __slots__ = ("_fn", "_conf", "_trans", "_epi", "_args", "_keep", "_split_k", "_sliced", "_as_given", "d", "kernel_names")
 
-    def __init__(self, conf: Config, a, b, c, d, transforms: dict, epilogue, kernel, specialized=None):
+    def __init__(self, conf: Config, a, b, c, d, transforms: dict, epilogue, kernel, specialized=None, slices=False):
         if specialized is None and any(t.expr is not None for t in transforms.values()):
             specialized = SpecializedKernel(conf, transforms)       # expression hooks: a run-time compiled kernel
         lds = (_leading_dim(a, conf.global_a_layout), _leading_dim(b, conf.global_b_layout),
@@ -294,7 +304,7 @@ class Plan:
         if larger is not None:
             self._as_given, self._conf = self._conf, _lib.gk_config.from_buffer_copy(larger.to_c(*lds))
         self._epi = None
-        self._split_k = False
+        self._split_k, self._sliced = False, 0
         if epilogue.kind != Epilogue.DEFAULT:
             self._epi = _lib.gk_epilogue()
             self._epi.kind = epilogue.kind
@@ -309,7 +319,8 @@ class Plan:
                           ctypes.byref(self._trans) if self._trans is not None else None, epi_ref)
             self._split_k = True
         else:
-            self._fn = _lib.lib().gk_matmul
+            self._sliced = _sliced_bytes(self._conf, self._trans, self._epi) if slices else 0
+            self._fn = _lib.lib().gk_matmul_sliced if self._sliced else _lib.lib().gk_matmul
             self._args = (ctypes.byref(self._conf), _ptr(a), _ptr(b), _ptr(c), _ptr(d),
                           ctypes.byref(self._trans) if self._trans is not None else None, epi_ref, kernel.code)
         self._keep = (a, b, c, d, epilogue, specialized)
@@ -324,9 +335,13 @@ class Plan:
             if rc != _lib.GK_OK:
                 _raise(rc)
             return self.d
-        rc = self._fn(*self._args, stream)
-        if rc != _lib.GK_OK and self._as_given is not None:
-            rc = self._fn(ctypes.byref(self._as_given), *self._args[1:], stream)
+        if self._sliced:
+            workspace = _workspace(self._sliced, stream)
+            rc = self._fn(*self._args, *_span(workspace), stream)
+        else:
+            rc = self._fn(*self._args, stream)
+            if rc != _lib.GK_OK and self._as_given is not None:
+                rc = self._fn(ctypes.byref(self._as_given), *self._args[1:], stream)
         if rc != _lib.GK_OK:
             _raise(rc)
         return self.d
@@ -571,7 +586,9 @@ def _single_plan(C, tA: bool, tB: bool, A, B, alpha, beta, wmma=None) -> Plan:
         tiles = -(-ms.M // bs.M) * -(-ms.N // bs.N)
         if bs == split_k_block_shape(ms.M, ms.N, ms.K, 0, factor) or tiles <= 128 and ms.K >= 2048:
             kernel = Kernel.matmul_split_k
-    p = plan(conf, A, B, C, C, transform_shared_to_regs_a=ta, transform_shared_to_regs_c=tc, kernel=kernel)
+    # (floating-point FPUOp: the library takes slices of K where one chain per output would leave the chip idle, gk_matmul_sliced)
+    p = Plan(conf, A, B, C, C, _collect({**dict.fromkeys(_HOOKS), "transform_shared_to_regs_a": ta, "transform_shared_to_regs_c": tc}),
+             _DEFAULT_EPILOGUE, kernel, slices=conf.operator.kind == Operator.FPU)
     p.kernel_names = (kernel_name(conf, kernel, dict(transform_shared_to_regs_a=ta, transform_shared_to_regs_c=tc)),)
     return p
 
@@ -676,7 +693,7 @@ class _MulLaunch:
     stream and from any thread (nothing in it is written after it is made).  Lowering the same call again took 22 us of
     interpreter time, the whole of a small product: mul! at 256^3 in Float32 takes 5 us on the device."""
 
-    __slots__ = ("_fn", "_conf", "_trans", "_conf_ref", "_trans_ref", "_code", "_workspace")
+    __slots__ = ("_fn", "_conf", "_trans", "_conf_ref", "_trans_ref", "_code", "_workspace", "_sliced")
 
     def __init__(self, p: Plan):
         self._conf, self._trans = p._conf, p._trans         # (own the memory that the references point to)
@@ -685,9 +702,13 @@ class _MulLaunch:
         self._fn = p._fn
         self._workspace = _split_k_bytes(self._conf) if p._split_k else None
         self._code = None if p._split_k else p._args[-1]
+        self._sliced = p._sliced
 
     def __call__(self, a: int, b: int, c: int, stream: int) -> None:
-        if self._workspace is None:
+        if self._sliced:
+            workspace = _workspace(self._sliced, stream)
+            rc = self._fn(self._conf_ref, a, b, c, c, self._trans_ref, None, self._code, *_span(workspace), stream)
+        elif self._workspace is None:
             rc = self._fn(self._conf_ref, a, b, c, c, self._trans_ref, None, self._code, stream)
         else:
             workspace = _workspace(self._workspace, stream)
