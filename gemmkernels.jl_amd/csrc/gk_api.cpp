@@ -1308,12 +1308,14 @@ int fpu_slices(const gk::InstanceKey& key, int tiles, int K) {
 // How gk_matmul_sliced cuts the K of a launch (slices < 2: not at all), from its configuration, hooks and sizes alone.
 struct Sliced {
   gk::FamilyFn fn = nullptr;
+  gk::InstanceKey key{};
   int slices = 1, per = 0;
   size_t bytes = 0;
 };
 
-Sliced sliced_route(const gk::InstanceKey& key, const gk::GemmArgs& args) {
+Sliced sliced_route(const gk::InstanceKey& as_asked, const gk::GemmArgs& args) {
   Sliced r;
+  gk::InstanceKey& key = r.key = as_asked;
   if (args.a_kind == GK_LAYOUT_ZERO || args.b_kind == GK_LAYOUT_ZERO || args.K <= 0) return r;
   const long long all = (long long)args.nbm * args.nbn;
   if (all > (long long)(kSplitCounterBytes / sizeof(unsigned))) return r;
@@ -1322,6 +1324,16 @@ Sliced sliced_route(const gk::InstanceKey& key, const gk::GemmArgs& args) {
     if ((key.variant & ~2) != 0 || key.dtype != key.acc_dtype || (key.dtype != gk::DT_F32 && key.dtype != gk::DT_F64)) return r;
     r.fn = gk::family_fpu_mfma_splitk;
     r.slices = fpu_slices(key, tiles, args.K);
+  } else if ((key.family == gk::FAMILY_MFMA || key.family == gk::FAMILY_GETT) && key.BM == 64 && key.BN == 64) {
+    // (BLOCK_K = 32 where it runs on K tiles of 64 unsplit as well)
+    if (key.family == gk::FAMILY_MFMA && key.BK == 32 && args.K % 64 == 0 && deep_instance(key, args)) key.BK = 64;
+    if (key.BK != 64 || key.waves_m != 2 || key.waves_n != 2) return r;
+    // (us, one chain with the branches it had then -> slices: plans 704 x 320 x 5056 (55 tiles) 20.7 -> 11.1, 448 x 960 x 4544 (105) 20.8 -> 13.9, 384 x 448 x 1984 (42) 11.9 -> 9.2,
+    // 256 x 1536 x 2304 (96) 11.9 -> 9.3; contractions of M x N x K = 640 x 448 x 4096 (70) 24.2 -> 15.6, 640 x 1088 x 4096 (170) 24.2 -> 17.8, 1536 x 768 x 4096 (288, one chain) 29.6 -> 24.6.
+    // The lines are those of mul!, split_k_block_shape in config.py, less two slices of 171 to 256 tiles, which are level there.)
+    r.fn = key.family == gk::FAMILY_MFMA ? gk::family_mfma_splitk : gk::family_mfma_splitk_gett;
+    if (args.K >= (tiles <= 64 ? 1280 : (tiles <= 128 ? 2048 : 3000)) && tiles <= 170)
+      r.slices = split_k_slices(tiles, (args.K + 63) / 64, gk_shape{64, 64, 64}, key.fused == 1);
   }
   if (r.slices < 2) return r;
   const int k_tiles = (args.K + key.BK - 1) / key.BK;
@@ -1361,15 +1373,17 @@ int gk_matmul_sliced(const gk_config* conf, const void* a, const void* b, const 
   gk::FamilyFn fn = family_fn(L.key);
   dim3 grid((unsigned)L.gx, (unsigned)L.gy);
   const Sliced route = sliced_route(L.key, L.args);
+  gk::InstanceKey key = L.key;
   if (route.slices > 1 && workspace && workspace_bytes >= route.bytes && ((uintptr_t)workspace & 15u) == 0) {
     L.args.k_steps = route.per; L.args.k_slices = route.slices;
     L.args.ws_counters = (unsigned*)workspace;
     L.args.ws_partials = (char*)workspace + kSplitCounterBytes;
     grid.z = (unsigned)route.slices;
     fn = route.fn;
+    key = route.key;
   }
   hipError_t err = hipSuccess;
-  if (!fn || !fn(L.key, L.args, grid, (hipStream_t)stream, 1, &L.info, &err)) return fail(GK_ERR_UNSUPPORTED, "no compiled kernel instance");
+  if (!fn || !fn(key, L.args, grid, (hipStream_t)stream, 1, &L.info, &err)) return fail(GK_ERR_UNSUPPORTED, "no compiled kernel instance");
   if (err != hipSuccess) return fail(GK_ERR_HIP, "HIP launch of %s failed: %s", L.info.name, hipGetErrorString(err));
   return GK_OK;
 }

@@ -604,7 +604,7 @@ struct MfmaGemmConfig {
   static_assert((STAGES - 2) * DMA_PER_TILE <= 63, "vmcnt is a 6-bit counter");
   static_assert(FM * FN > 0, "empty wave tile");
   static_assert(!GETT || FIX == FIX_NONE, "contractions are real");
-  static_assert(!SPLITK || (!GETT && FIX == FIX_NONE), "K-split instances are plain real GEMMs");
+  static_assert(!SPLITK || FIX == FIX_NONE, "K-split instances are real");
   static_assert(!PLANAR || (MI_ == 16 && !opk_complex_k(A_KIND_) && !opk_complex_k(B_KIND_)), "planar complex: 16-row blocks on plain real planes");
   static_assert(!COMPLEX || FUSE_ == 0 || FUSE_ == 3, "complex products take hooks on C and D only");
   static_assert(!PAIR || (MI_ == 16 && A_KIND_ != OPK_KMAJOR && B_KIND_ != OPK_KMAJOR),

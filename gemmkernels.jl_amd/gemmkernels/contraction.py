@@ -167,7 +167,7 @@ def plan(spec: str, a, b, d, c=None, ab_type: Optional[DType] = None, cd_type: O
             reasons.append(("B as the A operand: " if swapped else "") + info)
             continue
         x, y = (b, a) if swapped else (a, b)
-        launch = Plan(conf, x, y, c, d, {k: _IDENTITY for k in _HOOKS}, _DEFAULT_EPILOGUE, Kernel.matmul_pipelined)
+        launch = Plan(conf, x, y, c, d, {k: _IDENTITY for k in _HOOKS}, _DEFAULT_EPILOGUE, Kernel.matmul_pipelined, slices=True)
         ms = conf.matmul_shape
         return ContractionPlan(spec, swapped, groups, conf, (ms.M, ms.N, ms.K), info, launch)
     raise ConfigError("contraction " + spec + " does not map onto the GEMM kernel: " + "; ".join(reasons))
@@ -193,17 +193,22 @@ class _Launch:
     the planner arrived at, no address and no tensor; nothing in it is written after it is made, and the library checks
     the addresses at every launch.  Planning again took 70 us of interpreter time a call, several times the kernel of a small contraction."""
 
-    __slots__ = ("_conf", "_conf_ref", "_swapped", "_fn", "_code")
+    __slots__ = ("_conf", "_conf_ref", "_swapped", "_fn", "_code", "_sliced")
 
     def __init__(self, p: ContractionPlan):
         self._conf = p._launch._conf                      # (owns the memory that the reference points to)
         self._conf_ref = ctypes.byref(self._conf)
         self._swapped = p.swapped
-        self._fn, self._code = p._launch._fn, p._launch._args[-1]
+        self._fn, self._code, self._sliced = p._launch._fn, p._launch._args[-1], p._launch._sliced
 
     def __call__(self, a: int, b: int, c: Optional[int], d: int, stream: int) -> None:
         x, y = (b, a) if self._swapped else (a, b)
-        rc = self._fn(self._conf_ref, x, y, c, d, None, None, self._code, stream)
+        if self._sliced:
+            from .matmul import _span, _workspace
+            workspace = _workspace(self._sliced, stream)
+            rc = self._fn(self._conf_ref, x, y, c, d, None, None, self._code, *_span(workspace), stream)
+        else:
+            rc = self._fn(self._conf_ref, x, y, c, d, None, None, self._code, stream)
         if rc != _lib.GK_OK:
             from .matmul import _raise
             _raise(rc)

@@ -319,7 +319,7 @@ class Plan:
                           ctypes.byref(self._trans) if self._trans is not None else None, epi_ref)
             self._split_k = True
         else:
-            self._sliced = _sliced_bytes(self._conf, self._trans, self._epi) if slices else 0
+            self._sliced = _sliced_bytes(self._conf, self._trans, self._epi) if slices and larger is None else 0
             self._fn = _lib.lib().gk_matmul_sliced if self._sliced else _lib.lib().gk_matmul
             self._args = (ctypes.byref(self._conf), _ptr(a), _ptr(b), _ptr(c), _ptr(d),
                           ctypes.byref(self._trans) if self._trans is not None else None, epi_ref, kernel.code)
@@ -369,7 +369,8 @@ def plan(conf: Config, a, b, c, d, *,
                                transform_shared_to_regs_b=transform_shared_to_regs_b,
                                transform_shared_to_regs_c=transform_shared_to_regs_c,
                                transform_regs_to_shared_d=transform_regs_to_shared_d))
-    return Plan(conf, a, b, c, d, transforms, _DEFAULT_EPILOGUE if epilogue is None else epilogue, kernel)
+    # (FPUOp: a configured launch is one fma chain per output, whatever its sizes)
+    return Plan(conf, a, b, c, d, transforms, _DEFAULT_EPILOGUE if epilogue is None else epilogue, kernel, slices=conf.operator.kind == Operator.MFMA)
 
 
 def matmul(conf: Config, a, b, c, d, *,
@@ -418,7 +419,17 @@ def matmul(conf: Config, a, b, c, d, *,
         larger = _launched_as(conf, a, b, c, d, ctrans is not None or cepi is not None)
         rc = _lib.lib().gk_matmul(ctypes.byref(larger.to_c(*lds)), *args) if larger is not None else _lib.GK_ERR_UNSUPPORTED
         if rc != _lib.GK_OK:
-            rc = _lib.lib().gk_matmul(ctypes.byref(cconf), *args)
+            need = 0
+            if larger is None and ctrans is None and cepi is None and conf.operator.kind == Operator.MFMA:
+                known = conf.__dict__.setdefault("_slices_of", {})           # (a Config is immutable once built)
+                need = known.get(lds)
+                if need is None:
+                    need = known[lds] = _sliced_bytes(cconf, None, None)
+            if need:
+                workspace = _workspace(need, stream)
+                rc = _lib.lib().gk_matmul_sliced(ctypes.byref(cconf), *args[:-1], *_span(workspace), stream)
+            else:
+                rc = _lib.lib().gk_matmul(ctypes.byref(cconf), *args)
     if rc != _lib.GK_OK:
         _raise(rc)
     return d

@@ -290,8 +290,9 @@ int gk_matmul_split_k(const gk_config* conf, const void* a, const void* b, const
                       size_t workspace_bytes, void* stream);
 
 /* gk_matmul for a caller that brings a workspace (as gk_matmul_split_k takes it, and may share it with) and leaves the order of the
- * sums to the library: the same launch, in slices of K on its own tile where that is estimated to be faster -- Float32 and Float64 products of FPUOp with few
- * output tiles and a long K, hooks of at most one scale on A, on B and on C.  The result does not change from run to run; it
+ * sums to the library: the same launch, in slices of K on its own tile where that is estimated to be faster: products with few
+ * output tiles and a long K, Float32 and Float64 ones of FPUOp with hooks of at most one scale on A, on B and on C, real MFMA ones on 64 x 64 x 64
+ * tiles with a K-split instance, contractions on that tile without hooks.  The result does not change from run to run; it
  * differs from that of gk_matmul, which is one chain over K, in the last bits.  gk_sliced_workspace_size gives the workspace the
  * launch needs, decided from the configuration, the hooks and the epilogue alone; 0: it is gk_matmul's launch, as it is with a workspace that is NULL or too small. */
 int gk_sliced_workspace_size(const gk_config* conf, const gk_transforms* transforms, const gk_epilogue* epilogue, size_t* bytes);
