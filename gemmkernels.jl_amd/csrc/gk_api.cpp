@@ -10,6 +10,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <new>
 #include <string>
 
 #include "gk_internal.hpp"
@@ -40,6 +41,7 @@ using gk_internal::fail;
 
 std::atomic<long long> g_lds_override{0};
 std::atomic<int> g_threads_override{0};
+std::atomic<unsigned long long> g_limits_set{0};       // how often the limits were set: a prepared launch is checked against those it was prepared under
 
 void device_limits(long long* lds, int* threads) {
   long long l = g_lds_override.load();
@@ -887,6 +889,7 @@ const char* gk_status_string(int status) {
 int gk_set_device_limits(int64_t lds_bytes, int32_t max_threads) {
   g_lds_override.store(lds_bytes > 0 ? lds_bytes : 0);
   g_threads_override.store(max_threads > 0 ? max_threads : 0);
+  g_limits_set.fetch_add(1);
   return GK_OK;
 }
 
@@ -1279,6 +1282,13 @@ int gk_matmul_split_k(const gk_config* conf, const void* a, const void* b, const
 
 namespace {
 
+// A launch that has passed every check but those of its addresses (gk_prepare).
+struct Prepared {
+  gk_internal::Launch launch;
+  gk::FamilyFn fn;
+  unsigned long long limits;
+};
+
 // Slices of K of a Float32 / Float64 product: the number with the shortest estimated launch, in us per 1000 k by the workgroups of a CU, plus what
 // the slices cost (workspace and counter; measured in fpu_mfma_splitk.hip).  `chain`: what one chain takes on the instances that such a launch runs on unsplit.
 // Slices are taken where they are estimated a tenth faster than one chain.
@@ -1387,6 +1397,41 @@ int gk_matmul_sliced(const gk_config* conf, const void* a, const void* b, const 
   if (err != hipSuccess) return fail(GK_ERR_HIP, "HIP launch of %s failed: %s", L.info.name, hipGetErrorString(err));
   return GK_OK;
 }
+
+int gk_prepare(const gk_config* conf, const gk_transforms* transforms, const gk_epilogue* epilogue, int32_t kernel, void** prepared) {
+  if (!prepared) return fail(GK_ERR_INVALID_ARGUMENT, "NULL argument");
+  *prepared = nullptr;
+  if (kernel == GK_KERNEL_SPLIT_K) return fail(GK_ERR_INVALID_ARGUMENT, "a K-split launch needs a workspace and is not prepared");
+  Prepared* p = new (std::nothrow) Prepared();
+  if (!p) return fail(GK_ERR_INVALID_ARGUMENT, "out of memory");
+  p->limits = g_limits_set.load();
+  void* aligned = (void*)(uintptr_t)4096;               // (any address on a 16-byte boundary: gk_run asks for those)
+  int rc = gk_internal::prepare_launch(conf, aligned, aligned, aligned, aligned, transforms, epilogue, kernel, nullptr, &p->launch);
+  hipError_t err = hipSuccess;
+  if (rc == GK_OK) {
+    p->fn = family_fn(p->launch.key);
+    if (!p->fn || !p->fn(p->launch.key, p->launch.args, dim3(1), nullptr, 0, &p->launch.info, &err)) rc = fail(GK_ERR_UNSUPPORTED, "no compiled kernel instance");
+  }
+  if (rc != GK_OK) { delete p; return rc; }
+  *prepared = p;
+  return GK_OK;
+}
+
+int gk_run(const void* prepared, const void* a, const void* b, const void* c, void* d, void* stream) {
+  const Prepared* p = (const Prepared*)prepared;
+  if (!p || !a || !b || !d || (p->launch.args.c_mode != 0 && !c)) return fail(GK_ERR_INVALID_ARGUMENT, "NULL argument");
+  if ((((uintptr_t)a | (uintptr_t)b | (uintptr_t)c | (uintptr_t)d) & 15u) != 0) return fail(GK_ERR_ALIGNMENT, "a prepared launch takes operands on 16-byte boundaries");
+  if (p->limits != g_limits_set.load()) return fail(GK_ERR_UNSUPPORTED, "prepared under other device limits");
+  gk::GemmArgs args = p->launch.args;
+  args.a = a; args.b = b; args.c = c; args.d = d;
+  gk::InstanceInfo info;
+  hipError_t err = hipSuccess;
+  if (!p->fn(p->launch.key, args, dim3((unsigned)p->launch.gx, (unsigned)p->launch.gy), (hipStream_t)stream, 1, &info, &err)) return fail(GK_ERR_UNSUPPORTED, "no compiled kernel instance");
+  if (err != hipSuccess) return fail(GK_ERR_HIP, "HIP launch of %s failed: %s", info.name, hipGetErrorString(err));
+  return GK_OK;
+}
+
+void gk_prepared_free(void* prepared) { delete (Prepared*)prepared; }
 
 int gk_stream_capture(void* stream, int32_t* capturing, uint64_t* id) {
   if (!capturing || !id) return fail(GK_ERR_INVALID_ARGUMENT, "NULL argument");

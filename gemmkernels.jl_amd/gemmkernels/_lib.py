@@ -116,6 +116,10 @@ _SIGNATURES = {
     "gk_matmul_sliced": (ctypes.c_int, [ctypes.POINTER(gk_config), ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                                         ctypes.POINTER(gk_transforms), ctypes.POINTER(gk_epilogue), ctypes.c_int32, ctypes.c_void_p,
                                         ctypes.c_size_t, ctypes.c_void_p]),
+    "gk_prepare": (ctypes.c_int, [ctypes.POINTER(gk_config), ctypes.POINTER(gk_transforms), ctypes.POINTER(gk_epilogue), ctypes.c_int32,
+                                  ctypes.POINTER(ctypes.c_void_p)]),
+    "gk_run": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]),
+    "gk_prepared_free": (None, [ctypes.c_void_p]),
     "gk_stream_capture": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_uint64)]),
     "gk_split_k_noalloc_capacity": (ctypes.c_size_t, []),
     "gk_matmul_split_k_noalloc": (ctypes.c_int, [ctypes.POINTER(gk_config), ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,

@@ -1,0 +1,49 @@
+"""The module between torch tensors and the library (csrc/gk_torch.cpp): what a call that was seen before does, in C++.  ``load()`` gives it bound to the library, or
+None where it was not built for this interpreter and its torch; the package's own Python then does the same."""
+from __future__ import annotations
+
+import ctypes
+import importlib.util
+import os
+
+from . import _lib
+
+_PATH = os.path.join(os.path.dirname(_lib.LIB_PATH), "gk_torch.so")
+class Prepared:
+    """A launch that has passed every check but those of its addresses (gk_prepare), or one without a handle where the library makes none."""
+
+    __slots__ = ("handle", "_free", "_keep")
+
+    def __init__(self, conf_c, trans, epi, code: int, keep=None):
+        handle = ctypes.c_void_p()
+        lib = _lib.lib()
+        rc = lib.gk_prepare(ctypes.byref(conf_c), ctypes.byref(trans) if trans is not None else None, ctypes.byref(epi) if epi is not None else None, code, ctypes.byref(handle))
+        self.handle = handle.value if rc == _lib.GK_OK else None
+        self._free, self._keep = lib.gk_prepared_free, keep          # (keep: the bias of the epilogue)
+
+    def __del__(self):
+        if getattr(self, "handle", None):
+            self._free(self.handle)
+            self.handle = None
+
+
+_module = None
+_tried = False
+
+
+def load():
+    global _module, _tried
+    if not _tried:
+        lib = _lib.lib()
+        _tried = True
+        if os.path.exists(_PATH):
+            try:
+                spec = importlib.util.spec_from_file_location("gk_torch", _PATH)
+                module = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(module)
+            except ImportError:
+                return None
+            address = lambda fn: ctypes.cast(fn, ctypes.c_void_p).value
+            module.bind(*(address(fn) for fn in (lib.gk_matmul, lib.gk_matmul_sliced, lib.gk_matmul_split_k, lib.gk_stream_capture, lib.gk_run)))
+            _module = module
+    return _module

@@ -25,6 +25,7 @@ from . import _lib
 from . import kernel as Kernel
 from . import layout as Layout
 from . import operator as Operator
+from ._native import load as native
 from .config import _GETT_TILES, _mfma_cost, get_config
 from .dtypes import BFloat16, DType, Float16, Float32
 from .errors import ConfigError
@@ -184,7 +185,8 @@ def contract(spec: str, a, b, d, c=None, stream=None):
         if len(_launches) >= _LAUNCHES_MAX:
             _launches.clear()
         _launches[key] = launch
-    launch(a.data_ptr(), b.data_ptr(), None if c is None else c.data_ptr(), d.data_ptr(), _current_stream() if stream is None else int(stream))
+    if stream is not None or launch.run is None or not launch.run(launch.handle, *((b, a) if launch._swapped else (a, b)), c, d):
+        launch(a.data_ptr(), b.data_ptr(), None if c is None else c.data_ptr(), d.data_ptr(), _current_stream() if stream is None else int(stream))
     return d
 
 
@@ -193,13 +195,17 @@ class _Launch:
     the planner arrived at, no address and no tensor; nothing in it is written after it is made, and the library checks
     the addresses at every launch.  Planning again took 70 us of interpreter time a call, several times the kernel of a small contraction."""
 
-    __slots__ = ("_conf", "_conf_ref", "_swapped", "_fn", "_code", "_sliced")
+    __slots__ = ("_conf", "_conf_ref", "_swapped", "_fn", "_code", "_sliced", "_prepared", "handle", "run")
 
     def __init__(self, p: ContractionPlan):
         self._conf = p._launch._conf                      # (owns the memory that the reference points to)
         self._conf_ref = ctypes.byref(self._conf)
         self._swapped = p.swapped
         self._fn, self._code, self._sliced = p._launch._fn, p._launch._args[-1], p._launch._sliced
+        # (the launch checked once and gk_torch's way to it, for operands on 16-byte boundaries)
+        self._prepared = p._launch._prepared
+        self.handle = self._prepared.handle if self._prepared is not None else None
+        self.run = native().run if self.handle is not None else None
 
     def __call__(self, a: int, b: int, c: Optional[int], d: int, stream: int) -> None:
         x, y = (b, a) if self._swapped else (a, b)
@@ -208,7 +214,8 @@ class _Launch:
             workspace = _workspace(self._sliced, stream)
             rc = self._fn(self._conf_ref, x, y, c, d, None, None, self._code, *_span(workspace), stream)
         else:
-            rc = self._fn(self._conf_ref, x, y, c, d, None, None, self._code, stream)
+            from .matmul import _gk_matmul
+            rc = _gk_matmul(self._conf, x, y, c, d, None, None, self._code, stream)
         if rc != _lib.GK_OK:
             from .matmul import _raise
             _raise(rc)

@@ -24,6 +24,7 @@ from . import transform as Transform
 from .config import _MFMA_TILE_COST, Config, _mfma_cost, default_block_shape, get_config as _get_config, larger_tile, split_k_block_shape
 from .dtypes import BFloat16, DType, Float16, Float32, Float64, from_torch, promote_type
 from .errors import ConfigError, DimensionMismatch
+from ._native import Prepared, load as load_native
 from .tiling import NT
 
 _HOOKS = ("transform_global_to_shared_a", "transform_global_to_shared_b", "transform_global_to_shared_c",
@@ -78,10 +79,23 @@ def _leading_dim(x, layout) -> int:
 def _current_stream() -> int:
     """Raw handle of torch's current HIP stream."""
     import torch
+    if _native is not None:
+        return _native.current_stream()
     try:
         return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
     except AttributeError:
         return torch.cuda.current_stream().cuda_stream
+
+
+_native = None              # the module gk_torch, once a call has been made (None as well where it is not built)
+
+
+def _gk_matmul(conf_c, a, b, c, d, trans, epi, code: int, stream: int) -> int:
+    """gk_matmul on descriptors and addresses; its status."""
+    if _native is not None:
+        return _native.matmul(ctypes.addressof(conf_c), a, b, c, d, None if trans is None else ctypes.addressof(trans), None if epi is None else ctypes.addressof(epi), code, stream)
+    return _lib.lib().gk_matmul(ctypes.byref(conf_c), a, b, c, d, ctypes.byref(trans) if trans is not None else None,
+                                ctypes.byref(epi) if epi is not None else None, code, stream)
 
 
 _workspaces = {}            # (device, stream) -> buffer of eager launches
@@ -185,6 +199,8 @@ def _workspace(need: int, stream: int):
     if buf is None or buf.numel() < need:
         with _on(stream):
             buf = _workspaces[key] = torch.zeros(max(need, 1 << 20), dtype=torch.uint8, device="cuda")
+        if _native is not None:
+            _native.use_workspace(key[0], stream, buf.data_ptr(), buf.numel(), buf)
     return buf
 
 
@@ -289,7 +305,7 @@ class Plan:
     other means while it is in use.  For loops that launch the same GEMM many times, where the
     microseconds a general ``matmul`` call spends on lowering would rival the kernel itself."""
 
-    __slots__ = ("_fn", "_conf", "_trans", "_epi", "_args", "_keep", "_split_k", "_sliced", "_as_given", "d", "kernel_names")
+    __slots__ = ("_fn", "_conf", "_trans", "_epi", "_args", "_keep", "_split_k", "_sliced", "_as_given", "_direct", "_prepared", "d", "kernel_names")
 
     def __init__(self, conf: Config, a, b, c, d, transforms: dict, epilogue, kernel, specialized=None, slices=False):
         if specialized is None and any(t.expr is not None for t in transforms.values()):
@@ -324,6 +340,11 @@ class Plan:
             self._args = (ctypes.byref(self._conf), _ptr(a), _ptr(b), _ptr(c), _ptr(d),
                           ctypes.byref(self._trans) if self._trans is not None else None, epi_ref, kernel.code)
         self._keep = (a, b, c, d, epilogue, specialized)
+        self._direct = self._prepared = None
+        if _load_native() is not None and specialized is None and not self._split_k and not self._sliced:
+            self._prepared = Prepared(self._conf, self._trans, self._epi, kernel.code)
+            if self._prepared.handle is not None:
+                self._direct = (self._prepared.handle, *self._args[1:5])
         self.d = d
         self.kernel_names = ()      # filled in by the BLAS-level front end
 
@@ -339,6 +360,8 @@ class Plan:
             workspace = _workspace(self._sliced, stream)
             rc = self._fn(*self._args, *_span(workspace), stream)
         else:
+            if self._direct is not None and _native.run_at(*self._direct, stream) == _lib.GK_OK:
+                return self.d
             rc = self._fn(*self._args, stream)
             if rc != _lib.GK_OK and self._as_given is not None:
                 rc = self._fn(ctypes.byref(self._as_given), *self._args[1:], stream)
@@ -373,6 +396,24 @@ def plan(conf: Config, a, b, c, d, *,
     return Plan(conf, a, b, c, d, transforms, _DEFAULT_EPILOGUE if epilogue is None else epilogue, kernel, slices=conf.operator.kind == Operator.MFMA)
 
 
+_PREPARED_MAX = 64
+
+
+def _prepare(conf: Config, cconf, lds, kernel) -> None:
+    """Keeps the launch that ``matmul`` made for operands of these leading dimensions (no address) with its configuration."""
+    kept = conf.__dict__.get("_prepared")
+    if _load_native() is None or kept is not None and (lds, kernel) in kept:
+        return
+    made = Prepared(cconf, None, None, kernel.code)
+    if made.handle is None:
+        return
+    if kept is None or len(kept) > _PREPARED_MAX:
+        forms = {**dict.fromkeys(_NO_LD, 0), **dict.fromkeys(_INTERLEAVED, 2), **dict.fromkeys(_SPLIT, 3)}
+        kept = {"forms": tuple(forms.get(l.kind, 1) for l in (conf.global_a_layout, conf.global_b_layout, conf.global_c_layout, conf.global_d_layout))}
+    kept[(lds, kernel)] = made
+    conf.__dict__["_prepared"] = kept
+
+
 def matmul(conf: Config, a, b, c, d, *,
            transform_global_to_shared_a=None, transform_global_to_shared_b=None,
            transform_global_to_shared_c=None, transform_shared_to_global_d=None,
@@ -381,6 +422,16 @@ def matmul(conf: Config, a, b, c, d, *,
            epilogue=None, kernel=Kernel.matmul_singlestage, stream=None):
     """reference src/matmul.jl:7-44: launch geometry, checks (ConfigError) and the asynchronous
     launch on the current stream.  Same positional and keyword arguments as the reference."""
+    plain = (epilogue is None and transform_global_to_shared_a is None and transform_global_to_shared_b is None and
+             transform_global_to_shared_c is None and transform_shared_to_global_d is None and transform_shared_to_regs_a is None and
+             transform_shared_to_regs_b is None and transform_shared_to_regs_c is None and transform_regs_to_shared_d is None)
+    prepared = conf.__dict__.get("_prepared") if plain else None
+    if prepared is not None and stream is None:
+        # (a launch of these leading dimensions was made before: a Config is immutable once built)
+        lds = _native.leading_dims(prepared["forms"], a, b, c, d)
+        again = prepared.get((lds, kernel)) if lds is not None else None
+        if again is not None and _native.run(again.handle, a, b, c, d):
+            return d
     from . import complex_planar
     if complex_planar.is_planar(conf) and not complex_planar.planes_adjacent(a, b, c, d):
         return complex_planar.PlanarComplexPlan(conf, a, b, c, d)(stream)
@@ -414,10 +465,9 @@ def matmul(conf: Config, a, b, c, d, *,
                                           ctypes.byref(cepi) if cepi is not None else None,
                                           *_span(workspace), stream)
     else:
-        args = (_ptr(a), _ptr(b), _ptr(c), _ptr(d), ctypes.byref(ctrans) if ctrans is not None else None,
-                ctypes.byref(cepi) if cepi is not None else None, kernel.code, stream)
+        args = (_ptr(a), _ptr(b), _ptr(c), _ptr(d), ctrans, cepi, kernel.code, stream)
         larger = _launched_as(conf, a, b, c, d, ctrans is not None or cepi is not None)
-        rc = _lib.lib().gk_matmul(ctypes.byref(larger.to_c(*lds)), *args) if larger is not None else _lib.GK_ERR_UNSUPPORTED
+        rc = _gk_matmul(larger.to_c(*lds), *args) if larger is not None else _lib.GK_ERR_UNSUPPORTED
         if rc != _lib.GK_OK:
             need = 0
             if larger is None and ctrans is None and cepi is None and conf.operator.kind == Operator.MFMA:
@@ -427,9 +477,13 @@ def matmul(conf: Config, a, b, c, d, *,
                     need = known[lds] = _sliced_bytes(cconf, None, None)
             if need:
                 workspace = _workspace(need, stream)
-                rc = _lib.lib().gk_matmul_sliced(ctypes.byref(cconf), *args[:-1], *_span(workspace), stream)
+                rc = _lib.lib().gk_matmul_sliced(ctypes.byref(cconf), *args[:4], None, None, kernel.code, *_span(workspace), stream)
             else:
-                rc = _lib.lib().gk_matmul(ctypes.byref(cconf), *args)
+                rc = _gk_matmul(cconf, *args)
+                if rc == _lib.GK_OK and plain:
+                    _prepare(conf, cconf, lds, kernel)
+        elif plain:
+            _prepare(conf, larger.to_c(*lds), lds, kernel)
     if rc != _lib.GK_OK:
         _raise(rc)
     return d
@@ -623,6 +677,8 @@ def matmatmul_(C, transA: str, transB: str, A, B, alpha, beta, *, wmma=None):
                alpha, beta, wmma, a % 16 == 0, b % 16 == 0, c % 16 == 0)
         hit = _mul_launches.get(key)
         if hit is not None:
+            if wmma is None:
+                _remember(C, A, B, tA, tB, alpha, beta, hit)
             hit(a, b, c, _current_stream())
             return C
     p = _single_plan(C, tA, tB, A, B, alpha, beta, wmma)
@@ -634,7 +690,43 @@ def matmatmul_(C, transA: str, transB: str, A, B, alpha, beta, *, wmma=None):
             _mul_launches.clear()
         _mul_launches[key] = launch
     launch(a, b, c, _current_stream())
+    if key is not None and wmma is None:
+        _remember(C, A, B, tA, tB, alpha, beta, launch)
     return C
+
+
+def _load_native():
+    global _native, _native_mul
+    if _native is None:
+        _native = load_native()
+        if _native is not None:
+            _native_mul = _native.mul
+    return _native
+
+
+def _native_mul(C, A, B, tA, tB, alpha, beta) -> bool:
+    """gk_torch's ``mul`` once it is loaded: True when the call is on its way."""
+    return False
+
+
+def _remember(C, A, B, tA, tB, alpha, beta, launch) -> None:
+    """Leaves the launch of this kind of operands with gk_torch, which makes the next ones (``mul_``), and the workspace of the stream."""
+    native = _load_native()
+    if native is None or type(launch) is not _MulLaunch or type(alpha) is not float or type(beta) is not float:
+        return
+    import torch
+    form, need = (2, launch._workspace) if launch._workspace is not None else (1, launch._sliced) if launch._sliced else (0, 0)
+    what, trans = ctypes.addressof(launch._conf), 0 if launch._trans is None else ctypes.addressof(launch._trans)
+    if form == 0 and all(x.data_ptr() % 16 == 0 for x in (A, B, C)):           # (part of the kind)
+        if launch._prepared is None:
+            launch._prepared = Prepared(launch._conf, launch._trans, None, launch._code)
+        if launch._prepared.handle is not None:
+            form, what = 3, launch._prepared.handle
+    if native.remember(C, A, B, tA, tB, alpha, beta, form, what, trans, launch._code or 0, need, launch) and need:
+        key = (torch.cuda.current_device(), _current_stream())
+        buf = _workspaces.get(key)
+        if buf is not None:
+            native.use_workspace(*key, buf.data_ptr(), buf.numel(), buf)
 
 
 _PLAIN_NUMBERS = (float, int, bool)
@@ -704,7 +796,7 @@ class _MulLaunch:
     stream and from any thread (nothing in it is written after it is made).  Lowering the same call again took 22 us of
     interpreter time, the whole of a small product: mul! at 256^3 in Float32 takes 5 us on the device."""
 
-    __slots__ = ("_fn", "_conf", "_trans", "_conf_ref", "_trans_ref", "_code", "_workspace", "_sliced")
+    __slots__ = ("_fn", "_conf", "_trans", "_conf_ref", "_trans_ref", "_code", "_workspace", "_sliced", "_prepared")
 
     def __init__(self, p: Plan):
         self._conf, self._trans = p._conf, p._trans         # (own the memory that the references point to)
@@ -714,6 +806,7 @@ class _MulLaunch:
         self._workspace = _split_k_bytes(self._conf) if p._split_k else None
         self._code = None if p._split_k else p._args[-1]
         self._sliced = p._sliced
+        self._prepared = None
 
     def __call__(self, a: int, b: int, c: int, stream: int) -> None:
         if self._sliced:
@@ -808,5 +901,11 @@ Adjoint = Transpose
 def mul_(C, A, B, alpha=True, beta=False):
     """``mul!`` (reference src/matmul.jl:207-215): unwraps Transpose/Adjoint and forwards."""
     tA, tB = isinstance(A, Transpose), isinstance(B, Transpose)
-    return matmatmul_(C, 'T' if tA else 'N', 'T' if tB else 'N', A.parent if tA else A, B.parent if tB else B,
-                      float(alpha), float(beta))
+    if tA:
+        A = A.parent
+    if tB:
+        B = B.parent
+    alpha, beta = float(alpha), float(beta)
+    if _native_mul(C, A, B, tA, tB, alpha, beta):
+        return C
+    return matmatmul_(C, 'T' if tA else 'N', 'T' if tB else 'N', A, B, alpha, beta)

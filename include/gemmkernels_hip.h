@@ -300,6 +300,14 @@ int gk_matmul_sliced(const gk_config* conf, const void* a, const void* b, const 
                      const gk_transforms* transforms, const gk_epilogue* epilogue, int32_t kernel, void* workspace,
                      size_t workspace_bytes, void* stream);
 
+/* gk_matmul in two parts, for launches that repeat: gk_prepare makes every check of gk_matmul that does not depend on the operands'
+ * addresses, and gk_run launches on operands at 16-byte boundaries (GK_ERR_ALIGNMENT for others: gk_matmul takes them where the layouts do;
+ * GK_ERR_UNSUPPORTED after gk_set_device_limits).  Nothing of the configuration and the hooks is referred to after gk_prepare but the bias of the epilogue.  A prepared launch
+ * may be run from any number of threads, on any streams, and is freed by gk_prepared_free. */
+int gk_prepare(const gk_config* conf, const gk_transforms* transforms, const gk_epilogue* epilogue, int32_t kernel, void** prepared);
+int gk_run(const void* prepared, const void* a, const void* b, const void* c, void* d, void* stream);
+void gk_prepared_free(void* prepared);
+
 /* Whether `stream` (NULL: the default stream) is being captured into a HIP graph, and the id of that capture: a launch that is
  * captured needs a workspace that lives as long as the graph and is not in use by launches outside of it, which only
  * the stream that is launched on can tell. */

@@ -32,7 +32,7 @@ def test_which_launches_are_cut():
     for dtype in TYPES:
         assert sliced_bytes(96, 96, 100, dtype) == 0 and sliced_bytes(256, 256, 64, dtype) == 0
         assert sliced_bytes(2048, 2048, 2048, dtype) == 0 and sliced_bytes(1000, 1000, 1000, dtype) == 0
-    conf = configs.mfma_config(512, 512, 4096).to_c()
+    conf = configs.mfma_config(4096, 4096, 4096).to_c()
     need = ctypes.c_size_t(1)
     assert _lib.lib().gk_sliced_workspace_size(ctypes.byref(conf), None, None, ctypes.byref(need)) == _lib.GK_OK and need.value == 0
     assert _lib.lib().gk_sliced_workspace_size(None, None, None, ctypes.byref(need)) == _lib.GK_ERR_INVALID_ARGUMENT
