@@ -493,20 +493,33 @@ def larger_tile(conf: Config, hooks: bool) -> Optional[Config]:
     2368 x 3072 x 896 with C 28.4 and 30.0 (0.90).  ``hooks``: transforms or a bias, which tiles of 256 x 256 over the edges run on eight waves (5376 x 2176 x 768 with C 47.5 and 53.0,
     3520 x 2432 x 2048 72.4 and 76.1, so not those) and which the estimates leave out: 5696 x 5760 x 4160 with C 440 and 320 on 128 x 128 (0.57), 4992 x 1344 x 4416 99.6 and 73.7 (0.70), 4608 x 832 x 6080 75.5
     and 61.6 (0.71); beyond the line 5056 x 768 x 2176 29.1 and 31.0 (0.85)."""
-    if not conf.__dict__.get("_tile_left_open"):
+    if not conf.__dict__.get("_tile_left_open") or conf.operator.kind != Operator.MFMA or conf.global_a_layout.kind not in _ANY_SIZE:
         return None
-    key = "_larger_tile_with_hooks" if hooks else "_larger_tile"
-    if key not in conf.__dict__:
-        conf.__dict__[key] = _find_larger_tile(conf, hooks)
-    return conf.__dict__[key]
+    name = "_larger_tile_with_hooks" if hooks else "_larger_tile"
+    if name not in conf.__dict__:
+        op, layouts = conf.operator, (conf.global_a_layout, conf.global_b_layout, conf.global_c_layout, conf.global_d_layout)
+        shared = (conf.shared_a_layout, conf.shared_b_layout, conf.shared_c_layout, conf.shared_d_layout)
+        # (kept by value: a program that makes a configuration for every product finds the answer of the ones before)
+        key = (*conf.matmul_shape.values(), *conf.block_shape.values(), hooks, op.kind, op.M, op.N, op.K, op.CT.name, op.AT.name, conf.is_a_col_major, conf.is_b_col_major,
+               *((l.kind, l.T.name, l.pad) for l in layouts + shared))
+        found = _larger_tiles.get(key, False)
+        if found is False:
+            found = _find_larger_tile(tuple(conf.matmul_shape.values()), tuple(conf.block_shape.values()), op, layouts, shared,
+                                      conf.is_a_col_major, conf.is_b_col_major, hooks)
+            if len(_larger_tiles) >= 256:
+                _larger_tiles.clear()
+            _larger_tiles[key] = found
+        conf.__dict__[name] = found
+    return conf.__dict__[name]
 
 
-def _find_larger_tile(conf: Config, hooks: bool) -> Optional[Config]:
-    layouts = (conf.global_a_layout, conf.global_b_layout, conf.global_c_layout, conf.global_d_layout)
-    if conf.operator.kind != Operator.MFMA or any(l.kind not in _ANY_SIZE and not (i == 2 and l.kind == Layout.ZERO) for i, l in enumerate(layouts)):
+_larger_tiles = {}
+
+
+def _find_larger_tile(shape, own, operator, layouts, shared, is_a_col_major, is_b_col_major, hooks) -> Optional[Config]:
+    if operator.kind != Operator.MFMA or any(l.kind not in _ANY_SIZE and not (i == 2 and l.kind == Layout.ZERO) for i, l in enumerate(layouts)):
         return None
-    M, N, K = (conf.matmul_shape[x] for x in "MNK")
-    own = tuple(conf.block_shape[x] for x in "MNK")
+    M, N, K = shape
     if own not in _MFMA_TILE_COST:
         return None
     a_kmajor, b_kmajor = layouts[0].kind == Layout.ALIGNED_ROW_MAJOR, layouts[1].kind == Layout.ALIGNED_COL_MAJOR
@@ -515,10 +528,10 @@ def _find_larger_tile(conf: Config, hooks: bool) -> Optional[Config]:
         return None
     a, b, c, d = (_ANY_SIZE[l.kind][l.T] if l.kind in _ANY_SIZE else l for l in layouts)
     try:
-        return get_config(gemm_shape=conf.matmul_shape, operator=conf.operator, block_shape=NT(M=best[0], N=best[1], K=best[2]),
+        return get_config(gemm_shape=NT(M=M, N=N, K=K), operator=operator, block_shape=NT(M=best[0], N=best[1], K=best[2]),
                           global_a_layout=a, global_b_layout=b, global_c_layout=c, global_d_layout=d,
-                          shared_a_layout=conf.shared_a_layout, shared_b_layout=conf.shared_b_layout, shared_c_layout=conf.shared_c_layout,
-                          shared_d_layout=conf.shared_d_layout, is_a_col_major=conf.is_a_col_major, is_b_col_major=conf.is_b_col_major)
+                          shared_a_layout=shared[0], shared_b_layout=shared[1], shared_c_layout=shared[2], shared_d_layout=shared[3],
+                          is_a_col_major=is_a_col_major, is_b_col_major=is_b_col_major)
     except ConfigError:
         return None
 

@@ -25,7 +25,7 @@ from . import _lib
 from . import kernel as Kernel
 from . import layout as Layout
 from . import operator as Operator
-from ._native import load as native
+from ._native import Prepared, load as native
 from .config import _GETT_TILES, _mfma_cost, get_config
 from .dtypes import BFloat16, DType, Float16, Float32
 from .errors import ConfigError
@@ -185,17 +185,18 @@ def contract(spec: str, a, b, d, c=None, stream=None):
         if len(_launches) >= _LAUNCHES_MAX:
             _launches.clear()
         _launches[key] = launch
-    if stream is not None or launch.run is None or not launch.run(launch.handle, *((b, a) if launch._swapped else (a, b)), c, d):
+    ready = launch.ready if stream is None else None             # (held while it is used)
+    if ready is None or not ready[0](ready[1].handle, *((b, a) if launch._swapped else (a, b)), c, d):
         launch(a.data_ptr(), b.data_ptr(), None if c is None else c.data_ptr(), d.data_ptr(), _current_stream() if stream is None else int(stream))
     return d
 
 
 class _Launch:
     """What ``contract`` hands to the library for operands of one kind (mode string, element types, extents, strides): the descriptor
-    the planner arrived at, no address and no tensor; nothing in it is written after it is made, and the library checks
-    the addresses at every launch.  Planning again took 70 us of interpreter time a call, several times the kernel of a small contraction."""
+    the planner arrived at, no address and no tensor; the library checks the addresses at every launch.  (What is written after it is made is how often it was
+    called and, from the second call on, the launch checked once: threads that meet there make one too many.)  Planning again took 70 us of interpreter time a call, several times the kernel of a small contraction."""
 
-    __slots__ = ("_conf", "_conf_ref", "_swapped", "_fn", "_code", "_sliced", "_prepared", "handle", "run")
+    __slots__ = ("_conf", "_conf_ref", "_swapped", "_fn", "_code", "_sliced", "ready", "_calls")
 
     def __init__(self, p: ContractionPlan):
         self._conf = p._launch._conf                      # (owns the memory that the reference points to)
@@ -203,11 +204,15 @@ class _Launch:
         self._swapped = p.swapped
         self._fn, self._code, self._sliced = p._launch._fn, p._launch._args[-1], p._launch._sliced
         # (the launch checked once and gk_torch's way to it, for operands on 16-byte boundaries)
-        self._prepared = p._launch._prepared
-        self.handle = self._prepared.handle if self._prepared is not None else None
-        self.run = native().run if self.handle is not None else None
+        self.ready = None
+        self._calls = 0
 
     def __call__(self, a: int, b: int, c: Optional[int], d: int, stream: int) -> None:
+        self._calls += 1
+        if self._calls == 2 and not self._sliced and native() is not None:
+            prepared = Prepared(self._conf, None, None, self._code)
+            if prepared.handle is not None:
+                self.ready = native().run, prepared
         x, y = (b, a) if self._swapped else (a, b)
         if self._sliced:
             from .matmul import _span, _workspace

@@ -305,7 +305,7 @@ class Plan:
     other means while it is in use.  For loops that launch the same GEMM many times, where the
     microseconds a general ``matmul`` call spends on lowering would rival the kernel itself."""
 
-    __slots__ = ("_fn", "_conf", "_trans", "_epi", "_args", "_keep", "_split_k", "_sliced", "_as_given", "_direct", "_prepared", "d", "kernel_names")
+    __slots__ = ("_fn", "_conf", "_trans", "_epi", "_args", "_keep", "_split_k", "_sliced", "_as_given", "_direct", "_calls", "d", "kernel_names")
 
     def __init__(self, conf: Config, a, b, c, d, transforms: dict, epilogue, kernel, specialized=None, slices=False):
         if specialized is None and any(t.expr is not None for t in transforms.values()):
@@ -340,15 +340,24 @@ class Plan:
             self._args = (ctypes.byref(self._conf), _ptr(a), _ptr(b), _ptr(c), _ptr(d),
                           ctypes.byref(self._trans) if self._trans is not None else None, epi_ref, kernel.code)
         self._keep = (a, b, c, d, epilogue, specialized)
-        self._direct = self._prepared = None
-        if _load_native() is not None and specialized is None and not self._split_k and not self._sliced:
-            self._prepared = Prepared(self._conf, self._trans, self._epi, kernel.code)
-            if self._prepared.handle is not None:
-                self._direct = (self._prepared.handle, *self._args[1:5])
+        self._direct = None           # (from the second call on, see prepare)
+        self._calls = 0 if specialized is None and not self._split_k and not self._sliced else 2
         self.d = d
         self.kernel_names = ()      # filled in by the BLAS-level front end
 
+    def prepare(self):
+        """Has the library check the launch once for all calls to come (gk_prepare): a few microseconds, which a plan that is called once does not pay."""
+        self._calls = 2
+        if _load_native() is not None:
+            prepared = Prepared(self._conf, self._trans, self._epi, self._args[-1])
+            if prepared.handle is not None:
+                self._direct = prepared, (prepared.handle, *self._args[1:5])         # (one object: a thread that uses it holds it)
+
     def __call__(self, stream=None):
+        if self._calls < 2:
+            self._calls += 1
+            if self._calls == 2:
+                self.prepare()
         stream = _current_stream() if stream is None else int(stream)
         if self._split_k:
             workspace = split_k_workspace(self._conf, stream)
@@ -360,7 +369,8 @@ class Plan:
             workspace = _workspace(self._sliced, stream)
             rc = self._fn(*self._args, *_span(workspace), stream)
         else:
-            if self._direct is not None and _native.run_at(*self._direct, stream) == _lib.GK_OK:
+            direct = self._direct
+            if direct is not None and _native.run_at(*direct[1], stream) == _lib.GK_OK:
                 return self.d
             rc = self._fn(*self._args, stream)
             if rc != _lib.GK_OK and self._as_given is not None:
@@ -403,6 +413,9 @@ def _prepare(conf: Config, cconf, lds, kernel) -> None:
     """Keeps the launch that ``matmul`` made for operands of these leading dimensions (no address) with its configuration."""
     kept = conf.__dict__.get("_prepared")
     if _load_native() is None or kept is not None and (lds, kernel) in kept:
+        return
+    if conf.__dict__.get("_launched") != (lds, kernel):             # (a configuration that is launched once does not pay for it)
+        conf.__dict__["_launched"] = (lds, kernel)
         return
     made = Prepared(cconf, None, None, kernel.code)
     if made.handle is None:
@@ -716,13 +729,14 @@ def _remember(C, A, B, tA, tB, alpha, beta, launch) -> None:
         return
     import torch
     form, need = (2, launch._workspace) if launch._workspace is not None else (1, launch._sliced) if launch._sliced else (0, 0)
-    what, trans = ctypes.addressof(launch._conf), 0 if launch._trans is None else ctypes.addressof(launch._trans)
+    what, owner, trans = ctypes.addressof(launch._conf), None, 0 if launch._trans is None else ctypes.addressof(launch._trans)
     if form == 0 and all(x.data_ptr() % 16 == 0 for x in (A, B, C)):           # (part of the kind)
-        if launch._prepared is None:
-            launch._prepared = Prepared(launch._conf, launch._trans, None, launch._code)
-        if launch._prepared.handle is not None:
-            form, what = 3, launch._prepared.handle
-    if native.remember(C, A, B, tA, tB, alpha, beta, form, what, trans, launch._code or 0, need, launch) and need:
+        owner = launch._prepared
+        if owner is None:
+            owner = launch._prepared = Prepared(launch._conf, launch._trans, None, launch._code)
+        if owner.handle is not None:
+            form, what = 3, owner.handle
+    if native.remember(C, A, B, tA, tB, alpha, beta, form, what, trans, launch._code or 0, need, (launch, owner)) and need:
         key = (torch.cuda.current_device(), _current_stream())
         buf = _workspaces.get(key)
         if buf is not None:
