@@ -1146,7 +1146,7 @@ static_assert(kSplitCounterBytes / sizeof(unsigned) >= 2 * (size_t)gk::kNumCUs -
 //   'T','N' 4 13.8, 6 12.9; BF16 with op lists on A (level 2) 4 66.5, 6 61.6, 8 57.0, 7 x 7 x 20000 (1) 19 54.2, 31 46.6.  BF16 with one factor (level 1),
 //   whose loop is little longer, lies within 5 % of its best on the same slices: 4096 x 64 x 4096 'N','N' 4 15.9, 6 16.1, 8 16.3; 7 x 7 x 20000 19 17.1, 31 16.2;
 //   512 x 512 x 4096 (64) 4 15.2, 6 14.1, 8 13.7; 2048 x 128 x 8192 (64) 6 20.5, 8 18.2, 10 23.6; 960 x 384 x 4096 (90) 3 18.0, 5 15.6, 6 19.2; 8192 x 64 x 4096 (128) 2 23.3, 4 24.2.
-// 128 x 128 x 64, whose partial tiles are four times as large: 768 deep (1024 above 64 tiles), sixteen slices or 2048 deep:
+// 128 x 128 x 64 (figures on two LDS stages), whose partial tiles are four times as large: 768 deep (1024 above 64 tiles), sixteen slices or 2048 deep:
 //   512 x 512 x 4096 (16) 4 22.7, 5 22.0, 6 21.8; 2048 x 512 x 4096 (64) 4 25.3, 5 25.3, 6 26.2; 1536 x 1024 x 4096 (96) 4 29.5, 5 30.6;
 //   256 x 256 x 16384 (4) 12 34.4, 16 35.5, 25 40.2.
 // Other tiles (64 x 64 x 32): 4096 x 64 x 4096 (64) 4 24.4, 6 21.1, 7 20.6, 8 21.3.
@@ -1344,6 +1344,11 @@ Sliced sliced_route(const gk::InstanceKey& as_asked, const gk::GemmArgs& args) {
     r.fn = key.family == gk::FAMILY_MFMA ? gk::family_mfma_splitk : gk::family_mfma_splitk_gett;
     if (args.K >= (tiles <= 64 ? 1280 : (tiles <= 128 ? 2048 : 3000)) && tiles <= 170)
       r.slices = split_k_slices(tiles, (args.K + 63) / 64, gk_shape{64, 64, 64}, key.fused == 1);
+  } else if (key.family == gk::FAMILY_MFMA && key.BM == 128 && key.BN == 128 && key.BK == 64 && key.waves_m == 2 && key.waves_n == 2) {
+    // One workgroup of four LDS stages per CU, of slices that are 768 deep (1024 above 85 tiles, of which a CU each is left for two).  (As many as two per CU, which a K-split launch of this tile takes, whose callers chose its error: the time
+    // of one per CU is 0.98 of it with up to 32 tiles, 0.87 with 33 to 64, 0.83 with 65 to 85, 0.92 with 86 to 128, averages over 180 drawn products.)
+    r.fn = gk::family_mfma_splitk;
+    if (tiles <= gk::kNumCUs / 2 && args.K >= 2048) r.slices = std::min(gk::kNumCUs / tiles, args.K / (tiles <= 85 ? 768 : 1024));
   }
   if (r.slices < 2) return r;
   const int k_tiles = (args.K + key.BK - 1) / key.BK;

@@ -28,7 +28,10 @@ int family_mfma_splitk(const InstanceKey& key, const GemmArgs& args, dim3 grid, 
   GK_SK_T(bm_, bn_, bk_, wm_, wn_, st_, __bf16, DT_BF16, 0, "_bf16")  \
   GK_SK_T(bm_, bn_, bk_, wm_, wn_, st_, __bf16, DT_BF16, 1, "_bf16_fused")  \
   GK_SK_T(bm_, bn_, bk_, wm_, wn_, st_, __bf16, DT_BF16, 3, "_bf16_fused_cd")
-  GK_SK_TILE(128, 128, 64, 2, 2, 2)
+  // (four LDS stages as where a workgroup has a CU to itself unsplit: the slices of such a launch are chosen to.  us on two stages, two workgroups per CU, and on four with one:
+  // 824 x 1408 x 5958 'T','T' 32.5 and 26.3, 1058 x 704 x 4383 'T','N' 35.4 and 25.5, 7268 x 256 x 3200 'T','T' 36.5 and 27.2; four stages and two workgroups one behind the other
+  // 0.88 (up to 32 tiles) to 0.98 of two and two side by side)
+  GK_SK_TILE(128, 128, 64, 2, 2, 4)
   GK_SK_TILE(64, 64, 64, 2, 2, 4)
   // (op lists on A and B)
   GK_SK_T(64, 64, 64, 2, 2, 4, __bf16, DT_BF16, 2, "_bf16_fused_ab")

@@ -253,6 +253,20 @@ def split_k_block_shape(M, N, K, widest_ld=0, factor=None) -> Optional[NT]:
     return NT(M=64, N=64, K=64) if worth else None
 
 
+def sliced_block_shape(M, N, K, widest_ld=0, odd=False) -> Optional[NT]:
+    """128 x 128 x 64 for a 16-bit product whose tiles of that size leave CUs idle and whose K is long enough for slices of them to be ahead of tiles of 64 x 64, cut or not
+    (``gk_matmul_sliced``), or None.  A 64 x 64 tile brings twice the bytes per product into a CU, and more than 256 of them are not cut (a few more than 256 take as long as 512).
+    us, 64 x 64 -> 128 x 128 in slices, inputs that rotate: 1472 x 768 x 5888 'N','T' 34.2 -> 24.0, 1088 x 1088 x 5248 'N','T' 31.5 -> 24.3, 704 x 1664 x 4544 'T','T' 26.6 -> 22.3, 2944 x 384 x 3712 24.0 -> 19.2;
+    below the line 384 x 4160 x 2496 18.0 and 21.5, 1088 x 1728 x 3136 21.6 and 26.7.  ``odd``: an operand whose columns start off 16-byte boundaries, whose rows of a small tile lie on
+    relatively more lines: 326 x 3462 x 3056 'T','T' 26.6 -> 19.5, 2048 x 560 x 2542 'T','N' 22.3 -> 18.5, 2624 x 517 x 3296 32.1 -> 24.1, 539 x 2592 x 7990 with a factor 79.9 -> 50.7.  Error
+    against 64 bits: never larger than that of the one chain it replaces (two slices or three).
+    ``widest_ld``: the largest leading dimension; the kernel keeps the offsets in a tile in 32 bits."""
+    tiles, small = -(-M // 128) * -(-N // 128), -(-M // 64) * -(-N // 64)
+    if small <= 256 or tiles > 128 or K < (2500 if odd else 3500) or 128 * widest_ld * 2 >= 1 << 31:
+        return None
+    return NT(M=128, N=128, K=64)
+
+
 # Estimated launch time of a tile, in microseconds: what a launch costs whatever its size, per 1000 k and round, per further tile of
 # a CU, for a partial last K tile (times the square root of the rounds), for tiles over the edges.  Fitted, weighted towards the tiles near the
 # best, to timings of every tile at 61 sizes from 1000 x 1000 x 64 to 4416 x 4416 x 1024 ('N','N' and 'T','N'; whole tiles, multiples of 64 and odd ones; inputs
@@ -481,7 +495,7 @@ _TILE_CHOICES = ("block_shape", "warps_per_block", "compute_warp", "mem_a_warp",
 _ANY_SIZE = {Layout.ALIGNED_COL_MAJOR: Layout.ColMajor, Layout.ALIGNED_ROW_MAJOR: Layout.RowMajor}
 
 
-def larger_tile(conf: Config, hooks: bool) -> Optional[Config]:
+def larger_tile(conf: Config, hooks: bool, slices: bool = False) -> Optional[Config]:
     """The configuration that a launch of ``conf`` runs on where the tile was left to the default and one that does not divide the sizes is faster, or None.
 
     Aligned layouts ask for sizes in whole tiles (reference src/config.jl:268-275), so most multiples of 64 leave only the 64 x 64 tiles, which bring every
@@ -492,20 +506,20 @@ def larger_tile(conf: Config, hooks: bool) -> Optional[Config]:
     1600 x 4480 x 2048 'N','T' with C 54.9 and 47.5 (0.75), 5632 x 2240 x 384 24.2 and 20.7 (0.84), 5120 x 4224 x 5888 with C 285.8 and 269.4 (0.84); beyond the line 1920 x 1856 x 2368 27.9 and 29.2 (0.90),
     2368 x 3072 x 896 with C 28.4 and 30.0 (0.90).  ``hooks``: transforms or a bias, which tiles of 256 x 256 over the edges run on eight waves (5376 x 2176 x 768 with C 47.5 and 53.0,
     3520 x 2432 x 2048 72.4 and 76.1, so not those) and which the estimates leave out: 5696 x 5760 x 4160 with C 440 and 320 on 128 x 128 (0.57), 4992 x 1344 x 4416 99.6 and 73.7 (0.70), 4608 x 832 x 6080 75.5
-    and 61.6 (0.71); beyond the line 5056 x 768 x 2176 29.1 and 31.0 (0.85)."""
+    and 61.6 (0.71); beyond the line 5056 x 768 x 2176 29.1 and 31.0 (0.85).  ``slices``: the launch may run in slices of K (``sliced_block_shape``)."""
     if not conf.__dict__.get("_tile_left_open") or conf.operator.kind != Operator.MFMA or conf.global_a_layout.kind not in _ANY_SIZE:
         return None
-    name = "_larger_tile_with_hooks" if hooks else "_larger_tile"
+    name = ("_larger_tile_with_hooks" if hooks else "_larger_tile") + ("_in_slices" if slices else "")
     if name not in conf.__dict__:
         op, layouts = conf.operator, (conf.global_a_layout, conf.global_b_layout, conf.global_c_layout, conf.global_d_layout)
         shared = (conf.shared_a_layout, conf.shared_b_layout, conf.shared_c_layout, conf.shared_d_layout)
         # (kept by value: a program that makes a configuration for every product finds the answer of the ones before)
-        key = (*conf.matmul_shape.values(), *conf.block_shape.values(), hooks, op.kind, op.M, op.N, op.K, op.CT.name, op.AT.name, conf.is_a_col_major, conf.is_b_col_major,
+        key = (*conf.matmul_shape.values(), *conf.block_shape.values(), hooks, slices, op.kind, op.M, op.N, op.K, op.CT.name, op.AT.name, conf.is_a_col_major, conf.is_b_col_major,
                *((l.kind, l.T.name, l.pad) for l in layouts + shared))
         found = _larger_tiles.get(key, False)
         if found is False:
             found = _find_larger_tile(tuple(conf.matmul_shape.values()), tuple(conf.block_shape.values()), op, layouts, shared,
-                                      conf.is_a_col_major, conf.is_b_col_major, hooks)
+                                      conf.is_a_col_major, conf.is_b_col_major, hooks, slices)
             if len(_larger_tiles) >= 256:
                 _larger_tiles.clear()
             _larger_tiles[key] = found
@@ -516,16 +530,20 @@ def larger_tile(conf: Config, hooks: bool) -> Optional[Config]:
 _larger_tiles = {}
 
 
-def _find_larger_tile(shape, own, operator, layouts, shared, is_a_col_major, is_b_col_major, hooks) -> Optional[Config]:
+def _find_larger_tile(shape, own, operator, layouts, shared, is_a_col_major, is_b_col_major, hooks, slices) -> Optional[Config]:
     if operator.kind != Operator.MFMA or any(l.kind not in _ANY_SIZE and not (i == 2 and l.kind == Layout.ZERO) for i, l in enumerate(layouts)):
         return None
     M, N, K = shape
     if own not in _MFMA_TILE_COST:
         return None
     a_kmajor, b_kmajor = layouts[0].kind == Layout.ALIGNED_ROW_MAJOR, layouts[1].kind == Layout.ALIGNED_COL_MAJOR
-    best = min(_mfma_tiles(a_kmajor, b_kmajor), key=lambda t: math.inf if hooks and t[:2] == (256, 256) else _mfma_cost(t, M, N, K))
-    if best == own or _mfma_cost(best, M, N, K) > (0.8 if hooks else 0.86) * _mfma_cost(own, M, N, K):
-        return None
+    sliced = sliced_block_shape(M, N, K) if slices and own[:2] == (64, 64) else None
+    if sliced is not None:
+        best = tuple(sliced.values())
+    else:
+        best = min(_mfma_tiles(a_kmajor, b_kmajor), key=lambda t: math.inf if hooks and t[:2] == (256, 256) else _mfma_cost(t, M, N, K))
+        if best == own or _mfma_cost(best, M, N, K) > (0.8 if hooks else 0.86) * _mfma_cost(own, M, N, K):
+            return None
     a, b, c, d = (_ANY_SIZE[l.kind][l.T] if l.kind in _ANY_SIZE else l for l in layouts)
     try:
         return get_config(gemm_shape=NT(M=M, N=N, K=K), operator=operator, block_shape=NT(M=best[0], N=best[1], K=best[2]),

@@ -21,7 +21,7 @@ from . import kernel as Kernel
 from . import layout as Layout
 from . import operator as Operator
 from . import transform as Transform
-from .config import _MFMA_TILE_COST, Config, _mfma_cost, default_block_shape, get_config as _get_config, larger_tile, split_k_block_shape
+from .config import _MFMA_TILE_COST, Config, _mfma_cost, default_block_shape, get_config as _get_config, larger_tile, sliced_block_shape, split_k_block_shape
 from .dtypes import BFloat16, DType, Float16, Float32, Float64, from_torch, promote_type
 from .errors import ConfigError, DimensionMismatch
 from ._native import Prepared, load as load_native
@@ -282,9 +282,9 @@ def specialize(conf: Config, *,
     return SpecializedKernel(conf, {k: (Transform.Elementwise(expr=v) if isinstance(v, str) else v) for k, v in given.items()})
 
 
-def _launched_as(conf: Config, a, b, c, d, hooks: bool) -> Optional[Config]:
+def _launched_as(conf: Config, a, b, c, d, hooks: bool, slices: bool = False) -> Optional[Config]:
     """``larger_tile`` of ``conf`` where the operands are what the aligned layouts of ``conf`` ask for (the library refuses others, and is left to), or None."""
-    larger = larger_tile(conf, hooks)
+    larger = larger_tile(conf, hooks, slices)
     if larger is None:
         return None
     for x, layout in ((a, conf.global_a_layout), (b, conf.global_b_layout), (c, conf.global_c_layout), (d, conf.global_d_layout)):
@@ -316,7 +316,7 @@ class Plan:
         self._trans = None if specialized is not None else lower_transforms(transforms)
         self._as_given = None                                      # (what is launched where the library refuses the larger tile)
         hooks = self._trans is not None or epilogue.kind != Epilogue.DEFAULT
-        larger = _launched_as(conf, a, b, c, d, hooks) if specialized is None and kernel is not Kernel.matmul_split_k else None
+        larger = _launched_as(conf, a, b, c, d, hooks, slices) if specialized is None and kernel is not Kernel.matmul_split_k else None
         if larger is not None:
             self._as_given, self._conf = self._conf, _lib.gk_config.from_buffer_copy(larger.to_c(*lds))
         self._epi = None
@@ -335,7 +335,7 @@ class Plan:
                           ctypes.byref(self._trans) if self._trans is not None else None, epi_ref)
             self._split_k = True
         else:
-            self._sliced = _sliced_bytes(self._conf, self._trans, self._epi) if slices and larger is None else 0
+            self._sliced = _sliced_bytes(self._conf, self._trans, self._epi) if slices else 0
             self._fn = _lib.lib().gk_matmul_sliced if self._sliced else _lib.lib().gk_matmul
             self._args = (ctypes.byref(self._conf), _ptr(a), _ptr(b), _ptr(c), _ptr(d),
                           ctypes.byref(self._trans) if self._trans is not None else None, epi_ref, kernel.code)
@@ -368,6 +368,8 @@ class Plan:
         if self._sliced:
             workspace = _workspace(self._sliced, stream)
             rc = self._fn(*self._args, *_span(workspace), stream)
+            if rc != _lib.GK_OK and self._as_given is not None:
+                rc = _lib.lib().gk_matmul(ctypes.byref(self._as_given), *self._args[1:], stream)
         else:
             direct = self._direct
             if direct is not None and _native.run_at(*direct[1], stream) == _lib.GK_OK:
@@ -479,14 +481,18 @@ def matmul(conf: Config, a, b, c, d, *,
                                           *_span(workspace), stream)
     else:
         args = (_ptr(a), _ptr(b), _ptr(c), _ptr(d), ctrans, cepi, kernel.code, stream)
-        larger = _launched_as(conf, a, b, c, d, ctrans is not None or cepi is not None)
-        rc = _gk_matmul(larger.to_c(*lds), *args) if larger is not None else _lib.GK_ERR_UNSUPPORTED
-        if rc != _lib.GK_OK:
-            need = 0
-            if larger is None and ctrans is None and cepi is None and conf.operator.kind == Operator.MFMA:
-                known = conf.__dict__.setdefault("_slices_of", {})           # (a Config is immutable once built)
+        hooks = ctrans is not None or cepi is not None
+        larger, rc = _launched_as(conf, a, b, c, d, hooks, not hooks), _lib.GK_ERR_UNSUPPORTED
+        for of in (larger, conf):                                   # (the tile asked for where the library refuses the larger one)
+            if of is None or rc == _lib.GK_OK:
+                continue
+            cconf, need = of.to_c(*lds), 0
+            if not hooks and of.operator.kind == Operator.MFMA:
+                known = of.__dict__.setdefault("_slices_of", {})             # (a Config is immutable once built)
                 need = known.get(lds)
                 if need is None:
+                    if len(known) >= 64:
+                        known.clear()
                     need = known[lds] = _sliced_bytes(cconf, None, None)
             if need:
                 workspace = _workspace(need, stream)
@@ -495,8 +501,6 @@ def matmul(conf: Config, a, b, c, d, *,
                 rc = _gk_matmul(cconf, *args)
                 if rc == _lib.GK_OK and plain:
                     _prepare(conf, cconf, lds, kernel)
-        elif plain:
-            _prepare(conf, larger.to_c(*lds), lds, kernel)
     if rc != _lib.GK_OK:
         _raise(rc)
     return d
@@ -604,7 +608,7 @@ def create_config(A: DType, sizeA, stridesA, transA: bool, B: DType, sizeB, stri
                                  else compute_type in (Float16, Float32, Float64))
     block_shape = None
     if use_mfma and edge_ok:
-        block_shape = split_k_block_shape(m, n, k, max(0 if transA else stridesA[1], stridesB[1] if transB else 0), factor)
+        block_shape = sliced_block_shape(m, n, k, max(stridesA[1], stridesB[1]), not (a_aligned and b_aligned)) or split_k_block_shape(m, n, k, max(0 if transA else stridesA[1], stridesB[1] if transB else 0), factor)
     if block_shape is None:
         block_shape = default_block_shape(operator, NT(M=m, N=n, K=k), tile_sized=not edge_ok, a_kmajor=transA, b_kmajor=not transB)
     global_a_layout, global_b_layout, global_c_layout, global_d_layout = layouts_for(block_shape)
@@ -662,11 +666,14 @@ def _single_plan(C, tA: bool, tB: bool, A, B, alpha, beta, wmma=None) -> Plan:
         # ordered, so the result is the same on every run, like the reference's mul!.
         bs, ms = conf.block_shape, conf.matmul_shape
         tiles = -(-ms.M // bs.M) * -(-ms.N // bs.N)
-        if bs == split_k_block_shape(ms.M, ms.N, ms.K, 0, factor) or tiles <= 128 and ms.K >= 2048:
+        sliced = (bs.M, bs.N, bs.K) == (128, 128, 64) and tiles <= 128 and ms.K >= 2048
+        if not sliced and (bs == split_k_block_shape(ms.M, ms.N, ms.K, 0, factor) or tiles <= 128 and ms.K >= 2048):
             kernel = Kernel.matmul_split_k
-    # (floating-point FPUOp: the library takes slices of K where one chain per output would leave the chip idle, gk_matmul_sliced)
+    else:
+        sliced = conf.operator.kind == Operator.FPU
+    # (floating-point FPUOp and 128 x 128: the library takes slices of K where one chain per output would leave the chip idle, gk_matmul_sliced)
     p = Plan(conf, A, B, C, C, _collect({**dict.fromkeys(_HOOKS), "transform_shared_to_regs_a": ta, "transform_shared_to_regs_c": tc}),
-             _DEFAULT_EPILOGUE, kernel, slices=conf.operator.kind == Operator.FPU)
+             _DEFAULT_EPILOGUE, kernel, slices=sliced)
     p.kernel_names = (kernel_name(conf, kernel, dict(transform_shared_to_regs_a=ta, transform_shared_to_regs_c=tc)),)
     return p
 
@@ -696,7 +703,7 @@ def matmatmul_(C, transA: str, transB: str, A, B, alpha, beta, *, wmma=None):
             return C
     p = _single_plan(C, tA, tB, A, B, alpha, beta, wmma)
     # (an alpha that is infinite in A's type would make NaN of the zeros that fill a copy up)
-    packed = packed_leading_dims(p._conf, a, b) if not p._split_k and math.isfinite(_round_to(from_torch(A.dtype), float(alpha))) else None
+    packed = packed_leading_dims(p._conf, a, b) if not p._split_k and not p._sliced and math.isfinite(_round_to(from_torch(A.dtype), float(alpha))) else None
     launch = _MulLaunch(p) if packed is None else _MulLaunchOnCopies(p, packed)
     if key is not None:
         if len(_mul_launches) >= _MUL_LAUNCHES_MAX:
