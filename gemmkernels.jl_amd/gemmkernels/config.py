@@ -280,6 +280,53 @@ _MFMA_TILE_COST = {(256, 256, 64): (12.0, 16.4, 39.0, 21.0, 1.2), (256, 256, 32)
                    (256, 192, 64): (5.4, 17.1, 19.3, 9.1, 7.9), (192, 256, 64): (5.0, 17.1, 15.3, 10.4, 7.9)}
 
 
+# The same for plain products on any leading dimension, closer: the five above, per operand whose columns start off 16-byte boundaries (contiguous along k, along m or n) what the K loop takes
+# longer, per MB of C and D, and of the smaller tiles how many tile times one to two (a + b (tiles per CU - 1)) and more of them in a CU take.  Fitted to 1500 products
+# drawn like those that `mul_` is timed on, every tile of each, and the sliced launches of 128 x 128 x 64 (us, per 1000 k, per slice, per workgroup of a CU, for a partial last K tile).
+_PRODUCT_COST = {(256, 256, 64): (1.89, 20.31, 8.62, 2.54, 3.74, 0.22, 0.08, 0.16), (256, 256, 32): (0, 23.88, 4.11, 1.26, 5.98, 0.17, 0.01, 0.19),
+                 (256, 128, 64): (4.72, 12.53, 5.58, 2.69, 1.4, 0.18, 0.08, 0.13), (128, 256, 64): (4.74, 13, 5.41, 3, 1.35, 0.18, 0.1, 0.13),
+                 (128, 128, 32): (3.71, 7.92, 1.13, 0.9, 0.82, 0.34, 0.08, 0.12), (128, 128, 64): (3.65, 7.93, 0.99, 1.52, 0.78, 0.22, 0.11, 0.12),
+                 (64, 64, 64): (2.88, 3.35, 0, 0.76, 0.52, 0.22, 0.22, 0.11), (64, 64, 32): (3.05, 3.56, 0.03, 0.44, 0.39, 0.23, 0.19, 0.11),
+                 (256, 192, 64): (0.06, 18.16, 2.52, 1.82, 4.96, 0.2, 0.08, 0.19), (192, 256, 64): (3.72, 19.02, 2.44, 2.94, 0.35, 0.15, 0.14, 0.19)}
+_PRODUCT_ROUNDS = {(128, 128, 32): (0.75, 0.09, 1.59), (128, 128, 64): (0.49, 0.23, 1.66), (64, 64, 64): (0.75, 0.33, 1.08), (64, 64, 32): (0.62, 0.41, 1.12)}
+_PRODUCT_IN_SLICES = (2.88, 8.35, 1.06, 3.36, 0.04)
+
+
+def _product_cost(t, M, N, K, odd, cd_bytes):
+    """Estimated microseconds of a plain product; ``odd``: operands whose columns start off 16-byte boundaries, contiguous along k and not; ``cd_bytes``: of C and D per output."""
+    fixed, per_k, further, tail, edges, odd_k, odd_mn, per_mb = _PRODUCT_COST[t]
+    tiles = -(-M // t[0]) * -(-N // t[1])
+    per_k *= 1.0 + odd_k * odd[0] + odd_mn * odd[1]
+    always = per_mb * 1e-6 * M * N * cd_bytes + (edges if M % t[0] or N % t[1] else 0.0)
+    if t == (128, 128, 64) and tiles <= 128 and K >= 2048:
+        slices = min(NUM_CUS // tiles, K // (768 if tiles <= 85 else 1024))
+        own = _PRODUCT_IN_SLICES
+        return always + own[0] + own[1] * per_k / _PRODUCT_COST[t][1] * -(-K // (64 * slices)) * 0.064 + own[2] * slices + own[3] * slices * tiles / NUM_CUS + (own[4] if K % 64 else 0.0)
+    per_cu = tiles / NUM_CUS
+    if t not in _PRODUCT_ROUNDS:
+        rounds = -(-tiles // NUM_CUS)
+    elif per_cu <= 1:
+        rounds = 1.0
+    else:
+        second, more, full = _PRODUCT_ROUNDS[t]
+        rounds = 1.0 + second + more * (per_cu - 1.0) if per_cu <= 2 else full * (-(-tiles // (2 * NUM_CUS)) if t[0] == 128 else per_cu)
+    return always + fixed + rounds * per_k * K * 1e-3 + further * max(per_cu - 1.0, 0.0) + (tail * rounds ** 0.5 if K % t[2] else 0.0)
+
+
+def product_block_shape(block, M, N, K, a_kmajor, b_kmajor, odd, cd_bytes) -> NT:
+    """The tile of a plain 16-bit product whose default is ``block``: another one where the closer estimate has it 8 % ahead, which it was at every one of 344 products that the fit had not seen
+    (at 5 % one in a hundred was slower, by up to 7 %).  Not for products small enough to end within the launch and its ends, nor for odd operands of a product that may run on copies of them.
+    us on the default and on this one, inputs that rotate: 1110 x 6976 x 1284 'T','N' 43.7 and 34.1, 646 x 5207 x 960 'N','T' 23.2 and 18.7, 2336 x 266 x 7288 'N','T' 34.5 and 24.7 (in slices),
+    6236 x 96 x 6584 35.3 and 27.6 (in slices), 2632 x 2392 x 259 with C 20.5 and 18.1; the other 51 of 60 drawn ones within 2 %."""
+    work = M * N * K
+    if work < 5e8 or sum(odd) and work >= 2.4e10:
+        return block
+    own = (block.M, block.N, block.K)
+    cost = {t: _product_cost(t, M, N, K, odd, cd_bytes) for t in _mfma_tiles(a_kmajor, b_kmajor)}
+    best = min(cost, key=cost.get)
+    return NT(M=best[0], N=best[1], K=best[2]) if own in cost and cost[best] < 0.92 * cost[own] else block
+
+
 def _rounds(t, tiles):
     """How many tile times a launch of ``tiles`` tiles of shape ``t`` takes.  A CU holds one workgroup of the tiles with
     144 or 128 KiB of LDS at a time: whole rounds.  The 128 x 128 tiles run one per CU on four LDS stages where every tile has a CU,

@@ -21,7 +21,7 @@ from . import kernel as Kernel
 from . import layout as Layout
 from . import operator as Operator
 from . import transform as Transform
-from .config import _MFMA_TILE_COST, Config, _mfma_cost, default_block_shape, get_config as _get_config, larger_tile, sliced_block_shape, split_k_block_shape
+from .config import _MFMA_TILE_COST, Config, _mfma_cost, default_block_shape, get_config as _get_config, larger_tile, product_block_shape, sliced_block_shape, split_k_block_shape
 from .dtypes import BFloat16, DType, Float16, Float32, Float64, from_torch, promote_type
 from .errors import ConfigError, DimensionMismatch
 from ._native import Prepared, load as load_native
@@ -611,6 +611,9 @@ def create_config(A: DType, sizeA, stridesA, transA: bool, B: DType, sizeB, stri
         block_shape = sliced_block_shape(m, n, k, max(stridesA[1], stridesB[1]), not (a_aligned and b_aligned)) or split_k_block_shape(m, n, k, max(0 if transA else stridesA[1], stridesB[1] if transB else 0), factor)
     if block_shape is None:
         block_shape = default_block_shape(operator, NT(M=m, N=n, K=k), tile_sized=not edge_ok, a_kmajor=transA, b_kmajor=not transB)
+        if use_mfma and edge_ok:
+            odd = (not a_aligned and transA) + (not b_aligned and not transB), (not a_aligned and not transA) + (not b_aligned and transB)
+            block_shape = product_block_shape(block_shape, m, n, k, transA, not transB, odd, C.size * (1 if zeroBeta else 2))
     global_a_layout, global_b_layout, global_c_layout, global_d_layout = layouts_for(block_shape)
     if not edge_ok and any(l.kind in (Layout.COL_MAJOR, Layout.ROW_MAJOR) for l in (global_a_layout, global_b_layout, global_c_layout, global_d_layout)):
         # some operand needs bounds checks (and C = beta C, the zero alpha): one tile shape
