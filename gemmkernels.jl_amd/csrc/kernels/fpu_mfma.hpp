@@ -21,7 +21,7 @@
 // LDS stages and leave the CU to several workgroups; the Float32 tiles of 128 x 128, and of 32 x 32 on four waves, three, with
 // the first fragments of the next tile read in front of the barrier, because they often have a CU to themselves.
 //
-// Measured (beta = 0, one box; before, on the vector ALUs): Float32 256^3 12.2 -> 4.7 us, 1024^3 71 -> 23, 2048^3
+// Measured (beta = 0, one box; before, on the vector ALUs): Float32 256^3 12.2 -> 4.4 us, 1024^3 71 -> 23, 2048^3
 // 293 -> 134, 3001 x 3003 x 2999 -> 461 (0.79 of the instruction's rate), 4096^3 1900 -> 1028 us (134 TFLOP/s, 0.90);
 // Float64 1000^3 115 -> 41 us, 2048^3 -> 270 (64 TFLOP/s, 0.83).  What is left: the last round of tiles (2560^3 has 1600
 // tiles of 64 x 64 for 256 CUs: 7 rounds where 6.25 would do), and the ends of a launch.

@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+import struct
 from dataclasses import dataclass, fields
 from typing import Optional
 
@@ -60,27 +61,15 @@ class Config:
         c = _lib.gk_config()
         cache[key] = c
 
-        def shape(dst, src):
-            dst.M, dst.N, dst.K = int(src.get("M", 0)), int(src.get("N", 0)), int(src.get("K", 0))
-
-        shape(c.matmul_shape, self.matmul_shape)
-        shape(c.block_shape, self.block_shape)
+        # (whole structs at their offsets: member by member this was half of a first launch's time on the host)
+        mine = self.__dict__
+        for name, at in _SHAPES_AT:
+            src = mine[name].get
+            _SHAPE.pack_into(c, at, int(src("M", 0)), int(src("N", 0)), int(src("K", 0)))
         c.warps_per_block = int(self.warps_per_block)
-        for name in ("mem_a_warp", "mem_a_thread", "mem_b_warp", "mem_b_thread", "mem_cd_warp", "mem_cd_thread",
-                     "compute_warp", "compute_op_shape"):
-            shape(getattr(c, name), getattr(self, name))
-
-        def lay(dst, src: Layout.LayoutType, ld=0):
-            dst.kind, dst.eltype, dst.pad, dst.ld = src.kind, src.T.code, src.pad, int(ld)
-
-        lay(c.global_a_layout, self.global_a_layout, lda)
-        lay(c.global_b_layout, self.global_b_layout, ldb)
-        lay(c.global_c_layout, self.global_c_layout, ldc)
-        lay(c.global_d_layout, self.global_d_layout, ldd)
-        lay(c.shared_a_layout, self.shared_a_layout)
-        lay(c.shared_b_layout, self.shared_b_layout)
-        lay(c.shared_c_layout, self.shared_c_layout)
-        lay(c.shared_d_layout, self.shared_d_layout)
+        for (name, at), ld in zip(_LAYOUTS_AT, (lda, ldb, ldc, ldd, 0, 0, 0, 0)):
+            src = mine[name]
+            _LAYOUT.pack_into(c, at, src.kind, src.T.code, src.pad, 0, int(ld))
         op = self.operator
         c.op.kind, c.op.M, c.op.N, c.op.K = op.kind, op.M, op.N, op.K
         c.op.mb, c.op.nb, c.op.kb = op.mb, op.nb, op.kb
@@ -99,6 +88,14 @@ class Config:
                 for i, (e, s0, s1) in enumerate(src):
                     dst.extent[i], dst.stride0[i], dst.stride1[i] = int(e), int(s0), int(s1)
         return c
+
+
+_SHAPE, _LAYOUT = struct.Struct("=3i"), struct.Struct("=4iq")
+_SHAPES_AT = tuple((name, getattr(_lib.gk_config, name).offset) for name in (
+    "matmul_shape", "block_shape", "mem_a_warp", "mem_a_thread", "mem_b_warp", "mem_b_thread", "mem_cd_warp", "mem_cd_thread", "compute_warp", "compute_op_shape"))
+_LAYOUTS_AT = tuple((name, getattr(_lib.gk_config, name).offset) for name in (
+    "global_a_layout", "global_b_layout", "global_c_layout", "global_d_layout", "shared_a_layout", "shared_b_layout", "shared_c_layout", "shared_d_layout"))
+assert _SHAPE.size == ctypes.sizeof(_lib.gk_shape) and _LAYOUT.size == ctypes.sizeof(_lib.gk_layout)
 
 
 def heuristic_block_shape(shared_a_layout, shared_b_layout, shared_c_layout, shared_d_layout) -> NT:

@@ -124,6 +124,9 @@ def _split_k_bytes(conf_c) -> int:
 
 def _sliced_bytes(conf_c, trans, epi) -> int:
     """Workspace of a launch that runs in slices of K (``gk_matmul_sliced``), 0 of any other."""
+    shape, block = conf_c.matmul_shape, conf_c.block_shape
+    if conf_c.op.kind == Operator.MFMA and (shape.K < 1280 or block.M != block.N or -(-shape.M // block.M) * -(-shape.N // block.N) > 170):
+        return 0              # (what the library cuts has fewer tiles and a longer K: a first launch need not ask)
     need = ctypes.c_size_t()
     rc = _lib.lib().gk_sliced_workspace_size(ctypes.byref(conf_c), ctypes.byref(trans) if trans is not None else None,
                                              ctypes.byref(epi) if epi is not None else None, ctypes.byref(need))
@@ -300,8 +303,8 @@ def _launched_as(conf: Config, a, b, c, d, hooks: bool, slices: bool = False) ->
 class Plan:
     """One launch with everything but the stream lowered ahead of time: the descriptors of the
     configuration, the transforms and the epilogue, and the operand addresses.  Calling the plan is
-    one call into the library (which still runs every launch-time check of reference
-    src/matmul.jl:28-41).  The plan keeps its operands alive; they must not be resized or freed by
+    one call into the library, which runs every launch-time check of reference
+    src/matmul.jl:28-41 on the first call and, where the launch needs no workspace, keeps what they found from the second on (``prepare``).  The plan keeps its operands alive; they must not be resized or freed by
     other means while it is in use.  For loops that launch the same GEMM many times, where the
     microseconds a general ``matmul`` call spends on lowering would rival the kernel itself."""
 
@@ -486,7 +489,7 @@ def matmul(conf: Config, a, b, c, d, *,
         for of in (larger, conf):                                   # (the tile asked for where the library refuses the larger one)
             if of is None or rc == _lib.GK_OK:
                 continue
-            cconf, need = of.to_c(*lds), 0
+            cconf, need = cconf if of is conf else of.to_c(*lds), 0
             if not hooks and of.operator.kind == Operator.MFMA:
                 known = of.__dict__.setdefault("_slices_of", {})             # (a Config is immutable once built)
                 need = known.get(lds)
@@ -817,7 +820,7 @@ _PACK_MAX_ROWS = 255 * 512          # of one launch of gk_pack_columns
 class _MulLaunch:
     """What ``matmatmul_`` hands to the library for operands of one kind (element types, sizes, strides, alignment) and one
     pair of factors: descriptors only, no address and no tensor, so any operands of that kind can use it, on any
-    stream and from any thread (nothing in it is written after it is made).  Lowering the same call again took 22 us of
+    stream and from any thread (nothing in it is written after it is made).  Lowering the same call again takes 22 us of
     interpreter time, the whole of a small product: mul! at 256^3 in Float32 takes 5 us on the device."""
 
     __slots__ = ("_fn", "_conf", "_trans", "_conf_ref", "_trans_ref", "_code", "_workspace", "_sliced", "_prepared")
