@@ -1232,6 +1232,8 @@ int launch_split_k(const gk_config* conf, const void* a, const void* b, const vo
   // (a tile or hooks without a K-split instance: unsplit, see has_split_k_instance)
   gk::FamilyFn sk_fn = L.key.family == gk::FAMILY_MFMA_CHECKED ? fn : gk::family_mfma_splitk;
   bool split = plan.slices > 1 && sk_fn && sk_fn(L.key, L.args, dim3(1), nullptr, 0, &sk_info, &err);
+  // (128 x 128 x 64 in slices takes 128 KiB of LDS, unsplit 64 KiB where no more is allowed)
+  if (split && sk_info.lds_bytes > 64 * 1024 && g_lds_override.load() > 0 && sk_info.lds_bytes > g_lds_override.load()) split = false;
   // a product whose last K tile runs outside the pipeline does not insist on a workspace: without it, it is the launch unsplit
   if (L.ragged && (!workspace || workspace_bytes < plan.bytes || ((uintptr_t)workspace & 15u) != 0)) split = false;
   if (split) {

@@ -95,3 +95,22 @@ def test_refused_and_other_tiles(gpu):
     half = lambda m, n: torch.empty(n, m, device="cuda", dtype=torch.float16).t()
     launch = gk.plan(conf, half(1024, 4096), half(4096, 2048), None, gk.colmajor_empty((1024, 2048), torch.float32), kernel=Kernel.matmul_pipelined)
     assert launch._sliced == 0 and launch._conf.block_shape.M == 64
+
+
+def test_k_split_launches_of_the_tile_within_a_limit_of_lds(gpu):
+    """Their slices have four LDS stages (128 KiB); where less is allowed the launch runs unsplit on two, and is not refused."""
+    import torch
+    from gemmkernels import _lib
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    M, N, K = 512, 384, 4096
+    a, b = whole(gen, M, K, torch.float16), whole(gen, K, N, torch.float16)
+    conf = configs.mfma_config(M, N, K, block_shape=(128, 128, 64), zero_c=True)
+    want = a.double() @ b.double()
+    try:
+        for limit in (0, 65536):
+            _lib.lib().gk_set_device_limits(limit, 0)
+            d = gk.colmajor_empty((M, N), torch.float32)
+            gk.matmul(conf, a, b, None, d, kernel=Kernel.matmul_split_k)
+            assert torch.equal(d.double(), want), limit
+    finally:
+        _lib.lib().gk_set_device_limits(0, 0)
