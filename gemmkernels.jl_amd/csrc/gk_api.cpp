@@ -921,6 +921,15 @@ int gk_cta_swizzle(const gk_config* conf, int32_t block_x, int32_t block_y, int3
   return GK_OK;
 }
 
+void gk_internal_tail_chunks(int32_t k_major, int32_t rows, int32_t cols, int32_t ld, int32_t rows_valid, int32_t tail_k, int32_t* from, int32_t* shift,
+                             int32_t* keep) {
+  for (int row = 0; row < rows; ++row)
+    for (int col = 0; col < cols; col += 8) {
+      const gk::TailChunk c = k_major ? gk::tail_chunk<true>(row, col, ld, rows, rows_valid, tail_k) : gk::tail_chunk<false>(row, col, ld, rows, rows_valid, tail_k);
+      *from++ = c.from; *shift++ = c.shift; *keep++ = c.keep;
+    }
+}
+
 int64_t gk_shmem_size(const gk_config* conf, int32_t kernel) {
   (void)kernel;
   if (!conf) { fail(GK_ERR_INVALID_ARGUMENT, "config is NULL"); return -1; }

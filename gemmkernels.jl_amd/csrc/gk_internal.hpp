@@ -28,3 +28,8 @@ int launch_split_k(const gk_config* conf, const void* a, const void* b, const vo
                    const gk_epilogue* epilogue, void* workspace, size_t workspace_bytes, const char* whose, void* stream);
 
 }  // namespace gk_internal
+
+// tail_chunk of every chunk of a tile on the host, with the code that the kernels inline, for tests of its arithmetic: `rows` x `cols` / 8 chunks, row by row
+// (a K-major tile: rows of M or N, k along them; else rows of k).
+extern "C" void gk_internal_tail_chunks(int32_t k_major, int32_t rows, int32_t cols, int32_t ld, int32_t rows_valid, int32_t tail_k, int32_t* from,
+                                        int32_t* shift, int32_t* keep);

@@ -105,6 +105,42 @@ __host__ __device__ inline void gett_offsets32_flat(const GettDim& d, int idx, l
   }
 }
 
+// A 16-byte chunk (8 elements) of a K tile that runs outside the pipeline of the matrix-core products: where a lane fetches it from, in elements from the
+// operand's first element in the tile, and what it repairs once the chunk has landed.  `row` and `col` are the chunk's place in the tile (K-major: row along M or N, col along k;
+// otherwise row along k, col along M or N); `tile_rows` are the rows of a K-major tile, `rows_valid` is what is left of the operand along M or N from the tile on, `tail_k` its k values in the tile.
+// Rows and k values outside read valid ones; a chunk that would reach past the operand's last element is fetched `shift` (0 .. 7) elements further back; the first
+// `keep` (0 .. 8) elements keep their value, the others are k values that are not there.
+// The arithmetic is in 32 bits: the rows of a tile lie less than 2^30 elements apart (the host refuses others).  That bounds the tile, not what is left of the operand
+// (131072 rows of 16400 are 2^31 elements), so of the rows behind the tile only the first counts: an end that lies there or further on is out of the reach of every chunk alike.
+struct TailChunk {
+  int from, shift, keep;
+};
+template <bool KMAJOR>
+__host__ __device__ inline TailChunk tail_chunk(int row, int col, int ld, int tile_rows, int rows_valid, int tail_k) {
+  TailChunk c;
+  int end;                                     // one past the operand's last element
+  if (KMAJOR) {
+    const int rows = rows_valid > tile_rows ? tile_rows + 1 : rows_valid;
+    row = row > rows - 1 ? rows - 1 : row;
+    c.keep = tail_k - col;
+    c.keep = c.keep < 0 ? 0 : (c.keep > 8 ? 8 : c.keep);
+    const int last = ((tail_k - 1) >> 3) << 3;
+    col = col > last ? last : col;
+    end = (rows - 1) * ld + tail_k;
+  } else {
+    const int last = ((rows_valid - 1) >> 3) << 3;
+    col = col > last ? last : col;
+    c.keep = row < tail_k ? 8 : 0;
+    row = row < tail_k ? row : tail_k - 1;
+    end = (tail_k - 1) * ld + rows_valid;
+  }
+  c.from = row * ld + col;
+  c.shift = c.from + 8 - end;
+  c.shift = c.shift < 0 ? 0 : c.shift;
+  c.from -= c.shift;
+  return c;
+}
+
 __host__ __device__ inline void gett_offsets(const GettDim& d, long long idx, long long& off0, long long& off1) {
   off0 = 0; off1 = 0;
   for (int i = 0; i < d.nmodes; ++i) {

@@ -907,10 +907,8 @@ __global__ void __launch_bounds__(Cfg::THREADS) mfma_gemm_kernel(const GemmArgs 
     }
   }
 
-  // The last K tile when it stands outside the pipeline (tail_k): every lane fetches its 16-byte chunks with coordinates clamped to
-  // valid ones -- a chunk that would reach past the last element of the operand is fetched from 1 .. 7 elements further back -- and
-  // repairs its own chunks in LDS once they have landed: shifted into place, values whose k is beyond K set to zero.  Offsets in a tile
-  // fit 32 bits (the host refuses others).
+  // The last K tile when it stands outside the pipeline (tail_k): every lane fetches its 16-byte chunks from where tail_chunk says
+  // and repairs its own chunks in LDS once they have landed: shifted into place, values whose k is beyond K set to zero.
   // per chunk: elements it was fetched too far back (0 .. 7), leading elements that keep their value (0 .. 8)
   [[maybe_unused]] int tail_shift[RAGGED_K ? DPT : 1], tail_keep[RAGGED_K ? DPT : 1];
   [[maybe_unused]] auto issue_tail = [&](int stage, auto gta, auto gtb) __attribute__((always_inline)) {
@@ -923,25 +921,10 @@ __global__ void __launch_bounds__(Cfg::THREADS) mfma_gemm_kernel(const GemmArgs 
       typedef decltype(geom) G;
       int row, col;
       dma_lane_coords<G, KIND>(q, l, row, col);
-      int& r = KIND == OPK_KMAJOR ? row : col;           // index along M (A) or N (B), from the tile origin
-      int& k = KIND == OPK_KMAJOR ? col : row;
-      const int last_r = KIND == OPK_KMAJOR ? rows_valid - 1 : ((rows_valid - 1) >> 3) << 3;
-      r = r > last_r ? last_r : r;
-      if (KIND == OPK_KMAJOR) {                          // the chunk runs along k
-        keep = tail_k - k;
-        keep = keep < 0 ? 0 : (keep > 8 ? 8 : keep);
-        const int last_k = ((tail_k - 1) >> 3) << 3;
-        k = k > last_k ? last_k : k;
-      } else {
-        keep = k < tail_k ? 8 : 0;
-        k = k < tail_k ? k : tail_k - 1;
-      }
-      const int e = row * ld + col;
-      // one past the last element of the operand, counted from the tile origin
-      const int end = KIND == OPK_KMAJOR ? (rows_valid - 1) * ld + tail_k : (tail_k - 1) * ld + rows_valid;
-      shift = e + 8 - end;
-      shift = shift < 0 ? 0 : shift;
-      __builtin_amdgcn_global_load_lds(GK_GLOBAL_PTR(g + (long long)(e - shift) * 2), GK_LDS_PTR(void, dst + q * 1024), 16, 0, 0);
+      const TailChunk c = tail_chunk<KIND == OPK_KMAJOR>(row, col, ld, G::LDS_ROWS, rows_valid, tail_k);
+      shift = c.shift;
+      keep = c.keep;
+      __builtin_amdgcn_global_load_lds(GK_GLOBAL_PTR(g + (long long)c.from * 2), GK_LDS_PTR(void, dst + q * 1024), 16, 0, 0);
     };
 #pragma unroll
     for (int i = 0; i < DMA_A; ++i)
