@@ -311,16 +311,20 @@ def _product_cost(t, M, N, K, odd, cd_bytes):
     return always + fixed + rounds * per_k * K * 1e-3 + further * max(per_cu - 1.0, 0.0) + (tail * rounds ** 0.5 if K % t[2] else 0.0)
 
 
-def product_block_shape(block, M, N, K, a_kmajor, b_kmajor, odd, cd_bytes) -> NT:
+def product_block_shape(block, M, N, K, a_kmajor, b_kmajor, odd, cd_bytes, lda=0, ldb=0) -> NT:
     """The tile of a plain 16-bit product whose default is ``block``: another one where the closer estimate has it 8 % ahead, which it was at every one of 344 products that the fit had not seen
     (at 5 % one in a hundred was slower, by up to 7 %).  Not for products small enough to end within the launch and its ends, nor for odd operands of a product that may run on copies of them.
     us on the default and on this one, inputs that rotate: 1110 x 6976 x 1284 'T','N' 43.7 and 34.1, 646 x 5207 x 960 'N','T' 23.2 and 18.7, 2336 x 266 x 7288 'N','T' 34.5 and 24.7 (in slices),
-    6236 x 96 x 6584 35.3 and 27.6 (in slices), 2632 x 2392 x 259 with C 20.5 and 18.1; the other 51 of 60 drawn ones within 2 %."""
+    6236 x 96 x 6584 35.3 and 27.6 (in slices), 2632 x 2392 x 259 with C 20.5 and 18.1; the other 51 of 60 drawn ones within 2 %.
+
+    ``lda``, ``ldb``: a tile whose rows lie too far apart for the kernels' offsets in 32 bits is refused by the library, so it is none of the candidates."""
     work = M * N * K
     if work < 5e8 or sum(odd) and work >= 2.4e10:
         return block
     own = (block.M, block.N, block.K)
-    cost = {t: _product_cost(t, M, N, K, odd, cd_bytes) for t in _mfma_tiles(a_kmajor, b_kmajor)}
+    tiles = _mfma_tiles(a_kmajor, b_kmajor)
+    tiles = [t for t in tiles if t == own or max((t[0] if a_kmajor else t[2]) * lda, (t[1] if b_kmajor else t[2]) * ldb) * 2 < 1 << 31]
+    cost = {t: _product_cost(t, M, N, K, odd, cd_bytes) for t in tiles}
     best = min(cost, key=cost.get)
     return NT(M=best[0], N=best[1], K=best[2]) if own in cost and cost[best] < 0.92 * cost[own] else block
 

@@ -616,7 +616,8 @@ def create_config(A: DType, sizeA, stridesA, transA: bool, B: DType, sizeB, stri
         block_shape = default_block_shape(operator, NT(M=m, N=n, K=k), tile_sized=not edge_ok, a_kmajor=transA, b_kmajor=not transB)
         if use_mfma and edge_ok:
             odd = (not a_aligned and transA) + (not b_aligned and not transB), (not a_aligned and not transA) + (not b_aligned and transB)
-            block_shape = product_block_shape(block_shape, m, n, k, transA, not transB, odd, C.size * (1 if zeroBeta else 2))
+            block_shape = product_block_shape(block_shape, m, n, k, transA, not transB, odd, C.size * (1 if zeroBeta else 2),
+                                              stridesA[1], stridesB[1])
     global_a_layout, global_b_layout, global_c_layout, global_d_layout = layouts_for(block_shape)
     if not edge_ok and any(l.kind in (Layout.COL_MAJOR, Layout.ROW_MAJOR) for l in (global_a_layout, global_b_layout, global_c_layout, global_d_layout)):
         # some operand needs bounds checks (and C = beta C, the zero alpha): one tile shape

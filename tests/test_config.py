@@ -392,6 +392,38 @@ def test_wide_leading_dimensions_keep_a_tile_that_takes_them(ta, tb):
     assert block(4096, 1 << 24) == (narrow if tb else split)
 
 
+def _product(M, N, K, ta, tb, lda, ldb):
+    """The tile of a mul! on these leading dimensions, and whether the library takes the launch."""
+    conf, _, kernel = create_config(Float16, (K, M) if ta else (M, K), (1, lda), ta, Float16, (N, K) if tb else (K, N), (1, ldb), tb, Float32, (M, N), (1, M), float, False, float, True)
+    prepared = ctypes.c_void_p()
+    rc = _lib.lib().gk_prepare(ctypes.byref(conf.to_c(lda, ldb, M, M)), None, None, kernel.code, ctypes.byref(prepared))
+    _lib.lib().gk_prepared_free(prepared)
+    return tuple(conf.block_shape.values()), rc == _lib.GK_OK
+
+
+def test_a_tile_in_the_place_of_the_default_takes_the_same_leading_dimensions(monkeypatch):
+    """Whatever runs on the default tile, or on 64 x 64 x 64 in slices, is not refused for the rows of a larger one, which lie 2^31 bytes apart earlier."""
+    import random
+    import sys
+    named = [(30377976, 23, 23, False, True, 30377976, 23), (820, 6777, 876, True, False, 876, 13095080), (430, 1876, 5605, True, True, 5605, 26034496),
+             (991, 3293, 565, True, False, 1 << 23, 565), (1352, 5510, 223, False, False, 1352, 1 << 24), (47, 3591, 6956, False, False, 47, 1 << 24)]
+    rng = random.Random(5)
+    for _ in range(1500):
+        M, N, K = (int(16 * 512 ** rng.random()) for _ in range(3))
+        ta, tb = rng.random() < 0.5, rng.random() < 0.5
+        lda, ldb = K if ta else M, N if tb else K
+        wide = rng.choice((1 << 20, 1 << 21, 1 << 22, 1 << 23, 1 << 24)) + rng.choice((-8, 0, 0, 1, 8))
+        which = rng.randrange(3)
+        named.append((M, N, K, ta, tb, wide if which != 1 else lda, wide if which != 0 else ldb))
+    mm = sys.modules["gemmkernels.matmul"]
+    now = [_product(*p) for p in named]
+    monkeypatch.setattr(mm, "product_block_shape", lambda block, *args: block)
+    monkeypatch.setattr(mm, "sliced_block_shape", lambda *args: None)
+    before = [_product(*p) for p in named]
+    assert all(ok for (_, ok), (_, was) in zip(now, before) if was), [(p, n, b) for p, n, b in zip(named, now, before) if b[1] and not n[1]]
+    assert sum(n[0] != b[0] for n, b in zip(now, before)) > 40 and sum(not b[1] for b in before) > 20
+
+
 @pytest.mark.parametrize("dims,tile,scale,slices", [((4096, 64, 4096), (64, 64, 64), None, 4), ((4096, 64, 4096), (64, 64, 64), 1.5, 6), ((64, 64, 8000), (64, 64, 64), None, 12),
                                                     ((8192, 64, 4096), (64, 64, 64), None, 2), ((960, 384, 4096), (64, 64, 64), None, 5), ((1792, 64, 7168), (64, 64, 64), None, 8),
                                                     ((832, 640, 4096), (64, 64, 64), None, 3), ((1024, 1024, 4096), (64, 64, 64), None, 2), ((320, 192, 9984), (64, 64, 64), None, 9),
