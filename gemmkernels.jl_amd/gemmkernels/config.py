@@ -288,6 +288,13 @@ _PRODUCT_COST = {(256, 256, 64): (1.89, 20.31, 8.62, 2.54, 3.74, 0.22, 0.08, 0.1
                  (256, 192, 64): (0.06, 18.16, 2.52, 1.82, 4.96, 0.2, 0.08, 0.19), (192, 256, 64): (3.72, 19.02, 2.44, 2.94, 0.35, 0.15, 0.14, 0.19)}
 _PRODUCT_ROUNDS = {(128, 128, 32): (0.75, 0.09, 1.59), (128, 128, 64): (0.49, 0.23, 1.66), (64, 64, 64): (0.75, 0.33, 1.08), (64, 64, 32): (0.62, 0.41, 1.12)}
 _PRODUCT_IN_SLICES = (2.88, 8.35, 1.06, 3.36, 0.04)
+_PRODUCT_FITTED_TO = 8192
+
+
+def _product_slices(t, M, N, K) -> int:
+    """How many slices of K the library cuts a plain product on this tile into (``gk_matmul_sliced``; 128 x 128 x 64 only)."""
+    tiles = -(-M // t[0]) * -(-N // t[1])
+    return min(NUM_CUS // tiles, K // (768 if tiles <= 85 else 1024)) if t == (128, 128, 64) and tiles <= 128 and K >= 2048 else 1
 
 
 def _product_cost(t, M, N, K, odd, cd_bytes):
@@ -296,8 +303,8 @@ def _product_cost(t, M, N, K, odd, cd_bytes):
     tiles = -(-M // t[0]) * -(-N // t[1])
     per_k *= 1.0 + odd_k * odd[0] + odd_mn * odd[1]
     always = per_mb * 1e-6 * M * N * cd_bytes + (edges if M % t[0] or N % t[1] else 0.0)
-    if t == (128, 128, 64) and tiles <= 128 and K >= 2048:
-        slices = min(NUM_CUS // tiles, K // (768 if tiles <= 85 else 1024))
+    slices = _product_slices(t, M, N, K)
+    if slices > 1:
         own = _PRODUCT_IN_SLICES
         return always + own[0] + own[1] * per_k / _PRODUCT_COST[t][1] * -(-K // (64 * slices)) * 0.064 + own[2] * slices + own[3] * slices * tiles / NUM_CUS + (own[4] if K % 64 else 0.0)
     per_cu = tiles / NUM_CUS
@@ -317,12 +324,16 @@ def product_block_shape(block, M, N, K, a_kmajor, b_kmajor, odd, cd_bytes, lda=0
     us on the default and on this one, inputs that rotate: 1110 x 6976 x 1284 'T','N' 43.7 and 34.1, 646 x 5207 x 960 'N','T' 23.2 and 18.7, 2336 x 266 x 7288 'N','T' 34.5 and 24.7 (in slices),
     6236 x 96 x 6584 35.3 and 27.6 (in slices), 2632 x 2392 x 259 with C 20.5 and 18.1; the other 51 of 60 drawn ones within 2 %.
 
+    The fit knows extents up to 8192.  Beyond (to 262144), of 70 drawn products that it moved 17 were slower, none of them in slices (1387 x 169454 x 71 253.6 and 424.4, 14832 x 552 x 64584 1391
+    and 1559), so only the slices are taken there: of 50 others all faster, on average 1.7 times (1792 x 464 x 65960 309 and 195, 568 x 1424 x 37808 227 and 111).
     ``lda``, ``ldb``: a tile whose rows lie too far apart for the kernels' offsets in 32 bits is refused by the library, so it is none of the candidates."""
     work = M * N * K
     if work < 5e8 or sum(odd) and work >= 2.4e10:
         return block
     own = (block.M, block.N, block.K)
     tiles = _mfma_tiles(a_kmajor, b_kmajor)
+    if max(M, N, K) > _PRODUCT_FITTED_TO:
+        tiles = [t for t in tiles if t == own or _product_slices(t, M, N, K) > 1]
     tiles = [t for t in tiles if t == own or max((t[0] if a_kmajor else t[2]) * lda, (t[1] if b_kmajor else t[2]) * ldb) * 2 < 1 << 31]
     cost = {t: _product_cost(t, M, N, K, odd, cd_bytes) for t in tiles}
     best = min(cost, key=cost.get)

@@ -424,6 +424,14 @@ def test_a_tile_in_the_place_of_the_default_takes_the_same_leading_dimensions(mo
     assert sum(n[0] != b[0] for n, b in zip(now, before)) > 40 and sum(not b[1] for b in before) > 20
 
 
+@pytest.mark.parametrize("dims,ta,tb,tile", [((1387, 169454, 71), False, False, (128, 128, 32)), ((14832, 552, 64584), False, True, (256, 256, 64)), ((554, 14494, 403), True, True, (64, 64, 32)),
+                                             ((192512, 16, 7744), True, False, (64, 64, 64)), ((85096, 2638, 71), True, True, (128, 128, 32)),
+                                             ((568, 1424, 37808), True, True, (128, 128, 64)), ((68, 6169, 14597), False, True, (128, 128, 64))])
+def test_extents_beyond_those_of_the_fit_keep_the_default_or_run_in_slices(dims, ta, tb, tile):
+    M, N, K = dims
+    assert _product(M, N, K, ta, tb, K if ta else M, N if tb else K) == (tile, True)
+
+
 @pytest.mark.parametrize("dims,tile,scale,slices", [((4096, 64, 4096), (64, 64, 64), None, 4), ((4096, 64, 4096), (64, 64, 64), 1.5, 6), ((64, 64, 8000), (64, 64, 64), None, 12),
                                                     ((8192, 64, 4096), (64, 64, 64), None, 2), ((960, 384, 4096), (64, 64, 64), None, 5), ((1792, 64, 7168), (64, 64, 64), None, 8),
                                                     ((832, 640, 4096), (64, 64, 64), None, 3), ((1024, 1024, 4096), (64, 64, 64), None, 2), ((320, 192, 9984), (64, 64, 64), None, 9),
