@@ -50,6 +50,13 @@ class Config:
         width = max(len(f.name) for f in fields(self)) + 2
         return "\n".join(f"{(f.name + ':').ljust(width)}{getattr(self, f.name)}" for f in fields(self)) + "\n"
 
+    def __getstate__(self):
+        # (copies and pickles: the fields and whether the tile was left open; descriptors and launches that were kept are made again)
+        mine = {f.name: getattr(self, f.name) for f in fields(self)}
+        if "_tile_left_open" in self.__dict__:
+            mine["_tile_left_open"] = self.__dict__["_tile_left_open"]
+        return mine
+
     def to_c(self, lda: int = 0, ldb: int = 0, ldc: int = 0, ldd: int = 0) -> _lib.gk_config:
         """Lower to the POD of the C ABI; leading dimensions come from the arrays of the call.
         The result is cached per set of leading dimensions (a Config is immutable once built)."""

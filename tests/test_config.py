@@ -493,3 +493,24 @@ def test_the_slices_a_product_is_launched_in(dims, dtype, alpha, slices):
     if slices > 1:
         most = (need - 2048) // (tiles * bs.M * bs.N * 4)
         assert most == slices or tiles <= 128 and most > slices
+
+
+def test_a_configuration_that_was_launched_is_copied_and_pickled_like_any_other():
+    """What a launch keeps with its configuration (descriptors, launches checked once, the larger tile) is not part of it."""
+    import copy
+    import pickle
+    import sys
+    from gemmkernels import configs
+    mm = sys.modules["gemmkernels.matmul"]
+    conf = configs.mfma_config(2240, 5568, 2304)
+    lds = (2240, 2304, 2240, 2240)
+    for _ in range(2):                                 # (what matmul() does with its first and its second launch)
+        mm._prepare(conf, conf.to_c(*lds), lds, Kernel.matmul_pipelined)
+    assert (lds, Kernel.matmul_pipelined) in conf.__dict__["_prepared"]
+    larger = cfgmod.larger_tile(conf, False)
+    for again in (copy.copy(conf), copy.deepcopy(conf), pickle.loads(pickle.dumps(conf))):
+        assert again == conf and again is not conf and "_prepared" not in again.__dict__
+        assert cfgmod.larger_tile(again, False) == larger and larger is not None
+        assert bytes(again.to_c(*lds)) == bytes(conf.to_c(*lds)) and again.to_c(*lds) is not conf.to_c(*lds)
+    own = pickle.loads(pickle.dumps(configs.mfma_config(2240, 5568, 2304, block_shape=(64, 64, 64))))
+    assert cfgmod.larger_tile(own, False) is None      # (a tile that was asked for)
