@@ -313,4 +313,7 @@ PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "gk_torch", nullptr, -1, g_method
 
 }  // namespace
 
+// The interpreter and the torch that this was built for: at::Tensor is read inline, so no other may load it (_native.py compares).
+extern "C" const char gk_torch_built_for[] = GK_BUILT_FOR;
+
 PyMODINIT_FUNC PyInit_gk_torch(void) { return PyModule_Create(&g_module); }

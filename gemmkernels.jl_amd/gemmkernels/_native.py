@@ -5,10 +5,15 @@ from __future__ import annotations
 import ctypes
 import importlib.util
 import os
+import sys
+from typing import Optional
 
 from . import _lib
+from ._built_for import built_for
 
 _PATH = os.path.join(os.path.dirname(_lib.LIB_PATH), "gk_torch.so")
+
+
 class Prepared:
     """A launch that has passed every check but those of its addresses (gk_prepare), or one without a handle where the library makes none."""
 
@@ -31,13 +36,24 @@ _module = None
 _tried = False
 
 
+def _built_for_of(path: str) -> Optional[str]:
+    try:
+        return ctypes.string_at(ctypes.addressof(ctypes.c_char.in_dll(ctypes.CDLL(path), "gk_torch_built_for"))).decode()
+    except (OSError, ValueError):               # (not to be linked here; a module that does not say)
+        return None
+
+
 def load():
     global _module, _tried
-    if not _tried:
+    if not _tried and "torch" in sys.modules:                # (without it there are no tensors to read, and nothing to link against)
         lib = _lib.lib()
         _tried = True
         if os.path.exists(_PATH):
             try:
+                # (looked at before any of it runs: it would read the tensors of another torch at wrong offsets)
+                what = _built_for_of(_PATH)
+                if what is None or what != built_for():
+                    return None
                 spec = importlib.util.spec_from_file_location("gk_torch", _PATH)
                 module = importlib.util.module_from_spec(spec)
                 spec.loader.exec_module(module)
