@@ -300,6 +300,30 @@ def _launched_as(conf: Config, a, b, c, d, hooks: bool, slices: bool = False) ->
     return larger
 
 
+_AB_HOOKS = ("transform_global_to_shared_a", "transform_shared_to_regs_a", "transform_global_to_shared_b", "transform_shared_to_regs_b")
+_lists = {}
+
+
+def _lists_in_the_k_loop(conf: Config, transforms: dict) -> bool:
+    """Whether the hooks of A and B stay in the K loop as op lists (one factor per operand is folded or multiplied in, see the library's fused levels).  Such a launch
+    keeps its tile: its time is that of the lists, of which the estimates know nothing.  Of 67 drawn plans that a larger tile took 20 were slower on it, up to twice
+    (3648 x 3456 x 4032 'T','N' with a list on B 783 -> 1629 us), and those on the tile that stands for slices, of which there are none with lists, all were (1088 x 1088 x 5248 'N','T' with one on A 240 -> 437).
+    With hooks on C and D, a bias or factors all of 53 were faster."""
+    if conf.operator.kind != Operator.MFMA or all(transforms[h].is_identity for h in _AB_HOOKS):
+        return False
+    key = (conf.global_a_layout.kind, conf.global_a_layout.T.name, *(transforms[h].ops for h in _AB_HOOKS))
+    known = _lists.get(key)
+    if known is None:
+        if len(_lists) >= 256:
+            _lists.clear()
+        try:
+            known = kernel_name(conf, Kernel.matmul_pipelined, {h: transforms[h] for h in _AB_HOOKS}).endswith("_fused_ab")
+        except ConfigError:
+            return True                   # (what the launch says)
+        _lists[key] = known
+    return known
+
+
 class Plan:
     """One launch with everything but the stream lowered ahead of time: the descriptors of the
     configuration, the transforms and the epilogue, and the operand addresses.  Calling the plan is
@@ -319,7 +343,9 @@ class Plan:
         self._trans = None if specialized is not None else lower_transforms(transforms)
         self._as_given = None                                      # (what is launched where the library refuses the larger tile)
         hooks = self._trans is not None or epilogue.kind != Epilogue.DEFAULT
-        larger = _launched_as(conf, a, b, c, d, hooks, slices) if specialized is None and kernel is not Kernel.matmul_split_k else None
+        larger = None
+        if specialized is None and kernel is not Kernel.matmul_split_k and not (hooks and _lists_in_the_k_loop(conf, transforms)):
+            larger = _launched_as(conf, a, b, c, d, hooks, slices)
         if larger is not None:
             self._as_given, self._conf = self._conf, _lib.gk_config.from_buffer_copy(larger.to_c(*lds))
         self._epi = None
@@ -485,7 +511,9 @@ def matmul(conf: Config, a, b, c, d, *,
     else:
         args = (_ptr(a), _ptr(b), _ptr(c), _ptr(d), ctrans, cepi, kernel.code, stream)
         hooks = ctrans is not None or cepi is not None
-        larger, rc = _launched_as(conf, a, b, c, d, hooks, not hooks), _lib.GK_ERR_UNSUPPORTED
+        larger, rc = None, _lib.GK_ERR_UNSUPPORTED
+        if ctrans is None or not _lists_in_the_k_loop(conf, collected):
+            larger = _launched_as(conf, a, b, c, d, hooks, not hooks)
         for of in (larger, conf):                                   # (the tile asked for where the library refuses the larger one)
             if of is None or rc == _lib.GK_OK:
                 continue

@@ -26,6 +26,25 @@ def test_the_rule():
         assert gk.kernel_name(conf, Kernel.matmul_pipelined)
 
 
+LIST = Transform.Elementwise(lambda x: x * 0.5 + 0.25)
+
+
+@pytest.mark.parametrize("M,N,K,larger", [(1088, 1088, 5248, (128, 128, 64)), (2240, 5568, 2304, (128, 128, 64)), (3648, 3456, 4032, (128, 256, 64))])
+@pytest.mark.parametrize("hooks,moves", [(dict(transform_shared_to_regs_a=Transform.Elementwise(lambda x: x * 1.5)), True), (dict(transform_global_to_shared_b=Transform.Elementwise(lambda x: -x)), True),
+                                         (dict(transform_shared_to_global_d=LIST), True), (dict(transform_global_to_shared_a=LIST), False),
+                                         (dict(transform_shared_to_regs_b=Transform.Elementwise(Transform.relu)), False),
+                                         (dict(transform_global_to_shared_a=Transform.Elementwise(lambda x: x * 1.5), transform_shared_to_regs_a=Transform.Elementwise(lambda x: x * 3)), False)])
+def test_op_lists_in_the_k_loop_keep_their_tile(M, N, K, larger, hooks, moves):
+    # (no GPU: a plan is lowered, not launched)
+    torch = pytest.importorskip("torch")
+    conf = configs.mfma_config(M, N, K, zero_c=True)
+    half = lambda m, n: torch.empty((n, m), dtype=torch.float16).t()
+    launch = gk.plan(conf, half(M, K), half(K, N), None, torch.empty((N, M)).t(), kernel=Kernel.matmul_pipelined, **hooks)
+    block = launch._conf.block_shape
+    assert (block.M, block.N, block.K) == (larger if moves else shape(conf))
+    assert (launch._sliced > 0) == (moves and M == 1088)
+
+
 CASES = [(2240, 5568, 2304, False), (4544, 2048, 2368, False), (2368, 5376, 384, False), (2752, 3712, 1984, True), (1152, 5184, 4800, True), (2240, 2496, 5696, True)]
 
 
