@@ -332,7 +332,7 @@ class Plan:
     other means while it is in use.  For loops that launch the same GEMM many times, where the
     microseconds a general ``matmul`` call spends on lowering would rival the kernel itself."""
 
-    __slots__ = ("_fn", "_conf", "_trans", "_epi", "_args", "_keep", "_split_k", "_sliced", "_as_given", "_direct", "_calls", "d", "kernel_names")
+    __slots__ = ("_fn", "_conf", "_trans", "_epi", "_args", "_keep", "_split_k", "_sliced", "_slices", "_as_given", "_direct", "_calls", "d", "kernel_names")
 
     def __init__(self, conf: Config, a, b, c, d, transforms: dict, epilogue, kernel, specialized=None, slices=False):
         if specialized is None and any(t.expr is not None for t in transforms.values()):
@@ -349,7 +349,7 @@ class Plan:
         if larger is not None:
             self._as_given, self._conf = self._conf, _lib.gk_config.from_buffer_copy(larger.to_c(*lds))
         self._epi = None
-        self._split_k, self._sliced = False, 0
+        self._split_k, self._sliced, self._slices = False, 0, slices
         if epilogue.kind != Epilogue.DEFAULT:
             self._epi = _lib.gk_epilogue()
             self._epi.kind = epilogue.kind
@@ -397,15 +397,18 @@ class Plan:
         if self._sliced:
             workspace = _workspace(self._sliced, stream)
             rc = self._fn(*self._args, *_span(workspace), stream)
-            if rc != _lib.GK_OK and self._as_given is not None:
-                rc = _lib.lib().gk_matmul(ctypes.byref(self._as_given), *self._args[1:], stream)
         else:
             direct = self._direct
             if direct is not None and _native.run_at(*direct[1], stream) == _lib.GK_OK:
                 return self.d
             rc = self._fn(*self._args, stream)
-            if rc != _lib.GK_OK and self._as_given is not None:
-                rc = self._fn(ctypes.byref(self._as_given), *self._args[1:], stream)
+        if rc != _lib.GK_OK and self._as_given is not None:
+            need = _sliced_bytes(self._as_given, self._trans, self._epi) if self._slices else 0
+            if need:
+                workspace = _workspace(need, stream)
+                rc = _lib.lib().gk_matmul_sliced(ctypes.byref(self._as_given), *self._args[1:], *_span(workspace), stream)
+            else:
+                rc = _lib.lib().gk_matmul(ctypes.byref(self._as_given), *self._args[1:], stream)
         if rc != _lib.GK_OK:
             _raise(rc)
         return self.d
@@ -513,12 +516,14 @@ def matmul(conf: Config, a, b, c, d, *,
         hooks = ctrans is not None or cepi is not None
         larger, rc = None, _lib.GK_ERR_UNSUPPORTED
         if ctrans is None or not _lists_in_the_k_loop(conf, collected):
-            larger = _launched_as(conf, a, b, c, d, hooks, not hooks)
+            larger = _launched_as(conf, a, b, c, d, hooks, conf.operator.kind == Operator.MFMA)
         for of in (larger, conf):                                   # (the tile asked for where the library refuses the larger one)
             if of is None or rc == _lib.GK_OK:
                 continue
             cconf, need = cconf if of is conf else of.to_c(*lds), 0
-            if not hooks and of.operator.kind == Operator.MFMA:
+            if of.operator.kind == Operator.MFMA and hooks:                  # (what a plan with these arguments launches)
+                need = _sliced_bytes(cconf, ctrans, cepi)
+            elif of.operator.kind == Operator.MFMA:
                 known = of.__dict__.setdefault("_slices_of", {})             # (a Config is immutable once built)
                 need = known.get(lds)
                 if need is None:
@@ -527,7 +532,8 @@ def matmul(conf: Config, a, b, c, d, *,
                     need = known[lds] = _sliced_bytes(cconf, None, None)
             if need:
                 workspace = _workspace(need, stream)
-                rc = _lib.lib().gk_matmul_sliced(ctypes.byref(cconf), *args[:4], None, None, kernel.code, *_span(workspace), stream)
+                rc = _lib.lib().gk_matmul_sliced(ctypes.byref(cconf), *args[:4], ctypes.byref(ctrans) if ctrans is not None else None,
+                                                 ctypes.byref(cepi) if cepi is not None else None, kernel.code, *_span(workspace), stream)
             else:
                 rc = _gk_matmul(cconf, *args)
                 if rc == _lib.GK_OK and plain:
