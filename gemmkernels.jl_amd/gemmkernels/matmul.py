@@ -207,6 +207,28 @@ def _workspace(need: int, stream: int):
     return buf
 
 
+_RETRY_AFTER = 256          # calls, after an allocation that failed: each one gives the allocator's cache back and waits for the device
+_calls_without = {}         # (device, stream) -> calls that go without before memory is asked for again
+
+
+def _workspace_if_any(need: int, stream: int):
+    """``_workspace`` for a launch that is in slices of K without having been asked to: None where there is no memory for it (the library then
+    launches it unsplit)."""
+    import torch
+    key = (torch.cuda.current_device(), int(stream))
+    waiting = _calls_without.get(key, 0)
+    if waiting > 0:
+        buf = _workspaces.get(key)
+        if buf is None or buf.numel() < need:
+            _calls_without[key] = waiting - 1
+            return None
+    try:
+        return _workspace(need, stream)
+    except torch.OutOfMemoryError:
+        _calls_without[key] = _RETRY_AFTER - 1
+        return None
+
+
 _IDENTITY = Transform.Elementwise()
 _DEFAULT_EPILOGUE = Epilogue.Default()
 _lowered = {}
@@ -395,7 +417,7 @@ class Plan:
                 _raise(rc)
             return self.d
         if self._sliced:
-            workspace = _workspace(self._sliced, stream)
+            workspace = _workspace_if_any(self._sliced, stream)
             rc = self._fn(*self._args, *_span(workspace), stream)
         else:
             direct = self._direct
@@ -405,7 +427,7 @@ class Plan:
         if rc != _lib.GK_OK and self._as_given is not None:
             need = _sliced_bytes(self._as_given, self._trans, self._epi) if self._slices else 0
             if need:
-                workspace = _workspace(need, stream)
+                workspace = _workspace_if_any(need, stream)
                 rc = _lib.lib().gk_matmul_sliced(ctypes.byref(self._as_given), *self._args[1:], *_span(workspace), stream)
             else:
                 rc = _lib.lib().gk_matmul(ctypes.byref(self._as_given), *self._args[1:], stream)
@@ -531,7 +553,7 @@ def matmul(conf: Config, a, b, c, d, *,
                         known.clear()
                     need = known[lds] = _sliced_bytes(cconf, None, None)
             if need:
-                workspace = _workspace(need, stream)
+                workspace = _workspace_if_any(need, stream)
                 rc = _lib.lib().gk_matmul_sliced(ctypes.byref(cconf), *args[:4], ctypes.byref(ctrans) if ctrans is not None else None,
                                                  ctypes.byref(cepi) if cepi is not None else None, kernel.code, *_span(workspace), stream)
             else:
@@ -872,7 +894,7 @@ class _MulLaunch:
 
     def __call__(self, a: int, b: int, c: int, stream: int) -> None:
         if self._sliced:
-            workspace = _workspace(self._sliced, stream)
+            workspace = _workspace_if_any(self._sliced, stream)
             rc = self._fn(self._conf_ref, a, b, c, c, self._trans_ref, None, self._code, *_span(workspace), stream)
         elif self._workspace is None:
             rc = self._fn(self._conf_ref, a, b, c, c, self._trans_ref, None, self._code, stream)
@@ -893,8 +915,6 @@ class _MulLaunchOnCopies(_MulLaunch):
     after the launch is made: threads that meet on it try once more or less.)"""
 
     __slots__ = ("_packed", "_packed_ref", "_copies", "_copy_bytes", "_calls_without")
-
-    _RETRY_AFTER = 256
 
     def __init__(self, p: Plan, packed):
         super().__init__(p)
@@ -927,7 +947,7 @@ class _MulLaunchOnCopies(_MulLaunch):
         try:
             copies = torch.empty(self._copy_bytes, dtype=torch.uint8, device="cuda")
         except torch.OutOfMemoryError:
-            self._calls_without = self._RETRY_AFTER - 1
+            self._calls_without = _RETRY_AFTER - 1
             return False
         base, operands, jobs = copies.data_ptr(), [a, b], []
         for which, at, source, copy in self._copies:
