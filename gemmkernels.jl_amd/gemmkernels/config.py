@@ -66,13 +66,14 @@ class Config:
         if hit is not None:
             return hit
         c = _lib.gk_config()
-        cache[key] = c
-
         # (whole structs at their offsets: member by member this was half of a first launch's time on the host)
         mine = self.__dict__
         for name, at in _SHAPES_AT:
             src = mine[name].get
-            _SHAPE.pack_into(c, at, int(src("M", 0)), int(src("N", 0)), int(src("K", 0)))
+            try:
+                _SHAPE.pack_into(c, at, int(src("M", 0)), int(src("N", 0)), int(src("K", 0)))
+            except struct.error:
+                raise ConfigError(f"{name} must be below 2^31, got {tuple(mine[name].values())}") from None
         c.warps_per_block = int(self.warps_per_block)
         for (name, at), ld in zip(_LAYOUTS_AT, (lda, ldb, ldc, ldd, 0, 0, 0, 0)):
             src = mine[name]
@@ -94,6 +95,7 @@ class Config:
                 dst.nmodes = len(src)
                 for i, (e, s0, s1) in enumerate(src):
                     dst.extent[i], dst.stride0[i], dst.stride1[i] = int(e), int(s0), int(s1)
+        cache[key] = c                      # (whole: other threads may look for it meanwhile)
         return c
 
 

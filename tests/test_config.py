@@ -495,6 +495,18 @@ def test_the_slices_a_product_is_launched_in(dims, dtype, alpha, slices):
         assert most == slices or tiles <= 128 and most > slices
 
 
+@pytest.mark.parametrize("shape", [(1 << 31, 64, 64), (64, (1 << 31) + 64, 64), (64, 64, 1 << 31), ((1 << 32) + 64, 64, 64)])
+def test_extents_beyond_32_bits_are_refused(shape):
+    """As a ConfigError, like any other extent that does not fit (2^32 + 64 rows were 64 once)."""
+    from gemmkernels import configs
+    with pytest.raises(ConfigError, match="matmul_shape must be"):
+        configs.mfma_config(*shape)
+    M, N, K = shape
+    for dtype in (Float16, Float32):
+        with pytest.raises(ConfigError, match="matmul_shape must be"):
+            create_config(dtype, (M, K), (1, M), False, dtype, (K, N), (1, K), False, Float32, (M, N), (1, M), float, False, float, True)
+
+
 def test_a_configuration_that_was_launched_is_copied_and_pickled_like_any_other():
     """What a launch keeps with its configuration (descriptors, launches checked once, the larger tile) is not part of it."""
     import copy
