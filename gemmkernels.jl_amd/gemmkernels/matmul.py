@@ -326,7 +326,7 @@ _AB_HOOKS = ("transform_global_to_shared_a", "transform_shared_to_regs_a", "tran
 _lists = {}
 
 
-def _lists_in_the_k_loop(conf: Config, transforms: dict) -> bool:
+def _lists_in_the_k_loop(conf: Config, cconf, trans, transforms: dict) -> bool:
     """Whether the hooks of A and B stay in the K loop as op lists (one factor per operand is folded or multiplied in, see the library's fused levels).  Such a launch
     keeps its tile: its time is that of the lists, of which the estimates know nothing.  Of 67 drawn plans that a larger tile took 20 were slower on it, up to twice
     (3648 x 3456 x 4032 'T','N' with a list on B 783 -> 1629 us), and those on the tile that stands for slices, of which there are none with lists, all were (1088 x 1088 x 5248 'N','T' with one on A 240 -> 437).
@@ -338,11 +338,10 @@ def _lists_in_the_k_loop(conf: Config, transforms: dict) -> bool:
     if known is None:
         if len(_lists) >= 256:
             _lists.clear()
-        try:
-            known = kernel_name(conf, Kernel.matmul_pipelined, {h: transforms[h] for h in _AB_HOOKS}).endswith("_fused_ab")
-        except ConfigError:
-            return True                   # (what the launch says)
-        _lists[key] = known
+        name = ctypes.create_string_buffer(256)
+        if _lib.lib().gk_kernel_name(ctypes.byref(cconf), ctypes.byref(trans), None, Kernel.matmul_pipelined.code, name, len(name)) != _lib.GK_OK:
+            return True                   # (refused: the launch says why)
+        known = _lists[key] = name.value.endswith(b"_fused_ab")
     return known
 
 
@@ -366,7 +365,7 @@ class Plan:
         self._as_given = None                                      # (what is launched where the library refuses the larger tile)
         hooks = self._trans is not None or epilogue.kind != Epilogue.DEFAULT
         larger = None
-        if specialized is None and kernel is not Kernel.matmul_split_k and not (hooks and _lists_in_the_k_loop(conf, transforms)):
+        if specialized is None and kernel is not Kernel.matmul_split_k and not (self._trans is not None and _lists_in_the_k_loop(conf, self._conf, self._trans, transforms)):
             larger = _launched_as(conf, a, b, c, d, hooks, slices)
         if larger is not None:
             self._as_given, self._conf = self._conf, _lib.gk_config.from_buffer_copy(larger.to_c(*lds))
@@ -537,7 +536,7 @@ def matmul(conf: Config, a, b, c, d, *,
         args = (_ptr(a), _ptr(b), _ptr(c), _ptr(d), ctrans, cepi, kernel.code, stream)
         hooks = ctrans is not None or cepi is not None
         larger, rc = None, _lib.GK_ERR_UNSUPPORTED
-        if ctrans is None or not _lists_in_the_k_loop(conf, collected):
+        if ctrans is None or not _lists_in_the_k_loop(conf, cconf, ctrans, collected):
             larger = _launched_as(conf, a, b, c, d, hooks, conf.operator.kind == Operator.MFMA)
         for of in (larger, conf):                                   # (the tile asked for where the library refuses the larger one)
             if of is None or rc == _lib.GK_OK:
