@@ -1142,23 +1142,25 @@ static_assert(kSplitCounterBytes / sizeof(unsigned) >= 2 * (size_t)gk::kNumCUs -
 // workgroup's path), so slices are at least 640 deep in K, and no more workgroups start than two per CU, what a CU holds of
 // these tiles at a time.
 //
-// 64 x 64 x 64 without hooks on A or B: as many slices as give every CU one workgroup, rather than some CUs two (us by slices):
-//   4096 x 64 x 4096 (64 tiles) 3 12.0, 4 12.5, 6 13.1, 8 14.3; 1024 x 256 x 16384 (64) 4 23.9, 8 27.1; 287 x 589 x 7104 (50) 5 15.0,
-//   10 16.8; 8192 x 64 x 4096 (128) 2 18.7, 4 21.0; 2560 x 128 x 5120 (80) 3 13.4, 6 14.4;
+// (us by slices, inputs that rotate through 400 MB, in brackets the tiles)
+// 64 x 64 x 64 without hooks on A or B: as many slices as give every CU one workgroup, rather than some CUs two:
+//   4096 x 64 x 4096 (64) 3 14.7, 4 14.0, 6 15.8, 8 15.6; 287 x 589 x 7104 (50) 5 15.7, 10 17.2; 8192 x 64 x 4096 (128) 2 20.5, 4 22.1;
+//   2560 x 128 x 5120 (80) 3 17.7, 6 17.6; the other way 1024 x 256 x 16384 (64) 4 31.0, 8 29.2;
 // two per CU where one leaves a fifth of the CUs idle and two no more than a sixth:
-//   960 x 384 x 4096 (90) 2 14.1, 5 12.4; 1600 x 256 x 8192 (100) 2 21.8, 5 18.5; 3000 x 128 x 6000 (94) 2 21.9, 5 20.1;
-//   700 x 900 x 3001 (165) 1 34.4, 2 24.4, 3 20.0;
+//   960 x 384 x 4096 (90) 2 14.9, 3 14.4, 5 14.0; 1600 x 256 x 8192 (100) 2 24.2, 5 21.2; 3000 x 128 x 6000 (94) 2 28.1, 5 24.7;
+//   700 x 900 x 3001 (165) 1 26.2, 2 24.2, 3 20.5;
 // and with few tiles, whose slices all end at once, not many unless they are 1024 deep:
-//   1776 x 33 x 7392 (28) 7 14.4, 8 14.4, 11 16.0; 300 x 200 x 9001 (20) 9 15.4, 14 18.9; 1085 x 47 x 6136 (17) 6 15.0, 9 13.9;
-//   64 x 64 x 8000 (1) 7 10.6, 12 10.0; 64 x 64 x 32768 (1) 24 15.3, 32 15.8, 51 18.0.
-// A factor on A or B (AB_HOOKS) makes the K loop longer and what a slice costs weigh less: up to two per CU.  FP16 4096 x 64 x 4096
-//   'T','N' 4 13.8, 6 12.9; BF16 with op lists on A (level 2) 4 66.5, 6 61.6, 8 57.0, 7 x 7 x 20000 (1) 19 54.2, 31 46.6.  BF16 with one factor (level 1),
-//   whose loop is little longer, lies within 5 % of its best on the same slices: 4096 x 64 x 4096 'N','N' 4 15.9, 6 16.1, 8 16.3; 7 x 7 x 20000 19 17.1, 31 16.2;
-//   512 x 512 x 4096 (64) 4 15.2, 6 14.1, 8 13.7; 2048 x 128 x 8192 (64) 6 20.5, 8 18.2, 10 23.6; 960 x 384 x 4096 (90) 3 18.0, 5 15.6, 6 19.2; 8192 x 64 x 4096 (128) 2 23.3, 4 24.2.
-// 128 x 128 x 64 (figures on two LDS stages), whose partial tiles are four times as large: 768 deep (1024 above 64 tiles), sixteen slices or 2048 deep:
-//   512 x 512 x 4096 (16) 4 22.7, 5 22.0, 6 21.8; 2048 x 512 x 4096 (64) 4 25.3, 5 25.3, 6 26.2; 1536 x 1024 x 4096 (96) 4 29.5, 5 30.6;
-//   256 x 256 x 16384 (4) 12 34.4, 16 35.5, 25 40.2.
-// Other tiles (64 x 64 x 32): 4096 x 64 x 4096 (64) 4 24.4, 6 21.1, 7 20.6, 8 21.3.
+//   1776 x 33 x 7392 (28) 7 14.0, 8 13.7, 11 16.9; 300 x 200 x 9001 (20) 9 15.9, 14 17.7; 1085 x 47 x 6136 (17) 6 15.1, 9 14.0;
+//   64 x 64 x 8000 (1) 7 9.4, 12 9.1; 64 x 64 x 32768 (1) 24 16.2, 32 16.2, 51 18.3.
+// A factor on A or B (AB_HOOKS) makes the K loop longer and what a slice costs weigh less: up to two per CU.  That line is from op lists, BF16
+//   4096 x 64 x 4096 4 66.5, 6 61.6, 8 57.0, 7 x 7 x 20000 (1) 19 54.2, 31 46.6.  One factor (level 1), whose loop is little longer, lies between the two:
+//   BF16 4096 x 64 x 4096 4 14.6, 6 16.5, 8 16.2 (FP16 'T','N' 4 13.2, 6 14.9); 7 x 7 x 20000 19 14.8, 31 15.0; 512 x 512 x 4096 (64) 4 14.1, 6 14.3, 8 13.2;
+//   2048 x 128 x 8192 (64) 6 23.4, 8 20.8, 10 24.3; 960 x 384 x 4096 (90) 3 17.4, 5 14.8, 6 18.7; 8192 x 64 x 4096 (128) 2 20.5, 4 22.9.
+// 128 x 128 x 64, whose partial tiles are four times as large: 768 deep (1024 above 64 tiles), sixteen slices or 2048 deep.  (On four LDS stages, one
+//   workgroup per CU, fewer are ahead with 33 to 128 tiles; the callers who ask for the kind have chosen its error, see sliced_route for those who have not.)
+//   512 x 512 x 4096 (16) 4 17.8, 5 16.8, 6 16.4; 2048 x 512 x 4096 (64) 3 23.9, 4 21.4, 5 29.0; 1536 x 1024 x 4096 (96) 2 28.8, 4 33.7, 5 32.4;
+//   256 x 256 x 16384 (4) 12 25.7, 16 25.1, 25 27.5.
+// Other tiles (64 x 64 x 32): 4096 x 64 x 4096 (64) 4 25.8, 6 25.6, 7 25.8, 8 25.9.
 //
 // Where the partial tiles of that many slices would not fit the library's static workspace (512 tiles of 128 x 128 and the
 // counters are 2 KiB more than it holds) the slices are 1024 deep: what fits it at that depth is not refused.
@@ -1301,8 +1303,9 @@ struct Prepared {
 };
 
 // Slices of K of a Float32 / Float64 product: the number with the shortest estimated launch, in us per 1000 k by the workgroups of a CU, plus what
-// the slices cost (workspace and counter; measured in fpu_mfma_splitk.hip).  `chain`: what one chain takes on the instances that such a launch runs on unsplit.
-// Slices are taken where they are estimated a tenth faster than one chain.
+// the slices cost (workspace and counter; measured in fpu_mfma_splitk.hip).  `chain`: what one chain takes on the instances that such a launch runs
+// on unsplit.  Slices are taken where they are estimated a tenth faster than one chain (300 drawn products, extents from 8, K from 200 to 60000: all
+// faster but one that is level, 1.3 times on average below K = 800, 3.5 times above).
 int fpu_slices(const gk::InstanceKey& key, int tiles, int K) {
   const bool f64 = key.dtype == gk::DT_F64, large = key.BM == 64;
   if ((large && f64) || tiles > (int)(kSplitCounterBytes / sizeof(unsigned))) return 1;
@@ -1349,15 +1352,16 @@ Sliced sliced_route(const gk::InstanceKey& as_asked, const gk::GemmArgs& args) {
     // (BLOCK_K = 32 where it runs on K tiles of 64 unsplit as well)
     if (key.family == gk::FAMILY_MFMA && key.BK == 32 && args.K % 64 == 0 && deep_instance(key, args)) key.BK = 64;
     if (key.BK != 64 || key.waves_m != 2 || key.waves_n != 2) return r;
-    // (us, one chain with the branches it had then -> slices: plans 704 x 320 x 5056 (55 tiles) 20.7 -> 11.1, 448 x 960 x 4544 (105) 20.8 -> 13.9, 384 x 448 x 1984 (42) 11.9 -> 9.2,
-    // 256 x 1536 x 2304 (96) 11.9 -> 9.3; contractions of M x N x K = 640 x 448 x 4096 (70) 24.2 -> 15.6, 640 x 1088 x 4096 (170) 24.2 -> 17.8, 1536 x 768 x 4096 (288, one chain) 29.6 -> 24.6.
-    // The lines are those of mul!, split_k_block_shape in config.py, less two slices of 171 to 256 tiles, which are level there.)
+    // (us, one chain -> slices, inputs that rotate through 400 MB: plans 704 x 320 x 5056 (55 tiles) 23.7 -> 12.4, 256 x 1024 x 5184 (64) 24.6 -> 12.4, 448 x 960 x 4544
+    // (105) 21.8 -> 15.9, 256 x 1536 x 2304 (96) 13.0 -> 10.9, 384 x 448 x 1984 (42) 8.4 -> 8.2; contractions of M x N x K = 640 x 448 x 4096 (70) 20.1 -> 13.5,
+    // 640 x 1088 x 4096 (170) 25.3 -> 21.3.  The lines are those of mul!, split_k_block_shape in config.py, less two slices of 171 to 256 tiles, which are level there.)
     r.fn = key.family == gk::FAMILY_MFMA ? gk::family_mfma_splitk : gk::family_mfma_splitk_gett;
     if (args.K >= (tiles <= 64 ? 1280 : (tiles <= 128 ? 2048 : 3000)) && tiles <= 170)
       r.slices = split_k_slices(tiles, (args.K + 63) / 64, gk_shape{64, 64, 64}, key.fused == 1);
   } else if (key.family == gk::FAMILY_MFMA && key.BM == 128 && key.BN == 128 && key.BK == 64 && key.waves_m == 2 && key.waves_n == 2) {
-    // One workgroup of four LDS stages per CU, of slices that are 768 deep (1024 above 85 tiles, of which a CU each is left for two).  (As many as two per CU, which a K-split launch of this tile takes, whose callers chose its error: the time
-    // of one per CU is 0.98 of it with up to 32 tiles, 0.87 with 33 to 64, 0.83 with 65 to 85, 0.92 with 86 to 128, averages over 180 drawn products.)
+    // One workgroup of four LDS stages per CU, of slices that are 768 deep (1024 above 85 tiles, of which a CU each is left for two).  (As many as two
+    // per CU, which a K-split launch of this tile takes, whose callers chose its error: the time of one per CU is 0.98 of it with up to 32 tiles,
+    // 0.87 with 33 to 64, 0.83 with 65 to 85, 0.92 with 86 to 128, averages over 180 drawn products.)
     r.fn = gk::family_mfma_splitk;
     if (tiles <= gk::kNumCUs / 2 && args.K >= 2048) r.slices = std::min(gk::kNumCUs / tiles, args.K / (tiles <= 85 ? 768 : 1024));
   }

@@ -72,7 +72,7 @@ std::unordered_map<Kind, Launch, KindHash> g_launches;
 std::unordered_map<uint64_t, Workspace> g_workspaces[16];     // per device: by stream
 constexpr size_t kMaxLaunches = 1024;
 
-// A plain matrix on the current device; false: not for this module.
+// A plain matrix on a device; false: not for this module.
 bool read_matrix(PyObject* obj, int which, Kind* kind, char** address) {
   if (!THPVariable_CheckExact(obj)) return false;
   const at::Tensor& t = THPVariable_Unpack(obj);

@@ -15,16 +15,18 @@ _PATH = os.path.join(os.path.dirname(_lib.LIB_PATH), "gk_torch.so")
 
 
 class Prepared:
-    """A launch that has passed every check but those of its addresses (gk_prepare), or one without a handle where the library makes none."""
+    """A launch that has passed every check but those of its addresses (gk_prepare), or one without a handle where the library makes none.
+    (The bias of an epilogue is the caller's to keep.)"""
 
-    __slots__ = ("handle", "_free", "_keep")
+    __slots__ = ("handle", "_free")
 
-    def __init__(self, conf_c, trans, epi, code: int, keep=None):
+    def __init__(self, conf_c, trans, epi, code: int):
         handle = ctypes.c_void_p()
         lib = _lib.lib()
-        rc = lib.gk_prepare(ctypes.byref(conf_c), ctypes.byref(trans) if trans is not None else None, ctypes.byref(epi) if epi is not None else None, code, ctypes.byref(handle))
+        rc = lib.gk_prepare(ctypes.byref(conf_c), ctypes.byref(trans) if trans is not None else None, ctypes.byref(epi) if epi is not None else None, code,
+                            ctypes.byref(handle))
         self.handle = handle.value if rc == _lib.GK_OK else None
-        self._free, self._keep = lib.gk_prepared_free, keep          # (keep: the bias of the epilogue)
+        self._free = lib.gk_prepared_free
 
     def __del__(self):
         if getattr(self, "handle", None):

@@ -234,21 +234,28 @@ def default_block_shape(operator, gemm_shape, tile_sized: bool = True, gett: boo
 
 def split_k_block_shape(M, N, K, widest_ld=0, factor=None) -> Optional[NT]:
     """The tile of a 16-bit product with few output tiles and a long K, which is cut into slices of K (``Kernel.matmul_split_k``), or None (the
-    default tile, and one chain over K).  In us, slices against unsplit with four LDS stages: 64 tiles K = 1280 7.5 and 7.5, 2048 8.7 and 10.5, 4096
-    11.1 and 17.6; 128 tiles K = 1280 8.6 and 7.9, 2048 9.8 and 10.7; three slices of 165 tiles K = 3072 13.0 and 14.7, 4096 14.3 and 18.1.
-    (The K loop without branches, on which both sides run now, takes about a tenth off each of the figures here: 64 tiles K = 4096 with C 11.3.)
+    default tile, and one chain over K).  us, slices and unsplit on four LDS stages, inputs that rotate through 400 MB, 'N','N':
+        64 tiles (4096 x 64)        K = 1280 9.6 and 10.7, 2048 10.4 and 14.3, 4096 14.0 and 25.6
+        128 tiles (8192 x 64)       K = 1280 10.6 and 11.1, 2048 13.7 and 14.8
+        165 tiles, three slices     K = 3072 15.5 and 17.0, 4096 17.9 and 21.3
 
-    171 to 256 tiles leave two slices, which are there for the error as well: half the chain has 2.9e-7 of the norm where the whole has 4.1e-7 (K = 4096,
-    FP16 uniform in [-1, 1); 1.5e-7 and 3e-7 on values of one sign; 4.1 and 5.7e-7, 2.2 and 4.3e-7 at K = 8192).  Their time, 'N','N' / 'T','N':
-    K = 8192 180 tiles 29.5 and 32.1 / 28.1 and 31.1, 210 tiles 30.0 and 32.3 / 28.4 and 31.3, 256 tiles 32.3 and 32.4 / 28.2 and 31.8; K = 16384 256 tiles
-    80.0 and 86.1 / 67.5 and 72.6; K = 4096 180 tiles 18.0 and 18.1 / 17.0 and 17.6, 256 tiles 19.2 and 18.1 / 17.6 and 17.8; 256 tiles K = 3072 16.2 and 14.7
-    / 15.4 and 14.4; 1001 x 704 x 3328 20.9 and 18.1 / 15.7 and 16.0; 1024 x 768 x 4004 21.5 and 22.4 / 25.3 and 24.3.  Not where K and the output are both
-    ragged (1001 x 700 x 3333, 1000 x 1000 x 4000).
+    171 to 256 tiles leave two slices, which are there for the error as well: half the chain has 2.9e-7 of the norm where the whole has 4.1e-7
+    (K = 4096, FP16 uniform in [-1, 1); 1.5e-7 and 3e-7 on values of one sign; 4.1 and 5.7e-7, 2.2 and 4.3e-7 at K = 8192).  Their time, two
+    slices and unsplit, 'N','N' / 'T','N':
+        K = 3072     256 tiles 21.0 and 19.3 / 19.2 and 17.2
+        K = 4096     180 tiles 19.4 and 21.7 / 18.4 and 20.6, 256 tiles 25.3 and 24.3 / 22.6 and 20.6
+        K = 8192     180 tiles 32.1 and 39.3 / 30.7 and 35.8, 210 tiles 32.4 and 38.7 / 31.5 and 36.3, 256 tiles 43.4 and 44.9 / 36.9 and 36.5
+        K = 16384    256 tiles 79.9 and 86.4 / 68.4 and 70.7
+        K = 3328     1001 x 704 24.8 and 23.4 / 19.3 and 18.0;    K = 4004     1024 x 768 26.2 and 30.7 / 32.6 and 32.1
+    Not where K and the output are both ragged (1001 x 700 x 3333, 1000 x 1000 x 4000).
 
-    ``factor``: alpha stays in the K loop (None: it does not), which makes it longer, and two slices pay whatever the extents: FP16 111 x 2629 x 1477 (84 tiles) 15.7
-    and 19.9; two slices, BF16, 1024 x 1024 x 4096 24.4 and 32.9, 768 x 1024 x 4096 23.8 and 32.5, 1001 x 1001 x 5001 37.6 and 43.5, 960 x 896 x 8192 41.2 and 61.5, 1000 x 900 x 3001
-    25.0 and 29.0, 70 x 7000 x 3500 31.0 and 32.3, 12000 x 64 x 4096 33.1 and 34.3 ('T','N' 33.6 and 33.4).  ``widest_ld``: the larger leading dimension of the operands whose rows are the k of a tile; the kernel keeps the offsets in a tile
-    in 32 bits, so 64 rows of 2^24 elements are left to a tile with fewer."""
+    ``factor``: alpha stays in the K loop (None: it does not), which makes it longer, and two slices are taken whatever the extents.  FP16
+    111 x 2629 x 1477 (84 tiles) 12.9 and 16.4.  BF16, two slices and unsplit: 768 x 1024 x 4096 23.6 and 26.5, 960 x 896 x 8192 41.0 and 49.0,
+    1024 x 1024 x 4096 26.6 and 26.9, 1001 x 1001 x 5001 42.2 and 41.6, 1000 x 900 x 3001 26.4 and 26.1; and with an extent that fills no tile or
+    one, where the slices are behind, 70 x 7000 x 3500 28.9 and 26.1, 12000 x 64 x 4096 32.3 and 27.8.
+
+    ``widest_ld``: the larger leading dimension of the operands whose rows are the k of a tile; the kernel keeps the offsets in a tile in 32
+    bits, so 64 rows of 2^24 elements are left to a tile with fewer."""
     if 64 * widest_ld * 2 >= 1 << 31:
         return None
     tiles = -(-M // 64) * -(-N // 64)
@@ -261,12 +268,15 @@ def split_k_block_shape(M, N, K, widest_ld=0, factor=None) -> Optional[NT]:
 
 
 def sliced_block_shape(M, N, K, widest_ld=0, odd=False) -> Optional[NT]:
-    """128 x 128 x 64 for a 16-bit product whose tiles of that size leave CUs idle and whose K is long enough for slices of them to be ahead of tiles of 64 x 64, cut or not
-    (``gk_matmul_sliced``), or None.  A 64 x 64 tile brings twice the bytes per product into a CU, and more than 256 of them are not cut (a few more than 256 take as long as 512).
-    us, 64 x 64 -> 128 x 128 in slices, inputs that rotate: 1472 x 768 x 5888 'N','T' 34.2 -> 24.0, 1088 x 1088 x 5248 'N','T' 31.5 -> 24.3, 704 x 1664 x 4544 'T','T' 26.6 -> 22.3, 2944 x 384 x 3712 24.0 -> 19.2;
-    below the line 384 x 4160 x 2496 18.0 and 21.5, 1088 x 1728 x 3136 21.6 and 26.7.  ``odd``: an operand whose columns start off 16-byte boundaries, whose rows of a small tile lie on
-    relatively more lines: 326 x 3462 x 3056 'T','T' 26.6 -> 19.5, 2048 x 560 x 2542 'T','N' 22.3 -> 18.5, 2624 x 517 x 3296 32.1 -> 24.1, 539 x 2592 x 7990 with a factor 79.9 -> 50.7.  Error
-    against 64 bits: never larger than that of the one chain it replaces (two slices or three).
+    """128 x 128 x 64 for a 16-bit product whose tiles of that size leave CUs idle and whose K is long enough for slices of them to be ahead of
+    tiles of 64 x 64, cut or not (``gk_matmul_sliced``), or None.  A 64 x 64 tile brings twice the bytes per product into a CU, and more than 256 of
+    them are not cut (a few more than 256 take as long as 512).  us, 64 x 64 -> 128 x 128 in slices, inputs that rotate:
+        1472 x 768 x 5888 'N','T' 34.2 -> 24.0, 1088 x 1088 x 5248 'N','T' 31.5 -> 24.3, 704 x 1664 x 4544 'T','T' 26.6 -> 22.3,
+        2944 x 384 x 3712 24.0 -> 19.2; below the line 384 x 4160 x 2496 18.0 and 21.5, 1088 x 1728 x 3136 21.6 and 26.7.
+    ``odd``: an operand whose columns start off 16-byte boundaries, whose rows of a small tile lie on relatively more lines:
+        326 x 3462 x 3056 'T','T' 26.6 -> 19.5, 2048 x 560 x 2542 'T','N' 22.3 -> 18.5, 2624 x 517 x 3296 32.1 -> 24.1,
+        539 x 2592 x 7990 with a factor 79.9 -> 50.7.
+    Error against 64 bits: never larger than that of the one chain it replaces (two slices or three).
     ``widest_ld``: the largest leading dimension; the kernel keeps the offsets in a tile in 32 bits."""
     tiles, small = -(-M // 128) * -(-N // 128), -(-M // 64) * -(-N // 64)
     if small <= 256 or tiles > 128 or K < (2500 if odd else 3500) or 128 * widest_ld * 2 >= 1 << 31:
@@ -287,9 +297,11 @@ _MFMA_TILE_COST = {(256, 256, 64): (12.0, 16.4, 39.0, 21.0, 1.2), (256, 256, 32)
                    (256, 192, 64): (5.4, 17.1, 19.3, 9.1, 7.9), (192, 256, 64): (5.0, 17.1, 15.3, 10.4, 7.9)}
 
 
-# The same for plain products on any leading dimension, closer: the five above, per operand whose columns start off 16-byte boundaries (contiguous along k, along m or n) what the K loop takes
-# longer, per MB of C and D, and of the smaller tiles how many tile times one to two (a + b (tiles per CU - 1)) and more of them in a CU take.  Fitted to 1500 products
-# drawn like those that `mul_` is timed on, every tile of each, and the sliced launches of 128 x 128 x 64 (us, per 1000 k, per slice, per workgroup of a CU, for a partial last K tile).
+# The same for plain products on any leading dimension, closer: the five above, per operand whose columns start off 16-byte boundaries (contiguous
+# along k, along m or n) what the K loop takes longer, per MB of C and D, and of the smaller tiles how many tile times one to two (a + b (tiles per
+# CU - 1)) and more of them in a CU take.  Fitted to 1500 products drawn like those that `mul_` is timed on, extents 16 to 8192, every tile of each,
+# and the sliced launches of 128 x 128 x 64 (us, per 1000 k, per slice, per workgroup of a CU, for a partial last K tile).  _MFMA_TILE_COST stays the
+# estimate of what this one knows nothing of: contractions, complex and configured products, copies, and the default that it has to be ahead of.
 _PRODUCT_COST = {(256, 256, 64): (1.89, 20.31, 8.62, 2.54, 3.74, 0.22, 0.08, 0.16), (256, 256, 32): (0, 23.88, 4.11, 1.26, 5.98, 0.17, 0.01, 0.19),
                  (256, 128, 64): (4.72, 12.53, 5.58, 2.69, 1.4, 0.18, 0.08, 0.13), (128, 256, 64): (4.74, 13, 5.41, 3, 1.35, 0.18, 0.1, 0.13),
                  (128, 128, 32): (3.71, 7.92, 1.13, 0.9, 0.82, 0.34, 0.08, 0.12), (128, 128, 64): (3.65, 7.93, 0.99, 1.52, 0.78, 0.22, 0.11, 0.12),
@@ -307,7 +319,8 @@ def _product_slices(t, M, N, K) -> int:
 
 
 def _product_cost(t, M, N, K, odd, cd_bytes):
-    """Estimated microseconds of a plain product; ``odd``: operands whose columns start off 16-byte boundaries, contiguous along k and not; ``cd_bytes``: of C and D per output."""
+    """Estimated microseconds of a plain product; ``odd``: operands whose columns start off 16-byte boundaries, contiguous along k and not;
+    ``cd_bytes``: of C and D per output."""
     fixed, per_k, further, tail, edges, odd_k, odd_mn, per_mb = _PRODUCT_COST[t]
     tiles = -(-M // t[0]) * -(-N // t[1])
     per_k *= 1.0 + odd_k * odd[0] + odd_mn * odd[1]
@@ -315,7 +328,8 @@ def _product_cost(t, M, N, K, odd, cd_bytes):
     slices = _product_slices(t, M, N, K)
     if slices > 1:
         own = _PRODUCT_IN_SLICES
-        return always + own[0] + own[1] * per_k / _PRODUCT_COST[t][1] * -(-K // (64 * slices)) * 0.064 + own[2] * slices + own[3] * slices * tiles / NUM_CUS + (own[4] if K % 64 else 0.0)
+        chain = own[1] * per_k / _PRODUCT_COST[t][1] * -(-K // (64 * slices)) * 0.064
+        return always + own[0] + chain + own[2] * slices + own[3] * slices * tiles / NUM_CUS + (own[4] if K % 64 else 0.0)
     per_cu = tiles / NUM_CUS
     if t not in _PRODUCT_ROUNDS:
         rounds = -(-tiles // NUM_CUS)
@@ -328,14 +342,18 @@ def _product_cost(t, M, N, K, odd, cd_bytes):
 
 
 def product_block_shape(block, M, N, K, a_kmajor, b_kmajor, odd, cd_bytes, lda=0, ldb=0) -> NT:
-    """The tile of a plain 16-bit product whose default is ``block``: another one where the closer estimate has it 8 % ahead, which it was at every one of 344 products that the fit had not seen
-    (at 5 % one in a hundred was slower, by up to 7 %).  Not for products small enough to end within the launch and its ends, nor for odd operands of a product that may run on copies of them.
-    us on the default and on this one, inputs that rotate: 1110 x 6976 x 1284 'T','N' 43.7 and 34.1, 646 x 5207 x 960 'N','T' 23.2 and 18.7, 2336 x 266 x 7288 'N','T' 34.5 and 24.7 (in slices),
+    """The tile of a plain 16-bit product whose default is ``block``: another one where the closer estimate has it 8 % ahead, which it was at every
+    one of 344 products that the fit had not seen (at 5 % one in a hundred was slower, by up to 7 %).  Not for products small enough to end within
+    the launch and its ends, nor for odd operands of a product that may run on copies of them.  us on the default and on this one, inputs that
+    rotate: 1110 x 6976 x 1284 'T','N' 43.7 and 34.1, 646 x 5207 x 960 'N','T' 23.2 and 18.7, 2336 x 266 x 7288 'N','T' 34.5 and 24.7 (in slices),
     6236 x 96 x 6584 35.3 and 27.6 (in slices), 2632 x 2392 x 259 with C 20.5 and 18.1; the other 51 of 60 drawn ones within 2 %.
 
-    The fit knows extents up to 8192.  Beyond (to 262144), of 70 drawn products that it moved 17 were slower, none of them in slices (1387 x 169454 x 71 253.6 and 424.4, 14832 x 552 x 64584 1391
-    and 1559), so only the slices are taken there: of 50 others all faster, on average 1.7 times (1792 x 464 x 65960 309 and 195, 568 x 1424 x 37808 227 and 111).
-    ``lda``, ``ldb``: a tile whose rows lie too far apart for the kernels' offsets in 32 bits is refused by the library, so it is none of the candidates."""
+    The fit knows extents up to 8192.  Beyond (to 262144), of 70 drawn products that it moved 17 were slower, none of them in slices
+    (1387 x 169454 x 71 253.6 and 424.4, 14832 x 552 x 64584 1391 and 1559), so only the slices are taken there: of 50 others all faster, on
+    average 1.7 times (1792 x 464 x 65960 309 and 195, 568 x 1424 x 37808 227 and 111).
+
+    ``lda``, ``ldb``: a tile whose rows lie too far apart for the kernels' offsets in 32 bits is refused by the library, so it is none of the
+    candidates."""
     work = M * N * K
     if work < 5e8 or sum(odd) and work >= 2.4e10:
         return block
@@ -565,17 +583,23 @@ _ANY_SIZE = {Layout.ALIGNED_COL_MAJOR: Layout.ColMajor, Layout.ALIGNED_ROW_MAJOR
 
 
 def larger_tile(conf: Config, hooks: bool, slices: bool = False) -> Optional[Config]:
-    """The configuration that a launch of ``conf`` runs on where the tile was left to the default and one that does not divide the sizes is faster, or None.
+    """The configuration that a launch of ``conf`` runs on where the tile was left to the default and one that does not divide the sizes is faster,
+    or None.
 
-    Aligned layouts ask for sizes in whole tiles (reference src/config.jl:268-275), so most multiples of 64 leave only the 64 x 64 tiles, which bring every
-    operand into the CUs four times as often as 256 x 256 ones do.  The kernels take tiles over the edges on any layout (one
-    launch, the same bits: every output is summed in the same order), so the launch is that of the bounds-checked layouts on the tile with the shortest
-    estimate, once the operands have passed for what the aligned ones ask (``matmul``).  us on the tile that divides and on the larger one, and the ratio of the
-    estimates, inputs that rotate: 2240 x 5568 x 2304 'N','N' with C 100.0 and 69.9 (0.52), 4544 x 2048 x 2368 'T','N' 70.8 and 47.9 (0.68), 1344 x 2880 x 5696 'T','T' 64.7 and 58.3 (0.71),
-    1600 x 4480 x 2048 'N','T' with C 54.9 and 47.5 (0.75), 5632 x 2240 x 384 24.2 and 20.7 (0.84), 5120 x 4224 x 5888 with C 285.8 and 269.4 (0.84); beyond the line 1920 x 1856 x 2368 27.9 and 29.2 (0.90),
-    2368 x 3072 x 896 with C 28.4 and 30.0 (0.90).  ``hooks``: transforms or a bias, which tiles of 256 x 256 over the edges run on eight waves (5376 x 2176 x 768 with C 47.5 and 53.0,
-    3520 x 2432 x 2048 72.4 and 76.1, so not those) and which the estimates leave out: 5696 x 5760 x 4160 with C 440 and 320 on 128 x 128 (0.57), 4992 x 1344 x 4416 99.6 and 73.7 (0.70), 4608 x 832 x 6080 75.5
-    and 61.6 (0.71); beyond the line 5056 x 768 x 2176 29.1 and 31.0 (0.85).  ``slices``: the launch may run in slices of K (``sliced_block_shape``)."""
+    Aligned layouts ask for sizes in whole tiles (reference src/config.jl:268-275), so most multiples of 64 leave only the 64 x 64 tiles, which
+    bring every operand into the CUs four times as often as 256 x 256 ones do.  The kernels take tiles over the edges on any layout, so the launch
+    is that of the bounds-checked layouts on the tile with the shortest estimate, once the operands have passed for what the aligned ones ask
+    (``matmul``): every output is summed in the same order, except in slices.  us on the tile that divides and on the larger one, and the ratio of
+    the estimates, inputs that rotate:
+        2240 x 5568 x 2304 'N','N' with C 100.0 and 69.9 (0.52), 4544 x 2048 x 2368 'T','N' 70.8 and 47.9 (0.68), 1344 x 2880 x 5696 'T','T' 64.7 and
+        58.3 (0.71), 1600 x 4480 x 2048 'N','T' with C 54.9 and 47.5 (0.75), 5632 x 2240 x 384 24.2 and 20.7 (0.84), 5120 x 4224 x 5888 with C 285.8
+        and 269.4 (0.84); beyond the line 1920 x 1856 x 2368 27.9 and 29.2 (0.90), 2368 x 3072 x 896 with C 28.4 and 30.0 (0.90).
+    Extents up to 131072, with and without hooks: 81 drawn ones all faster, 1.01 to 2.5 times.
+    ``hooks``: transforms or a bias, which tiles of 256 x 256 over the edges run on eight waves (5376 x 2176 x 768 with C 47.5 and 53.0,
+    3520 x 2432 x 2048 72.4 and 76.1, so not those) and which the estimates leave out: 5696 x 5760 x 4160 with C 440 and 320 on 128 x 128 (0.57),
+    4992 x 1344 x 4416 99.6 and 73.7 (0.70), 4608 x 832 x 6080 75.5 and 61.6 (0.71); beyond the line 5056 x 768 x 2176 29.1 and 31.0 (0.85).  (Not for
+    op lists on A or B, see ``matmul``.)
+    ``slices``: the launch may run in slices of K (``sliced_block_shape``)."""
     if not conf.__dict__.get("_tile_left_open") or conf.operator.kind != Operator.MFMA or conf.global_a_layout.kind not in _ANY_SIZE:
         return None
     name = ("_larger_tile_with_hooks" if hooks else "_larger_tile") + ("_in_slices" if slices else "")

@@ -22,6 +22,7 @@ from . import layout as Layout
 from . import operator as Operator
 from . import transform as Transform
 from .config import _MFMA_TILE_COST, Config, _mfma_cost, default_block_shape, get_config as _get_config, larger_tile, product_block_shape, sliced_block_shape, split_k_block_shape
+from .config import _product_slices
 from .dtypes import BFloat16, DType, Float16, Float32, Float64, from_torch, promote_type
 from .errors import ConfigError, DimensionMismatch
 from ._native import Prepared, load as load_native
@@ -728,7 +729,7 @@ def _single_plan(C, tA: bool, tB: bool, A, B, alpha, beta, wmma=None) -> Plan:
         # ordered, so the result is the same on every run, like the reference's mul!.
         bs, ms = conf.block_shape, conf.matmul_shape
         tiles = -(-ms.M // bs.M) * -(-ms.N // bs.N)
-        sliced = (bs.M, bs.N, bs.K) == (128, 128, 64) and tiles <= 128 and ms.K >= 2048
+        sliced = _product_slices((bs.M, bs.N, bs.K), ms.M, ms.N, ms.K) > 1
         if not sliced and (bs == split_k_block_shape(ms.M, ms.N, ms.K, 0, factor) or tiles <= 128 and ms.K >= 2048):
             kernel = Kernel.matmul_split_k
     else:
@@ -876,7 +877,8 @@ _PACK_MAX_ROWS = 255 * 512          # of one launch of gk_pack_columns
 class _MulLaunch:
     """What ``matmatmul_`` hands to the library for operands of one kind (element types, sizes, strides, alignment) and one
     pair of factors: descriptors only, no address and no tensor, so any operands of that kind can use it, on any
-    stream and from any thread (nothing in it is written after it is made).  Lowering the same call again takes 22 us of
+    stream and from any thread.  (What is written after it is made is the launch checked once for gk_torch: threads that meet there make one too
+    many.)  Lowering the same call again takes 22 us of
     interpreter time, the whole of a small product: mul! at 256^3 in Float32 takes 5 us on the device."""
 
     __slots__ = ("_fn", "_conf", "_trans", "_conf_ref", "_trans_ref", "_code", "_workspace", "_sliced", "_prepared")

@@ -290,20 +290,21 @@ int gk_matmul_split_k(const gk_config* conf, const void* a, const void* b, const
                       size_t workspace_bytes, void* stream);
 
 /* gk_matmul for a caller that brings a workspace (as gk_matmul_split_k takes it, and may share it with) and leaves the order of the
- * sums to the library: the same launch, in slices of K on its own tile where that is estimated to be faster: products with few
- * output tiles and a long K, Float32 and Float64 ones of FPUOp with hooks of at most one scale on A, on B and on C, real MFMA ones on 64 x 64 x 64
- * tiles with a K-split instance, contractions on that tile without hooks.  The result does not change from run to run; it
- * differs from that of gk_matmul, which is one chain over K, in the last bits.  gk_sliced_workspace_size gives the workspace the
- * launch needs, decided from the configuration, the hooks and the epilogue alone; 0: it is gk_matmul's launch, as it is with a workspace that is NULL or too small. */
+ * sums to the library: the same launch, in slices of K on its own tile where that is estimated to be faster.  That is products with
+ * few output tiles and a long K: Float32 and Float64 ones of FPUOp with hooks of at most one scale on A, on B and on C; real MFMA ones
+ * on 64 x 64 x 64 (and 64 x 64 x 32 where it runs on K tiles of 64) and on 128 x 128 x 64 tiles with a K-split instance; contractions on
+ * 64 x 64 x 64 without hooks.  The result does not change from run to run; it differs from that of gk_matmul, which is one chain over K,
+ * in the last bits.  gk_sliced_workspace_size gives the workspace the launch needs, decided from the configuration, the hooks and the
+ * epilogue alone; 0: it is gk_matmul's launch, as it is with a workspace that is NULL or too small. */
 int gk_sliced_workspace_size(const gk_config* conf, const gk_transforms* transforms, const gk_epilogue* epilogue, size_t* bytes);
 int gk_matmul_sliced(const gk_config* conf, const void* a, const void* b, const void* c, void* d,
                      const gk_transforms* transforms, const gk_epilogue* epilogue, int32_t kernel, void* workspace,
                      size_t workspace_bytes, void* stream);
 
 /* gk_matmul in two parts, for launches that repeat: gk_prepare makes every check of gk_matmul that does not depend on the operands'
- * addresses, and gk_run launches on operands at 16-byte boundaries (GK_ERR_ALIGNMENT for others: gk_matmul takes them where the layouts do;
- * GK_ERR_UNSUPPORTED after gk_set_device_limits).  Nothing of the configuration and the hooks is referred to after gk_prepare but the bias of the epilogue.  A prepared launch
- * may be run from any number of threads, on any streams, and is freed by gk_prepared_free. */
+ * addresses, and gk_run launches on operands at 16-byte boundaries (GK_ERR_ALIGNMENT for others: gk_matmul takes them where the layouts
+ * do; GK_ERR_UNSUPPORTED after gk_set_device_limits).  Nothing of the configuration and the hooks is referred to after gk_prepare but the
+ * bias of the epilogue.  A prepared launch may be run from any number of threads, on any streams, and is freed by gk_prepared_free. */
 int gk_prepare(const gk_config* conf, const gk_transforms* transforms, const gk_epilogue* epilogue, int32_t kernel, void** prepared);
 int gk_run(const void* prepared, const void* a, const void* b, const void* c, void* d, void* stream);
 void gk_prepared_free(void* prepared);

@@ -526,3 +526,25 @@ def test_a_configuration_that_was_launched_is_copied_and_pickled_like_any_other(
         assert bytes(again.to_c(*lds)) == bytes(conf.to_c(*lds)) and again.to_c(*lds) is not conf.to_c(*lds)
     own = pickle.loads(pickle.dumps(configs.mfma_config(2240, 5568, 2304, block_shape=(64, 64, 64))))
     assert cfgmod.larger_tile(own, False) is None      # (a tile that was asked for)
+
+
+@pytest.mark.parametrize("tile", [(64, 64, 64), (128, 128, 64), (256, 128, 64)])
+def test_the_package_and_the_library_cut_the_same_launches(tile):
+    """The tile rules weigh slices of K that the library decides on, and a first launch does not ask where there are none."""
+    import random
+    import sys
+    from gemmkernels import configs
+    mm = sys.modules["gemmkernels.matmul"]
+    rng, cut = random.Random(tile[0]), 0
+    for _ in range(300):
+        M, N = (tile[i] * rng.randint(1, 12) * rng.choice((1, 1, 2)) for i in (0, 1))
+        K = 64 * int(8 * 256 ** rng.random()) + rng.choice((0, 0, 64))
+        c = configs.mfma_config(M, N, K, rng.random() < 0.5, rng.random() < 0.5, block_shape=tile, zero_c=True).to_c(max(M, K), max(N, K), M, M)
+        need = ctypes.c_size_t()
+        assert _lib.lib().gk_sliced_workspace_size(ctypes.byref(c), None, None, ctypes.byref(need)) == _lib.GK_OK
+        assert mm._sliced_bytes(c, None, None) == need.value, (M, N, K)
+        cut += need.value > 0
+        if tile[0] > 64:
+            slices = cfgmod._product_slices(tile, M, N, K)
+            assert need.value == (2048 + -(-M // tile[0]) * -(-N // tile[1]) * -(-(K // 64) // -(-(K // 64) // slices)) * tile[0] * tile[1] * 4 if slices > 1 else 0), (M, N, K)
+    assert (20 < cut < 280) if tile[0] == tile[1] else cut == 0
