@@ -98,6 +98,18 @@ bool read_call(PyObject* const* args, Kind* kind, char** a, char** b, char** c) 
   return true;
 }
 
+// The buffer of eager launches on a stream of the current device; false where there is none of that size, or the stream is being captured.
+bool find_workspace(void* stream, size_t bytes, Workspace* space) {
+  int32_t capturing = 0;
+  uint64_t id = 0;
+  const int device = c10::hip::current_device();
+  if (device >= 16 || g_capture(stream, &capturing, &id) != 0 || capturing != 0) return false;
+  const auto found = g_workspaces[device].find((uint64_t)(uintptr_t)stream);
+  if (found == g_workspaces[device].end() || found->second.bytes < bytes) return false;
+  *space = found->second;
+  return true;
+}
+
 PyObject* error_of(const std::exception& e) {
   PyErr_SetString(PyExc_RuntimeError, e.what());
   return nullptr;
@@ -172,15 +184,7 @@ PyObject* mul(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const Launch launch = hit->second;
     void* stream = (void*)c10::hip::getCurrentHIPStream().stream();
     Workspace space{nullptr, 0, nullptr};
-    if (launch.workspace > 0) {
-      int32_t capturing = 0;
-      uint64_t id = 0;
-      if (g_capture(stream, &capturing, &id) != 0 || capturing != 0 || kind.device >= 16) Py_RETURN_FALSE;
-      const auto& spaces = g_workspaces[kind.device];
-      const auto found = spaces.find((uint64_t)(uintptr_t)stream);
-      if (found == spaces.end() || found->second.bytes < launch.workspace) Py_RETURN_FALSE;
-      space = found->second;
-    }
+    if (launch.workspace > 0 && !find_workspace(stream, launch.workspace, &space)) Py_RETURN_FALSE;
     // (other threads may forget the launch, or put a larger workspace in the place of this one, while the GIL is given up)
     Py_INCREF(launch.owner);
     Py_XINCREF(space.owner);
@@ -292,6 +296,56 @@ PyObject* run_at(PyObject*, PyObject* const* args, Py_ssize_t n) {
   return PyLong_FromLong(rc);
 }
 
+// A launch in slices of K on the workspace of a stream, which other threads may replace by a larger one while the GIL is given up; -1: there is none.
+int launch_sliced(const void* conf, void* const* p, const void* transforms, const void* epilogue, int32_t kernel, size_t bytes, void* stream) {
+  Workspace space{nullptr, 0, nullptr};
+  if (!find_workspace(stream, bytes, &space)) return -1;
+  Py_INCREF(space.owner);
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = g_sliced(conf, p[0], p[1], p[2], p[3], transforms, epilogue, kernel, space.address, space.bytes, stream);
+  Py_END_ALLOW_THREADS
+  Py_DECREF(space.owner);
+  return rc;
+}
+
+// sliced_at(conf, a, b, c, d, transforms, epilogue, kernel, workspace, stream): gk_matmul_sliced on addresses, with the workspace of that stream if it
+// holds so many bytes; its status, or -1 where there is none and the Python side makes one
+PyObject* sliced_at(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  if (n != 10) { PyErr_SetString(PyExc_TypeError, "sliced_at takes ten arguments"); return nullptr; }
+  void* p[10];
+  for (int i = 0; i < 10; ++i) p[i] = args[i] == Py_None ? nullptr : PyLong_AsVoidPtr(args[i]);
+  if (PyErr_Occurred()) return nullptr;
+  try {
+    return PyLong_FromLong(launch_sliced(p[0], p + 1, p[5], p[6], (int32_t)(intptr_t)p[7], (size_t)(uintptr_t)p[8], p[9]));
+  } catch (const std::exception&) {
+    return PyLong_FromLong(-1);
+  }
+}
+
+// run_sliced(conf, kernel, workspace, a, b, c, d): the same without hooks on tensors at 16-byte boundaries and torch's current stream; True when it is on
+// its way, False when it is the Python side's
+PyObject* run_sliced(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  if (n != 7) Py_RETURN_FALSE;
+  const void* conf = PyLong_AsVoidPtr(args[0]);
+  const long kernel = PyLong_AsLong(args[1]);
+  const size_t bytes = PyLong_AsSize_t(args[2]);
+  if (PyErr_Occurred()) return nullptr;
+  try {
+    void* p[4] = {nullptr, nullptr, nullptr, nullptr};
+    for (int i = 0; i < 4; ++i) {
+      if (args[3 + i] == Py_None) continue;
+      const at::Tensor* t;
+      if (!read_tensor(args[3 + i], &t)) Py_RETURN_FALSE;
+      p[i] = t->data_ptr();
+      if (((uintptr_t)p[i] & 15u) != 0) Py_RETURN_FALSE;
+    }
+    return PyBool_FromLong(launch_sliced(conf, p, nullptr, nullptr, (int32_t)kernel, bytes, (void*)c10::hip::getCurrentHIPStream().stream()) == 0);
+  } catch (const std::exception&) {
+    Py_RETURN_FALSE;
+  }
+}
+
 // current_stream(): the handle of torch's current stream on the current device
 PyObject* current_stream(PyObject*, PyObject*) {
   try {
@@ -307,6 +361,8 @@ PyMethodDef g_methods[] = {{"bind", (PyCFunction)(void*)bind, METH_FASTCALL, nul
                            {"leading_dims", (PyCFunction)(void*)leading_dims, METH_FASTCALL, nullptr},
                            {"run", (PyCFunction)(void*)run, METH_FASTCALL, nullptr},
                            {"run_at", (PyCFunction)(void*)run_at, METH_FASTCALL, nullptr},
+                           {"sliced_at", (PyCFunction)(void*)sliced_at, METH_FASTCALL, nullptr},
+                           {"run_sliced", (PyCFunction)(void*)run_sliced, METH_FASTCALL, nullptr},
                            {"current_stream", (PyCFunction)(void*)current_stream, METH_NOARGS, nullptr},
                            {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "gk_torch", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};

@@ -215,9 +215,8 @@ class _Launch:
                 self.ready = native().run, prepared
         x, y = (b, a) if self._swapped else (a, b)
         if self._sliced:
-            from .matmul import _span, _workspace_if_any
-            workspace = _workspace_if_any(self._sliced, stream)
-            rc = self._fn(self._conf_ref, x, y, c, d, None, None, self._code, *_span(workspace), stream)
+            from .matmul import _launch_sliced
+            rc = _launch_sliced(self._conf, x, y, c, d, None, None, self._code, self._sliced, stream)
         else:
             from .matmul import _gk_matmul
             rc = _gk_matmul(self._conf, x, y, c, d, None, None, self._code, stream)

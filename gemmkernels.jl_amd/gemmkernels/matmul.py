@@ -230,6 +230,24 @@ def _workspace_if_any(need: int, stream: int):
         return None
 
 
+def _launch_sliced(conf_c, a, b, c, d, trans, epi, code: int, need: int, stream: int) -> int:
+    """gk_matmul_sliced on descriptors and addresses, with the workspace of the stream; its status."""
+    native = _load_native()
+    if native is not None:
+        rc = native.sliced_at(ctypes.addressof(conf_c), a, b, c, d, None if trans is None else ctypes.addressof(trans),
+                              None if epi is None else ctypes.addressof(epi), code, need, stream)
+        if rc == _lib.GK_OK:
+            return rc
+    workspace = _workspace_if_any(need, stream)
+    if native is not None and workspace is not None:
+        import torch
+        key = (torch.cuda.current_device(), stream)
+        if _workspaces.get(key) is workspace:
+            native.use_workspace(*key, *_span(workspace), workspace)
+    return _lib.lib().gk_matmul_sliced(ctypes.byref(conf_c), a, b, c, d, ctypes.byref(trans) if trans is not None else None,
+                                       ctypes.byref(epi) if epi is not None else None, code, *_span(workspace), stream)
+
+
 _IDENTITY = Transform.Elementwise()
 _DEFAULT_EPILOGUE = Epilogue.Default()
 _lowered = {}
@@ -240,10 +258,17 @@ def lower_transforms(transforms: dict) -> Optional[_lib.gk_transforms]:
         return None
     if any(t.expr is not None for t in transforms.values()):
         raise ConfigError("expression transforms need a specialised kernel (gemmkernels.specialize)")
-    key = tuple(transforms[name].ops for name in _HOOKS)
+    return _lower(transforms)
+
+
+def _lower(transforms: dict) -> Optional[_lib.gk_transforms]:
+    """``lower_transforms`` of transforms without expressions.  (What it gives is kept for good: matmul() knows it by its identity.)"""
+    key = tuple([transforms[name].ops for name in _HOOKS])
     hit = _lowered.get(key)
     if hit is not None:
         return hit
+    if not any(key):
+        return None
     out = _lowered[key] = _lib.gk_transforms()
     for i, name in enumerate(_HOOKS):
         ops = transforms[name].ops
@@ -316,11 +341,14 @@ def _launched_as(conf: Config, a, b, c, d, hooks: bool, slices: bool = False) ->
     for x, layout in ((a, conf.global_a_layout), (b, conf.global_b_layout), (c, conf.global_c_layout), (d, conf.global_d_layout)):
         if layout.kind == Layout.ZERO:
             continue
-        ld = _leading_dim(x, layout)
-        # (the offsets in a tile are kept in 32 bits: 256 columns of 2^22 elements are left to a tile with fewer)
-        if x is None or _ptr(x) % 16 != 0 or ld * layout.T.size % 16 != 0 or ld >= 1 << 21:
+        if not _takes_larger_tile(x, layout, _leading_dim(x, layout)) or _ptr(x) % 16 != 0:
             return None
     return larger
+
+
+def _takes_larger_tile(x, layout, ld: int) -> bool:
+    # (the offsets in a tile are kept in 32 bits: 256 columns of 2^22 elements are left to a tile with fewer)
+    return x is not None and ld * layout.T.size % 16 == 0 and ld < 1 << 21
 
 
 _AB_HOOKS = ("transform_global_to_shared_a", "transform_shared_to_regs_a", "transform_global_to_shared_b", "transform_shared_to_regs_b")
@@ -344,6 +372,20 @@ def _lists_in_the_k_loop(conf: Config, cconf, trans, transforms: dict) -> bool:
             return True                   # (refused: the launch says why)
         known = _lists[key] = name.value.endswith(b"_fused_ab")
     return known
+
+
+def _routes_of(conf: Config, lds, cconf, trans, transforms, epi, operands):
+    """What a launch of ``conf`` on operands of these leading dimensions tries, in this order: descriptor, workspace (0: not in slices of K), and whether
+    it takes operands at 16-byte boundaries only."""
+    mfma = conf.operator.kind == Operator.MFMA
+    larger = None
+    if mfma and (trans is None or not _lists_in_the_k_loop(conf, cconf, trans, transforms)):
+        larger = larger_tile(conf, trans is not None or epi is not None, True)
+    layouts = (conf.global_a_layout, conf.global_b_layout, conf.global_c_layout, conf.global_d_layout)
+    if larger is not None and any(l.kind != Layout.ZERO and not _takes_larger_tile(x, l, ld) for x, l, ld in zip(operands, layouts, lds)):
+        larger = None
+    of = [cconf] if larger is None else [larger.to_c(*lds), cconf]
+    return [(c, _sliced_bytes(c, trans, epi) if mfma else 0, c is not cconf) for c in of]
 
 
 class Plan:
@@ -417,8 +459,7 @@ class Plan:
                 _raise(rc)
             return self.d
         if self._sliced:
-            workspace = _workspace_if_any(self._sliced, stream)
-            rc = self._fn(*self._args, *_span(workspace), stream)
+            rc = _launch_sliced(self._conf, *self._args[1:5], self._trans, self._epi, self._args[-1], self._sliced, stream)
         else:
             direct = self._direct
             if direct is not None and _native.run_at(*direct[1], stream) == _lib.GK_OK:
@@ -427,8 +468,7 @@ class Plan:
         if rc != _lib.GK_OK and self._as_given is not None:
             need = _sliced_bytes(self._as_given, self._trans, self._epi) if self._slices else 0
             if need:
-                workspace = _workspace_if_any(need, stream)
-                rc = _lib.lib().gk_matmul_sliced(ctypes.byref(self._as_given), *self._args[1:], *_span(workspace), stream)
+                rc = _launch_sliced(self._as_given, *self._args[1:5], self._trans, self._epi, self._args[-1], need, stream)
             else:
                 rc = _lib.lib().gk_matmul(ctypes.byref(self._as_given), *self._args[1:], stream)
         if rc != _lib.GK_OK:
@@ -465,7 +505,17 @@ def plan(conf: Config, a, b, c, d, *,
 _PREPARED_MAX = 64
 
 
-def _prepare(conf: Config, cconf, lds, kernel) -> None:
+class _Sliced:
+    """What gk_torch launches in slices of K where ``Prepared`` holds a launch checked once: the descriptor, the kind of kernel and the workspace."""
+
+    __slots__ = ("handle", "args", "_conf")
+
+    def __init__(self, conf_c, code: int, need: int):
+        self._conf = _lib.gk_config.from_buffer_copy(conf_c)
+        self.handle, self.args = None, (ctypes.addressof(self._conf), code, need)
+
+
+def _prepare(conf: Config, cconf, lds, kernel, need: int = 0) -> None:
     """Keeps the launch that ``matmul`` made for operands of these leading dimensions (no address) with its configuration."""
     kept = conf.__dict__.get("_prepared")
     if _load_native() is None or kept is not None and (lds, kernel) in kept:
@@ -473,8 +523,8 @@ def _prepare(conf: Config, cconf, lds, kernel) -> None:
     if conf.__dict__.get("_launched") != (lds, kernel):             # (a configuration that is launched once does not pay for it)
         conf.__dict__["_launched"] = (lds, kernel)
         return
-    made = Prepared(cconf, None, None, kernel.code)
-    if made.handle is None:
+    made = _Sliced(cconf, kernel.code, need) if need else Prepared(cconf, None, None, kernel.code)
+    if not need and made.handle is None:
         return
     if kept is None or len(kept) > _PREPARED_MAX:
         forms = {**dict.fromkeys(_NO_LD, 0), **dict.fromkeys(_INTERLEAVED, 2), **dict.fromkeys(_SPLIT, 3)}
@@ -491,24 +541,22 @@ def matmul(conf: Config, a, b, c, d, *,
            epilogue=None, kernel=Kernel.matmul_singlestage, stream=None):
     """reference src/matmul.jl:7-44: launch geometry, checks (ConfigError) and the asynchronous
     launch on the current stream.  Same positional and keyword arguments as the reference."""
-    plain = (epilogue is None and transform_global_to_shared_a is None and transform_global_to_shared_b is None and
-             transform_global_to_shared_c is None and transform_shared_to_global_d is None and transform_shared_to_regs_a is None and
-             transform_shared_to_regs_b is None and transform_shared_to_regs_c is None and transform_regs_to_shared_d is None)
+    hooked = not (transform_global_to_shared_a is None and transform_global_to_shared_b is None and
+                  transform_global_to_shared_c is None and transform_shared_to_global_d is None and transform_shared_to_regs_a is None and
+                  transform_shared_to_regs_b is None and transform_shared_to_regs_c is None and transform_regs_to_shared_d is None)
+    plain = epilogue is None and not hooked
     prepared = conf.__dict__.get("_prepared") if plain else None
     if prepared is not None and stream is None:
         # (a launch of these leading dimensions was made before: a Config is immutable once built)
         lds = _native.leading_dims(prepared["forms"], a, b, c, d)
         again = prepared.get((lds, kernel)) if lds is not None else None
-        if again is not None and _native.run(again.handle, a, b, c, d):
+        if again is not None and (_native.run(again.handle, a, b, c, d) if again.handle is not None else _native.run_sliced(*again.args, a, b, c, d)):
             return d
     from . import complex_planar
     if complex_planar.is_planar(conf) and not complex_planar.planes_adjacent(a, b, c, d):
         return complex_planar.PlanarComplexPlan(conf, a, b, c, d)(stream)
     ctrans = None
-    if not (transform_global_to_shared_a is None and transform_global_to_shared_b is None and
-            transform_global_to_shared_c is None and transform_shared_to_global_d is None and
-            transform_shared_to_regs_a is None and transform_shared_to_regs_b is None and
-            transform_shared_to_regs_c is None and transform_regs_to_shared_d is None):
+    if hooked:
         collected = _collect(dict(
             transform_global_to_shared_a=transform_global_to_shared_a, transform_global_to_shared_b=transform_global_to_shared_b,
             transform_global_to_shared_c=transform_global_to_shared_c, transform_shared_to_global_d=transform_shared_to_global_d,
@@ -516,7 +564,7 @@ def matmul(conf: Config, a, b, c, d, *,
             transform_shared_to_regs_c=transform_shared_to_regs_c, transform_regs_to_shared_d=transform_regs_to_shared_d))
         if any(t.expr is not None for t in collected.values()):
             return Plan(conf, a, b, c, d, collected, _DEFAULT_EPILOGUE if epilogue is None else epilogue, kernel)(stream)
-        ctrans = lower_transforms(collected)
+        ctrans = _lower(collected)
 
     lds = (_leading_dim(a, conf.global_a_layout), _leading_dim(b, conf.global_b_layout),
            _leading_dim(c, conf.global_c_layout), _leading_dim(d, conf.global_d_layout))
@@ -534,32 +582,23 @@ def matmul(conf: Config, a, b, c, d, *,
                                           ctypes.byref(cepi) if cepi is not None else None,
                                           *_span(workspace), stream)
     else:
-        args = (_ptr(a), _ptr(b), _ptr(c), _ptr(d), ctrans, cepi, kernel.code, stream)
-        hooks = ctrans is not None or cepi is not None
-        larger, rc = None, _lib.GK_ERR_UNSUPPORTED
-        if ctrans is None or not _lists_in_the_k_loop(conf, cconf, ctrans, collected):
-            larger = _launched_as(conf, a, b, c, d, hooks, conf.operator.kind == Operator.MFMA)
-        for of in (larger, conf):                                   # (the tile asked for where the library refuses the larger one)
-            if of is None or rc == _lib.GK_OK:
+        pointers = (_ptr(a), _ptr(b), _ptr(c), _ptr(d))
+        routes = conf.__dict__.setdefault("_routes", {})                 # (a Config is immutable once built, and lowered transforms are kept)
+        key = (lds, 0 if ctrans is None else id(ctrans), 0 if cepi is None else cepi.kind)
+        route = routes.get(key)
+        if route is None:
+            if len(routes) >= _PREPARED_MAX:
+                routes.clear()
+            route = routes[key] = _routes_of(conf, lds, cconf, ctrans, collected if ctrans is not None else None, cepi, (a, b, c, d))
+        rc = _lib.GK_ERR_UNSUPPORTED
+        for of, need, aligned in route:                                   # (the tile asked for where the library refuses the larger one)
+            if aligned and any(p is not None and p % 16 != 0 for p in pointers):
                 continue
-            cconf, need = cconf if of is conf else of.to_c(*lds), 0
-            if of.operator.kind == Operator.MFMA and hooks:                  # (what a plan with these arguments launches)
-                need = _sliced_bytes(cconf, ctrans, cepi)
-            elif of.operator.kind == Operator.MFMA:
-                known = of.__dict__.setdefault("_slices_of", {})             # (a Config is immutable once built)
-                need = known.get(lds)
-                if need is None:
-                    if len(known) >= 64:
-                        known.clear()
-                    need = known[lds] = _sliced_bytes(cconf, None, None)
-            if need:
-                workspace = _workspace_if_any(need, stream)
-                rc = _lib.lib().gk_matmul_sliced(ctypes.byref(cconf), *args[:4], ctypes.byref(ctrans) if ctrans is not None else None,
-                                                 ctypes.byref(cepi) if cepi is not None else None, kernel.code, *_span(workspace), stream)
-            else:
-                rc = _gk_matmul(cconf, *args)
-                if rc == _lib.GK_OK and plain:
-                    _prepare(conf, cconf, lds, kernel)
+            rc = _launch_sliced(of, *pointers, ctrans, cepi, kernel.code, need, stream) if need else _gk_matmul(of, *pointers, ctrans, cepi, kernel.code, stream)
+            if rc == _lib.GK_OK:
+                if plain:
+                    _prepare(conf, of, lds, kernel, need)
+                break
     if rc != _lib.GK_OK:
         _raise(rc)
     return d

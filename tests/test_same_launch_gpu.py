@@ -37,3 +37,56 @@ def test_the_same_bits(gpu, M, N, K, slices, hooks, bf16, bias):
         launch()
         gk.matmul(conf, a, b, c, other, kernel=Kernel.matmul_pipelined, **options)
         assert torch.equal(one, other)
+
+
+def test_repeated_launches_in_slices(gpu):
+    """From the third on they go from the tensors to the library in C++: on other operands, other streams and in several threads, under capture, and refused
+    where the first one would be."""
+    import threading
+    import torch
+    from gemmkernels import ConfigError
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    whole = lambda m, n: torch.randint(-3, 4, (n, m), generator=gen, device="cuda").to(torch.float16).t()
+    M, N, K = 1088, 1088, 5248
+    conf = configs.mfma_config(M, N, K, zero_c=True)
+    sets = []
+    for _ in range(3):
+        a, b = whole(M, K), whole(K, N)
+        sets.append((a, b, gk.colmajor_empty((M, N), torch.float32), a.double() @ b.double()))
+    run = lambda s: gk.matmul(conf, s[0], s[1], None, s[2], kernel=Kernel.matmul_pipelined)
+    for _ in range(3):
+        for s in sets:
+            s[2].fill_(float("nan"))
+            run(s)
+            assert torch.equal(s[2].double(), s[3])
+    assert any(getattr(x, "args", None) for x in conf.__dict__["_prepared"].values())
+    off = torch.empty(M * K + 8, dtype=torch.float16, device="cuda")[1:1 + M * K].view(K, M).t()               # starts off a 16-byte boundary
+    with pytest.raises(ConfigError, match="aligned"):
+        gk.matmul(conf, off, sets[0][1], None, sets[0][2], kernel=Kernel.matmul_pipelined)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run(sets[1])
+    for _ in range(3):
+        sets[1][2].fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(sets[1][2].double(), sets[1][3])
+        run(sets[0])
+        torch.cuda.synchronize()
+    failed = []
+
+    def work(s):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(20):
+                s[2].fill_(float("nan"))
+                run(s)
+                if not torch.equal(s[2].double(), s[3]):
+                    failed.append(s)
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=work, args=(s,)) for s in sets]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed

@@ -18,13 +18,17 @@ def test_a_plan_without_memory_seldom_asks_again(monkeypatch):
     launch = gk.plan(conf, half(384, 3776), half(3776, 256), None, torch.empty((256, 384)).t(), kernel=Kernel.matmul_pipelined)
     assert launch._sliced > 0
     ran, asked = [], []
-    launch._fn = lambda *args: ran.append(args[-3:]) or 0
+
+    class Library:
+        gk_matmul_sliced = staticmethod(lambda *args: ran.append(args[-3:]) or 0)
 
     def none(*args, **kwargs):
         asked.append(len(ran))
         raise torch.OutOfMemoryError("no memory")
     monkeypatch.setattr(torch, "zeros", none)
     monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(mm, "_load_native", lambda: None)
+    monkeypatch.setattr(mm._lib, "lib", lambda: Library)
     monkeypatch.setattr(mm, "_capture_of", lambda stream: None)
     monkeypatch.setattr(mm, "_on", lambda stream: contextlib.nullcontext())
     monkeypatch.setattr(mm, "_workspaces", {})
