@@ -333,15 +333,14 @@ def specialize(conf: Config, *,
     return SpecializedKernel(conf, {k: (Transform.Elementwise(expr=v) if isinstance(v, str) else v) for k, v in given.items()})
 
 
-def _launched_as(conf: Config, a, b, c, d, hooks: bool, slices: bool = False) -> Optional[Config]:
-    """``larger_tile`` of ``conf`` where the operands are what the aligned layouts of ``conf`` ask for (the library refuses others, and is left to), or None."""
+def _launched_as(conf: Config, operands, lds, cconf, trans, transforms, hooks: bool, slices: bool) -> Optional[Config]:
+    """``larger_tile`` of ``conf`` where the operands, but for their addresses, are what the aligned layouts of ``conf`` ask for (the library refuses others, and is
+    left to) and no op list keeps the launch on its tile, or None."""
     larger = larger_tile(conf, hooks, slices)
-    if larger is None:
+    if larger is None or trans is not None and _lists_in_the_k_loop(conf, cconf, trans, transforms):
         return None
-    for x, layout in ((a, conf.global_a_layout), (b, conf.global_b_layout), (c, conf.global_c_layout), (d, conf.global_d_layout)):
-        if layout.kind == Layout.ZERO:
-            continue
-        if not _takes_larger_tile(x, layout, _leading_dim(x, layout)) or _ptr(x) % 16 != 0:
+    for x, layout, ld in zip(operands, (conf.global_a_layout, conf.global_b_layout, conf.global_c_layout, conf.global_d_layout), lds):
+        if layout.kind != Layout.ZERO and not _takes_larger_tile(x, layout, ld):
             return None
     return larger
 
@@ -378,12 +377,7 @@ def _routes_of(conf: Config, lds, cconf, trans, transforms, epi, operands):
     """What a launch of ``conf`` on operands of these leading dimensions tries, in this order: descriptor, workspace (0: not in slices of K), and whether
     it takes operands at 16-byte boundaries only."""
     mfma = conf.operator.kind == Operator.MFMA
-    larger = None
-    if mfma and (trans is None or not _lists_in_the_k_loop(conf, cconf, trans, transforms)):
-        larger = larger_tile(conf, trans is not None or epi is not None, True)
-    layouts = (conf.global_a_layout, conf.global_b_layout, conf.global_c_layout, conf.global_d_layout)
-    if larger is not None and any(l.kind != Layout.ZERO and not _takes_larger_tile(x, l, ld) for x, l, ld in zip(operands, layouts, lds)):
-        larger = None
+    larger = _launched_as(conf, operands, lds, cconf, trans, transforms, trans is not None or epi is not None, mfma) if mfma else None
     of = [cconf] if larger is None else [larger.to_c(*lds), cconf]
     return [(c, _sliced_bytes(c, trans, epi) if mfma else 0, c is not cconf) for c in of]
 
@@ -408,8 +402,10 @@ class Plan:
         self._as_given = None                                      # (what is launched where the library refuses the larger tile)
         hooks = self._trans is not None or epilogue.kind != Epilogue.DEFAULT
         larger = None
-        if specialized is None and kernel is not Kernel.matmul_split_k and not (self._trans is not None and _lists_in_the_k_loop(conf, self._conf, self._trans, transforms)):
-            larger = _launched_as(conf, a, b, c, d, hooks, slices)
+        if specialized is None and kernel is not Kernel.matmul_split_k:
+            larger = _launched_as(conf, (a, b, c, d), lds, self._conf, self._trans, transforms, hooks, slices)
+            if larger is not None and any(x is not None and _ptr(x) % 16 != 0 for x in (a, b, c, d)):
+                larger = None
         if larger is not None:
             self._as_given, self._conf = self._conf, _lib.gk_config.from_buffer_copy(larger.to_c(*lds))
         self._epi = None
