@@ -7,8 +7,9 @@ import gemmkernels as gk
 pytestmark = pytest.mark.gpu
 
 # M, N, K, A transposed, leading dimension of the wide operand (0: dense).  Tiles of 128 x 256, 256 x 256 (four
-# waves), 256 x 128, and 64 x 64 in slices of K
-CASES = [(80, 131072, 16400, False, 0), (4096, 131072, 16400, False, 0), (65536, 72, 50264, True, 0), (10000, 64, 4100, True, 215000)]
+# waves), 256 x 128, 64 x 64 in slices of K, and 64 x 64 because the rows of larger tiles lie too far apart
+CASES = [(80, 131072, 16400, False, 0), (4096, 131072, 16400, False, 0), (65536, 72, 50264, True, 0), (10000, 64, 4100, True, 215000),
+         (991, 3293, 565, True, 1 << 23)]
 
 
 @pytest.mark.parametrize("case", range(len(CASES)))
@@ -19,8 +20,7 @@ def test_more_than_2_31_elements(gpu, case):
     gen = torch.Generator(device="cuda").manual_seed(case)
     wide = torch.empty((M if ta else N, ld or K), dtype=torch.float16, device="cuda")
     assert wide.numel() >= 2 ** 31
-    wide.random_(-3, 4, generator=gen)
-    wide = wide[:, :K].t()                                     # contiguous along k
+    wide = wide[:, :K].random_(-3, 4, generator=gen).t()       # contiguous along k
     other = torch.randint(-3, 4, (N, K) if ta else (K, M), generator=gen, device="cuda").to(torch.float16).t()        # K x N, or M x K
     c = gk.colmajor_empty((M, N), torch.float32)
     c.fill_(float("nan"))
